@@ -128,6 +128,15 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
             const int64_t* strides, float scale, int dtype, void* stream,
             RopeTables rope = RopeTables{nullptr, nullptr, 0, 0}) {
     const bool has_do = t.dO != nullptr, has_g = t.dTO != nullptr;
+    const void* ptrs[SJVP_B_COUNT] = {t.q, t.k, t.v, has_g ? t.tq : nullptr, has_g ? t.tk : nullptr,
+                                      has_g ? t.tv : nullptr, t.o, has_g ? t.to : nullptr, t.dO, t.dTO,
+                                      t.dq, t.dk, t.dv, has_g ? t.dtq : nullptr, has_g ? t.dtk : nullptr,
+                                      has_g ? t.dtv : nullptr};
+    const bool f32io = dtype == SJVP_FP32_BF16;
+    const int m = f32io ? 2 : 1;
+    VecCheck vc;
+    vc.unit = f32io || dtype == SJVP_FP32 ? 4 : 8;
+    for (int i = 0; i < SJVP_B_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
     if (dtype == SJVP_FP32) {
         BwdParamsF32 f{};
         f.q = view32(t.q, strides + 3 * SJVP_B_Q);
@@ -159,17 +168,8 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
         f.s4 = f.lse2 + (size_t)B * H * f.Lr;
         f.s7d = f.s4 + (size_t)B * H * f.Lr;
         f.scale = resolve_scale(scale, D);
-        return bwd_f32(f, B * H, has_do, has_g, parts, static_cast<hipStream_t>(stream));
+        return bwd_f32(f, B * H, has_do, has_g, parts, vc.ok && D % 4 == 0, static_cast<hipStream_t>(stream));
     }
-    const void* ptrs[SJVP_B_COUNT] = {t.q, t.k, t.v, has_g ? t.tq : nullptr, has_g ? t.tk : nullptr,
-                                      has_g ? t.tv : nullptr, t.o, has_g ? t.to : nullptr, t.dO, t.dTO,
-                                      t.dq, t.dk, t.dv, has_g ? t.dtq : nullptr, has_g ? t.dtk : nullptr,
-                                      has_g ? t.dtv : nullptr};
-    const bool f32io = dtype == SJVP_FP32_BF16;
-    const int m = f32io ? 2 : 1;
-    VecCheck vc;
-    vc.unit = f32io ? 4 : 8;
-    for (int i = 0; i < SJVP_B_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
 
     BwdParams p{};
     p.q = view(t.q, strides + 3 * SJVP_B_Q, m);
@@ -292,6 +292,12 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
     int rc = check_common(B, H, Lq, Lk, D, dtype, scale);
     if (rc != SJVP_OK) return rc;
 
+    const void* ptrs[SJVP_F_COUNT] = {q, k, v, tq, tk, tv, o, to};
+    const bool f32io = dtype == SJVP_FP32_BF16;
+    const int m = f32io ? 2 : 1;
+    VecCheck vc;
+    vc.unit = f32io || dtype == SJVP_FP32 ? 4 : 8;
+    for (int i = 0; i < SJVP_F_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
     if (dtype == SJVP_FP32) {
         FwdParamsF32 f{};
         f.q = view32(q, strides + 3 * SJVP_F_Q);
@@ -313,14 +319,8 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
         f.D = D;
         f.Lr = round_up(Lq, 128);
         f.scale = resolve_scale(scale, D);
-        return fwd_f32(f, B * H, jvp, static_cast<hipStream_t>(stream));
+        return fwd_f32(f, B * H, jvp, vc.ok && D % 4 == 0, static_cast<hipStream_t>(stream));
     }
-    const void* ptrs[SJVP_F_COUNT] = {q, k, v, tq, tk, tv, o, to};
-    const bool f32io = dtype == SJVP_FP32_BF16;
-    const int m = f32io ? 2 : 1;
-    VecCheck vc;
-    vc.unit = f32io ? 4 : 8;
-    for (int i = 0; i < SJVP_F_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
 
     FwdParams p{};
     p.q = view(q, strides + 3 * SJVP_F_Q, m);
