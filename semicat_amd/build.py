@@ -28,10 +28,12 @@ HIPCC_FLAGS = [
     # keep the compiler from forming packed-fp32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-# Flags of single units.  The row-owned and column-owned backward kernels gain about 1 % from the
+# Flags of single units.  The row-owned and column-owned backward kernels gain 1 to 4 % from the
 # scheduler that orders for instruction-level parallelism (measured on the MI355X at head dimensions 64 and
-# 128); the single-launch backward loses 2 % with it and the forward is unchanged, so they keep the default.
-UNIT_FLAGS = {"sjvp_tu_pair16.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]}
+# 128); the single-launch backward loses 2 % with it, the forward is unchanged on aligned rows and loses up
+# to 20 % on staged ones, so they keep the default.
+_ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
+UNIT_FLAGS = {name: _ILP for name in ("sjvp_tu_pair16.hip", "sjvp_tu_pair_staged16.hip", "sjvp_f32io_pair.hip")}
 
 
 def hipcc_path() -> str:

@@ -197,8 +197,6 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
     p.Lk = Lk;
     p.D = D;
     p.Lr = round_up(Lq, 128);
-    p.q_blocks = p.Lr / kOwned;
-    p.k_blocks = round_up(Lk, kOwned) / kOwned;
     p.lse2 = ws;
     p.s4 = p.lse2 + (size_t)B * H * p.Lr;
     p.s7d = p.s4 + (size_t)B * H * p.Lr;
@@ -217,7 +215,7 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
         p.q_side_uniform = !f32io && fits(SJVP_B_Q, p.Lr) && same(SJVP_B_Q, SJVP_B_TQ) && same(SJVP_B_Q, SJVP_B_O) &&
                            same(SJVP_B_Q, SJVP_B_TO) && (!has_do || same(SJVP_B_Q, SJVP_B_DO)) &&
                            (!has_g || same(SJVP_B_Q, SJVP_B_DTO));
-        p.k_side_uniform = !f32io && fits(SJVP_B_K, round_up(Lk, kOwned)) && same(SJVP_B_K, SJVP_B_V) &&
+        p.k_side_uniform = !f32io && fits(SJVP_B_K, round_up(Lk, kOwned16)) && same(SJVP_B_K, SJVP_B_V) &&
                            same(SJVP_B_K, SJVP_B_TK) && same(SJVP_B_K, SJVP_B_TV);
     }
     p.rowfix = g_row_sum_repair.load(std::memory_order_relaxed);
@@ -341,7 +339,7 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
     p.Lk = Lk;
     p.D = D;
     p.Lr = round_up(Lq, 128);
-    p.q_blocks = p.Lr / kOwned;  // covers every statistic row below Lr
+    p.q_blocks = p.Lr / kOwned16;  // covers every statistic row below Lr
     p.scale = resolve_scale(scale, D);
     p.vec = (vc.ok && D % 8 == 0) ? 1 : 0;
     p.rope = rope;
@@ -350,7 +348,7 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
     const int grid = B * H * p.q_blocks;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (f32io) return fwd_f32io(p, grid, jvp, s);
-    // LDS-DMA streaming needs 16-byte aligned rows; anything else takes the register-staged path
+    // LDS-DMA streaming needs 16-byte aligned rows; anything else is copied through registers
     if (p.vec) return dtype == SJVP_BF16 ? fwd_vec<Bf16>(p, grid, jvp, s) : fwd_vec<Fp16>(p, grid, jvp, s);
     return dtype == SJVP_BF16 ? fwd_any<Bf16>(p, grid, jvp, s) : fwd_any<Fp16>(p, grid, jvp, s);
 }

@@ -1,12 +1,12 @@
-// Attention-JVP backward for key axes beyond one workgroup, 16-wide form (gfx950; inputs with 16-byte
-// aligned rows): the row-owned and column-owned pair of sjvp_bwd.hpp (same mathematics, the same
-// workspace arrays lse*log2e, s4, s7d, the two sums negated here) with 16 owned positions per wavefront,
+// Attention-JVP backward for key axes beyond one workgroup, 16-wide form (gfx950): a row-owned and a
+// column-owned launch (mathematics in sjvp_bwd.hpp) with 16 owned positions per wavefront,
 // so that several wavefronts share a SIMD and a workgroup's copies overlap another's arithmetic.
 //   bwd_row16_kernel   4 waves x 16 queries; streams K, V (, K_dot, V_dot)        -> dQ (, dQ_dot)
 //   bwd_col16_kernel   4 waves x 16 keys;    streams Q (, Q_dot, G) (, dO) + stats -> dK, dV (, dK_dot, dV_dot)
 // (workgroups of four waves: at 160-200 registers two or three of them share a CU)
 // The owned rows are loaded straight into registers (each lane its own 16-byte pieces), the streamed
-// side goes through an LDS ring filled by LDS-DMA.  Each gradient is accumulated in fp32 registers by
+// side goes through an LDS ring filled by LDS-DMA (IO = kIoDma), or, where the rows do not start on 16-byte boundaries
+// or hold fp32 elements, through registers one stage ahead (sjvp_staged16.hpp).  Each gradient is accumulated in fp32 registers by
 // exactly one wavefront and written once: deterministic, no atomics.
 //
 // Row sums.  The row-owned kernel starts from s4' = rowsum(G*O), s7d' = rowsum(G*TO) + rowsum(dO*O),
@@ -27,7 +27,7 @@
 // launch (PASS = 1) only measures (the reference's preprocess + backward structure).
 #pragma once
 #include "sjvp_bwd.hpp"
-#include "sjvp_w16.hpp"
+#include "sjvp_staged16.hpp"
 
 namespace sjvp {
 
@@ -36,10 +36,14 @@ constexpr int kXThreads16 = 64 * kXWaves16;
 constexpr int kXOwned16 = 16 * kXWaves16;  // owned positions per workgroup
 
 // B operands (all head-dimension chunks of 32) of one owned row, straight from global memory.
-template <int HD>
+template <typename T, int HD, int IO>
 __device__ __forceinline__ void load_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
+    if constexpr (IO != kIoDma) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
 #pragma unroll
-    for (int c = 0; c < HD / 32; ++c) out[c] = load8(row, 32 * c + 8 * g, D, valid, true);
+    for (int c = 0; c < HD / 32; ++c) {
+        out[c] = u32x4{0u, 0u, 0u, 0u};
+        if (valid && 32 * c + 8 * g < D) out[c] = *reinterpret_cast<const u32x4*>(row + 32 * c + 8 * g);
+    }
 }
 
 // The same from a uniform slice pointer and the lane's byte offset in the slice: whole rows of HD elements
@@ -74,8 +78,9 @@ struct Row16Smem {
 
 // (the body of the kernel as a function of the workgroup's index and the number of workgroups, so that the
 // second launch can also ride at the end of the column-owned launch, see bwd_col16_repair_kernel)
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO>
 __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int block, const int blocks) {
+    constexpr bool DMA = IO == kIoDma;
     constexpr bool SECOND = PASS == 2;   // second launch: sums from the workspace, flagged workgroups only
     constexpr bool MEASURE = PASS == 1;  // first launch of "always": residues and sums only, no gradients
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -110,7 +115,7 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     u32x4 oR[KC], toR[KC];
     float s4 = 0.f, s7d = 0.f;
     const int64_t so = (int64_t)bh * p.Lr + qrow;  // rows below Lr exist in every statistic
-    if (p.q_side_uniform && p.D == HD && q0 + kXOwned16 <= p.Lq) {
+    if (DMA && p.q_side_uniform && p.D == HD && q0 + kXOwned16 <= p.Lq) {
         // the common case: whole rows that all exist, every tensor with q's strides
         const int64_t slice = b * p.q.sb + h * p.q.sh;
         const uint32_t at = ((uint32_t)qrow * (uint32_t)p.q.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
@@ -123,30 +128,31 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         }
         if constexpr (HAS_DO) load_b_operands16_at<HD>(doB, p.dO.ptr + slice, at);
     } else {
-        load_b_operands16<HD>(qB, p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qvalid);
-        if constexpr (!SECOND) load_b_operands16<HD>(oR, p.o.head(b, h) + (int64_t)qrow * p.o.sl, g, p.D, qvalid);
+        load_b_operands16<T, HD, IO>(qB, p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qvalid);
+        if constexpr (!SECOND) load_b_operands16<T, HD, IO>(oR, p.o.head(b, h) + (int64_t)qrow * p.o.sl, g, p.D, qvalid);
         if constexpr (HAS_G) {
-            load_b_operands16<HD>(tqB, p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qvalid);
-            load_b_operands16<HD>(gB, p.dTO.head(b, h) + (int64_t)qrow * p.dTO.sl, g, p.D, qvalid);
-            if constexpr (!SECOND) load_b_operands16<HD>(toR, p.to.head(b, h) + (int64_t)qrow * p.to.sl, g, p.D, qvalid);
+            load_b_operands16<T, HD, IO>(tqB, p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qvalid);
+            load_b_operands16<T, HD, IO>(gB, p.dTO.head(b, h) + (int64_t)qrow * p.dTO.sl, g, p.D, qvalid);
+            if constexpr (!SECOND) load_b_operands16<T, HD, IO>(toR, p.to.head(b, h) + (int64_t)qrow * p.to.sl, g, p.D, qvalid);
         }
-        if constexpr (HAS_DO) load_b_operands16<HD>(doB, p.dO.head(b, h) + (int64_t)qrow * p.dO.sl, g, p.D, qvalid);
+        if constexpr (HAS_DO) load_b_operands16<T, HD, IO>(doB, p.dO.head(b, h) + (int64_t)qrow * p.dO.sl, g, p.D, qvalid);
     }
     float lse_in = p.lse[so];  // requested with the rows: they are awaited together
     float mu_in = HAS_G ? p.mu[so] : 0.f;
 
-    using StagePlan = CopyPlan<HD, SM::nt, 1, kXThreads16>;
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
+                                         StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
     constexpr int SPT = StagePlan::N;
     StagePlan plan;
     if constexpr (HAS_G)
-        plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl},
+        init_plan(plan, tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl},
                   Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
     else
-        plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
+        init_plan(plan, tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
     const int ns = (p.Lk + kStageRows - 1) / kStageRows;
     int issued = 0;
     auto issue_next = [&]() {
-        plan.issue(ring + (issued % R) * SM::slot, p.Lk - issued * kStageRows,
+        issue_plan(plan, ring + (issued % R) * SM::slot, p.Lk - issued * kStageRows,
                    p.D == HD && (issued + 1) * kStageRows <= p.Lk);
         ++issued;
     };
@@ -182,7 +188,11 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     // cores ready for use.
     float n4 = -s4, n7 = -s7d;
     asm volatile("" : "+v"(lse2), "+v"(mu), "+v"(n4), "+v"(n7));  // every load so far is awaited here
-    while (issued < R && issued < ns) issue_next();
+    if constexpr (DMA) {
+        while (issued < R && issued < ns) issue_next();
+    } else {
+        plan.commit();
+    }
     // every row below Lr gets its workspace entries (zeros beyond Lq except lse2, which is finite): the
     // column-owned kernel, which runs after this one, stages 32-row groups
     if constexpr (!SECOND) {
@@ -299,10 +309,11 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     auto stage = [&](int i, auto ragged_tag) {
         // copies issued after stage i: the later stages; anything else in flight (the own rows'
         // loads, the statistics) only makes the wait stricter
-        wait_stages<SPT>(issued - 1 - i);
+        if constexpr (DMA) wait_stages<SPT>(issued - 1 - i);
         workgroup_barrier();  // stage i has landed for every wave; stage i-1 is fully consumed
-        if (i > 0 && issued < ns) issue_next();
+        if ((i > 0 || !DMA) && issued < ns) issue_next();
         if (wave_active) compute(ring + (i % R) * SM::slot, i * kStageRows, ragged_tag);
+        if constexpr (!DMA) plan.commit();
     };
     for (int i = 0; i < ns - 1; ++i) stage(i, std::false_type{});
     stage(ns - 1, std::true_type{});
@@ -329,14 +340,14 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     if (!wave_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
     const int row0 = q0 + wave * 16;
-    store_tile16<T, HD>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq, p.scale, lane);
+    store_rows16<T, HD, IO>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq, p.scale, lane);
     if constexpr (HAS_G)
-        store_tile16<T, HD>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq, p.scale, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq, p.scale, lane);
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_row16_kernel(const BwdParams p) {
-    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -354,8 +365,9 @@ struct Col16Smem {
     static_assert(R * slot >= kXWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART, int IO>
 __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int block, const int blocks) {
+    constexpr bool DMA = IO == kIoDma;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     using SM = Col16Smem<HD, R, HAS_DO, HAS_G>;
     constexpr bool DO_K = (PART & 1) != 0, DO_V = (PART & 2) != 0;
@@ -379,7 +391,8 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     const bool kvalid = krow < p.Lk;
     const bool wave_active = (key0 + wave * 16) < p.Lk;
 
-    using StagePlan = CopyPlan<HD, SM::nt, 1, kXThreads16>;
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
+                                         StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
     constexpr int SPT = StagePlan::N + 1;  // plus one 4-byte copy of statistics
     StagePlan plan;
     const int ns = (p.Lq + kStageRows - 1) / kStageRows;
@@ -387,7 +400,7 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     auto issue_next = [&]() {
         elem_t* slot = ring + (issued % R) * SM::slot;
         const int row0 = issued * kStageRows;
-        plan.issue(slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
+        issue_plan(plan, slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
         // the four statistic arrays (lse2, mu, s4, s7d) of the stage's rows, one per wave, 32 lanes
         // each (rows < Lr exist in all of them); every wave issues exactly one 4-byte LDS-DMA
         // (the three workspace arrays lie one behind the other: chosen by arithmetic, which stays in scalar
@@ -405,19 +418,19 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         {
             const Src q{p.q.head(b, h), p.q.sl};
             if constexpr (HAS_G && HAS_DO)
-                plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                           Src{p.dTO.head(b, h), p.dTO.sl}, Src{p.dO.head(b, h), p.dO.sl});
             else if constexpr (HAS_G)
-                plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                           Src{p.dTO.head(b, h), p.dTO.sl});
             else
-                plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
+                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
         }
         issue_next();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
     u32x4 kB[KC], vB[KC], tkB[KC], tvB[KC];
-    if (p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
+    if (DMA && p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
         // the common case: whole rows that all exist, every tensor with k's strides
         const int64_t slice = b * p.k.sb + h * p.k.sh;
         const uint32_t at = ((uint32_t)krow * (uint32_t)p.k.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
@@ -429,11 +442,11 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         }
         begin_copies();
     } else {
-        load_b_operands16<HD>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
-        if constexpr (DO_K) load_b_operands16<HD>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
+        load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
+        if constexpr (DO_K) load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
         if constexpr (HAS_G) {
-            load_b_operands16<HD>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
-            if constexpr (DO_K) load_b_operands16<HD>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
+            if constexpr (DO_K) load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
         }
         begin_copies();
     }
@@ -446,7 +459,11 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             if constexpr (DO_K) asm volatile("" : "+v"(tvB[c]));
         }
     }
-    while (issued < R && issued < ns) issue_next();
+    if constexpr (DMA) {
+        while (issued < R && issued < ns) issue_next();
+    } else {
+        plan.commit();
+    }
     const float sl2 = p.scale * kLog2e;
     f32x4 dk[DT], dv[DT], dtk[DT], dtv[DT];
 #pragma unroll
@@ -609,30 +626,31 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     };
 
     for (int i = 0; i < ns; ++i) {
-        wait_stages<SPT>(issued - 1 - i);
+        wait_stages<SPT>(DMA ? issued - 1 - i : 0);  // staged: the statistics still come by LDS-DMA
         workgroup_barrier();  // stage i has landed for every wave; stage i-1 is fully consumed
-        if (i > 0 && issued < ns) issue_next();
+        if ((i > 0 || !DMA) && issued < ns) issue_next();
         if (wave_active) compute(ring + (i % R) * SM::slot);
+        if constexpr (!DMA) plan.commit();
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!wave_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
     const int row0 = key0 + wave * 16;
     if constexpr (DO_K) {
-        store_tile16<T, HD>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane);
         if constexpr (HAS_G)
-            store_tile16<T, HD>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane);
+            store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane);
     }
     if constexpr (DO_V) {
-        store_tile16<T, HD>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
         if constexpr (HAS_G)
-            store_tile16<T, HD>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
+            store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
     }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART, int OCC>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART, int OCC, int IO = kIoDma>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdParams p) {
-    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, PART>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, PART, IO>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The column-owned launch with the second launch of the row-owned kernel at its end: workgroups
@@ -640,13 +658,13 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdPa
 // not depend on the column pass (it rewrites dQ, dQ_dot of flagged workgroups from the sums the first pass
 // left).  Nearly all of those workgroups leave at once; dealt out behind the column pass they fill the time in
 // which its last workgroups run alone, where a launch of their own costs a few microseconds.
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks)
-        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, 3>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, 3, IO>(p, (int)blockIdx.x, col_blocks);
     else
-        bwd_row16_body<T, HD, R, HAS_DO, HAS_G, 2>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
+        bwd_row16_body<T, HD, R, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -670,8 +688,9 @@ struct Col16pSmem {
     static_assert(R * slot >= kWaves16 * StoreStage16<64>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO>
 __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int block, const int blocks) {
+    constexpr bool DMA = IO == kIoDma;
     static_assert(HD == 128, "the paired form exists for the head dimension that needs it");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     using SM = Col16pSmem<HD, R, HAS_DO, HAS_G>;
@@ -697,7 +716,8 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     const bool kvalid = krow < p.Lk;
     const bool pair_active = (key0 + pr * 16) < p.Lk;
 
-    using StagePlan = CopyPlan<HD, SM::nt, 1, kThreads16>;
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kThreads16>,
+                                         StagedPlan<T, HD, SM::nt, kThreads16, IO>>;
     constexpr int SPT = StagePlan::N + 1;  // plus one 4-byte copy of statistics (or its placeholder)
     StagePlan plan;
     const int ns = (p.Lq + kStageRows - 1) / kStageRows;
@@ -705,7 +725,7 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     auto issue_next = [&]() {
         elem_t* slot = ring + (issued % R) * SM::slot;
         const int row0 = issued * kStageRows;
-        plan.issue(slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
+        issue_plan(plan, slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
         // the four statistic arrays of the stage's rows by waves 0..3; the others issue a placeholder
         if (wave < 4) {
             const int64_t plane = p.s4 - p.lse2;  // see bwd_col16_body
@@ -713,7 +733,7 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
             if (HAS_G && wave == 1) src = p.mu;
             float* st = reinterpret_cast<float*>(slot + oST);
             if (lane < 32) dma4(src + (int64_t)bh * p.Lr + row0 + lane, lds_addr(st) + (uint32_t)(wave * 32 * 4));
-        } else {
+        } else if constexpr (DMA) {
             if (lane == 0) dma4(plan.any, plan.sink);
         }
         ++issued;
@@ -723,18 +743,18 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     auto begin_copies = [&]() __attribute__((always_inline)) {
         const Src q{p.q.head(b, h), p.q.sl};
         if constexpr (HAS_G && HAS_DO)
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                       Src{p.dTO.head(b, h), p.dTO.sl}, Src{p.dO.head(b, h), p.dO.sl});
         else if constexpr (HAS_G)
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                       Src{p.dTO.head(b, h), p.dTO.sl});
         else
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
         issue_next();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
     u32x4 kB[KC], vB[KC], tkB[KC], tvB[KC];
-    if (p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
+    if (DMA && p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
         // the common case: whole rows that all exist, every tensor with k's strides
         const int64_t slice = b * p.k.sb + h * p.k.sh;
         const uint32_t at = ((uint32_t)krow * (uint32_t)p.k.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
@@ -746,11 +766,11 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
         }
         begin_copies();
     } else {
-        load_b_operands16<HD>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
-        load_b_operands16<HD>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
+        load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
+        load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
         if constexpr (HAS_G) {
-            load_b_operands16<HD>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
-            load_b_operands16<HD>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
         }
         begin_copies();
     }
@@ -759,7 +779,11 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
         asm volatile("" : "+v"(kB[c]), "+v"(vB[c]));
         if constexpr (HAS_G) asm volatile("" : "+v"(tkB[c]), "+v"(tvB[c]));
     }
-    while (issued < R && issued < ns) issue_next();
+    if constexpr (DMA) {
+        while (issued < R && issued < ns) issue_next();
+    } else {
+        plan.commit();
+    }
     const float sl2 = p.scale * kLog2e;
     f32x4 dk[DH], dv[DH], dtk[DH], dtv[DH];
 #pragma unroll
@@ -868,44 +892,46 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     };
 
     for (int i = 0; i < ns; ++i) {
-        wait_stages<SPT>(issued - 1 - i);
+        wait_stages<SPT>(DMA ? issued - 1 - i : 0);  // staged: the statistics still come by LDS-DMA
         workgroup_barrier();  // stage i has landed for every wave; stage i-1 and the exchange area are free
-        if (i > 0 && issued < ns) issue_next();
+        if ((i > 0 || !DMA) && issued < ns) issue_next();
         const elem_t* slot = ring + (i % R) * SM::slot;
         if (pair_active) scores(slot);
         workgroup_barrier();  // the partner's tiles are visible
         if (pair_active) outputs(slot);
+        if constexpr (!DMA) plan.commit();
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!pair_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<64>::elems;
     const int row0 = key0 + pr * 16;
     const int dcol = 64 * m;
+    const int doff = IO == kIoF32 ? 2 * dcol : dcol;  // in the units of the views
     const int Dm = p.D - dcol;  // columns of this member's half that exist (may be <= 0)
-    store_tile16<T, 64>(stage_tile, p.dk.head(b, h) + dcol, p.dk.sl, row0, p.Lk, Dm, dk, p.scale, lane);
+    store_rows16<T, 64, IO>(stage_tile, p.dk.head(b, h) + doff, p.dk.sl, row0, p.Lk, Dm, dk, p.scale, lane);
     if constexpr (HAS_G)
-        store_tile16<T, 64>(stage_tile, p.dtk.head(b, h) + dcol, p.dtk.sl, row0, p.Lk, Dm, dtk, p.scale, lane);
-    store_tile16<T, 64>(stage_tile, p.dv.head(b, h) + dcol, p.dv.sl, row0, p.Lk, Dm, dv, 1.0f, lane);
+        store_rows16<T, 64, IO>(stage_tile, p.dtk.head(b, h) + doff, p.dtk.sl, row0, p.Lk, Dm, dtk, p.scale, lane);
+    store_rows16<T, 64, IO>(stage_tile, p.dv.head(b, h) + doff, p.dv.sl, row0, p.Lk, Dm, dv, 1.0f, lane);
     if constexpr (HAS_G)
-        store_tile16<T, 64>(stage_tile, p.dtv.head(b, h) + dcol, p.dtv.sl, row0, p.Lk, Dm, dtv, 1.0f, lane);
+        store_rows16<T, 64, IO>(stage_tile, p.dtv.head(b, h) + doff, p.dtv.sl, row0, p.Lk, Dm, dtv, 1.0f, lane);
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO = kIoDma>
 __global__ __launch_bounds__(kThreads16, 2) void bwd_col16p_kernel(const BwdParams p) {
-    bwd_col16p_body<T, HD, R, HAS_DO, HAS_G>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The paired column-owned launch with the second pass of the row-owned kernel at its end (see
 // bwd_col16_repair_kernel).  The row-owned kernel's workgroups have four waves, these eight: in a workgroup that
 // takes a row item the upper four leave at once, and the barriers of the others count the waves that are left.
-template <typename T, int HD, int R, int RROW, bool HAS_DO, bool HAS_G>
+template <typename T, int HD, int R, int RROW, bool HAS_DO, bool HAS_G, int IO = kIoDma>
 __global__ __launch_bounds__(kThreads16, 2) void bwd_col16p_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks) {
-        bwd_col16p_body<T, HD, R, HAS_DO, HAS_G>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, col_blocks);
     } else {
         if ((int)threadIdx.x >= kXThreads16) return;
-        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
+        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
     }
 }
 

@@ -1,6 +1,6 @@
-// Fused attention-JVP forward, 16-wide form (gfx950; inputs with 16-byte aligned rows).
+// Fused attention-JVP forward, 16-wide form (gfx950).
 //
-// Same mathematics and outputs as fwd_kernel (semicat/jvp_utils/ryu_triton.py:73-291: O, TO, M = lse,
+// Computes what the reference forward does (semicat/jvp_utils/ryu_triton.py:73-291: O, TO, M = lse,
 // MU, LI in one online-softmax pass), decomposed for occupancy: a workgroup of eight wavefronts owns
 // 128 queries of one (batch, head), 16 per wavefront as MFMA columns, and walks over the keys in
 // stages of 32 streamed through an LDS ring by LDS-DMA.  A wavefront needs fewer than 128 registers,
@@ -8,7 +8,7 @@
 // workgroups per CU overlap one's copies with the other's arithmetic.
 #pragma once
 #include "sjvp_fwd.hpp"
-#include "sjvp_w16.hpp"
+#include "sjvp_staged16.hpp"
 
 namespace sjvp {
 
@@ -18,11 +18,11 @@ namespace sjvp {
 // moves into registers before the first stage is consumed, land in slots 2 and 3 (exactly their
 // size), which then join the ring.  After the last stage the ring doubles as the per-wave staging
 // tiles of the output stores.
-template <int HD, int R, bool JVP, int SPB = 1>
+template <int HD, int R, bool JVP, int SPB = 1, bool DMA = true>
 struct Fwd16Smem {
     static constexpr int nt = JVP ? 4 : 2;
     static constexpr int slot = nt * Slab<HD>::elems;
-    static constexpr int own = (JVP ? 2 : 1) * 4 * Slab<HD>::elems;
+    static constexpr int own = DMA ? (JVP ? 2 : 1) * 4 * Slab<HD>::elems : 0;
     static_assert(SPB == 1 || (SPB == 2 && R == 4 && own == 2 * slot), "SPB = 2 needs a ring of four slots");
     static constexpr int own_off = SPB == 2 ? 2 * slot : 0;
     static constexpr int ring_off = SPB == 2 ? 0 : own;
@@ -35,11 +35,15 @@ struct Fwd16Smem {
 // stage per barrier): the own rows in registers, each stage's K (, K_dot) slab in place in LDS.  Meant
 // for key axes that one workgroup per (batch, head) walks once (every workgroup rotates the K rows it
 // streams).
-template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false>
+// IO: how the tensors lie in memory (sjvp_staged16.hpp); anything but kIoDma copies its stages through registers,
+// one stage ahead, and loads its own rows straight into registers.
+template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma>
 __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams p) {
     static_assert(!ROPE || (HD == 64 && SPB == 1), "the folded rotation covers HD = 64, one stage per barrier");
+    constexpr bool DMA = IO == kIoDma;
+    static_assert(DMA || (SPB == 1 && !ROPE), "staged copies run one stage ahead, unrotated");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    using SM = Fwd16Smem<HD, R, JVP, SPB>;
+    using SM = Fwd16Smem<HD, R, JVP, SPB, DMA>;
     elem_t* own = reinterpret_cast<elem_t*>(smem_raw) + SM::own_off;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw) + SM::ring_off;
     constexpr int SE = Slab<HD>::elems;
@@ -61,33 +65,53 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     const int qrow = q0 + wave * 16 + n;
     const bool wave_active = (q0 + wave * 16) < p.Lq;
 
-    // own rows first (issued before the stages, so they land first), then the ring
-    {
-        CopyPlan<HD, JVP ? 8 : 4, 4> own_plan;
-        if constexpr (JVP)
-            own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl},
-                          Src{p.tq.head(b, h), p.tq.sl});
-        else
-            own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl});
-        own_plan.issue(own, p.Lq - q0, p.D == HD && q0 + kOwned16 <= p.Lq);
-    }
-    using StagePlan = CopyPlan<HD, SM::nt, 1>;
+    u32x4 qB[KC], tqB[KC];
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1>, StagedPlan<T, HD, SM::nt, kThreads16, IO>>;
     constexpr int SPT = StagePlan::N;
     StagePlan plan;
     // slot layout K | V | K_dot | V_dot (primal only: K | V)
-    if constexpr (JVP)
-        plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl},
-                  Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
-    else
-        plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
+    const Src sk{p.k.head(b, h), p.k.sl}, sv{p.v.head(b, h), p.v.sl};
+    if constexpr (DMA) {
+        // own rows first (issued before the stages, so they land first), then the ring
+        {
+            CopyPlan<HD, JVP ? 8 : 4, 4> own_plan;
+            if constexpr (JVP)
+                own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl},
+                              Src{p.tq.head(b, h), p.tq.sl});
+            else
+                own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl});
+            own_plan.issue(own, p.Lq - q0, p.D == HD && q0 + kOwned16 <= p.Lq);
+        }
+        if constexpr (JVP)
+            plan.init(tid, 0, p.D, smem_raw + SM::sink, sk, sv, Src{p.tk.head(b, h), p.tk.sl},
+                      Src{p.tv.head(b, h), p.tv.sl});
+        else
+            plan.init(tid, 0, p.D, smem_raw + SM::sink, sk, sv);
+    } else {
+        staged_b_operands16<T, HD, IO>(qB, p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
+        if constexpr (JVP) {
+            staged_b_operands16<T, HD, IO>(tqB, p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
+            plan.init(tid, p.D, sk, sv, Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
+        } else {
+            plan.init(tid, p.D, sk, sv);
+        }
+    }
     const int ns = (p.Lk + kStageRows - 1) / kStageRows;
     int issued = 0;
     auto issue_next = [&]() {
-        plan.issue(ring + (issued % R) * SM::slot, p.Lk - issued * kStageRows,
-                   p.D == HD && (issued + 1) * kStageRows <= p.Lk);
+        elem_t* slot = ring + (issued % R) * SM::slot;
+        if constexpr (DMA)
+            plan.issue(slot, p.Lk - issued * kStageRows, p.D == HD && (issued + 1) * kStageRows <= p.Lk);
+        else
+            plan.issue(slot, p.Lk - issued * kStageRows);
         ++issued;
     };
-    while (issued < (SPB == 2 ? 2 : R) && issued < ns) issue_next();
+    if constexpr (DMA) {
+        while (issued < (SPB == 2 ? 2 : R) && issued < ns) issue_next();
+    } else {
+        issue_next();
+        plan.commit();
+    }
 
     const float sl2 = p.scale * kLog2e;
     float m_i = -INFINITY;     // reference maximum (same in the four lanes of a query)
@@ -104,10 +128,9 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     }
 
     // SPB = 1: the own rows and stage 0 were issued before the other stages; SPB = 2: everything
-    wait_stages<SPT>(SPB == 2 ? 0 : issued - 1);
+    if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1);
     workgroup_barrier();
-    u32x4 qB[KC], tqB[KC];
-    {
+    if constexpr (DMA) {
         const int r = 16 * (wave & 1) + n;
         read_b_operands16<HD>(qB, own + (wave >> 1) * SE, r, g);
         if constexpr (JVP) read_b_operands16<HD>(tqB, own + (4 + (wave >> 1)) * SE, r, g);
@@ -216,17 +239,21 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
             if (i >= ns) break;
             if (i > 0) {
                 // the stages of this step have landed for every wave; those of the last step are consumed
-                wait_stages<SPT>(SPB == 2 ? 0 : issued - 1 - i);
+                if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1 - i);
                 workgroup_barrier();
+            }
+            if (i > 0 || !DMA) {
 #pragma unroll
                 for (int u = 0; u < SPB; ++u)
                     if (issued < ns) issue_next();
-                rotate_stage(ring + h * SM::slot, i * kStageRows);
             }
-            if (!wave_active) continue;
+            if (i > 0) rotate_stage(ring + h * SM::slot, i * kStageRows);
+            if (wave_active) {
 #pragma unroll
-            for (int u = 0; u < SPB; ++u)
-                if (i + u < ns) compute(ring + (h + u) * SM::slot, (i + u) * kStageRows);
+                for (int u = 0; u < SPB; ++u)
+                    if (i + u < ns) compute(ring + (h + u) * SM::slot, (i + u) * kStageRows);
+            }
+            if constexpr (!DMA) plan.commit();
         }
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
@@ -264,9 +291,9 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     }
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
     const int row0 = q0 + wave * 16;
-    store_tile16<T, HD>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc, inv_l, lane);
+    store_rows16<T, HD, IO>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc, inv_l, lane);
     if constexpr (JVP)
-        store_tile16<T, HD>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc, inv_l, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc, inv_l, lane);
 }
 
 }  // namespace sjvp

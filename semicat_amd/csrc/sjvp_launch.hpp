@@ -62,16 +62,16 @@ int launch(K kernel, int grid, int smem_bytes, hipStream_t stream, const P& para
     return rc == hipSuccess ? SJVP_OK : SJVP_ERR_LAUNCH;
 }
 
-// Forward: 16-wide LDS-DMA kernels (16-byte aligned rows) and the 32-wide register-staged ones.
+// Forward: stages by LDS-DMA (16-byte aligned rows), or through registers (any alignment).
 template <typename T> int fwd_vec(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 template <typename T> int fwd_any(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 
-// Backward: the single launch (short key axes, D <= 64), the 16-wide pair and the 32-wide pair.
+// Backward: the single launch (short key axes, D <= 64), and the row + column pair on rows as above.
 template <typename T> int bwd_fused(const BwdParams& p, int BH, bool has_do, bool has_g, hipStream_t stream);
 template <typename T> int bwd_pair_vec(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 template <typename T> int bwd_pair_any(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 
-// fp32 tensors with bf16 arithmetic (the cast folded into the loads and stores): 32-wide kernels.
+// fp32 tensors with bf16 arithmetic (the cast folded into the loads and stores).
 // The views carry fp32 pointers cast to elem_t* and strides counted in 2-byte units.
 int fwd_f32io(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 int bwd_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);

@@ -1,0 +1,77 @@
+// Launches of the 16-wide row-owned + column-owned backward pair, for every way the tensors may lie in memory
+// (IO, sjvp_staged16.hpp).
+#pragma once
+#include "sjvp_bwd16x.hpp"
+#include "sjvp_launch.hpp"
+
+namespace sjvp {
+
+template <typename T, int HD, bool HAS_DO, bool HAS_G, int IO>
+int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
+    // the row-owned kernel first (besides dQ, dQ_dot it leaves the row sums in the workspace), then
+    // the column-owned one; workgroups of four waves own 64 positions
+    constexpr int XR = HD == 128 || IO != kIoDma ? 2 : 3;  // ring depth (staged copies run one stage ahead)
+    int rc = SJVP_OK;
+    bool rides = false;
+    if (parts & SJVP_BWD_ROW) {
+        // (fp32 rows at HD = 128 are staged in 64 registers: one wave per SIMD, or they spill)
+        constexpr int OCC = HD == 128 && IO == kIoF32 ? 1 : HD == 128 || IO != kIoDma ? 2 : 3;
+        const int grid = BH * (p.Lr / kXOwned16);
+        constexpr int smem = Row16Smem<HD, XR, HAS_G>::bytes;
+        // "always": a launch that measures the row-sum residues, then one that computes with the corrected
+        // sums; otherwise the pass itself and, unless switched off, a second launch in which the workgroups
+        // whose residues call for it run again
+        if (p.rowfix == 2) rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 1, IO>, grid, smem, stream, p, kXThreads16);
+        else rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 0, IO>, grid, smem, stream, p, kXThreads16);
+        // The second launch does not depend on the column-owned pass.  Where nearly all of its workgroups leave
+        // at once (repair of flagged workgroups only), they ride at the end of that launch instead of paying for
+        // one of their own.
+        // (not at D = 128 with the cotangent on O only: the row-owned body needs more registers than that
+        // column-owned kernel, which would lose a resident workgroup per compute unit to it; nor on fp32 rows there)
+        rides = p.rowfix == 1 && (parts & SJVP_BWD_COL) && (HD != 128 || (HAS_G && IO != kIoF32));
+        if (rc == SJVP_OK && p.rowfix != 0 && !rides)
+            rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 2, IO>, grid, smem, stream, p, kXThreads16);
+    }
+    if (rc != SJVP_OK || !(parts & SJVP_BWD_COL)) return rc;
+    const int grid = BH * ((p.Lk + kXOwned16 - 1) / kXOwned16);
+    using CS = Col16Smem<HD, XR, HAS_DO, HAS_G>;
+    if constexpr (HD == 128) {
+        // eight waves: wave pairs share 16 keys, split the score-side tiles by query tile and the
+        // gradients by head-dimension half (one launch, nothing computed twice)
+        constexpr int PR = 2;  // ring depths 2, 3, 4 measure the same (the kernel is issue-bound)
+        using PS = Col16pSmem<HD, PR, HAS_DO, HAS_G>;
+        if (rides) {
+            BwdParams pr = p;
+            pr.col_workgroups = grid;
+            constexpr int smem = PS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? PS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
+            return launch(bwd_col16p_repair_kernel<T, HD, PR, XR, HAS_DO, HAS_G, IO>, grid + BH * (p.Lr / kXOwned16), smem,
+                          stream, pr, kThreads16);
+        }
+        return launch(bwd_col16p_kernel<T, HD, PR, HAS_DO, HAS_G, IO>, grid, PS::bytes, stream, p, kThreads16);
+    } else {
+        if (rides) {
+            BwdParams pr = p;
+            pr.col_workgroups = grid;
+            constexpr int smem = CS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? CS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
+            return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO>, grid + BH * (p.Lr / kXOwned16), smem,
+                          stream, pr, kXThreads16);
+        }
+        return launch(bwd_col16_kernel<T, HD, XR, HAS_DO, HAS_G, 3, 2, IO>, grid, CS::bytes, stream, p, kXThreads16);
+    }
+}
+
+template <typename T, int HD, int IO>
+int pair_hd(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+    if (has_do && has_g) return pair_mode<T, HD, true, true, IO>(p, BH, parts, stream);
+    if (has_g) return pair_mode<T, HD, false, true, IO>(p, BH, parts, stream);
+    return pair_mode<T, HD, true, false, IO>(p, BH, parts, stream);
+}
+
+template <typename T, int IO>
+int bwd_pair16(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+    if (p.D <= 32) return pair_hd<T, 32, IO>(p, BH, has_do, has_g, parts, stream);
+    if (p.D <= 64) return pair_hd<T, 64, IO>(p, BH, has_do, has_g, parts, stream);
+    return pair_hd<T, 128, IO>(p, BH, has_do, has_g, parts, stream);
+}
+
+}  // namespace sjvp

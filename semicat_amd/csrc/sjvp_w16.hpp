@@ -17,9 +17,8 @@ namespace sjvp {
 
 constexpr int kWaves16 = 8;
 constexpr int kThreads16 = 64 * kWaves16;
-constexpr int kOwned16 = 16 * kWaves16;  // owned positions per workgroup (== kOwned)
+constexpr int kOwned16 = 16 * kWaves16;  // owned positions per workgroup
 constexpr int kSink16 = 16;              // bytes of LDS that placeholder copies may overwrite
-static_assert(kOwned16 == kOwned, "both kernel families use the same workgroup grid");
 
 struct Src {
     const elem_t* ptr;  // [L][D] slice of one (batch, head)

@@ -1,0 +1,58 @@
+"""The 16-bit kernels on rows that LDS-DMA cannot read (odd head dimensions, pointers off the 16-byte grid) and on
+fp32 rows: the piece of a row that reaches beyond D at every remainder, stage edges on both axes, every
+head-dimension class, against the fp64 oracle, and that nothing outside the tensors is written."""
+import pytest
+import torch
+
+from oracle import attn_jvp_oracle as orc
+
+pytestmark = pytest.mark.gpu
+GRADS = ("dq", "dk", "dv", "dtq", "dtk", "dtv")
+TOL = 1e-2  # the gate of the 16-bit kernels; measured 2.6e-3 (bf16) and 3.3e-4 (fp16)
+CANARY = 12345.0
+
+
+def _place(t, offset):
+    """A copy of t inside a larger buffer, `offset` elements from its start, canaries on both sides."""
+    buf = torch.full((t.numel() + 64,), CANARY, device="cuda", dtype=t.dtype)
+    v = buf[offset:offset + t.numel()].view(t.shape)
+    v.copy_(t)
+    return v, buf
+
+
+@pytest.mark.parametrize("store", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("Lq,Lk,D,offset,mode", [
+    (33, 64, 17, 0, "both"), (65, 31, 22, 0, "both"), (32, 160, 31, 0, "dTO"), (64, 33, 33, 0, "both"),
+    (130, 65, 36, 0, "both"), (31, 97, 45, 0, "dO"), (97, 96, 54, 0, "both"), (200, 129, 63, 0, "dTO"),
+    (40, 70, 64, 3, "both"), (70, 40, 32, 1, "dO"), (66, 34, 65, 0, "both"), (35, 100, 91, 0, "dTO"),
+    (90, 61, 110, 0, "both"), (33, 65, 127, 0, "both"), (64, 32, 128, 1, "dO")])
+def test_staged_rows(store, Lq, Lk, D, offset, mode):
+    from semicat_amd import kernels as K
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}[store]
+    arith = "bf16" if store == "fp32" else None
+    x = orc.make_inputs(2, 3, Lq, Lk, D, seed=7, tangent_scale=0.3, dtype=dt)
+    # fp32 tensors are rounded to bf16 as they are loaded: the reference sees what the kernels compute with
+    y = {n: t.to(torch.bfloat16) for n, t in x.items()} if store == "fp32" else x
+    cot = {n: y[n] for n in ("dO", "dTO") if mode in ("both", n)}
+    ref = orc.attention_jvp_autograd(*[y[n] for n in orc.TENSOR_ORDER[:6]], **cot)
+    d = {n: _place(t, offset)[0] for n, t in x.items()}
+    print(f"[staged] {store} {(Lq, Lk, D, offset)} {mode}", flush=True)
+    out = [_place(torch.zeros_like(x["q"]), offset) for _ in range(2)]
+    tan = [d[n] for n in ("tq", "tk", "tv")]
+    o, to, lse, mu, _ = K.attention_jvp_forward(d["q"], d["k"], d["v"], *tan, o=out[0][0], to=out[1][0],
+                                                arithmetic=arith)
+    g = [_place(torch.zeros_like(x[n]), offset) for n in ("q", "k", "v", "tq", "tk", "tv")]
+    has_g = mode != "dO"
+    K.attention_jvp_backward(d["q"], d["k"], d["v"], *(tan if has_g else (None,) * 3), o, to if has_g else None, lse,
+                             mu if has_g else None, dO=d["dO"] if "dO" in cot else None,
+                             dTO=d["dTO"] if has_g else None, grads=tuple(v for v, _ in g), arithmetic=arith)
+    res = {"O": o, "TO": to, **{n: v for n, (v, _) in zip(GRADS, g) if has_g or not n.startswith("dt")}}
+    for n, t in res.items():
+        err = orc.rel_frobenius(t.cpu(), ref[n])
+        assert err <= TOL, (n, err)
+    for v, buf in out + g:
+        end = offset + v.numel()
+        assert (buf[:offset].float() == torch.tensor(CANARY).to(dt).float().item()).all()
+        assert (buf[end:].float() == torch.tensor(CANARY).to(dt).float().item()).all()
+    o2, _ = K.attention_forward(d["q"], d["k"], d["v"], arithmetic=arith)
+    assert orc.rel_frobenius(o2.cpu(), ref["O"]) <= TOL
