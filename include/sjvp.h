@@ -110,8 +110,12 @@ int sjvp_bwd(const void* q, const void* k, const void* v, const void* tq, const 
  * valid on a workspace that an earlier SJVP_BWD_ROW launch with the same arguments has filled.  (The second
  * pass of the row-owned kernel, see sjvp_set_row_sum_repair, belongs to SJVP_BWD_ROW; with SJVP_BWD_ALL its
  * workgroups are appended to the column-owned launch, since it depends on the first row-owned launch only.)
+ *
+ * SJVP_FP32_BF16 takes the pair for every shape, whose row sums are repaired (sjvp_set_row_sum_repair).
+ * SJVP_BWD_ALL | SJVP_BWD_FP32_SINGLE lets it take the single launch where 16-bit tensors do (faster, and with the
+ * row sums of the 16-bit route: what casting the tensors around sjvp_bwd() would give).
  */
-enum sjvp_bwd_part { SJVP_BWD_ROW = 1, SJVP_BWD_COL = 2, SJVP_BWD_ALL = 3 };
+enum sjvp_bwd_part { SJVP_BWD_ROW = 1, SJVP_BWD_COL = 2, SJVP_BWD_ALL = 3, SJVP_BWD_FP32_SINGLE = 4 };
 int sjvp_bwd_parts(int parts, const void* q, const void* k, const void* v, const void* tq,
                    const void* tk, const void* tv, const void* o, const void* to, const void* dO,
                    const void* dTO, const float* lse, const float* mu, void* dq, void* dk, void* dv,

@@ -29,6 +29,7 @@ SJVP_NOALLOC_MAX_ROWS = 1 << 20
 SJVP_BWD_ROW = 1
 SJVP_BWD_COL = 2
 SJVP_BWD_ALL = 3
+SJVP_BWD_FP32_SINGLE = 4  # with SJVP_BWD_ALL and SJVP_FP32_BF16: the single launch where 16-bit tensors take it
 
 F_TENSORS = ("q", "k", "v", "tq", "tk", "tv", "o", "to")
 B_TENSORS = ("q", "k", "v", "tq", "tk", "tv", "o", "to", "dO", "dTO",

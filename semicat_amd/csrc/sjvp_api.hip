@@ -90,10 +90,8 @@ int compute_units() {
     return n;
 }
 
-// Kernel selection of the backward: the single launch where it fits, else the row + column pair.
-template <typename T>
-int bwd_select(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
-    if (!p.vec) return bwd_pair_any<T>(p, BH, has_do, has_g, parts, stream);
+// Whether the backward takes the single launch, else the row + column pair.
+bool bwd_single(const BwdParams& p, int BH, int parts) {
     // the single launch takes its row sums from the 16-bit outputs and cannot repair them: a caller who
     // asked for the repair everywhere gets the pair (the folded rotation exists in the single launch only)
     const bool single = parts == SJVP_BWD_ALL && p.Lk <= kOwned16 && p.D <= 64;
@@ -101,8 +99,13 @@ int bwd_select(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, h
     // pairs with a long query axis would leave most of the chip idle, while the row-owned launch of the
     // pair spreads the queries over Lq / 64 workgroups per pair.
     const bool few_long = 2 * BH <= compute_units() && p.Lq >= 4 * kOwned16 && !p.rope.cos;
-    if (single && !few_long && (p.rowfix != SJVP_REPAIR_ALWAYS || p.rope.cos))
-        return bwd_fused<T>(p, BH, has_do, has_g, stream);
+    return single && !few_long && (p.rowfix != SJVP_REPAIR_ALWAYS || p.rope.cos);
+}
+
+template <typename T>
+int bwd_select(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+    if (!p.vec) return bwd_pair_any<T>(p, BH, has_do, has_g, parts, stream);
+    if (bwd_single(p, BH, parts)) return bwd_fused<T>(p, BH, has_do, has_g, stream);
     return bwd_pair_vec<T>(p, BH, has_do, has_g, parts, stream);
 }
 
@@ -115,7 +118,9 @@ struct BwdTensors {
 
 int check_bwd(int parts, const BwdTensors& t, int B, int H, int Lq, int Lk, int D, const int64_t* strides,
               float scale, int dtype) {
-    if (parts < SJVP_BWD_ROW || parts > SJVP_BWD_ALL) return SJVP_ERR_PARTS;
+    const int extra = parts & ~SJVP_BWD_ALL;
+    if (!(parts & SJVP_BWD_ALL) || (extra != 0 && (extra != SJVP_BWD_FP32_SINGLE || dtype != SJVP_FP32_BF16)))
+        return SJVP_ERR_PARTS;
     if (!t.dO && !t.dTO) return SJVP_ERR_COTANGENT;
     if (!t.q || !t.k || !t.v || !t.o || !t.lse || !t.dq || !t.dk || !t.dv || !strides) return SJVP_ERR_NULL;
     if (t.dTO && (!t.tq || !t.tk || !t.tv || !t.to || !t.mu || !t.dtq || !t.dtk || !t.dtv)) return SJVP_ERR_NULL;
@@ -223,7 +228,12 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
     if (rope.cos && (!p.vec || parts != SJVP_BWD_ALL)) return SJVP_ERR_ROTARY;  // the single launch only
 
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (f32io) return bwd_f32io(p, B * H, has_do, has_g, parts, s);
+    if (f32io) {
+        // the row sums of the pair are repaired, those of the single launch are not: the caller has to allow it
+        if ((parts & SJVP_BWD_FP32_SINGLE) && bwd_single(p, B * H, parts & SJVP_BWD_ALL))
+            return bwd_fused_f32io(p, B * H, has_do, has_g, s);
+        return bwd_pair_f32io(p, B * H, has_do, has_g, parts & SJVP_BWD_ALL, s);
+    }
     return dtype == SJVP_BF16 ? bwd_select<Bf16>(p, B * H, has_do, has_g, parts, s)
                               : bwd_select<Fp16>(p, B * H, has_do, has_g, parts, s);
 }

@@ -16,7 +16,7 @@
 // Results are deterministic.
 #pragma once
 #include "sjvp_bwd.hpp"
-#include "sjvp_w16.hpp"
+#include "sjvp_staged16.hpp"
 
 namespace sjvp {
 
@@ -55,10 +55,17 @@ __device__ __forceinline__ int bounce_swz(int key) { return 4 * ((key >> 2) & 1)
 // ROPE: q, k and their tangents are rotated by p.rope once they are in LDS (own K, K_dot rows in the
 // prologue, each stage's Q, Q_dot slabs by the threads that do not form row sums), and the gradients
 // dQ, dQ_dot, dK, dK_dot go back through the inverse rotation on their way out (head dimension 64).
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, bool ROPE = false>
-__global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(const BwdParams p) {
+// IO: how the tensors lie in memory (sjvp_staged16.hpp): aligned 16-bit rows, or fp32 rows, which go through
+// registers: stage i + 2 is requested behind the barrier of iteration i and written behind its step 3, where the
+// registers of step 2 are free.  (16-bit rows of any alignment take the row + column pair: it repairs the row
+// sums, and the single launch measured no faster on them, 68 against 58 us forward + backward at B=64 H=12 L=128
+// D=20.)  fp32 rows, B=64 H=12 L=128 D=64: 100 us, the pair 126.
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, bool ROPE = false, int IO = kIoDma>
+__global__ __launch_bounds__(kThreads16, HAS_G || IO != kIoDma ? 2 : 4) void bwd_fused16_kernel(const BwdParams p) {
     static_assert(HD <= 64, "the accumulators of four gradients must fit the register file");
     static_assert(!ROPE || HD == 64, "the folded rotation covers a head dimension of 64");
+    constexpr bool DMA = IO == kIoDma;
+    static_assert(DMA || (IO == kIoF32 && R == 3 && !ROPE), "staged copies: fp32 rows, two stages ahead, unrotated");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     using SM = Fused16Smem<HD, R, HAS_DO, HAS_G>;
     constexpr int SE = Slab<HD>::elems;
@@ -106,43 +113,43 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
         return v;
     };
 
-    using StagePlan = CopyPlan<HD, SM::nt, 1>;
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1>, StagedPlan<T, HD, SM::nt, kThreads16, IO>>;
     constexpr int SPT = StagePlan::N + 1;  // plus one 4-byte copy of statistics
     StagePlan plan;
     {
         const Src q{p.q.head(b, h), p.q.sl}, o{p.o.head(b, h), p.o.sl};
         if constexpr (HAS_G && HAS_DO)
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                       Src{p.dTO.head(b, h), p.dTO.sl}, Src{p.dO.head(b, h), p.dO.sl}, o,
                       Src{p.to.head(b, h), p.to.sl});
         else if constexpr (HAS_G)
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                       Src{p.dTO.head(b, h), p.dTO.sl}, o, Src{p.to.head(b, h), p.to.sl});
         else
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl}, o);
+            init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl}, o);
     }
     const int ns = (p.Lq + kStageRows - 1) / kStageRows;
     int issued = 0;
     auto issue_next = [&]() {
         elem_t* slot = ring + (issued % R) * SM::slot;
         const int row0 = issued * kStageRows;
-        plan.issue(slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
+        issue_plan(plan, slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
         // raw lse (wave 0) and mu (wave 1) of the stage's rows (rows < Lr exist); every wave issues
         // exactly one 4-byte LDS-DMA instruction, the others as a placeholder into the sink
         float* raw = reinterpret_cast<float*>(slot + oST);
         if (wave < 2) {
             const float* src = (wave == 1 && HAS_G) ? p.mu : p.lse;
             if (lane < 32) dma4(src + (int64_t)bh * p.Lr + row0 + lane, lds_addr(raw) + (uint32_t)(wave * 32 * 4));
-        } else {
+        } else if constexpr (DMA) {
             if (lane == 0) dma4(plan.any, plan.sink);
         }
         ++issued;
     };
-    issue_next();
     // The first stage is issued before the own rows: it lands first and its row sums are formed while the
     // own rows (four times its size) are still on their way.
     constexpr int OWN = (HAS_G ? 16 : 8) * Slab<HD>::chunks / kThreads16;  // own-row copies per wave
-    {
+    if constexpr (DMA) {
+        issue_next();
         CopyPlan<HD, HAS_G ? 16 : 8, 4> own_plan;
         if constexpr (HAS_G)
             own_plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl},
@@ -152,6 +159,24 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
             own_plan.init(tid, 0, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl},
                           Src{p.v.head(b, h), p.v.sl});
         own_plan.issue(ownK, p.Lk, p.D == HD && p.Lk == kOwned16);
+    } else {
+        // slab s of every own tensor at a time, the next window's loads under the writes of the last
+        StagedPlan<T, HD, HAS_G ? 4 : 2, kThreads16, IO, 4 * SE> own_plan;
+        if constexpr (HAS_G)
+            own_plan.init(tid, p.D, Src{p.k.head(b, h), p.k.sl}, Src{p.tk.head(b, h), p.tk.sl},
+                          Src{p.v.head(b, h), p.v.sl}, Src{p.tv.head(b, h), p.tv.sl});
+        else
+            own_plan.init(tid, p.D, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
+        issue_next();
+        for (int s = 0; s < 4; ++s) {
+            own_plan.issue(ownK + s * SE, p.Lk - 32 * s);
+            if (s == 0) {
+                plan.commit();
+                if (issued < ns) issue_next();
+            }
+            own_plan.commit();
+        }
+        plan.commit();
     }
     const float sl2 = p.scale * kLog2e;
 
@@ -334,7 +359,7 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
     // Step 3: 16 x 16 tiles (head-dimension tile dt, query tile qt) of dQ and dQ_dot for the stage.
     // HD = 64: wave w forms tile w of both; HD = 32: waves 0..3 form dQ, waves 4..7 dQ_dot.
     constexpr int NTILES = 2 * DT;
-    auto row_outputs = [&](const elem_t* bounceS, elem_t* qstage_i, auto full_tag) {
+    auto row_outputs = [&](const elem_t* bounceS, elem_t* qstage_i, int row0, auto full_tag) {
         const elem_t* bounceT = bounceS + oBT;
         constexpr bool FULL = decltype(full_tag)::value;  // all four key slabs hold keys
         const int tq = wave;                           // dQ tile of this wave
@@ -370,6 +395,16 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
         // lane = query 16*qt + n, registers = columns 16*dt + 4g .. + 3: into the staging tile, from
         // where flush_rows() sends whole rows after the next barrier
         elem_t* st = qstage_i + (16 * qt + (lane_l & 15)) * SM::qpitch + 16 * dt + 4 * (lane_l >> 4);
+        if constexpr (IO == kIoF32) {
+            // fp32 rows leave unrounded from here: four lanes hold 64 consecutive bytes of a row
+            const int row = row0 + 16 * qt + (lane_l & 15), d = 16 * dt + 4 * (lane_l >> 4);
+            if (row < p.Lq) {
+                a0 += a1;
+                if (do_q) store_f32x4(p.dq.head(b, h) + (int64_t)row * p.dq.sl, a0 * p.scale, d, p.D);
+                if (do_t) store_f32x4(p.dtq.head(b, h) + (int64_t)row * p.dtq.sl, a2 * p.scale, d, p.D);
+            }
+            return;
+        }
         if (do_q) {
             a0 += a1;
             *reinterpret_cast<u32x2*>(st) =
@@ -384,6 +419,7 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
     // of a row per thread (HD / 8 pieces per row).  Issued before the stage copy of the iteration, so
     // the stores are older than every copy a later wait_stages() still allows to be outstanding.
     auto flush_rows = [&](int row0, const elem_t* qstage_i) {
+        if constexpr (IO == kIoF32) return;
         constexpr int CH = HD / 8;
         const int tid_l = wave * 64 + lane_now();
         const int half = tid_l >> 8, t = tid_l & 255;
@@ -402,12 +438,14 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
 
     // Only stage 0 and the own rows are waited for here; the later stages are issued once these
     // have landed, so that their copies run under the arithmetic instead of ahead of it.
-    wait_stages<OWN>(1);  // everything but the OWN youngest copies of this wave: stage 0
+    if constexpr (DMA) wait_stages<OWN>(1);  // everything but the OWN youngest copies of this wave: stage 0
+    else wait_stages<SPT>(0);
     workgroup_barrier();
     row_sums(ring);
-    wait_stages<SPT>(0);
+    if constexpr (DMA) wait_stages<SPT>(0);
     workgroup_barrier();
-    if (issued < ns) issue_next();
+    if constexpr (DMA)
+        if (issued < ns) issue_next();
     // ROPE: Q (, Q_dot) of a landed stage, one item per thread of the upper half of the workgroup
     auto rotate_stage = [&](elem_t* slot, int row0) {
         if constexpr (ROPE) {
@@ -440,13 +478,13 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
     // dK, dV (, dK_dot, dV_dot) of this wave's sixteen keys through its staging tile
     auto key_gradients = [&](elem_t* stage_tile) {
         const int row0 = wave * 16;
-        store_tile16<T, HD, ROPE>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane, &p.rope);
+        store_rows16<T, HD, IO, ROPE>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane, &p.rope);
         if constexpr (HAS_G)
-            store_tile16<T, HD, ROPE>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane,
+            store_rows16<T, HD, IO, ROPE>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane,
                                       &p.rope);
-        store_tile16<T, HD>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
         if constexpr (HAS_G)
-            store_tile16<T, HD>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
+            store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
     };
     // One workgroup barrier per stage.  Iteration i: step 2 of stage i (tiles into bounce buffer i % 2), the
     // barrier, then the row sums of stage i+1, step 3 of stage i (bounce buffer i % 2 -> staging buffer i % 2)
@@ -470,7 +508,7 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
     };
     workgroup_barrier();  // every wave has read V, V_dot, whose memory the bounce tiles take over
     for (int i = 0; i < ns; ++i) {
-        if (issued < ns && issued < i + R) issue_next();  // into the slot of stage issued - R <= i - 1
+        if (DMA && issued < ns && issued < i + R) issue_next();  // into the slot of stage issued - R <= i - 1
         elem_t* slot = ring + (i % R) * SM::slot;
         elem_t* bounce_i = bounce0 + (i & 1) * BBUF;
         if (i >= 1) await_announced(SIG * (unsigned)i);
@@ -484,8 +522,11 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
             static_assert(R >= 3 && SM::slot >= 4 * StoreStage16<HD>::elems, "two spare slots hold the staging tiles");
             key_gradients(ring + ((i + 1 + (wave >> 2)) % R) * SM::slot + (wave & 3) * StoreStage16<HD>::elems);
         }
-        if (i + 1 < ns) wait_stages<SPT>(issued - 2 - i);  // stage i+1 has landed (this wave's part)
+        // stage i+1 has landed (this wave's part; staged copies: its statistics, the only part that came by LDS-DMA)
+        if (i + 1 < ns) wait_stages<SPT>(DMA ? issued - 2 - i : 0);
         workgroup_barrier();  // bounce buffer i % 2 is complete; stage i+1 is in LDS; stage i's slot is free
+        if constexpr (!DMA)
+            if (issued < ns) issue_next();  // stage i+2, into the slot of stage i-1
         if (i >= 1) flush_rows((i - 1) * kStageRows, qstage + ((i - 1) & 1) * SM::qstage_one);
         if (i + 1 < ns) {
             row_sums(ring + ((i + 1) % R) * SM::slot);
@@ -493,8 +534,9 @@ __global__ __launch_bounds__(kThreads16, HAS_G ? 2 : 4) void bwd_fused16_kernel(
             if (ROPE || tid < 256) announce();
         }
         elem_t* qstage_i = qstage + (i & 1) * SM::qstage_one;
-        if (key_slabs == 4) row_outputs(bounce_i, qstage_i, std::true_type{});
-        else row_outputs(bounce_i, qstage_i, std::false_type{});
+        if (key_slabs == 4) row_outputs(bounce_i, qstage_i, i * kStageRows, std::true_type{});
+        else row_outputs(bounce_i, qstage_i, i * kStageRows, std::false_type{});
+        if constexpr (!DMA) plan.commit();
     }
     workgroup_barrier();  // the last stage's dQ (, dQ_dot) tiles are in their staging tile; the ring is free
     flush_rows((ns - 1) * kStageRows, qstage + ((ns - 1) & 1) * SM::qstage_one);

@@ -3,7 +3,7 @@
 
 namespace sjvp {
 
-int bwd_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+int bwd_pair_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
     return bwd_pair16<Bf16, kIoF32>(p, BH, has_do, has_g, parts, stream);
 }
 

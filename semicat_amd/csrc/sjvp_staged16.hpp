@@ -10,7 +10,7 @@
 //
 // Measured, forward + backward (one element at a time through one stage of LDS under 32-wide tiles before):
 //   bf16 B=8 H=8 L=300 D=36 158 -> 62 us (the aligned D = 40: 54), B=64 H=12 L=128 D=20 174 -> 58,
-//   B=8 H=16 L=512 D=100 1579 -> 325; fp32 rows B=64 H=12 L=128 D=64 248 -> 158 us, B=128 H=12 L=256 1637 -> 745.
+//   B=8 H=16 L=512 D=100 1579 -> 325; fp32 rows B=64 H=12 L=128 D=64 248 -> 139 us, B=128 H=12 L=256 1637 -> 745.
 // The shorter life of a stage in registers (one ahead instead of a ring of two or three) costs 15 % against the
 // LDS-DMA form; what is left is bound as that one is.
 #pragma once
@@ -76,8 +76,8 @@ __device__ __forceinline__ void staged_b_operands16(u32x4* out, const elem_t* ro
 }
 
 // CopyPlan (sjvp_w16.hpp) through registers: issue() requests the next window, commit() writes it to the region it
-// was issued for.
-template <typename T, int HD, int NS, int NT, int IO>
+// was issued for, slab j of the window PITCH elements behind slab j - 1.
+template <typename T, int HD, int NS, int NT, int IO, int PITCH = Slab<HD>::elems>
 struct StagedPlan {
     static constexpr int chunks = Slab<HD>::chunks;
     static constexpr int total = NS * chunks;
@@ -86,15 +86,16 @@ struct StagedPlan {
     const elem_t* src[N];  // first column this thread reads of its row in the next window
     int64_t adv[N];        // elements from one window to the next (wave-uniform)
     int row[N];
-    int pos8;              // element offset of this thread's first chunk position; the others follow NT positions apart
+    int pos8;              // element offset of this thread's first chunk position
     int shift;             // of every chunk: a thread's positions are the same columns of successive slabs or rows
     bool shifted;          // wave-uniform: D does not fill the slabs
     elem_t* region;
     bool pending;
     Raw8<IO> raw[N];
 
-    __device__ __forceinline__ void init(int tid, int D, Src t0, Src t1, Src t2 = Src{nullptr, 0}, Src t3 = Src{nullptr, 0}) {
-        static_assert(NS <= 4, "at most four tensors per copy");
+    __device__ __forceinline__ void init(int tid, int D, Src t0, Src t1, Src t2 = Src{nullptr, 0}, Src t3 = Src{nullptr, 0},
+                                         Src t4 = Src{nullptr, 0}, Src t5 = Src{nullptr, 0}) {
+        static_assert(NS <= 6, "at most six tensors per copy");
         constexpr int CH = HD / 8;
         const int q0 = tid % chunks;
         const int c8 = 8 * ((q0 % CH) ^ swz<HD>(q0 / CH));
@@ -103,13 +104,20 @@ struct StagedPlan {
         const int col = (IO == kIoF32 ? 2 : 1) * piece_col(c8, D);
         shift = piece_shift(c8, D);
         shifted = D != HD;
-        pos8 = 8 * tid;
+        pos8 = j0 * PITCH + 8 * q0;
         pending = false;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const int j = NT >= chunks ? j0 + (NT / chunks) * i : i / (chunks / NT);
             const int r = NT >= chunks ? q0 / CH : q0 / CH + (NT / CH) * (i % (chunks / NT));
-            const Src s = j <= 0 ? t0 : j == 1 ? t1 : j == 2 ? t2 : t3;
+            // the tensor of slab j: one of SPI neighbours, chosen by the (wave-uniform) slab of position 0
+            constexpr int SPI = NT >= chunks ? NT / chunks : 1;
+            const Src ts[6] = {t0, t1, t2, t3, t4, t5};
+            const int first = NT >= chunks ? SPI * i : i / (chunks / NT);
+            Src s = ts[first < NS ? first : 0];
+#pragma unroll
+            for (int k = 1; k < SPI; ++k)
+                if (first + k < NS && j0 == k) s = ts[first + k < NS ? first + k : 0];
             row[i] = j < NS ? r : 1 << 30;  // a position beyond the last slab has no row
             src[i] = s.ptr + (int64_t)r * s.sl + col;
             adv[i] = 32 * s.sl;
@@ -140,26 +148,50 @@ struct StagedPlan {
             if (total % NT != 0 && row[i] >= kStageRows) continue;
             u32x4 v = raw[i].template get<T>();
             if (shifted) v = shift_down(v, shift);
-            *reinterpret_cast<u32x4*>(region + pos8 + 8 * NT * i) = v;
+            constexpr int PPS = NT >= chunks ? 1 : chunks / NT;    // positions per slab
+            constexpr int SPI = NT >= chunks ? NT / chunks : 1;    // slabs from one position to the next
+            *reinterpret_cast<u32x4*>(region + pos8 + (i / PPS) * SPI * PITCH + (i % PPS) * 8 * NT) = v;
         }
     }
 };
+
+// One 16-byte piece (columns 8c ..) of a 16-bit row of any alignment, masked at D.
+__device__ __forceinline__ void store_piece(elem_t* dst, u32x4 v, int d, int D) {
+    if (d + 8 <= D) {
+        __builtin_memcpy(dst, &v, sizeof(v));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 7; ++e)
+            if (d + e < D) dst[e] = (elem_t)(v[e >> 1] >> (16 * (e & 1)));
+    }
+}
+// Four consecutive fp32 elements at columns d .., masked at D.
+__device__ __forceinline__ void store_f32x4(elem_t* row, f32x4 v, int d, int D) {
+    float* dst = reinterpret_cast<float*>(row) + d;
+    if (d + 4 <= D) {
+        __builtin_memcpy(dst, &v, sizeof(v));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (d + e < D) dst[e] = v[e];
+    }
+}
 
 // One spelling for both kinds of plan.
 template <int HD, int NS, int NT, typename... S>
 __device__ __forceinline__ void init_plan(CopyPlan<HD, NS, 1, NT>& plan, int tid, int D, const void* sink, S... srcs) {
     plan.init(tid, 0, D, sink, srcs...);
 }
-template <typename T, int HD, int NS, int NT, int IO, typename... S>
-__device__ __forceinline__ void init_plan(StagedPlan<T, HD, NS, NT, IO>& plan, int tid, int D, const void*, S... srcs) {
+template <typename T, int HD, int NS, int NT, int IO, int P, typename... S>
+__device__ __forceinline__ void init_plan(StagedPlan<T, HD, NS, NT, IO, P>& plan, int tid, int D, const void*, S... srcs) {
     plan.init(tid, D, srcs...);
 }
 template <int HD, int NS, int NT>
 __device__ __forceinline__ void issue_plan(CopyPlan<HD, NS, 1, NT>& plan, elem_t* slot, int rows_left, bool whole) {
     plan.issue(slot, rows_left, whole);
 }
-template <typename T, int HD, int NS, int NT, int IO>
-__device__ __forceinline__ void issue_plan(StagedPlan<T, HD, NS, NT, IO>& plan, elem_t* slot, int rows_left, bool) {
+template <typename T, int HD, int NS, int NT, int IO, int P>
+__device__ __forceinline__ void issue_plan(StagedPlan<T, HD, NS, NT, IO, P>& plan, elem_t* slot, int rows_left, bool) {
     plan.issue(slot, rows_left);
 }
 
@@ -171,19 +203,9 @@ __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, i
     const int n = lane & 15, g = lane >> 4;
     if constexpr (IO == kIoF32) {
         if (row0 + n >= L) return;
-        float* row = reinterpret_cast<float*>(gp + (int64_t)(row0 + n) * sl);
+        elem_t* row = gp + (int64_t)(row0 + n) * sl;
 #pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt) {
-            const int d = 16 * dt + 4 * g;
-            const f32x4 v = acc[dt] * mul;
-            if (d + 4 <= D) {
-                __builtin_memcpy(row + d, &v, sizeof(v));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 3; ++e)
-                    if (d + e < D) row[d + e] = v[e];
-            }
-        }
+        for (int dt = 0; dt < HD / 16; ++dt) store_f32x4(row, acc[dt] * mul, 16 * dt + 4 * g, D);
     } else {
         constexpr int P = StoreStage16<HD>::pitch;
 #pragma unroll
@@ -199,24 +221,17 @@ __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, i
             const int c = lane % CH;
             if ((RPI <= 16 || r < 16) && row0 + r < L && 8 * c < D) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(stage + r * P + 8 * c);
-                elem_t* dst = gp + (int64_t)(row0 + r) * sl + 8 * c;
-                if (8 * c + 8 <= D) {
-                    __builtin_memcpy(dst, &v, sizeof(v));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 7; ++e)
-                        if (8 * c + e < D) dst[e] = (elem_t)(v[e >> 1] >> (16 * (e & 1)));
-                }
+                store_piece(gp + (int64_t)(row0 + r) * sl + 8 * c, v, 8 * c, D);
             }
         }
     }
 }
 
 // The wave's 16 rows of an output tensor, whatever its storage.
-template <typename T, int HD, int IO>
+template <typename T, int HD, int IO, bool ROPE = false>
 __device__ __forceinline__ void store_rows16(elem_t* stage, elem_t* gp, int64_t sl, int row0, int L, int D,
-                                             const f32x4* acc, float mul, int lane) {
-    if constexpr (IO == kIoDma) store_tile16<T, HD>(stage, gp, sl, row0, L, D, acc, mul, lane);
+                                             const f32x4* acc, float mul, int lane, const RopeTables* rt = nullptr) {
+    if constexpr (IO == kIoDma) store_tile16<T, HD, ROPE>(stage, gp, sl, row0, L, D, acc, mul, lane, rt);
     else staged_store_tile16<T, HD, IO>(stage, gp, sl, row0, L, D, acc, mul, lane);
 }
 

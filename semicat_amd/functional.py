@@ -35,23 +35,28 @@ import torch.autograd.forward_ad as fwAD
 from torch import Tensor
 
 from . import kernels
+from ._lib import SJVP_BWD_ALL, SJVP_BWD_FP32_SINGLE
 
 
 AUTOGRAD_WIRING = "fused"  # or "reference"
 # How safe_sdpa_jvp serves float32 callers with bf16 arithmetic (functional.py:318-332):
-#   "torch"   (default) torch casts around the 16-bit LDS-DMA kernels, as the reference does;
-#   "library" the library's multi-tensor cast launches around them (half the launches, no kernel that is
-#             not the library's own; the same speed on large problems, more host time on small ones);
-#   "folded"  the float32 tensors handed to the kernels, which round as they load and store float32
-#             (SJVP_FP32_BF16: register-staged kernels, no cast at all, but 1.1 to 2.4 times slower).
-# Measured on an MI355X, forward + backward in microseconds, 16-bit callers / torch / library / folded:
-#   B=64 H=12 L=128 D=64: 70 / 218 / 207 / 244;  B=128 H=12 L=256: 502 / 936 / 934 / 1609;
-#   B=8 H=16 L=1024: 514 / 687 / 668 / 1614;  B=2 H=4 L=256 (host-bound): 41 / 76 / 212 / 86.
+#   "torch"   (default) the reference's casts around the op: on a GPU they are folded into the kernels, which
+#             round the float32 tensors as they load them and store float32 (SJVP_FP32_BF16, with the launches that
+#             16-bit tensors of the shape would take); elsewhere they are torch casts;
+#   "folded"  the float32 tensors handed to the launchers wherever they live;
+#   "library" the library's multi-tensor cast launches around the 16-bit kernels.
+# Measured on an MI355X, launches of forward + backward in microseconds, 16-bit callers / folded / torch casts:
+#   B=64 H=12 L=128 D=64: 66 / 139 / 214;  B=128 H=12 L=256: 443 / 745 / 889;  B=8 H=16 L=1024: 438 / 590 / 618.
 FP32_CALLERS = "torch"
 
 
 def _has_tangent(t: Tensor) -> bool:
     return fwAD.unpack_dual(t).tangent is not None
+
+
+def _backward_launches(q: Tensor, arith: Optional[str]) -> dict:
+    """Float32 tensors with folded casts take the launches that 16-bit tensors of the shape would take."""
+    return {"parts": SJVP_BWD_ALL | SJVP_BWD_FP32_SINGLE} if arith == "bf16" and q.is_cuda else {}
 
 
 class SDPAJVPFlashBackwardFunction(torch.autograd.Function):
@@ -75,7 +80,7 @@ class SDPABackwardFunction(torch.autograd.Function):
     def forward(ctx, q, k, v, o, do, M, arith=None, cos=None, sin=None):
         dq, dk, dv, _, _, _ = kernels.attention_jvp_backward(
             q, k, v, None, None, None, o, None, M, None, dO=do, dTO=None, arithmetic=arith,
-            rope=None if cos is None else (cos, sin))
+            rope=None if cos is None else (cos, sin), **_backward_launches(q, arith))
         return dq, dk, dv
 
     @staticmethod
@@ -200,7 +205,8 @@ class SDPAJVPFusedBackwardFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, t_q, t_k, t_v, y, t_y, M, MU, d_y, d_t_y, arith=None, cos=None, sin=None):
         return kernels.attention_jvp_backward(q, k, v, t_q, t_k, t_v, y, t_y, M, MU, dO=d_y, dTO=d_t_y,
-                                              arithmetic=arith, rope=None if cos is None else (cos, sin))
+                                              arithmetic=arith, rope=None if cos is None else (cos, sin),
+                                              **_backward_launches(q, arith))
 
     @staticmethod
     def backward(ctx, *grads):
@@ -254,10 +260,9 @@ def _sdpa(q: Tensor, k: Tensor, v: Tensor, seq_major: bool, arith: Optional[str]
 
 def safe_sdpa_jvp(q: Tensor, k: Tensor, v: Tensor, precise: bool = False) -> Tensor:
     """``[B,S,H,D]`` wrapper with the reference's dtype policy (functional.py:310-332): inputs that
-    are neither bf16 nor fp16 are computed in bfloat16 and the result comes back in their dtype, cast
-    with torch as in the reference; for float32 inputs ``FP32_CALLERS`` selects two other routes (the
-    library's own cast launches, or float32 tensors handed to the kernels as they are), both measured
-    slower or equal (figures beside ``FP32_CALLERS``).  ``precise=True`` runs float32 inputs in the
+    are neither bf16 nor fp16 are computed in bfloat16 and the result comes back in their dtype.  On a GPU the
+    casts of float32 tensors are folded into the kernels; ``FP32_CALLERS`` selects other routes (figures
+    beside it).  ``precise=True`` runs float32 inputs in the
     library's fp32 mode instead (fp32 arithmetic throughout, about 1e-6 against fp64, much slower
     than the MFMA kernels)."""
     orig_dtype = q.dtype
@@ -269,7 +274,7 @@ def safe_sdpa_jvp(q: Tensor, k: Tensor, v: Tensor, precise: bool = False) -> Ten
         q, k, v = cast_tensors((q, k, v), torch.bfloat16)
         y = _sdpa(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), seq_major=True).transpose(1, 2)
         return cast_tensors(y, orig_dtype)
-    if fp32_bf16 and FP32_CALLERS == "folded":
+    if fp32_bf16 and (FP32_CALLERS == "folded" or (FP32_CALLERS == "torch" and q.is_cuda)):
         arith = "bf16"
     elif orig_dtype != torch.bfloat16 and orig_dtype != torch.float16 and not (precise and orig_dtype == torch.float32):
         q = q.to(torch.bfloat16)

@@ -24,7 +24,7 @@ def _place(t, offset):
 @pytest.mark.parametrize("Lq,Lk,D,offset,mode", [
     (33, 64, 17, 0, "both"), (65, 31, 22, 0, "both"), (32, 160, 31, 0, "dTO"), (64, 33, 33, 0, "both"),
     (130, 65, 36, 0, "both"), (31, 97, 45, 0, "dO"), (97, 96, 54, 0, "both"), (200, 129, 63, 0, "dTO"),
-    (40, 70, 64, 3, "both"), (70, 40, 32, 1, "dO"), (66, 34, 65, 0, "both"), (35, 100, 91, 0, "dTO"),
+    (128, 128, 64, 0, "both"), (160, 100, 32, 0, "both"), (20, 17, 64, 0, "dTO"), (40, 70, 64, 3, "both"), (70, 40, 32, 1, "dO"), (66, 34, 65, 0, "both"), (35, 100, 91, 0, "dTO"),
     (90, 61, 110, 0, "both"), (33, 65, 127, 0, "both"), (64, 32, 128, 1, "dO")])
 def test_staged_rows(store, Lq, Lk, D, offset, mode):
     from semicat_amd import kernels as K
@@ -54,5 +54,19 @@ def test_staged_rows(store, Lq, Lk, D, offset, mode):
         end = offset + v.numel()
         assert (buf[:offset].float() == torch.tensor(CANARY).to(dt).float().item()).all()
         assert (buf[end:].float() == torch.tensor(CANARY).to(dt).float().item()).all()
+    if store == "fp32" and Lk <= 128 and D <= 64:  # the single launch on fp32 rows
+        from semicat_amd import _lib
+        for v, _ in g:
+            v.zero_()
+        K.attention_jvp_backward(d["q"], d["k"], d["v"], *(tan if has_g else (None,) * 3), o, to if has_g else None, lse,
+                                 mu if has_g else None, dO=d["dO"] if "dO" in cot else None,
+                                 dTO=d["dTO"] if has_g else None, grads=tuple(v for v, _ in g), arithmetic=arith,
+                                 parts=_lib.SJVP_BWD_ALL | _lib.SJVP_BWD_FP32_SINGLE)
+        for n, (v, buf) in zip(GRADS, g):
+            if n in ref and (has_g or not n.startswith("dt")):
+                err = orc.rel_frobenius(v.cpu(), ref[n])
+                assert err <= TOL, ("single launch", n, err)
+            end = offset + v.numel()
+            assert (buf[:offset] == CANARY).all() and (buf[end:] == CANARY).all()
     o2, _ = K.attention_forward(d["q"], d["k"], d["v"], arithmetic=arith)
     assert orc.rel_frobenius(o2.cpu(), ref["O"]) <= TOL
