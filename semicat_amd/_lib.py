@@ -3,6 +3,8 @@ missing or a call fails, an exception is raised."""
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 
 from . import build as _build
@@ -44,6 +46,7 @@ EXPORTS = ("sjvp_fwd", "sjvp_bwd", "sjvp_bwd_parts", "sjvp_bwd_noalloc", "sjvp_f
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 class SjvpError(RuntimeError):
@@ -55,7 +58,7 @@ class SjvpError(RuntimeError):
 def load() -> ctypes.CDLL:
     """Load the in-tree shared library; it is built first when it does not exist or is older than one
     of its sources (a stale binary is never loaded silently)."""
-    global _lib
+    global _lib, _host
     if _lib is not None:
         return _lib
     with _lock:
@@ -97,8 +100,30 @@ def load() -> ctypes.CDLL:
             lib.sjvp_build_id.restype = ctypes.c_char_p
             if lib.sjvp_build_id().decode() != "SJVP_BUILD_ID=" + _build.source_id():
                 raise RuntimeError(f"{path} was built from other sources than the ones in this tree")
+            _host = _load_host(lib)
             _lib = lib
     return _lib
+
+
+def _load_host(lib: ctypes.CDLL):
+    """The host extension (csrc/sjvp_host.cpp), bound to the entry points of the loaded library."""
+    import torch  # noqa: F401  (the extension links against its libraries)
+    path = _build.HOST_PATH
+    spec = importlib.util.spec_from_file_location(
+        "_sjvp_host", path, loader=importlib.machinery.ExtensionFileLoader("_sjvp_host", path))
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    if host.build_id != "SJVP_BUILD_ID=" + _build.source_id():
+        raise RuntimeError(f"{path} was built from other sources than the ones in this tree")
+    host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in
+                (lib.sjvp_fwd, lib.sjvp_fwd_rotary, lib.sjvp_bwd_parts, lib.sjvp_bwd_rotary,
+                 lib.sjvp_bwd_workspace_bytes)))
+    return host
+
+
+def host():
+    """The host extension; loads the library first."""
+    return _host if _host is not None else (load() and _host)
 
 
 def strerror(status: int) -> str:

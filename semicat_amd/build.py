@@ -1,7 +1,8 @@
 """Builds libsjvp.so (the gfx950 attention-JVP kernels + C ABI) in-tree with hipcc.
 
 The kernels are instantiated in several translation units (one per kernel family and element type)
-that are compiled in parallel and linked into one shared library."""
+that are compiled in parallel and linked into one shared library.  Beside it goes a small CPython extension,
+the host side of the entry points (csrc/sjvp_host.cpp)."""
 from __future__ import annotations
 
 import hashlib
@@ -10,6 +11,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -20,6 +22,9 @@ LIB_PATH = os.path.join(PKG_DIR, "libsjvp.so")
 UNITS = [(name, ("Bf16", "Fp16") if name.startswith("sjvp_tu_") else (None,))
          for name in sorted(os.listdir(CSRC)) if name.endswith(".hip")]
 SOURCES = [os.path.join(CSRC, name) for name, _ in UNITS]
+# The host side of the entry points: a CPython extension against torch's headers, no device code.
+HOST_SOURCE = os.path.join(CSRC, "sjvp_host.cpp")
+HOST_PATH = os.path.join(PKG_DIR, "_sjvp_host.so")
 HEADERS = sorted(os.path.join(CSRC, n) for n in os.listdir(CSRC) if n.endswith(".hpp")) + [
     os.path.join(os.path.dirname(PKG_DIR), "include", "sjvp.h")]
 
@@ -46,7 +51,7 @@ def hipcc_path() -> str:
 def source_id() -> str:
     """Identifier of the sources the library is built from: a hash of their contents and the flags."""
     h = hashlib.sha256((" ".join(HIPCC_FLAGS) + repr(sorted(UNIT_FLAGS.items()))).encode())
-    for path in SOURCES + HEADERS:
+    for path in SOURCES + HEADERS + [HOST_SOURCE]:
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
             h.update(f.read())
@@ -68,7 +73,20 @@ def _run(cmd, verbose):
         print(" ".join(cmd), file=sys.stderr)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+        raise RuntimeError("the compiler failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+
+
+def host_command(build_id: str) -> list[str]:
+    """The command that builds the host extension (host code only: g++)."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    return [shutil.which("g++") or "c++", "-O2", "-std=c++20", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", build_id,
+            "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(root, "include"),
+            "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + os.path.join(rocm, "include"),
+            HOST_SOURCE, "-o", HOST_PATH + ".tmp", "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu",
+            "-lc10_hip", "-lc10"]
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> str:
@@ -84,18 +102,20 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
             cmds.append([hipcc, *HIPCC_FLAGS, *UNIT_FLAGS.get(name, []), *define, "-c", os.path.join(CSRC, name),
                          "-o", obj])
             objs.append(obj)
+    cmds.insert(0, host_command(build_id))
     jobs = jobs or min(len(cmds), os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH + ".tmp", *objs], verbose)
     os.replace(LIB_PATH + ".tmp", LIB_PATH)
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     return LIB_PATH
 
 
 def is_stale() -> bool:
-    """True when no library is built or it was built from other sources than the ones in the tree
-    (compared by content, so copying or checking out the tree does not matter)."""
-    return built_id() != source_id()
+    """True when no library or no host extension is built or one was built from other sources than the ones in
+    the tree (compared by content, so copying or checking out the tree does not matter)."""
+    return any(built_id(path) != source_id() for path in (LIB_PATH, HOST_PATH))
 
 
 if __name__ == "__main__":

@@ -150,6 +150,21 @@ def _require_gpu(q: torch.Tensor, arithmetic: Optional[str] = None) -> int:
     return _DTYPES[q.dtype]
 
 
+def _on_gpu(q) -> bool:
+    """Whether the host extension (csrc/sjvp_host.cpp) is asked first.  It serves the calls that pass every check of
+    the general forms below, with the same results, and answers None to all others, which the general form then
+    refuses or takes.  Forward + backward of a 2x2x16x16x32 problem: 55 us through Python and ctypes alone,
+    15 us with it (toy problem in a loop, kernels included)."""
+    return isinstance(q, torch.Tensor) and q.is_cuda
+
+
+def _host_result(res):
+    """Results of the host extension, or its C ABI status as an error."""
+    if type(res) is int:
+        _lib.check(res)
+    return res
+
+
 def _stat(buf: Optional[torch.Tensor], name: str, B: int, H: int, Lr: int, device) -> torch.Tensor:
     if buf is None:
         return torch.empty((B, H, Lr), device=device, dtype=torch.float32)
@@ -168,6 +183,11 @@ def attention_jvp_forward(q, k, v, tq, tk, tv, scale: Optional[float] = None, o=
     ``arithmetic="bf16"`` on float32 tensors: see :func:`_require_gpu`.  ``rope=(cos, sin)``: q, k, tq,
     tk are given unrotated and the kernel applies the rotary embedding as it loads them
     (``sjvp_fwd_rotary``; see :func:`rotary_fusable` for the shapes this serves)."""
+    if not _plan and _on_gpu(q):
+        cos, sin = (None, None) if rope is None else rope
+        res = _lib.host().forward(q, k, v, tq, tk, tv, o, to, lse, mu, li, with_li, scale, arithmetic, cos, sin)
+        if res is not None:
+            return _host_result(res)
     dtype_tag = _require_gpu(q, arithmetic)
     B, H, Lq, D = q.shape
     Lk = k.shape[-2]
@@ -212,6 +232,12 @@ def attention_forward(q, k, v, scale: Optional[float] = None, o=None, lse=None,
                       arithmetic: Optional[str] = None, rope=None) -> Tuple[torch.Tensor, torch.Tensor]:
     """Primal-only forward (tangent contractions compiled out): returns (o, lse).  ``rope``: as in
     :func:`attention_jvp_forward`."""
+    if _on_gpu(q):
+        cos, sin = (None, None) if rope is None else rope
+        res = _lib.host().forward(q, k, v, None, None, None, o, None, lse, None, None, None, scale, arithmetic, cos, sin)
+        if res is not None:
+            o, _, lse, _, _ = _host_result(res)
+            return o, lse
     dtype_tag = _require_gpu(q, arithmetic)
     B, H, Lq, D = q.shape
     Lk = k.shape[-2]
@@ -256,6 +282,12 @@ def attention_jvp_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dO=None, dTO=Non
     serves up to ``SJVP_NOALLOC_MAX_ROWS`` statistic rows and calls overlapping on one GPU race.
     ``rope=(cos, sin)``: q, k, tq, tk are the unrotated tensors the forward was given with the same
     ``rope``; the gradients returned are those of the unrotated tensors (``sjvp_bwd_rotary``)."""
+    if not _plan and not static_scratch and _on_gpu(q):
+        cos, sin = (None, None) if rope is None else rope
+        res = _lib.host().backward(q, k, v, tq, tk, tv, o, to, lse, mu, dO, dTO, scale, grads, workspace, parts,
+                                   arithmetic, cos, sin)
+        if res is not None:
+            return _host_result(res)
     dtype_tag = _require_gpu(q, arithmetic)
     if dO is None and dTO is None:
         raise ValueError("attention_jvp_backward needs a cotangent on o, on to, or on both")
