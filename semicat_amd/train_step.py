@@ -79,7 +79,11 @@ def lag_self_distillation_loss(net: nn.Module, x0: Tensor, x1: Tensor, t: Option
     xst, dv = torch.func.jvp(lambda end: flow_map(net, xs, s, end, jvp_attention=True),
                              (t,), (torch.ones_like(t),))
     xst = xst.detach()
-    with torch.no_grad():
+    # Casts of the weights made without gradients must not enter the cache of the caller's autocast context: a network
+    # call behind this one would take them from there and lose its weights' gradients.
+    kind = xst.device.type
+    with torch.no_grad(), torch.autocast(kind, dtype=torch.get_autocast_dtype(kind),
+                                         enabled=torch.is_autocast_enabled(kind), cache_enabled=False):
         target = net(xst, t, t).softmax(dim=-1)
     return ((1.0 - _per_sample(t, xst)) * dv - target + xst).pow(2).sum(dim=-1).mean()
 
