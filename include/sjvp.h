@@ -222,6 +222,43 @@ int sjvp_rope(int n, const void* const* x, void* const* y, const int64_t* stride
               const float* cos, const float* sin, int64_t cs_stride, int B, int H, int L, int D,
               int rot_dim, int in_dtype, int out_dtype, int inverse, void* stream);
 
+/*
+ * The element-wise parts of an adaLN transformer block (semicat/net/duo.py:134-166) with forward-mode tangents and
+ * the reverse mode of both, bf16 storage and fp32 arithmetic:
+ *   y = a gate + x                          (a, gate NULL: skipped, the norm reads x)
+ *   h = LayerNorm(y; w, b) (1 + scale) + shift   (w NULL: skipped)
+ * x, a, y, h and what belongs to them: contiguous [B,S,W]; gate, scale, shift and their tangents: [B,W] with the row
+ * strides mod_stride = (gate, tgate, scale, tscale, shift, tshift) in elements; 4 <= W <= 1024, W and the strides
+ * multiples of 4, bf16 pointers 8-byte and w, b (fp32 [W]) 16-byte aligned; gradients of [B,W] inputs contiguous.
+ * A tangent or cotangent that is NULL is zero; a gradient that is NULL is not stored.  sjvp_adaln_bwd() takes the inputs again,
+ * with both a and w also y (and ty), and a workspace of sjvp_adaln_workspace_floats() floats (0: not served).
+ * No counterpart in the reference, which uses separate PyTorch operations.
+ */
+typedef struct sjvp_adaln {
+    const void *x, *tx, *a, *ta;
+    const void *gate, *tgate, *scale, *tscale, *shift, *tshift;
+    int64_t mod_stride[6];
+    const float *w, *b;
+    void *y, *ty, *h, *th;
+    const void *dy, *dty, *dh, *dth;
+    void *dx, *dtx, *da, *dta;
+    void *dgate, *dtgate, *dscale, *dtscale, *dshift, *dtshift;
+    float *dw, *db, *workspace;
+    int B, S, W;
+    float eps;
+} sjvp_adaln;
+size_t sjvp_adaln_workspace_floats(const sjvp_adaln* t);
+int sjvp_adaln_fwd(const sjvp_adaln* t, int jvp, void* stream);
+int sjvp_adaln_bwd(const sjvp_adaln* t, int jvp, void* stream);
+
+/*
+ * tanh GELU g of n bf16 elements (n a multiple of 8, pointers 16-byte aligned).  reverse = 0: y = g(u),
+ * ty = g'(u) tu; reverse = 1: y = g'(u) dy + g''(u) tu dty, ty = g'(u) dty.  NULL inputs other than u are zero,
+ * NULL outputs are not stored.
+ */
+int sjvp_gelu(const void* u, const void* tu, const void* dy, const void* dty, void* y, void* ty, int64_t n,
+              int reverse, void* stream);
+
 /* Static, NUL-terminated description of a status code. */
 const char* sjvp_strerror(int status);
 

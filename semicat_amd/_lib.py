@@ -42,7 +42,19 @@ SJVP_REPAIR_AUTO = 1
 SJVP_REPAIR_ALWAYS = 2
 
 EXPORTS = ("sjvp_fwd", "sjvp_bwd", "sjvp_bwd_parts", "sjvp_bwd_noalloc", "sjvp_fwd_rotary", "sjvp_bwd_rotary", "sjvp_bwd_workspace_bytes", "sjvp_rope",
+           "sjvp_adaln_fwd", "sjvp_adaln_bwd", "sjvp_adaln_workspace_floats", "sjvp_gelu",
            "sjvp_set_row_sum_repair", "sjvp_strerror", "sjvp_version", "sjvp_build_id")
+
+
+class AdaLn(ctypes.Structure):
+    """``struct sjvp_adaln``."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "tx", "a", "ta", "gate", "tgate", "scale", "tscale", "shift", "tshift")]
+                + [("mod_stride", ctypes.c_int64 * 6)]
+                + [(n, ctypes.c_void_p) for n in ("w", "b", "y", "ty", "h", "th", "dy", "dty", "dh", "dth", "dx", "dtx",
+                                                  "da", "dta", "dgate", "dtgate", "dscale", "dtscale", "dshift",
+                                                  "dtshift", "dw", "db", "workspace")]
+                + [("B", ctypes.c_int), ("S", ctypes.c_int), ("W", ctypes.c_int), ("eps", ctypes.c_float)])
+
 
 _lock = threading.Lock()
 _lib = None
@@ -90,6 +102,13 @@ def load() -> ctypes.CDLL:
             vpp = ctypes.POINTER(ctypes.c_void_p)
             lib.sjvp_rope.argtypes = [i, vpp, vpp, i64p, vp, vp, ctypes.c_int64] + [i] * 8 + [vp]
             lib.sjvp_rope.restype = i
+            ada = ctypes.POINTER(AdaLn)
+            lib.sjvp_adaln_fwd.argtypes = lib.sjvp_adaln_bwd.argtypes = [ada, i, vp]
+            lib.sjvp_adaln_fwd.restype = lib.sjvp_adaln_bwd.restype = i
+            lib.sjvp_adaln_workspace_floats.argtypes = [ada]
+            lib.sjvp_adaln_workspace_floats.restype = ctypes.c_size_t
+            lib.sjvp_gelu.argtypes = [vp] * 6 + [ctypes.c_int64, i, vp]
+            lib.sjvp_gelu.restype = i
             lib.sjvp_set_row_sum_repair.argtypes = [i]
             lib.sjvp_set_row_sum_repair.restype = i
             lib.sjvp_strerror.argtypes = [i]

@@ -1,0 +1,228 @@
+"""The element-wise parts of the DiT's blocks as single launches (csrc/sjvp_adaln.hip): LayerNorm with adaLN
+modulation, the gated residual in front of it, and the MLP's tanh GELU, each with forward-mode tangents and the
+reverse mode of both.
+
+As separate PyTorch operations these are what a training step spends its launches on: forward-mode LayerNorm
+alone is some twenty kernels and its reverse twice as many, and the step issues thousands of them, each
+shorter than the time the host takes to issue it.
+
+The functions serve what a step under bf16 autocast on a GPU has in hand: bf16 activations with fp32 LayerNorm
+parameters, outside every transform or inside exactly one ``torch.func.jvp``.  For anything else (other types, other
+transforms, tracing, dual numbers, tensor subclasses, modules with hooks) they return None and the caller runs its
+PyTorch operations.  To torch.compile they are opaque, like the attention op: a compiled network computes what the
+unwrapped one does.  Results are rounded where the PyTorch operations round (the residual stream) or where autocast would
+round behind them (the input of the next linear layer)."""
+from __future__ import annotations
+
+import ctypes
+from typing import Optional
+
+import torch
+import torch.autograd.forward_ad as fwAD
+from torch import Tensor, nn
+from torch._C import _functorch
+from torch.autograd.function import once_differentiable
+from torch.nn.modules import module as _module
+
+from . import _lib
+from .functional import _below_jvp, _dual_above
+
+_MOD = ("gate", "tgate", "scale", "tscale", "shift", "tshift")
+
+
+def _aligned(t: Optional[Tensor], bytes_: int = 16) -> Optional[Tensor]:
+    """The tensor as contiguous memory that starts on a boundary of ``bytes_``."""
+    if t is None:
+        return None
+    t = t.contiguous()
+    return t if t.data_ptr() % bytes_ == 0 else t.clone()
+
+
+def _mod_rows(t: Optional[Tensor]) -> Optional[Tensor]:
+    """``[B,1,W]`` with rows of unit stride that start on 8-byte boundaries; the rows of a chunked projection
+    are left where they are."""
+    if t is None:
+        return None
+    if t.stride(-1) == 1 and t.stride(0) % 4 == 0 and t.data_ptr() % 8 == 0:
+        return t
+    return t.contiguous().clone()
+
+
+@torch._dynamo.disable
+def _launch(fn, jvp: bool, shape, eps: float, tensors: dict) -> None:
+    """Fill the call's structure and launch on the current stream of the tensors' device.  ``tensors`` keeps every
+    buffer alive until the launch is queued."""
+    p = _lib.AdaLn()
+    p.B, p.S, p.W = shape
+    p.eps = eps
+    for name, t in tensors.items():
+        if t is not None:
+            setattr(p, name, t.data_ptr())
+    for i, name in enumerate(_MOD):
+        t = tensors.get(name)
+        if t is not None:
+            p.mod_stride[i] = t.stride(0)
+    with torch.cuda.device(tensors["x"].device):
+        if fn == "sjvp_adaln_bwd":
+            floats = _lib.load().sjvp_adaln_workspace_floats(ctypes.byref(p))
+            workspace = torch.empty(floats, device=tensors["x"].device, dtype=torch.float32)
+            p.workspace = workspace.data_ptr()
+        stream = torch.cuda.current_stream().cuda_stream
+        _lib.check(getattr(_lib.load(), fn)(ctypes.byref(p), int(jvp), stream))
+
+
+class GatedNormFunction(torch.autograd.Function):
+    """``y = a gate + x`` and ``h = norm(y) (1 + scale) + shift`` with their tangents ``ty, th``.  Without ``a`` the
+    norm reads ``x`` and ``y`` is None; without ``w`` there is no ``h``."""
+
+    @staticmethod
+    def forward(ctx, eps, jvp, x, a, gate, scale, shift, w, b, tx, ta, tgate, tscale, tshift):
+        ctx.set_materialize_grads(False)
+        ctx.eps, ctx.jvp = eps, jvp
+        names = dict(x=_aligned(x), a=_aligned(a), tx=_aligned(tx), ta=_aligned(ta), w=_aligned(w), b=_aligned(b),
+                     gate=_mod_rows(gate), tgate=_mod_rows(tgate), scale=_mod_rows(scale), tscale=_mod_rows(tscale),
+                     shift=_mod_rows(shift), tshift=_mod_rows(tshift))
+
+        def like(present):
+            return torch.empty(x.shape, device=x.device, dtype=x.dtype) if present else None
+
+        y, ty = like(a is not None), like(a is not None and jvp)
+        h, th = like(w is not None), like(w is not None and jvp)
+        _launch("sjvp_adaln_fwd", jvp, x.shape, eps, dict(names, y=y, ty=ty, h=h, th=th))
+        if a is not None:  # the reverse mode reads y in the place of x
+            names["tx"] = None
+        ctx.names = list(names) + ["y", "ty"]
+        ctx.save_for_backward(*names.values(), y, ty)
+        return y, h, ty, th
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy, dh, dty, dth):
+        if dy is None and dh is None and dty is None and dth is None:
+            return (None,) * 14
+        t = dict(zip(ctx.names, ctx.saved_tensors))
+        x, jvp = t["x"], ctx.jvp
+        B, S, W = x.shape
+        need = dict(zip(("x", "a", "gate", "scale", "shift", "w", "b", "tx", "ta", "tgate", "tscale", "tshift"),
+                        ctx.needs_input_grad[2:]))
+        out = {"d" + n: torch.empty((B, 1, W) if n in _MOD else (W,) if n in ("w", "b") else x.shape, device=x.device,
+                                    dtype=torch.float32 if n in ("w", "b") else x.dtype)
+               for n, wanted in need.items() if wanted}
+        _launch("sjvp_adaln_bwd", jvp, x.shape, ctx.eps,
+                dict(t, dy=_aligned(dy), dh=_aligned(dh), dty=_aligned(dty), dth=_aligned(dth), **out))
+        return (None, None, *(out.get("d" + n) for n in need))
+
+
+class GeluFunction(torch.autograd.Function):
+    """tanh GELU and its tangent as one launch, and the reverse mode of both as one launch."""
+
+    @staticmethod
+    def forward(ctx, u, tu):
+        ctx.set_materialize_grads(False)
+        u, tu = _aligned(u), _aligned(tu)
+        y, ty = torch.empty_like(u), None if tu is None else torch.empty_like(u)
+        _gelu(u, tu, None, None, y, ty, 0)
+        ctx.save_for_backward(u, tu)
+        return y, ty
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy, dty):
+        if dy is None and dty is None:
+            return None, None
+        u, tu = ctx.saved_tensors
+        du = torch.empty_like(u)
+        dtu = torch.empty_like(u) if tu is not None and dty is not None else None
+        _gelu(u, tu, _aligned(dy), _aligned(dty), du, dtu, 1)
+        return du, dtu
+
+
+@torch._dynamo.disable
+def _gelu(u, tu, dy, dty, y, ty, reverse) -> None:
+    with torch.cuda.device(u.device):
+        _lib.check(_lib.load().sjvp_gelu(*(None if t is None else t.data_ptr() for t in (u, tu, dy, dty, y, ty)), u.numel(),
+                                         reverse, torch.cuda.current_stream().cuda_stream))
+
+
+@torch._dynamo.disable
+def bare(*modules: nn.Module) -> bool:
+    """Whether calling the modules does nothing beyond their ``forward``: no hooks of any kind."""
+    return not _module._has_any_global_hook() and not any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+
+
+@torch._dynamo.disable
+def serves_block(x: Tensor) -> bool:
+    """Whether a block's activations are of the kind that the functions serve; cheap, asked once per block."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.ndim == 3 and x.shape[-1] % 8 == 0
+            and 8 <= x.shape[-1] <= 1024 and 0 < x.shape[0] <= 65535 and x.numel() > 0
+            and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and not torch.jit.is_tracing() and not torch.jit.is_scripting()
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
+
+
+def _unwrap(tensors):
+    """``(interpreter or None, primals, tangents)`` on the level where both can be computed, or None where the general
+    dispatch has to see the operations.  Absent tensors stay None."""
+    present = [t for t in tensors if t is not None]
+    if _functorch.get_interpreter_stack() is None:
+        if fwAD._current_level >= 0 or any(type(t) not in (Tensor, nn.Parameter) for t in present):
+            return None
+        return None, list(tensors), [None] * len(tensors)
+    below = _below_jvp(present)
+    if below is None:
+        return None
+    interpreter, duals = below
+    duals = iter(duals)
+    pairs = [(None, None) if t is None else next(duals) for t in tensors]
+    return interpreter, [p for p, _ in pairs], [t for _, t in pairs]
+
+
+@torch._dynamo.disable
+def gated_norm(x: Tensor, a: Optional[Tensor], gate: Optional[Tensor], norm: Optional[nn.LayerNorm],
+               scale: Optional[Tensor], shift: Optional[Tensor]):
+    """``(y, h)`` of :class:`GatedNormFunction` on dual or plain tensors, or None where it does not serve the call.
+    The caller has asked :func:`serves_block`."""
+    w = b = None
+    if norm is not None:
+        w, b = norm.weight, norm.bias
+        if type(norm) is not nn.LayerNorm or norm.normalized_shape != x.shape[-1:] or w is None or b is None:
+            return None
+    found = _unwrap((x, a, gate, scale, shift, w, b))
+    if found is None:
+        return None
+    interpreter, primals, tangents = found
+    if tangents[5] is not None or tangents[6] is not None:
+        return None
+    B, S, W = x.shape
+    for i, (p, t) in enumerate(zip(primals, tangents)):
+        if p is None:
+            continue
+        shape, dtype = ((W,), torch.float32) if i > 4 else ((B, S, W) if i < 2 else (B, 1, W), torch.bfloat16)
+        if any(z.shape != shape or z.dtype != dtype or z.device != primals[0].device for z in (p, t) if z is not None):
+            return None
+    eps = 0.0 if norm is None else norm.eps
+    if interpreter is None:
+        return GatedNormFunction.apply(eps, False, *primals, *tangents[:5])[:2]
+    with interpreter.lower():
+        y, h, ty, th = GatedNormFunction.apply(eps, True, *primals, *tangents[:5])
+    return tuple(None if p is None else _dual_above(interpreter, p, t) for p, t in ((y, ty), (h, th)))
+
+
+@torch._dynamo.disable
+def gelu(u: Tensor) -> Optional[Tensor]:
+    """tanh GELU of a dual or plain bf16 tensor, or None where it is not served.  The caller has asked
+    :func:`serves_block` on the block's input."""
+    if u.dtype != torch.bfloat16 or u.numel() % 8 or not u.is_cuda:
+        return None
+    found = _unwrap((u,))
+    if found is None:
+        return None
+    interpreter, (p,), (t,) = found
+    if interpreter is None:
+        return GeluFunction.apply(p, None)[0]
+    if t.dtype != p.dtype or t.shape != p.shape:
+        return None
+    with interpreter.lower():
+        y, ty = GeluFunction.apply(p, t)
+    return _dual_above(interpreter, y, ty)

@@ -7,7 +7,8 @@ the op can be exercised where the reference calls it: twelve times per step, fro
 primal and the tangent.  Module and parameter names follow the reference (``vocab_embed.seq``,
 ``s_map.mlp.{0,2}``, ``blocks.<i>.attn_qkv`` ...), so a reference ``state_dict`` loads unchanged.
 
-Only the arithmetic of attention runs in HIP kernels; every other layer is stock PyTorch.
+Attention runs in HIP kernels, and so do the element-wise parts of the blocks under bf16 autocast on a GPU
+(:mod:`semicat_amd.adaln`); every other layer is stock PyTorch.
 
 Rotary embedding: the reference calls ``flash_attn.layers.rotary.apply_rotary_emb_torch`` (duo.py:52-53;
 flash_attn 2.8.3, not vendored).  :func:`rotate_half_embedding` restates that routine's published
@@ -24,6 +25,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
+from . import adaln
 from .functional import safe_sdpa_jvp, safe_sdpa_jvp_rotary
 from .rotary import apply_rotary
 
@@ -110,11 +112,27 @@ class DDiTBlock(nn.Module):
         nn.init.zeros_(self.adaLN_modulation.weight)
         nn.init.zeros_(self.adaLN_modulation.bias)
 
+    def _fuses(self, x: Tensor) -> bool:
+        return (adaln.serves_block(x) and not (self.training and self.dropout.p > 0.0)
+                and type(self.mlp) is nn.Sequential and len(self.mlp) == 3 and type(self.mlp[1]) is nn.GELU
+                and self.mlp[1].approximate == "tanh"
+                and adaln.bare(self.norm1, self.norm2, self.dropout, self.mlp, self.mlp[1]))
+
+    def _norm(self, fused: bool, x: Tensor, a, gate, norm, scale, shift):
+        """``(y, h)``: the gated residual ``y = dropout(a gate) + x`` and ``h = norm(y) (1 + scale) + shift``."""
+        both = adaln.gated_norm(x, a, gate, norm, scale, shift) if fused else None
+        if both is None:
+            y = x if a is None else self.dropout(a * gate) + x
+            both = y, None if norm is None else norm(y) * (1.0 + scale) + shift
+        return both
+
     def forward(self, x: Tensor, cos: Tensor, sin: Tensor, c: Tensor,
                 attention: Callable[[Tensor, Tensor, Tensor], Tensor], rotary_kernel: bool = False) -> Tensor:
         B = x.shape[0]
         shift_a, scale_a, gate_a, shift_m, scale_m, gate_m = self.adaLN_modulation(c)[:, None].chunk(6, dim=2)
-        h = self.norm1(x) * (1.0 + scale_a) + shift_a
+        # one launch for each run of element-wise operations where the library serves them (adaln.py)
+        fused = rotary_kernel and attention is safe_sdpa_jvp and self._fuses(x)
+        h = self._norm(fused, x, None, None, self.norm1, scale_a, shift_a)[1]
         qkv = self.attn_qkv(h).view(B, self.seq_len, 3, self.n_heads, self.dim // self.n_heads)
         v = qkv[:, :, 2]
         if rotary_kernel and attention is safe_sdpa_jvp:
@@ -123,9 +141,12 @@ class DDiTBlock(nn.Module):
             # (shapes the folded rotation does not serve take the rotary kernel first)
             a = safe_sdpa_jvp_rotary(qkv[:, :, 0], qkv[:, :, 1], v, cos, sin)
             a = a.reshape(B, self.seq_len, self.dim)
-            x = self.dropout(self.attn_out(a) * gate_a) + x
-            h = self.norm2(x) * (1.0 + scale_m) + shift_m
-            return self.dropout(self.mlp(h) * gate_m) + x
+            x, h = self._norm(fused, x, self.attn_out(a), gate_a, self.norm2, scale_m, shift_m)
+            if not fused:
+                return self.dropout(self.mlp(h) * gate_m) + x
+            h = self.mlp[0](h)
+            g = adaln.gelu(h)
+            return self._norm(fused, x, self.mlp[2](self.mlp[1](h) if g is None else g), gate_m, None, None, None)[0]
         if rotary_kernel:
             # one launch rotates q and k (and their tangents) out of the fused projection and writes
             # the contiguous 16-bit tensors the attention kernels read
@@ -165,9 +186,11 @@ class DDiTFinalLayer(nn.Module):
             nn.init.zeros_(lin.weight)
             nn.init.zeros_(lin.bias)
 
-    def forward(self, x: Tensor, c: Tensor) -> Tensor:
+    def forward(self, x: Tensor, c: Tensor, fused: bool = False) -> Tensor:
         shift, scale = self.adaLN_modulation(c)[:, None].chunk(2, dim=2)
-        return self.linear(self.norm_final(x) * (1.0 + scale) + shift)
+        both = adaln.gated_norm(x, None, None, self.norm_final, scale, shift) \
+            if fused and adaln.serves_block(x) and adaln.bare(self.norm_final) else None
+        return self.linear(self.norm_final(x) * (1.0 + scale) + shift if both is None else both[1])
 
 
 class DIT(nn.Module):
@@ -226,4 +249,4 @@ class DIT(nn.Module):
         rotary_kernel = self.rotary == "hip"
         for block in self.blocks:
             h = block(h, cos, sin, cond, attention, rotary_kernel)
-        return self.output_layer(h, cond)
+        return self.output_layer(h, cond, rotary_kernel and attention is safe_sdpa_jvp)
