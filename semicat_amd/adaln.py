@@ -24,7 +24,7 @@ from torch._C import _functorch
 from torch.autograd.function import once_differentiable
 from torch.nn.modules import module as _module
 
-from . import _lib
+from . import _lib, functional, kernels
 from .functional import _below_jvp, _dual_above
 
 _MOD = ("gate", "tgate", "scale", "tscale", "shift", "tshift")
@@ -137,6 +137,68 @@ class GeluFunction(torch.autograd.Function):
         return du, dtu
 
 
+class ChunkFunction(torch.autograd.Function):
+    """``n`` equal pieces of the last axis of ``[B,nW]`` as ``[B,1,W]`` views; their gradients come back as one
+    concatenation, where slices would each fill, copy and add a tensor of the whole size."""
+
+    @staticmethod
+    def forward(ctx, n, x):
+        ctx.set_materialize_grads(False)
+        ctx.shape = x.shape
+        return tuple(x.detach()[:, None].chunk(n, dim=2))
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, *grads):
+        some = next((g for g in grads if g is not None), None)
+        if some is None:
+            return None, None
+        return None, torch.cat([torch.zeros_like(some) if g is None else g for g in grads], dim=2).view(ctx.shape)
+
+
+class PackedAttentionFunction(torch.autograd.Function):
+    """Attention with the rotary embedding folded in on one ``[B,S,3,H,D]`` projection and its tangent.  The backward
+    writes its gradients into one tensor of the projection's layout: three slices of it would each fill, copy
+    and add a tensor of the whole size."""
+
+    @staticmethod
+    def forward(ctx, qkv, t_qkv, cos, sin):
+        ctx.set_materialize_grads(False)
+        B, S, _, H, D = qkv.shape
+        out = [None if t is None else torch.empty((B, S, H, D), device=qkv.device, dtype=qkv.dtype) for t in (qkv, t_qkv)]
+        o, to = (None if t is None else t.transpose(1, 2) for t in out)
+        q, k, v = _heads(qkv)
+        mu = None
+        if t_qkv is None:
+            _, lse = kernels.attention_forward(q, k, v, o=o, rope=(cos, sin))
+        else:
+            _, _, lse, mu, _ = kernels.attention_jvp_forward(q, k, v, *_heads(t_qkv), o=o, to=to, with_li=False,
+                                                             rope=(cos, sin))
+        ctx.save_for_backward(qkv, t_qkv, cos, sin, *out, lse, mu)
+        return tuple(out)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, d_y, d_ty):
+        qkv, t_qkv, cos, sin, y, ty, lse, mu = ctx.saved_tensors
+        if d_y is None and d_ty is None:
+            return (None,) * 4
+        d_qkv = torch.empty_like(qkv)
+        d_t_qkv = None if d_ty is None else torch.empty_like(qkv)
+        o, to, d_o, d_to = (None if t is None else t.transpose(1, 2) for t in (y, ty, d_y, d_ty))
+        tangents = (None,) * 3 if d_ty is None else _heads(t_qkv)
+        if d_ty is None:
+            to = mu = None
+        kernels.attention_jvp_backward(*_heads(qkv), *tangents, o, to, lse, mu, dO=d_o, dTO=d_to, rope=(cos, sin),
+                                       grads=(*_heads(d_qkv), *((None,) * 3 if d_ty is None else _heads(d_t_qkv))))
+        return d_qkv, d_t_qkv, None, None
+
+
+def _heads(qkv: Tensor):
+    """The three ``[B,H,S,D]`` views of ``[B,S,3,H,D]``."""
+    return qkv.permute(2, 0, 3, 1, 4).unbind(0)
+
+
 @torch._dynamo.disable
 def _gelu(u, tu, dy, dty, y, ty, reverse) -> None:
     with torch.cuda.device(u.device):
@@ -225,4 +287,45 @@ def gelu(u: Tensor) -> Optional[Tensor]:
         return None
     with interpreter.lower():
         y, ty = GeluFunction.apply(p, t)
+    return _dual_above(interpreter, y, ty)
+
+
+@torch._dynamo.disable
+def chunk(x: Tensor, n: int):
+    """``x[:, None].chunk(n, dim=2)`` of a dual or plain ``[B,nW]`` tensor, or None where it is not served.  The caller has
+    asked :func:`serves_block`."""
+    found = _unwrap((x,)) if x.ndim == 2 and x.shape[1] % n == 0 and x.dtype == torch.bfloat16 else None
+    if found is None:
+        return None
+    interpreter, (p,), (t,) = found
+    if interpreter is None:
+        return ChunkFunction.apply(n, p)
+    with interpreter.lower():
+        primals, tangents = ChunkFunction.apply(n, p), ChunkFunction.apply(n, t)
+    return tuple(_dual_above(interpreter, a, b) for a, b in zip(primals, tangents))
+
+
+@torch._dynamo.disable
+def attention(qkv: Tensor, cos: Tensor, sin: Tensor) -> Optional[Tensor]:
+    """``safe_sdpa_jvp_rotary`` of the three slices of a dual or plain ``[B,S,3,H,D]`` projection, ``[B,S,H,D]``, or
+    None where it is not served.  The caller has asked :func:`serves_block`."""
+    # tables sliced inside the transform are wrapped like everything computed there
+    found = _unwrap((qkv, cos, sin)) if functional.AUTOGRAD_WIRING != "reference" else None
+    if found is None:
+        return None
+    interpreter, (p, cos, sin), (t, *tables) = found
+    if any(z is not None for z in tables) or (t is None) != (interpreter is None):
+        return None
+    if p.dtype != torch.bfloat16 or any(z.ndim != 5 or z.shape != p.shape or z.dtype != p.dtype or not z.is_contiguous()
+                                        for z in (p, t) if z is not None) or cos.requires_grad or sin.requires_grad:
+        return None
+    if interpreter is None:
+        q, k, v = _heads(p.detach())
+        return PackedAttentionFunction.apply(p, None, cos, sin)[0] \
+            if kernels.rotary_fusable(q, k, cos, (v,), sin=sin) else None
+    with interpreter.lower():
+        q, k, v = _heads(p.detach())
+        if not kernels.rotary_fusable(q, k, cos, (v, *_heads(t.detach())), sin=sin):
+            return None
+        y, ty = PackedAttentionFunction.apply(p, t, cos, sin)
     return _dual_above(interpreter, y, ty)

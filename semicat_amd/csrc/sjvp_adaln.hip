@@ -206,14 +206,23 @@ __global__ __launch_bounds__(64 * kWaves) void adaln_bwd_kernel(AdaParams p) {
     }
     for (int s = chunk * p.rows_per_block + wave; s < end; s += kWaves) {
         const int64_t at = (b * t.S + s) * W;
-        Row<NV> dy, dty, u;
+        // every load of the row is issued ahead of its first reduction
+        Row<NV> dy, dty, u, dh, e, ty, a, ta;
+        if constexpr (NORM) {
+            u.load(GATE ? t.y : t.x, at, lane, W);
+            if constexpr (JVP) ty.load(GATE ? t.ty : t.tx, at, lane, W);
+            dh.load(t.dh, at, lane, W);
+            if constexpr (JVP) e.load(t.dth, at, lane, W);
+        }
         dy.load(t.dy, at, lane, W);
         if constexpr (JVP) dty.load(t.dty, at, lane, W);
+        if constexpr (GATE) {
+            a.load(t.a, at, lane, W);
+            if constexpr (JVP) ta.load(t.ta, at, lane, W);
+        }
         if constexpr (NORM) {
-            Row<NV> xhat, dh;
-            u.load(GATE ? t.y : t.x, at, lane, W);
+            Row<NV> xhat;
             const float r = normalise(u, xhat, lane, W, t.eps);
-            dh.load(t.dh, at, lane, W);
 #pragma unroll
             for (int i = 0; i < NV * 4; ++i) {
                 sums[0].v[i] += dh.v[i] * xhat.v[i];
@@ -221,10 +230,8 @@ __global__ __launch_bounds__(64 * kWaves) void adaln_bwd_kernel(AdaParams p) {
                 dh.v[i] *= (1.f + sc.v[i]) * w.v[i];  // now the gradient of xhat
             }
             if constexpr (JVP) {
-                Row<NV> e, txhat;
-                u.load(GATE ? t.ty : t.tx, at, lane, W);
-                const float c1 = project(u, xhat, txhat, r, lane, W);
-                e.load(t.dth, at, lane, W);
+                Row<NV> txhat;
+                const float c1 = project(ty, xhat, txhat, r, lane, W);
 #pragma unroll
                 for (int i = 0; i < NV * 4; ++i) {
                     sums[0].v[i] += e.v[i] * txhat.v[i];
@@ -253,22 +260,20 @@ __global__ __launch_bounds__(64 * kWaves) void adaln_bwd_kernel(AdaParams p) {
         if constexpr (JVP) dty.store(t.dtx, at, lane, W);
         if constexpr (GATE) {
             Row<NV> da;
-            u.load(t.a, at, lane, W);
 #pragma unroll
             for (int i = 0; i < NV * 4; ++i) {
-                sums[4].v[i] += dy.v[i] * u.v[i];
+                sums[4].v[i] += dy.v[i] * a.v[i];
                 da.v[i] = dy.v[i] * g.v[i];
             }
             if constexpr (JVP) {
 #pragma unroll
                 for (int i = 0; i < NV * 4; ++i) {
-                    sums[5].v[i] += dty.v[i] * u.v[i];
+                    sums[5].v[i] += dty.v[i] * a.v[i];
                     da.v[i] += dty.v[i] * tg.v[i];
                 }
-                u.load(t.ta, at, lane, W);
 #pragma unroll
                 for (int i = 0; i < NV * 4; ++i) {
-                    sums[4].v[i] += dty.v[i] * u.v[i];
+                    sums[4].v[i] += dty.v[i] * ta.v[i];
                     dty.v[i] *= g.v[i];
                 }
                 dty.store(t.dta, at, lane, W);
@@ -292,13 +297,15 @@ __global__ __launch_bounds__(64 * kWaves) void adaln_bwd_kernel(AdaParams p) {
 }
 
 // One thread per (sample, column): the partial rows of a sample's workgroups, then what the sums stand for.
-__global__ __launch_bounds__(256) void adaln_mod_kernel(AdaParams p, int gate, int norm, int jvp) {
+template <bool gate, bool norm, bool jvp>
+__global__ __launch_bounds__(64) void adaln_mod_kernel(AdaParams p) {
     const sjvp_adaln& t = p.t;
-    const int c = blockIdx.x * 256 + threadIdx.x, W = t.W;
+    const int c = blockIdx.x * 64 + threadIdx.x, W = t.W;
     const int64_t b = blockIdx.y;
     if (c >= W) return;
     float s[kSums] = {};
     const float* in = t.workspace + b * p.chunks * kSums * W + c;
+#pragma unroll 4
     for (int k = 0; k < p.chunks; ++k, in += (int64_t)kSums * W) {
 #pragma unroll
         for (int i = 0; i < kSums; ++i)
@@ -406,9 +413,9 @@ __global__ __launch_bounds__(256) void gelu_kernel(const void* u, const void* tu
     store8(ty, i8 * 8, tx);
 }
 
-template <typename K, typename... A>
+template <int THREADS = 256, typename K, typename... A>
 int launch(K kernel, dim3 grid, void* stream, A... args) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), args...);
+    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), 0, static_cast<hipStream_t>(stream), args...);
     return hipGetLastError() == hipSuccess ? SJVP_OK : SJVP_ERR_LAUNCH;
 }
 
@@ -491,11 +498,16 @@ int sjvp_adaln_bwd(const sjvp_adaln* t, int jvp, void* stream) {
     if (!t->workspace || (t->a && t->w && (!t->y || (jvp && !t->ty)))) return SJVP_ERR_NULL;
     AdaParams p{*t, rows_per_block(*t), chunks_of(*t), nullptr};
     p.col_partial = t->workspace + (size_t)t->B * p.chunks * kSums * t->W;
-    const dim3 grid((unsigned)(t->B * p.chunks));
+    const dim3 grid((unsigned)(t->B * p.chunks)), per_column((t->W + 63) / 64, t->B);
     rc = jvp ? run<true, true>(p, grid, stream) : run<true, false>(p, grid, stream);
     if (rc != SJVP_OK) return rc;
-    rc = launch(adaln_mod_kernel, dim3((t->W + 255) / 256, t->B), stream, p, int(t->a != nullptr),
-                int(t->w != nullptr), jvp);
+    auto columns = [&](auto j) {
+        constexpr bool J = decltype(j)::value;
+        if (t->a && t->w) return launch<64>(adaln_mod_kernel<true, true, J>, per_column, stream, p);
+        if (t->a) return launch<64>(adaln_mod_kernel<true, false, J>, per_column, stream, p);
+        return launch<64>(adaln_mod_kernel<false, true, J>, per_column, stream, p);
+    };
+    rc = jvp ? columns(std::true_type{}) : columns(std::false_type{});
     if (rc != SJVP_OK || !t->w || (!t->dw && !t->db)) return rc;
     return launch(adaln_col_kernel, dim3((t->W + 31) / 32, 2), stream, p);
 }

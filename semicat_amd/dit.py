@@ -129,17 +129,20 @@ class DDiTBlock(nn.Module):
     def forward(self, x: Tensor, cos: Tensor, sin: Tensor, c: Tensor,
                 attention: Callable[[Tensor, Tensor, Tensor], Tensor], rotary_kernel: bool = False) -> Tensor:
         B = x.shape[0]
-        shift_a, scale_a, gate_a, shift_m, scale_m, gate_m = self.adaLN_modulation(c)[:, None].chunk(6, dim=2)
         # one launch for each run of element-wise operations where the library serves them (adaln.py)
         fused = rotary_kernel and attention is safe_sdpa_jvp and self._fuses(x)
+        mod = self.adaLN_modulation(c)
+        pieces = adaln.chunk(mod, 6) if fused else None
+        shift_a, scale_a, gate_a, shift_m, scale_m, gate_m = mod[:, None].chunk(6, dim=2) if pieces is None else pieces
         h = self._norm(fused, x, None, None, self.norm1, scale_a, shift_a)[1]
         qkv = self.attn_qkv(h).view(B, self.seq_len, 3, self.n_heads, self.dim // self.n_heads)
-        v = qkv[:, :, 2]
         if rotary_kernel and attention is safe_sdpa_jvp:
             # the attention kernels read q, k, v (and their tangents) as strided views of the fused
             # projection and rotate q, k on chip; gradients come back through the inverse rotation
             # (shapes the folded rotation does not serve take the rotary kernel first)
-            a = safe_sdpa_jvp_rotary(qkv[:, :, 0], qkv[:, :, 1], v, cos, sin)
+            a = adaln.attention(qkv, cos, sin) if fused else None
+            if a is None:
+                a = safe_sdpa_jvp_rotary(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], cos, sin)
             a = a.reshape(B, self.seq_len, self.dim)
             x, h = self._norm(fused, x, self.attn_out(a), gate_a, self.norm2, scale_m, shift_m)
             if not fused:
@@ -147,6 +150,7 @@ class DDiTBlock(nn.Module):
             h = self.mlp[0](h)
             g = adaln.gelu(h)
             return self._norm(fused, x, self.mlp[2](self.mlp[1](h) if g is None else g), gate_m, None, None, None)[0]
+        v = qkv[:, :, 2]
         if rotary_kernel:
             # one launch rotates q and k (and their tangents) out of the fused projection and writes
             # the contiguous 16-bit tensors the attention kernels read
@@ -187,9 +191,11 @@ class DDiTFinalLayer(nn.Module):
             nn.init.zeros_(lin.bias)
 
     def forward(self, x: Tensor, c: Tensor, fused: bool = False) -> Tensor:
-        shift, scale = self.adaLN_modulation(c)[:, None].chunk(2, dim=2)
-        both = adaln.gated_norm(x, None, None, self.norm_final, scale, shift) \
-            if fused and adaln.serves_block(x) and adaln.bare(self.norm_final) else None
+        fused = fused and adaln.serves_block(x) and adaln.bare(self.norm_final)
+        mod = self.adaLN_modulation(c)
+        pieces = adaln.chunk(mod, 2) if fused else None
+        shift, scale = mod[:, None].chunk(2, dim=2) if pieces is None else pieces
+        both = adaln.gated_norm(x, None, None, self.norm_final, scale, shift) if fused else None
         return self.linear(self.norm_final(x) * (1.0 + scale) + shift if both is None else both[1])
 
 

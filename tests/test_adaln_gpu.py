@@ -108,8 +108,12 @@ def test_training_step_with_and_without(monkeypatch, hook):
     if hook:
         net.blocks[0].norm1.register_forward_hook(lambda *_: seen.append(1))
     calls = []
-    gated_norm = adaln.gated_norm
-    monkeypatch.setattr(adaln, "gated_norm", lambda *a: calls.append(gated_norm(*a)) or calls[-1])
+    for name in ("gated_norm", "chunk", "attention", "gelu"):
+        def served(*a, f=getattr(adaln, name)):
+            out = f(*a)
+            calls.append((f.__name__, out is not None))
+            return out
+        monkeypatch.setattr(adaln, name, served)
 
     def step():
         net.zero_grad(set_to_none=True)
@@ -120,7 +124,8 @@ def test_training_step_with_and_without(monkeypatch, hook):
         return vf.item(), sd.item(), torch.cat([p.grad.flatten() for p in net.parameters()])
 
     got = step()
-    assert len(calls) == 3 * (4 if hook else 7) and all(c is not None for c in calls)
+    # three network calls; six functions per block and two in the output layer
+    assert len(calls) == 3 * (8 if hook else 14) and all(served for _, served in calls), calls
     assert len(seen) == (3 if hook else 0)
     monkeypatch.setattr(adaln, "serves_block", lambda x: False)
     ref = step()
