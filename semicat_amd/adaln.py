@@ -48,6 +48,24 @@ def _mod_rows(t: Optional[Tensor]) -> Optional[Tensor]:
     return t.contiguous().clone()
 
 
+def _pair(like: Tensor, first: bool = True, second: bool = True, shape=None):
+    """Uninitialised memory for a tensor and its tangent (or either), side by side, so that a linear layer behind
+    takes both as the rows of one product."""
+    shape = like.shape if shape is None else shape
+    both = torch.empty((int(first) + int(second), *shape), device=like.device, dtype=like.dtype).unbind(0)
+    return (both[0] if first else None), (both[-1] if second else None)
+
+
+def _stacked(p: Tensor, t: Tensor) -> Tensor:
+    """The rows of both tensors as one matrix, without a copy where they lie side by side."""
+    p, t = p.detach().contiguous(), t.detach().contiguous()
+    rows, W = p.numel() // p.shape[-1], p.shape[-1]
+    if t.data_ptr() == p.data_ptr() + p.numel() * p.element_size() \
+            and t.untyped_storage().data_ptr() == p.untyped_storage().data_ptr():
+        return p.as_strided((2 * rows, W), (W, 1))
+    return torch.cat((p.view(rows, W), t.view(rows, W)))
+
+
 @torch._dynamo.disable
 def _launch(fn, jvp: bool, shape, eps: float, tensors: dict) -> None:
     """Fill the call's structure and launch on the current stream of the tensors' device.  ``tensors`` keeps every
@@ -83,11 +101,8 @@ class GatedNormFunction(torch.autograd.Function):
                      gate=_mod_rows(gate), tgate=_mod_rows(tgate), scale=_mod_rows(scale), tscale=_mod_rows(tscale),
                      shift=_mod_rows(shift), tshift=_mod_rows(tshift))
 
-        def like(present):
-            return torch.empty(x.shape, device=x.device, dtype=x.dtype) if present else None
-
-        y, ty = like(a is not None), like(a is not None and jvp)
-        h, th = like(w is not None), like(w is not None and jvp)
+        y, ty = _pair(x, a is not None, a is not None and jvp)
+        h, th = _pair(x, w is not None, w is not None and jvp)
         _launch("sjvp_adaln_fwd", jvp, x.shape, eps, dict(names, y=y, ty=ty, h=h, th=th))
         if a is not None:  # the reverse mode reads y in the place of x
             names["tx"] = None
@@ -105,9 +120,13 @@ class GatedNormFunction(torch.autograd.Function):
         B, S, W = x.shape
         need = dict(zip(("x", "a", "gate", "scale", "shift", "w", "b", "tx", "ta", "tgate", "tscale", "tshift"),
                         ctx.needs_input_grad[2:]))
-        out = {"d" + n: torch.empty((B, 1, W) if n in _MOD else (W,) if n in ("w", "b") else x.shape, device=x.device,
-                                    dtype=torch.float32 if n in ("w", "b") else x.dtype)
-               for n, wanted in need.items() if wanted}
+        out = {}
+        for n in ("x", "a"):
+            out["d" + n], out["dt" + n] = _pair(x, need[n], need["t" + n])
+        for n in _MOD:
+            out["d" + n] = x.new_empty((B, 1, W)) if need[n] else None
+        for n in ("w", "b"):
+            out["d" + n] = torch.empty(W, device=x.device, dtype=torch.float32) if need[n] else None
         _launch("sjvp_adaln_bwd", jvp, x.shape, ctx.eps,
                 dict(t, dy=_aligned(dy), dh=_aligned(dh), dty=_aligned(dty), dth=_aligned(dth), **out))
         return (None, None, *(out.get("d" + n) for n in need))
@@ -120,7 +139,7 @@ class GeluFunction(torch.autograd.Function):
     def forward(ctx, u, tu):
         ctx.set_materialize_grads(False)
         u, tu = _aligned(u), _aligned(tu)
-        y, ty = torch.empty_like(u), None if tu is None else torch.empty_like(u)
+        y, ty = _pair(u, True, tu is not None)
         _gelu(u, tu, None, None, y, ty, 0)
         ctx.save_for_backward(u, tu)
         return y, ty
@@ -131,8 +150,7 @@ class GeluFunction(torch.autograd.Function):
         if dy is None and dty is None:
             return None, None
         u, tu = ctx.saved_tensors
-        du = torch.empty_like(u)
-        dtu = torch.empty_like(u) if tu is not None and dty is not None else None
+        du, dtu = _pair(u, True, tu is not None and dty is not None)
         _gelu(u, tu, _aligned(dy), _aligned(dty), du, dtu, 1)
         return du, dtu
 
@@ -165,7 +183,7 @@ class PackedAttentionFunction(torch.autograd.Function):
     def forward(ctx, qkv, t_qkv, cos, sin):
         ctx.set_materialize_grads(False)
         B, S, _, H, D = qkv.shape
-        out = [None if t is None else torch.empty((B, S, H, D), device=qkv.device, dtype=qkv.dtype) for t in (qkv, t_qkv)]
+        out = _pair(qkv, True, t_qkv is not None, (B, S, H, D))
         o, to = (None if t is None else t.transpose(1, 2) for t in out)
         q, k, v = _heads(qkv)
         mu = None
@@ -175,7 +193,7 @@ class PackedAttentionFunction(torch.autograd.Function):
             _, _, lse, mu, _ = kernels.attention_jvp_forward(q, k, v, *_heads(t_qkv), o=o, to=to, with_li=False,
                                                              rope=(cos, sin))
         ctx.save_for_backward(qkv, t_qkv, cos, sin, *out, lse, mu)
-        return tuple(out)
+        return out
 
     @staticmethod
     @once_differentiable
@@ -183,8 +201,7 @@ class PackedAttentionFunction(torch.autograd.Function):
         qkv, t_qkv, cos, sin, y, ty, lse, mu = ctx.saved_tensors
         if d_y is None and d_ty is None:
             return (None,) * 4
-        d_qkv = torch.empty_like(qkv)
-        d_t_qkv = None if d_ty is None else torch.empty_like(qkv)
+        d_qkv, d_t_qkv = _pair(qkv, True, d_ty is not None)
         o, to, d_o, d_to = (None if t is None else t.transpose(1, 2) for t in (y, ty, d_y, d_ty))
         tangents = (None,) * 3 if d_ty is None else _heads(t_qkv)
         if d_ty is None:
@@ -192,6 +209,51 @@ class PackedAttentionFunction(torch.autograd.Function):
         kernels.attention_jvp_backward(*_heads(qkv), *tangents, o, to, lse, mu, dO=d_o, dTO=d_to, rope=(cos, sin),
                                        grads=(*_heads(d_qkv), *((None,) * 3 if d_ty is None else _heads(d_t_qkv))))
         return d_qkv, d_t_qkv, None, None
+
+
+class LinearFunction(torch.autograd.Function):
+    """``x w^T + b`` and ``tx w^T``, without a bias as one matrix product over the rows of both; in reverse mode one
+    product for both inputs and one, summed over both in fp32, for the weight.  Through the general dispatch forward mode adds products
+    with the absent tangents of weight and bias, zero fills and sums: 9 products per layer and step instead of 3.
+    bf16 products on a bf16 copy of the fp32 weight, as autocast makes it."""
+
+    @staticmethod
+    def forward(ctx, x, tx, w, b):
+        ctx.set_materialize_grads(False)
+        w16 = w.to(x.dtype)
+        if b is None:
+            y, ty = torch.mm(_stacked(x, tx), w16.t()).view(2, *x.shape[:-1], w.shape[0]).unbind(0)
+        else:
+            # the bias enters the product's accumulator; added behind it, y would be rounded twice
+            y, ty = _pair(x, shape=(*x.shape[:-1], w.shape[0]))
+            torch.addmm(b.to(x.dtype), x.reshape(-1, w.shape[1]), w16.t(), out=y.view(-1, w.shape[0]))
+            torch.mm(tx.reshape(-1, w.shape[1]), w16.t(), out=ty.view(-1, w.shape[0]))
+        ctx.save_for_backward(x, tx, w16)
+        ctx.w_dtype = w.dtype
+        return y, ty
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy, dty):
+        x, tx, w16 = ctx.saved_tensors
+        if dy is None and dty is None:
+            return (None,) * 4
+        dx = dtx = dw = db = None
+        need_x, need_tx, need_w, need_b = ctx.needs_input_grad
+        if dy is not None and dty is not None:
+            g, rows = _stacked(dy, dty), lambda: _stacked(x, tx)
+        else:
+            g = (dy if dty is None else dty).reshape(-1, w16.shape[0])
+            rows = lambda: (x if dty is None else tx).reshape(-1, w16.shape[1])
+        if need_x or need_tx:
+            pieces = iter(torch.mm(g, w16).view(-1, *x.shape).unbind(0))
+            dx = None if dy is None else next(pieces)
+            dtx = None if dty is None else next(pieces)
+        if need_w:
+            dw = torch.mm(g.t(), rows()).to(ctx.w_dtype)
+        if need_b and dy is not None:
+            db = dy.reshape(-1, w16.shape[0]).sum(0).to(ctx.w_dtype)
+        return dx, dtx, dw, db
 
 
 def _heads(qkv: Tensor):
@@ -287,6 +349,26 @@ def gelu(u: Tensor) -> Optional[Tensor]:
         return None
     with interpreter.lower():
         y, ty = GeluFunction.apply(p, t)
+    return _dual_above(interpreter, y, ty)
+
+
+@torch._dynamo.disable
+def linear(layer: nn.Linear, x: Tensor) -> Optional[Tensor]:
+    """The layer on a dual tensor, or None where it is not served (a plain tensor included: that is one product
+    already).  The caller has asked :func:`serves_block`."""
+    w, b = layer.weight, layer.bias
+    if type(layer) is not nn.Linear or not bare(layer) or x.dtype != torch.bfloat16 \
+            or _functorch.get_interpreter_stack() is None:
+        return None
+    found = _unwrap((x, w, b))
+    if found is None:
+        return None
+    interpreter, (p, w, b), (t, *absent) = found
+    if t is None or any(z is not None for z in absent) or t.dtype != p.dtype or t.shape != p.shape or p.numel() == 0 \
+            or any(z.dtype != torch.float32 or z.device != p.device for z in (w, b) if z is not None):
+        return None
+    with interpreter.lower():
+        y, ty = LinearFunction.apply(p, t, w, b)
     return _dual_above(interpreter, y, ty)
 
 

@@ -91,6 +91,36 @@ def test_gelu_against_fp64(n):
         _check(name, got, ref)
 
 
+@pytest.mark.parametrize("adjacent", [False, True])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("cot", ["both", "y", "ty"])
+def test_linear_against_fp64(adjacent, bias, cot):
+    gen = torch.Generator("cuda").manual_seed(3)
+    x, tx = torch.randn(2, 3, 5, 24, generator=gen, device="cuda").bfloat16().unbind(0)
+    if not adjacent:
+        tx = tx.clone()
+    x.requires_grad_(), tx.requires_grad_()
+    w = torch.randn(40, 24, generator=gen, device="cuda").bfloat16().float().requires_grad_()
+    b = torch.randn(40, generator=gen, device="cuda").bfloat16().float().requires_grad_() if bias else None
+    outs = adaln.LinearFunction.apply(x, tx, w, b)
+    ref_in = [None if z is None else z.detach().double().requires_grad_() for z in (x, tx, w, b)]
+    refs = F.linear(ref_in[0], ref_in[2], ref_in[3]), F.linear(ref_in[1], ref_in[2])
+    keep = [i for i, name in enumerate(("y", "ty")) if cot in ("both", name)]
+    g = torch.randn(2, 3, 5, 40, generator=gen, device="cuda").bfloat16()
+    wrt = [i for i, z in enumerate((x, tx, w, b)) if z is not None]
+    got = torch.autograd.grad([outs[i] for i in keep], [(x, tx, w, b)[i] for i in wrt], [g[i] for i in keep],
+                              allow_unused=True)
+    ref = torch.autograd.grad([refs[i] for i in keep], [ref_in[i] for i in wrt], [g[i].double() for i in keep],
+                              allow_unused=True)
+    for i in range(2):
+        _check(f"output {i}", outs[i], refs[i])
+    for i, a, r in zip(wrt, got, ref):
+        assert (a is None) == (r is None)
+        if a is not None:
+            assert a.dtype == (x, tx, w, b)[i].dtype and a.shape == r.shape
+            _check(f"gradient {i}", a, r)
+
+
 @pytest.mark.parametrize("hook", [False, True])
 def test_training_step_with_and_without(monkeypatch, hook):
     """Both losses and every gradient through the kernels and through the PyTorch operations; a module with a hook keeps
@@ -127,6 +157,11 @@ def test_training_step_with_and_without(monkeypatch, hook):
     # three network calls; six functions per block and two in the output layer
     assert len(calls) == 3 * (8 if hook else 14) and all(served for _, served in calls), calls
     assert len(seen) == (3 if hook else 0)
+    layers = []
+    linear = adaln.linear
+    monkeypatch.setattr(adaln, "linear", lambda *a: layers.append(linear(*a) is not None) or linear(*a))
+    step()
+    assert sum(layers) == (7 if hook else 12)  # of the three network calls the one under forward-mode AD
     monkeypatch.setattr(adaln, "serves_block", lambda x: False)
     ref = step()
     # two blocks of bf16 products on either side, each rounding its operands: 2^-9 per product
