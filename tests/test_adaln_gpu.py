@@ -167,3 +167,42 @@ def test_training_step_with_and_without(monkeypatch, hook):
     # two blocks of bf16 products on either side, each rounding its operands: 2^-9 per product
     assert abs(got[0] - ref[0]) < 1e-2 * abs(ref[0]) and abs(got[1] - ref[1]) < 1e-2 * abs(ref[1])
     assert (got[2] - ref[2]).norm() < 3e-2 * ref[2].norm()
+
+
+@pytest.mark.parametrize("train", ["net", "dropout only"])
+def test_training_step_with_dropout(monkeypatch, train):
+    """A training block's dropout goes in front of the gate: the same masks as behind it, the same gradients, also
+    where only the dropout modules are in training mode."""
+    torch.manual_seed(0)
+    B, S, V = 4, 16, 48
+    net = DIT(V, 128, 16, 2, 2, 0.3, S).cuda()
+    for p in net.parameters():
+        if not p.any():
+            torch.nn.init.normal_(p, std=0.05)
+    if train != "net":
+        net.eval()
+        for block in net.blocks:
+            block.dropout.train()
+    x0, x1 = torch.randn(B, S, V, device="cuda"), torch.randint(0, V, (B, S), device="cuda")
+    t = torch.rand(B, device="cuda")
+    s = t * torch.rand(B, device="cuda")
+
+    def step():
+        torch.manual_seed(1)
+        net.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            vf = train_step.vfm_loss(net, x0[2:], x1[2:], t=t[2:])
+            sd = train_step.lag_self_distillation_loss(net, x0[:2], x1[:2], t=t[:2], s=s[:2])
+        (vf + sd).backward()
+        return vf.item(), sd.item(), torch.cat([p.grad.flatten() for p in net.parameters()])
+
+    calls = []
+    norm = adaln.gated_norm
+    monkeypatch.setattr(adaln, "gated_norm", lambda *a: (calls.append(1), norm(*a))[1])
+    got = step()
+    assert len(calls) == 3 * 7
+    monkeypatch.setattr(adaln, "serves_block", lambda x: False)
+    ref = step()
+    # as without dropout; another mask would differ by far more
+    assert abs(got[0] - ref[0]) < 1e-2 * abs(ref[0]) and abs(got[1] - ref[1]) < 1e-2 * abs(ref[1])
+    assert (got[2] - ref[2]).norm() < 3e-2 * ref[2].norm()
