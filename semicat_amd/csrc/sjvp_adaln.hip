@@ -15,6 +15,10 @@
 // sample and every lane keeps the column sums of its columns in registers over its rows; six of them are
 // enough for the gradients of gate, scale, shift, their tangents, w and b.  They leave as one partial row per
 // workgroup, which two small launches reduce in a fixed order (no atomics: results repeat bit by bit).
+// Measured at W = 768, S = 128, gated residual + norm: forward with tangents (B = 16, 25 MB) 15.8 us, reverse (38 MB)
+// 37.9; reverse without tangents (B = 48, 57 MB) 36.6 us = 1.5 TB/s.  The reverse is short of waves (one or two
+// workgroups per compute unit) and waits for its chain of row reductions.  gelu_kernel averages 12.8 us forward and
+// 21.2 us in reverse over the step's two shares.  In the place of PyTorch's kernels: LM1B training step 98 -> 67 ms.
 #include <type_traits>
 
 #include "../../include/sjvp.h"

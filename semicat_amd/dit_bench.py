@@ -98,7 +98,8 @@ def graph_step(args, net, opt, x1) -> int:
     library allocates nothing, records no memset and never synchronises, so its launches can be
     captured).  The replay time is what the kernels of a step take without the host issuing them one
     by one.  The random draws of a step come from the default generator, which graph capture
-    advances per replay."""
+    advances per replay.  A timing only: PyTorch's multi-block sums (the MLP's bias gradients) record a memset, and
+    from the second replay on they come out wrong, so the replayed losses mean nothing."""
     def step():
         opt.zero_grad(set_to_none=False)
         with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
@@ -130,7 +131,7 @@ def graph_step(args, net, opt, x1) -> int:
     print(json.dumps({
         "workload": f"LM1B DiT step: {args.blocks} blocks, width 768, 12x64 heads, seq {args.length}, "
                     f"vocab {args.vocab}, batch {args.batch}, sd_prop {args.sd_prop}, bf16 autocast, AdamW",
-        "launch": "HIP graph replay of one whole step",
+        "launch": "HIP graph replay of one whole step (timing only: bias gradients of replays are wrong)",
         "ms_per_step": e0.elapsed_time(e1) / args.steps,
         "plain_attention": args.plain_attention, "rotary": args.rotary,
         "vfm_loss": float(vf), "sd_loss": None if sd is None else float(sd),
