@@ -37,28 +37,25 @@ from torch._C import _functorch
 from torch._functorch.pyfunctorch import TransformType, retrieve_current_functorch_interpreter
 
 from . import kernels
-from ._lib import SJVP_BWD_ALL, SJVP_BWD_FP32_SINGLE
 
 
 AUTOGRAD_WIRING = "fused"  # or "reference"
 # How safe_sdpa_jvp serves float32 callers with bf16 arithmetic (functional.py:318-332):
-#   "torch"   (default) the reference's casts around the op: on a GPU they are folded into the kernels, which
-#             round the float32 tensors as they load them and store float32 (SJVP_FP32_BF16, with the launches that
-#             16-bit tensors of the shape would take); elsewhere they are torch casts;
-#   "folded"  the float32 tensors handed to the launchers wherever they live;
-#   "library" the library's multi-tensor cast launches around the 16-bit kernels.
-# Measured on an MI355X, launches of forward + backward in microseconds, 16-bit callers / folded / torch casts:
-#   B=64 H=12 L=128 D=64: 66 / 139 / 214;  B=128 H=12 L=256: 443 / 745 / 889;  B=8 H=16 L=1024: 438 / 590 / 618.
+#   "torch"   (default) torch casts around the 16-bit kernels, as the reference does;
+#   "library" the library's multi-tensor cast launches around them (half the launches, no kernel that is
+#             not the library's own);
+#   "folded"  the float32 tensors handed to the kernels, which round as they load and store float32 (SJVP_FP32_BF16).
+# "folded" is not the default: autograd keeps the caller's own tensors for it, so they (and the result) may not be
+# written to before the backward, they stay in memory at twice the size (B=64 H=12 L=128 D=64: 191 MB held by a call on
+# temporaries against 145), the last dimension has to have unit stride, and it is the faster route for short sequences
+# at D = 64 only.  Measured on an MI355X, forward + backward under torch.func.jvp in microseconds, folded / casts:
+#   D = 64:  B=64 H=12 L=128 187 / 280, B=8 H=16 L=1024 604 / 621, L=2048 2125 / 2010, L=4096 7936 / 7410;
+#   D = 128: B=8 H=16 L=1024 1508 / 1260, L=2048 5496 / 4136, L=4096 20085 / 14900.
 FP32_CALLERS = "torch"
 
 
 def _has_tangent(t: Tensor) -> bool:
     return fwAD.unpack_dual(t).tangent is not None
-
-
-def _backward_launches(q: Tensor, arith: Optional[str]) -> dict:
-    """Float32 tensors with folded casts take the launches that 16-bit tensors of the shape would take."""
-    return {"parts": SJVP_BWD_ALL | SJVP_BWD_FP32_SINGLE} if arith == "bf16" and q.is_cuda else {}
 
 
 class SDPAJVPFlashBackwardFunction(torch.autograd.Function):
@@ -82,7 +79,7 @@ class SDPABackwardFunction(torch.autograd.Function):
     def forward(ctx, q, k, v, o, do, M, arith=None, cos=None, sin=None):
         dq, dk, dv, _, _, _ = kernels.attention_jvp_backward(
             q, k, v, None, None, None, o, None, M, None, dO=do, dTO=None, arithmetic=arith,
-            rope=None if cos is None else (cos, sin), **_backward_launches(q, arith))
+            rope=None if cos is None else (cos, sin))
         return dq, dk, dv
 
     @staticmethod
@@ -207,8 +204,7 @@ class SDPAJVPFusedBackwardFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, t_q, t_k, t_v, y, t_y, M, MU, d_y, d_t_y, arith=None, cos=None, sin=None):
         return kernels.attention_jvp_backward(q, k, v, t_q, t_k, t_v, y, t_y, M, MU, dO=d_y, dTO=d_t_y,
-                                              arithmetic=arith, rope=None if cos is None else (cos, sin),
-                                              **_backward_launches(q, arith))
+                                              arithmetic=arith, rope=None if cos is None else (cos, sin))
 
     @staticmethod
     def backward(ctx, *grads):
@@ -234,36 +230,54 @@ class SDPAPrimalFunction(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None
 
 
+def _cast_all(tensors, dtypes):
+    """``[t.to(dtype)]`` of present tensors with one launch for all that change: 2.5 instead of 5.5 us of host time each."""
+    out = [t if t is None or t.dtype == dtype else torch.empty_like(t, dtype=dtype) for t, dtype in zip(tensors, dtypes)]
+    pairs = [(o, t) for o, t in zip(out, tensors) if o is not t]
+    if pairs:
+        torch._foreach_copy_(*map(list, zip(*pairs)))
+    return out
+
+
 class SDPASeqMajorFunction(torch.autograd.Function):
     """:class:`SDPAFusedFunction` on ``[B,S,H,D]`` tensors, for tensors below the forward-mode level (see
-    :func:`_below_jvp`): the change of axes happens in here, where it leaves no autograd nodes."""
+    :func:`_below_jvp`): the change of axes, and the casts to the dtype ``compute`` and back, happen in here, where they
+    leave no autograd nodes.  With ``compute`` only its copies are kept for the backward: the caller may write to its
+    own tensors and to the result."""
 
     @staticmethod
-    def forward(ctx, q, k, v, t_q, t_k, t_v, arith, cos, sin):
+    def forward(ctx, q, k, v, t_q, t_k, t_v, arith, cos, sin, compute):
         ctx.rope = None if cos is None else (cos, sin)
-        ctx.arith = arith
+        ctx.arith, ctx.compute = arith, compute
+        given = (q, k, v, t_q, t_k, t_v)
+        ctx.dtypes = [t.dtype for t in given]
+        if compute is not None:
+            given = _cast_all(given, (compute,) * 6)
         B, S, H, _ = q.shape
-        y, t_y = (torch.empty((B, S, H, v.shape[-1]), device=q.device, dtype=q.dtype) for _ in range(2))
-        *inputs, o, to = (t.transpose(1, 2) for t in (q, k, v, t_q, t_k, t_v, y, t_y))
+        y, t_y = (torch.empty((B, S, H, v.shape[-1]), device=q.device, dtype=given[0].dtype) for _ in range(2))
+        *inputs, o, to = (t.transpose(1, 2) for t in (*given, y, t_y))
         _, _, M, MU, _ = kernels.attention_jvp_forward(*inputs, o=o, to=to, with_li=False, arithmetic=arith,
                                                        rope=ctx.rope)
-        ctx.save_for_backward(q, k, v, t_q, t_k, t_v, y, t_y, M, MU, *(ctx.rope or ()))
+        ctx.save_for_backward(*given, y, t_y, M, MU, *(ctx.rope or ()))
         ctx.rope = ctx.rope is not None
         ctx.set_materialize_grads(False)
-        return y, t_y
+        return (y, t_y) if compute is None else tuple(_cast_all((y, t_y), (q.dtype,) * 2))
 
     @staticmethod
     def backward(ctx, d_y, d_t_y):
         if d_y is None and d_t_y is None:
-            return (None,) * 9
+            return (None,) * 10
         *tensors, M, MU = ctx.saved_tensors[:10]
         rope = ctx.saved_tensors[10:] if ctx.rope else None
         with torch.no_grad():
             q, k, v, t_q, t_k, t_v, y, t_y = (t.transpose(1, 2) for t in tensors)
+            if ctx.compute is not None:
+                d_y, d_t_y = _cast_all((d_y, d_t_y), (ctx.compute,) * 2)
             d_y, d_t_y = (None if d is None else d.transpose(1, 2) for d in (d_y, d_t_y))
             grads = kernels.attention_jvp_backward(q, k, v, t_q, t_k, t_v, y, t_y, M, MU, dO=d_y, dTO=d_t_y,
-                                                   arithmetic=ctx.arith, rope=rope, **_backward_launches(q, ctx.arith))
-            return *(None if g is None else g.transpose(1, 2) for g in grads), None, None, None
+                                                   arithmetic=ctx.arith, rope=rope)
+            grads = _cast_all([None if g is None else g.transpose(1, 2) for g in grads], ctx.dtypes)
+            return *grads, None, None, None, None
 
 
 def _below_jvp(tensors):
@@ -315,13 +329,22 @@ def _sdpa_seq_major(q: Tensor, k: Tensor, v: Tensor, arith: Optional[str] = None
     return _seq_major_below(below, arith, cos, sin)
 
 
-def _seq_major_below(below, arith, cos, sin) -> Tensor:
+def _seq_major_below(below, arith=None, cos=None, sin=None, compute=None) -> Tensor:
     interpreter, duals = below
     with interpreter.lower():
         primals = [p for p, _ in duals]
         tangents = [torch.zeros_like(p) if t is None else t for p, t in duals]
-        y, t_y = SDPASeqMajorFunction.apply(*primals, *tangents, arith, cos, sin)
+        y, t_y = SDPASeqMajorFunction.apply(*primals, *tangents, arith, cos, sin, compute)
     return _dual_above(interpreter, y, t_y)
+
+
+@torch._dynamo.disable
+def _sdpa_cast_below(q: Tensor, k: Tensor, v: Tensor) -> Optional[Tensor]:
+    """The op in bfloat16 with its casts below the level of one ``torch.func.jvp``, or None where the casts have to be
+    seen.  (As duals each of the casts and its derivative would go through the transform: forward + backward at
+    B=64 H=12 L=128 D=64 690 against 370 us.)"""
+    below = _below_jvp((q, k, v)) if AUTOGRAD_WIRING != "reference" else None
+    return None if below is None else _seq_major_below(below, compute=torch.bfloat16)
 
 
 @torch._dynamo.disable
@@ -352,9 +375,10 @@ def _sdpa(q: Tensor, k: Tensor, v: Tensor, seq_major: bool, arith: Optional[str]
 
 def safe_sdpa_jvp(q: Tensor, k: Tensor, v: Tensor, precise: bool = False) -> Tensor:
     """``[B,S,H,D]`` wrapper with the reference's dtype policy (functional.py:310-332): inputs that
-    are neither bf16 nor fp16 are computed in bfloat16 and the result comes back in their dtype.  On a GPU the
-    casts of float32 tensors are folded into the kernels; ``FP32_CALLERS`` selects other routes (figures
-    beside it).  ``precise=True`` runs float32 inputs in the
+    are neither bf16 nor fp16 are computed in bfloat16 and the result comes back in their dtype, cast
+    with torch as in the reference; for float32 inputs ``FP32_CALLERS`` selects two other routes (the
+    library's own cast launches, or float32 tensors handed to the kernels as they are; figures beside
+    it).  ``precise=True`` runs float32 inputs in the
     library's fp32 mode instead (fp32 arithmetic throughout, about 1e-6 against fp64, much slower
     than the MFMA kernels)."""
     orig_dtype = q.dtype
@@ -366,9 +390,12 @@ def safe_sdpa_jvp(q: Tensor, k: Tensor, v: Tensor, precise: bool = False) -> Ten
         q, k, v = cast_tensors((q, k, v), torch.bfloat16)
         y = _sdpa(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), seq_major=True).transpose(1, 2)
         return cast_tensors(y, orig_dtype)
-    if fp32_bf16 and (FP32_CALLERS == "folded" or (FP32_CALLERS == "torch" and q.is_cuda)):
+    if fp32_bf16 and FP32_CALLERS == "folded":
         arith = "bf16"
     elif orig_dtype != torch.bfloat16 and orig_dtype != torch.float16 and not (precise and orig_dtype == torch.float32):
+        y = _sdpa_cast_below(q, k, v)
+        if y is not None:
+            return y
         q = q.to(torch.bfloat16)
         k = k.to(torch.bfloat16)
         v = v.to(torch.bfloat16)

@@ -11,8 +11,8 @@ Prints one JSON line.  A companion measurement, not the headline figure.
 ``--dtype fp32io`` and ``fp32cast`` time the two ways of serving a float32 caller with bf16 arithmetic
 (the dtype policy of semicat/jvp_utils/functional.py:318-332): the casts folded into the kernels
 (float32 tensors handed over as they are, SJVP_FP32_BF16), or torch casts around the 16-bit kernels
-(six casts in, two out in the forward; two in, six out in the backward), or (``fp32lib``) the
-library's own multi-tensor cast launches around them, which is what ``safe_sdpa_jvp`` does.
+(six casts in, two out in the forward; two in, six out in the backward), which is what ``safe_sdpa_jvp``
+does, or (``fp32lib``) the library's own multi-tensor cast launches around them.
 """
 from __future__ import annotations
 
@@ -63,7 +63,7 @@ def main(argv=None) -> int:
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
         if a.dtype == "fp32lib":
-            # the route safe_sdpa_jvp takes for float32 callers: the library's multi-tensor cast launches
+            # safe_sdpa_jvp's "library" route for float32 callers: the library's multi-tensor cast launches
             # ([B,S,H,D] views in and out) around the 16-bit kernels
             lo = torch.bfloat16
             bshd = lambda t: t.transpose(1, 2)
