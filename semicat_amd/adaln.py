@@ -48,11 +48,19 @@ def _mod_rows(t: Optional[Tensor]) -> Optional[Tensor]:
     return t.contiguous().clone()
 
 
-def _pair(like: Tensor, first: bool = True, second: bool = True, shape=None):
-    """Uninitialised memory for a tensor and its tangent (or either), side by side, so that a linear layer behind
-    takes both as the rows of one product."""
+def _outputs(like: Tensor, first: bool = True, second: bool = True, shape=None):
+    """Uninitialised memory for an output and its tangent (or either), each with a storage of its own: of a tangent whose
+    storage offset or size differs from its primal's, ``make_dual`` keeps a copy in zeroed memory of the whole
+    storage's size."""
     shape = like.shape if shape is None else shape
-    both = torch.empty((int(first) + int(second), *shape), device=like.device, dtype=like.dtype).unbind(0)
+    return tuple(torch.empty(shape, device=like.device, dtype=like.dtype) if wanted else None
+                 for wanted in (first, second))
+
+
+def _pair(like: Tensor, first: bool = True, second: bool = True):
+    """Uninitialised memory for the gradients of a tensor and its tangent (or either), side by side, so that the
+    reverse mode of a linear layer in front takes both as the rows of one product."""
+    both = torch.empty((int(first) + int(second), *like.shape), device=like.device, dtype=like.dtype).unbind(0)
     return (both[0] if first else None), (both[-1] if second else None)
 
 
@@ -101,8 +109,8 @@ class GatedNormFunction(torch.autograd.Function):
                      gate=_mod_rows(gate), tgate=_mod_rows(tgate), scale=_mod_rows(scale), tscale=_mod_rows(tscale),
                      shift=_mod_rows(shift), tshift=_mod_rows(tshift))
 
-        y, ty = _pair(x, a is not None, a is not None and jvp)
-        h, th = _pair(x, w is not None, w is not None and jvp)
+        y, ty = _outputs(x, a is not None, a is not None and jvp)
+        h, th = _outputs(x, w is not None, w is not None and jvp)
         _launch("sjvp_adaln_fwd", jvp, x.shape, eps, dict(names, y=y, ty=ty, h=h, th=th))
         if a is not None:  # the reverse mode reads y in the place of x
             names["tx"] = None
@@ -139,7 +147,7 @@ class GeluFunction(torch.autograd.Function):
     def forward(ctx, u, tu):
         ctx.set_materialize_grads(False)
         u, tu = _aligned(u), _aligned(tu)
-        y, ty = _pair(u, True, tu is not None)
+        y, ty = _outputs(u, True, tu is not None)
         _gelu(u, tu, None, None, y, ty, 0)
         ctx.save_for_backward(u, tu)
         return y, ty
@@ -183,7 +191,7 @@ class PackedAttentionFunction(torch.autograd.Function):
     def forward(ctx, qkv, t_qkv, cos, sin):
         ctx.set_materialize_grads(False)
         B, S, _, H, D = qkv.shape
-        out = _pair(qkv, True, t_qkv is not None, (B, S, H, D))
+        out = _outputs(qkv, True, t_qkv is not None, (B, S, H, D))
         o, to = (None if t is None else t.transpose(1, 2) for t in out)
         q, k, v = _heads(qkv)
         mu = None
@@ -212,22 +220,24 @@ class PackedAttentionFunction(torch.autograd.Function):
 
 
 class LinearFunction(torch.autograd.Function):
-    """``x w^T + b`` and ``tx w^T``, without a bias as one matrix product over the rows of both; in reverse mode one
-    product for both inputs and one, summed over both in fp32, for the weight.  Through the general dispatch forward mode adds products
-    with the absent tangents of weight and bias, zero fills and sums: 9 products per layer and step instead of 3.
+    """``x w^T + b`` and ``tx w^T``; in reverse mode one product for both inputs and one, summed over both in fp32, for the
+    weight.  Through the general dispatch forward mode adds products with the absent tangents of weight and bias,
+    zero fills and sums: 9 products per layer and step instead of 4.
     bf16 products on a bf16 copy of the fp32 weight, as autocast makes it."""
 
     @staticmethod
     def forward(ctx, x, tx, w, b):
         ctx.set_materialize_grads(False)
         w16 = w.to(x.dtype)
+        # two products, so that each output has its own storage (see _outputs); the bias enters the product's
+        # accumulator: added behind it, y would be rounded twice
+        y, ty = _outputs(x, shape=(*x.shape[:-1], w.shape[0]))
+        rows, t_rows = x.reshape(-1, w.shape[1]), tx.reshape(-1, w.shape[1])
         if b is None:
-            y, ty = torch.mm(_stacked(x, tx), w16.t()).view(2, *x.shape[:-1], w.shape[0]).unbind(0)
+            torch.mm(rows, w16.t(), out=y.view(-1, w.shape[0]))
         else:
-            # the bias enters the product's accumulator; added behind it, y would be rounded twice
-            y, ty = _pair(x, shape=(*x.shape[:-1], w.shape[0]))
-            torch.addmm(b.to(x.dtype), x.reshape(-1, w.shape[1]), w16.t(), out=y.view(-1, w.shape[0]))
-            torch.mm(tx.reshape(-1, w.shape[1]), w16.t(), out=ty.view(-1, w.shape[0]))
+            torch.addmm(b.to(x.dtype), rows, w16.t(), out=y.view(-1, w.shape[0]))
+        torch.mm(t_rows, w16.t(), out=ty.view(-1, w.shape[0]))
         ctx.save_for_backward(x, tx, w16)
         ctx.w_dtype = w.dtype
         return y, ty
