@@ -280,9 +280,11 @@ def _gelu(u, tu, dy, dty, y, ty, reverse) -> None:
 
 @torch._dynamo.disable
 def bare(*modules: nn.Module) -> bool:
-    """Whether calling the modules does nothing beyond their ``forward``: no hooks of any kind."""
+    """Whether calling the modules does nothing beyond the ``forward`` of their classes: no hooks of any kind, no
+    ``forward`` of the instance's own, no compiled call."""
     return not _module._has_any_global_hook() and not any(
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+        or "forward" in m.__dict__ or m._compiled_call_impl is not None for m in modules)
 
 
 @torch._dynamo.disable
