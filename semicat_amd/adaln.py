@@ -112,10 +112,10 @@ class GatedNormFunction(torch.autograd.Function):
         y, ty = _outputs(x, a is not None, a is not None and jvp)
         h, th = _outputs(x, w is not None, w is not None and jvp)
         _launch("sjvp_adaln_fwd", jvp, x.shape, eps, dict(names, y=y, ty=ty, h=h, th=th))
-        if a is not None:  # the reverse mode reads y in the place of x
-            names["tx"] = None
+        if a is not None:  # the reverse mode reads y in the place of x, and without a norm neither
+            names["x"] = names["tx"] = None
         ctx.names = list(names) + ["y", "ty"]
-        ctx.save_for_backward(*names.values(), y, ty)
+        ctx.save_for_backward(*names.values(), *((None, None) if w is None else (y, ty)))
         return y, h, ty, th
 
     @staticmethod
@@ -124,6 +124,8 @@ class GatedNormFunction(torch.autograd.Function):
         if dy is None and dh is None and dty is None and dth is None:
             return (None,) * 14
         t = dict(zip(ctx.names, ctx.saved_tensors))
+        if t["x"] is None:
+            t["x"] = t["a"]  # not read, but the call names its shape, dtype and device by x
         x, jvp = t["x"], ctx.jvp
         B, S, W = x.shape
         need = dict(zip(("x", "a", "gate", "scale", "shift", "w", "b", "tx", "ta", "tgate", "tscale", "tshift"),
