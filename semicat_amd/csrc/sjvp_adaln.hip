@@ -417,10 +417,14 @@ __global__ __launch_bounds__(256) void gelu_kernel(const void* u, const void* tu
     store8(ty, i8 * 8, tx);
 }
 
-template <int THREADS = 256, typename K, typename... A>
-int launch(K kernel, dim3 grid, void* stream, A... args) {
-    hipLaunchKernelGGL(kernel, grid, dim3(THREADS), 0, static_cast<hipStream_t>(stream), args...);
-    return hipGetLastError() == hipSuccess ? SJVP_OK : SJVP_ERR_LAUNCH;
+// Launch with the status of this launch only (not the thread's sticky last error); the arguments take the types of the
+// kernel's parameters.
+template <int THREADS = 256, typename... P>
+int launch(void (*kernel)(P...), dim3 grid, void* stream, std::type_identity_t<P>... params) {
+    void* args[] = {&params...};
+    const hipError_t rc = hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, dim3(THREADS), args, 0,
+                                          static_cast<hipStream_t>(stream));
+    return rc == hipSuccess ? SJVP_OK : SJVP_ERR_LAUNCH;
 }
 
 bool misaligned(const void* p, int bytes) { return reinterpret_cast<uintptr_t>(p) % bytes != 0; }
