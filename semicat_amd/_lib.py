@@ -132,8 +132,8 @@ def _load_host(lib: ctypes.CDLL):
         "_sjvp_host", path, loader=importlib.machinery.ExtensionFileLoader("_sjvp_host", path))
     host = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(host)
-    if host.build_id != "SJVP_BUILD_ID=" + _build.source_id():
-        raise RuntimeError(f"{path} was built from other sources than the ones in this tree")
+    if host.build_id != "SJVP_BUILD_ID=" + _build.host_id():
+        raise RuntimeError(f"{path} was built from other sources than the ones in this tree, or against another torch")
     host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in
                 (lib.sjvp_fwd, lib.sjvp_fwd_rotary, lib.sjvp_bwd_parts, lib.sjvp_bwd_rotary,
                  lib.sjvp_bwd_workspace_bytes)))

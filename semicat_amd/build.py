@@ -25,8 +25,8 @@ SOURCES = [os.path.join(CSRC, name) for name, _ in UNITS]
 # The host side of the entry points: a CPython extension against torch's headers, no device code.
 HOST_SOURCE = os.path.join(CSRC, "sjvp_host.cpp")
 HOST_PATH = os.path.join(PKG_DIR, "_sjvp_host.so")
-HEADERS = sorted(os.path.join(CSRC, n) for n in os.listdir(CSRC) if n.endswith(".hpp")) + [
-    os.path.join(os.path.dirname(PKG_DIR), "include", "sjvp.h")]
+ABI_HEADER = os.path.join(os.path.dirname(PKG_DIR), "include", "sjvp.h")
+HEADERS = sorted(os.path.join(CSRC, n) for n in os.listdir(CSRC) if n.endswith(".hpp")) + [ABI_HEADER]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++20", "-fPIC",
@@ -48,14 +48,31 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found (expected on PATH or at /opt/rocm/bin/hipcc)")
 
 
-def source_id() -> str:
-    """Identifier of the sources the library is built from: a hash of their contents and the flags."""
-    h = hashlib.sha256((" ".join(HIPCC_FLAGS) + repr(sorted(UNIT_FLAGS.items()))).encode())
-    for path in SOURCES + HEADERS + [HOST_SOURCE]:
+# Flags of the host extension (g++; the include and library folders of torch, ROCm and Python come on top).
+HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+HOST_LIBS = ["-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
+def _hash(what: str, paths) -> str:
+    h = hashlib.sha256(what.encode())
+    for path in paths:
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
+
+
+def source_id() -> str:
+    """Identifier of the sources the library is built from: a hash of their contents and the flags."""
+    return _hash(" ".join(HIPCC_FLAGS) + repr(sorted(UNIT_FLAGS.items())), SOURCES + HEADERS)
+
+
+def host_id() -> str:
+    """Identifier of what the host extension is built from: its source, the C ABI it calls, the flags, and the torch and
+    interpreter whose headers it is compiled against (inlined accessors read torch's object layouts)."""
+    import torch
+    against = (torch.__version__, torch.version.hip, torch.compiled_with_cxx11_abi(), sysconfig.get_config_var("SOABI"))
+    return _hash(repr((HOST_FLAGS, HOST_LIBS, against)), [HOST_SOURCE, ABI_HEADER])
 
 
 def built_id(path: str = LIB_PATH) -> str | None:
@@ -76,17 +93,15 @@ def _run(cmd, verbose):
         raise RuntimeError("the compiler failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
 
 
-def host_command(build_id: str) -> list[str]:
+def host_command() -> list[str]:
     """The command that builds the host extension (host code only: g++)."""
     import torch
     root = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    return [shutil.which("g++") or "c++", "-O2", "-std=c++20", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", build_id,
-            "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(root, "include"),
+    return [shutil.which("g++") or "c++", *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            f'-DSJVP_BUILD_ID="SJVP_BUILD_ID={host_id()}"', "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(root, "include"),
             "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + os.path.join(rocm, "include"),
-            HOST_SOURCE, "-o", HOST_PATH + ".tmp", "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu",
-            "-lc10_hip", "-lc10"]
+            HOST_SOURCE, "-o", HOST_PATH + ".tmp", "-L" + os.path.join(root, "lib"), *HOST_LIBS]
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> str:
@@ -102,7 +117,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
             cmds.append([hipcc, *HIPCC_FLAGS, *UNIT_FLAGS.get(name, []), *define, "-c", os.path.join(CSRC, name),
                          "-o", obj])
             objs.append(obj)
-    cmds.insert(0, host_command(build_id))
+    cmds.insert(0, host_command())
     jobs = jobs or min(len(cmds), os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda c: _run(c, verbose), cmds))
@@ -114,8 +129,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
 
 def is_stale() -> bool:
     """True when no library or no host extension is built or one was built from other sources than the ones in
-    the tree (compared by content, so copying or checking out the tree does not matter)."""
-    return any(built_id(path) != source_id() for path in (LIB_PATH, HOST_PATH))
+    the tree (compared by content, so copying or checking out the tree does not matter), or the extension
+    against another torch or interpreter than the running ones."""
+    return built_id(LIB_PATH) != source_id() or built_id(HOST_PATH) != host_id()
 
 
 if __name__ == "__main__":
