@@ -6,6 +6,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import threading
+import warnings
 
 from . import build as _build
 
@@ -70,14 +71,14 @@ class SjvpError(RuntimeError):
 def load() -> ctypes.CDLL:
     """Load the in-tree shared library; it is built first when it does not exist or is older than one
     of its sources (a stale binary is never loaded silently)."""
-    global _lib, _host
+    global _lib
     if _lib is not None:
         return _lib
     with _lock:
         if _lib is None:
             path = _build.LIB_PATH
-            if _build.is_stale():
-                _build.build()
+            if _build.library_is_stale():
+                _build.build_library()
             lib = ctypes.CDLL(path)
             vp, fp, i, i64p = ctypes.c_void_p, ctypes.POINTER(ctypes.c_float), ctypes.c_int, \
                 ctypes.POINTER(ctypes.c_int64)
@@ -119,7 +120,6 @@ def load() -> ctypes.CDLL:
             lib.sjvp_build_id.restype = ctypes.c_char_p
             if lib.sjvp_build_id().decode() != "SJVP_BUILD_ID=" + _build.source_id():
                 raise RuntimeError(f"{path} was built from other sources than the ones in this tree")
-            _host = _load_host(lib)
             _lib = lib
     return _lib
 
@@ -141,8 +141,22 @@ def _load_host(lib: ctypes.CDLL):
 
 
 def host():
-    """The host extension; loads the library first."""
-    return _host if _host is not None else (load() and _host)
+    """The host extension, built first where it is stale; False, after one warning, where it cannot be built or loaded.  The
+    library does not depend on it: calls then go through ctypes, with the same results."""
+    global _host
+    if _host is None:
+        lib = load()
+        with _lock:
+            if _host is None:
+                try:
+                    if _build.host_is_stale():
+                        _build.build_host()
+                    _host = _load_host(lib)
+                except (RuntimeError, ImportError, OSError) as error:
+                    warnings.warn(f"semicat_amd: calls take the slower ctypes path, the host extension is not usable: {error}",
+                                  RuntimeWarning)
+                    _host = False
+    return _host
 
 
 def strerror(status: int) -> str:

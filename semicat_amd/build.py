@@ -104,8 +104,15 @@ def host_command() -> list[str]:
             HOST_SOURCE, "-o", HOST_PATH + ".tmp", "-L" + os.path.join(root, "lib"), *HOST_LIBS]
 
 
-def build(verbose: bool = False, jobs: int | None = None) -> str:
-    """Compile every translation unit unconditionally and link; returns the path of the library."""
+def build_host(verbose: bool = False) -> str:
+    """Compile the host extension; returns its path."""
+    _run(host_command(), verbose)
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
+    return HOST_PATH
+
+
+def build_library(verbose: bool = False, jobs: int | None = None) -> str:
+    """Compile every translation unit of the C library unconditionally and link; needs nothing but hipcc."""
     hipcc = hipcc_path()
     os.makedirs(OBJ_DIR, exist_ok=True)
     cmds, objs = [], []
@@ -117,22 +124,40 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
             cmds.append([hipcc, *HIPCC_FLAGS, *UNIT_FLAGS.get(name, []), *define, "-c", os.path.join(CSRC, name),
                          "-o", obj])
             objs.append(obj)
-    cmds.insert(0, host_command())
     jobs = jobs or min(len(cmds), os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH + ".tmp", *objs], verbose)
     os.replace(LIB_PATH + ".tmp", LIB_PATH)
-    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     return LIB_PATH
 
 
+def build(verbose: bool = False, jobs: int | None = None) -> str:
+    """Compile everything unconditionally; returns the path of the library.  Where the host extension fails to build, the
+    library is there all the same when the error comes."""
+    with ThreadPoolExecutor(max_workers=1) as beside:
+        host = beside.submit(build_host, verbose)
+        path = build_library(verbose, jobs)
+        host.result()
+    return path
+
+
+def library_is_stale() -> bool:
+    """True when no library is built or one from other sources than the ones in the tree (compared by content, so copying
+    or checking out the tree does not matter)."""
+    return built_id(LIB_PATH) != source_id()
+
+
+def host_is_stale() -> bool:
+    """The same of the host extension, which is also stale beside another torch or interpreter than its own."""
+    return built_id(HOST_PATH) != host_id()
+
+
 def is_stale() -> bool:
-    """True when no library or no host extension is built or one was built from other sources than the ones in
-    the tree (compared by content, so copying or checking out the tree does not matter), or the extension
-    against another torch or interpreter than the running ones."""
-    return built_id(LIB_PATH) != source_id() or built_id(HOST_PATH) != host_id()
+    """True when the library or the host extension is."""
+    return library_is_stale() or host_is_stale()
 
 
 if __name__ == "__main__":
-    print(build(verbose=True))
+    print(build_library(verbose=True))
+    print(build_host(verbose=True))
