@@ -283,3 +283,12 @@ def test_companion_benchmarks_refuse_to_run_without_gpu(capsys):
     assert shape_bench.main(["--shape", "2", "2", "64", "64"]) == 2
     assert dit_bench.main([]) == 2
     assert "needs the GPU" in capsys.readouterr().err
+
+
+def test_training_step_is_not_offered_as_a_graph(capsys):
+    """Replays of a captured training step compute wrong bias gradients (PyTorch's multi-block sums record a memset): the
+    companion benchmark has no mode that runs them."""
+    from semicat_amd import dit_bench
+    with pytest.raises(SystemExit):
+        dit_bench.main(["--graph"])
+    assert "--graph" in capsys.readouterr().err
