@@ -232,6 +232,10 @@ int sjvp_rope(int n, const void* const* x, void* const* y, const int64_t* stride
  * multiples of 4, bf16 pointers 8-byte and w, b (fp32 [W]) 16-byte aligned; gradients of [B,W] inputs contiguous.
  * A tangent or cotangent that is NULL is zero; a gradient that is NULL is not stored.  sjvp_adaln_bwd() takes the inputs again,
  * with both a and w also y (and ty), and a workspace of sjvp_adaln_workspace_floats() floats (0: not served).
+ * A convention to know: for a cotangent on th the row mean and reciprocal deviation of y inside the LayerNorm's tangent
+ * are held constant, as PyTorch's reverse mode of its forward-mode layer_norm holds them, so that a network's gradients do
+ * not depend on which of the two computes it.  Finite differences of th give another gradient of y, and through it of
+ * x, a and gate.  The outputs, the other gradients and calls without a cotangent on th are not affected.
  * No counterpart in the reference, which uses separate PyTorch operations.
  */
 typedef struct sjvp_adaln {

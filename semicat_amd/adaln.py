@@ -11,7 +11,11 @@ parameters, outside every transform or inside exactly one ``torch.func.jvp``.  F
 transforms, tracing, dual numbers, tensor subclasses, modules with hooks) they return None and the caller runs its
 PyTorch operations.  To torch.compile they are opaque, like the attention op: a compiled network computes what the
 unwrapped one does.  Results are rounded where the PyTorch operations round (the residual stream) or where autocast would
-round behind them (the input of the next linear layer)."""
+round behind them (the input of the next linear layer).
+
+The reverse mode of the normalised rows' tangent holds the mean and the reciprocal deviation of its input constant: that
+is what PyTorch's layer_norm does there, and a network's gradients are the same whichever of the two computes it.  It is
+not the full derivative of the tangent."""
 from __future__ import annotations
 
 import ctypes
