@@ -140,7 +140,7 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
     const bool f32io = dtype == SJVP_FP32_BF16;
     const int m = f32io ? 2 : 1;
     VecCheck vc;
-    vc.unit = f32io || dtype == SJVP_FP32 ? 4 : 8;
+    vc.unit = f32io ? 4 : 8;
     for (int i = 0; i < SJVP_B_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
     if (dtype == SJVP_FP32) {
         BwdParamsF32 f{};
@@ -173,7 +173,7 @@ int run_bwd(int parts, const BwdTensors& t, float* ws, int B, int H, int Lq, int
         f.s4 = f.lse2 + (size_t)B * H * f.Lr;
         f.s7d = f.s4 + (size_t)B * H * f.Lr;
         f.scale = resolve_scale(scale, D);
-        return bwd_f32(f, B * H, has_do, has_g, parts, vc.ok && D % 4 == 0, static_cast<hipStream_t>(stream));
+        return bwd_f32(f, B * H, has_do, has_g, parts, static_cast<hipStream_t>(stream));
     }
 
     BwdParams p{};
@@ -304,7 +304,7 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
     const bool f32io = dtype == SJVP_FP32_BF16;
     const int m = f32io ? 2 : 1;
     VecCheck vc;
-    vc.unit = f32io || dtype == SJVP_FP32 ? 4 : 8;
+    vc.unit = f32io ? 4 : 8;
     for (int i = 0; i < SJVP_F_COUNT; ++i) vc.add(ptrs[i], strides + 3 * i);
     if (dtype == SJVP_FP32) {
         FwdParamsF32 f{};
@@ -327,7 +327,7 @@ int fwd_impl(const void* q, const void* k, const void* v, const void* tq, const 
         f.D = D;
         f.Lr = round_up(Lq, 128);
         f.scale = resolve_scale(scale, D);
-        return fwd_f32(f, B * H, jvp, vc.ok && D % 4 == 0, static_cast<hipStream_t>(stream));
+        return fwd_f32(f, B * H, jvp, static_cast<hipStream_t>(stream));
     }
 
     FwdParams p{};

@@ -1,4 +1,6 @@
 // Translation unit: the fp32 kernels of the correctness mode.
+#include <type_traits>
+
 #include "sjvp_f32.hpp"
 #include "sjvp_launch.hpp"
 
@@ -22,71 +24,73 @@ inline int blocks(int rows, int split) {
     return (rows + per - 1) / per;
 }
 
-template <int HD, bool JVP, bool VEC>
+template <int HD, bool JVP, F32Columns COLS>
 int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
     p.blocks = blocks(p.Lr, sp);  // the statistics cover rows below Lr
     const int grid = BH * p.blocks;
-    if (sp == 4) return launch(fwd_f32_kernel<HD, JVP, 4, VEC>, grid, 0, stream, p, kF32Threads);
-    return launch(fwd_f32_kernel<HD, JVP, 1, VEC>, grid, 0, stream, p, kF32Threads);
+    if (sp == 4) return launch(fwd_f32_kernel<HD, JVP, 4, COLS>, grid, 0, stream, p, kF32Threads);
+    return launch(fwd_f32_kernel<HD, JVP, 1, COLS>, grid, 0, stream, p, kF32Threads);
 }
 
-template <int HD, bool HAS_DO, bool HAS_G, bool VEC>
+template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
     p.q_blocks = blocks(p.Lq, sp);
     const int grid = BH * p.q_blocks;
-    if (sp == 4) return launch(bwd_row_f32_kernel<HD, HAS_DO, HAS_G, 4, VEC>, grid, 0, stream, p, kF32Threads);
-    return launch(bwd_row_f32_kernel<HD, HAS_DO, HAS_G, 1, VEC>, grid, 0, stream, p, kF32Threads);
+    if (sp == 4) return launch(bwd_row_f32_kernel<HD, HAS_DO, HAS_G, 4, COLS>, grid, 0, stream, p, kF32Threads);
+    return launch(bwd_row_f32_kernel<HD, HAS_DO, HAS_G, 1, COLS>, grid, 0, stream, p, kF32Threads);
 }
 
-template <int HD, bool HAS_DO, bool HAS_G, bool VEC>
+template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int col_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lk, p.Lq);
     p.k_blocks = blocks(p.Lk, sp);
     const int grid = BH * p.k_blocks;
-    if (sp == 4) return launch(bwd_col_f32_kernel<HD, HAS_DO, HAS_G, 4, VEC>, grid, 0, stream, p, kF32Threads);
-    return launch(bwd_col_f32_kernel<HD, HAS_DO, HAS_G, 1, VEC>, grid, 0, stream, p, kF32Threads);
+    if (sp == 4) return launch(bwd_col_f32_kernel<HD, HAS_DO, HAS_G, 4, COLS>, grid, 0, stream, p, kF32Threads);
+    return launch(bwd_col_f32_kernel<HD, HAS_DO, HAS_G, 1, COLS>, grid, 0, stream, p, kF32Threads);
 }
 
-template <int HD, bool HAS_DO, bool HAS_G, bool VEC>
+template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int bwd_one(const BwdParamsF32& p, int BH, int parts, hipStream_t stream) {
     if (parts & SJVP_BWD_ROW) {
-        const int rc = row_one<HD, HAS_DO, HAS_G, VEC>(p, BH, stream);
+        const int rc = row_one<HD, HAS_DO, HAS_G, COLS>(p, BH, stream);
         if (rc != SJVP_OK) return rc;
     }
-    return parts & SJVP_BWD_COL ? col_one<HD, HAS_DO, HAS_G, VEC>(p, BH, stream) : SJVP_OK;
+    return parts & SJVP_BWD_COL ? col_one<HD, HAS_DO, HAS_G, COLS>(p, BH, stream) : SJVP_OK;
 }
 
-template <int HD, bool VEC>
-int bwd_mode(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
-    if (has_do && has_g) return bwd_one<HD, true, true, VEC>(p, BH, parts, stream);
-    if (has_g) return bwd_one<HD, false, true, VEC>(p, BH, parts, stream);
-    return bwd_one<HD, true, false, VEC>(p, BH, parts, stream);
+// Calls f with the compiled head dimension and the form of its columns as constants.
+template <int HD, typename F>
+int by_columns(int D, F&& f) {
+    constexpr std::integral_constant<int, HD> hd{};
+    if (D == HD) return f(hd, std::integral_constant<F32Columns, kColumnsAll>{});
+    if (D % 4 == 0) return f(hd, std::integral_constant<F32Columns, kColumnsWhole>{});
+    return f(hd, std::integral_constant<F32Columns, kColumnsCut>{});
 }
-
-template <bool VEC>
-int fwd_hd(const FwdParamsF32& p, int BH, bool jvp, hipStream_t stream) {
-    if (p.D <= 32) return jvp ? fwd_one<32, true, VEC>(p, BH, stream) : fwd_one<32, false, VEC>(p, BH, stream);
-    if (p.D <= 64) return jvp ? fwd_one<64, true, VEC>(p, BH, stream) : fwd_one<64, false, VEC>(p, BH, stream);
-    return jvp ? fwd_one<128, true, VEC>(p, BH, stream) : fwd_one<128, false, VEC>(p, BH, stream);
-}
-
-template <bool VEC>
-int bwd_hd(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
-    if (p.D <= 32) return bwd_mode<32, VEC>(p, BH, has_do, has_g, parts, stream);
-    if (p.D <= 64) return bwd_mode<64, VEC>(p, BH, has_do, has_g, parts, stream);
-    return bwd_mode<128, VEC>(p, BH, has_do, has_g, parts, stream);
+template <typename F>
+int by_head(int D, F&& f) {
+    return D <= 32 ? by_columns<32>(D, f) : D <= 64 ? by_columns<64>(D, f) : by_columns<128>(D, f);
 }
 
 }  // namespace
 
-int fwd_f32(const FwdParamsF32& p, int BH, bool jvp, bool vec, hipStream_t stream) {
-    return vec ? fwd_hd<true>(p, BH, jvp, stream) : fwd_hd<false>(p, BH, jvp, stream);
+int fwd_f32(const FwdParamsF32& p, int BH, bool jvp, hipStream_t stream) {
+    return by_head(p.D, [&](auto hd, auto cols) {
+        constexpr int HD = decltype(hd)::value;
+        constexpr F32Columns COLS = decltype(cols)::value;
+        return jvp ? fwd_one<HD, true, COLS>(p, BH, stream) : fwd_one<HD, false, COLS>(p, BH, stream);
+    });
 }
 
-int bwd_f32(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, bool vec, hipStream_t stream) {
-    return vec ? bwd_hd<true>(p, BH, has_do, has_g, parts, stream) : bwd_hd<false>(p, BH, has_do, has_g, parts, stream);
+int bwd_f32(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+    return by_head(p.D, [&](auto hd, auto cols) {
+        constexpr int HD = decltype(hd)::value;
+        constexpr F32Columns COLS = decltype(cols)::value;
+        if (has_do && has_g) return bwd_one<HD, true, true, COLS>(p, BH, parts, stream);
+        if (has_g) return bwd_one<HD, false, true, COLS>(p, BH, parts, stream);
+        return bwd_one<HD, true, false, COLS>(p, BH, parts, stream);
+    });
 }
 
 }  // namespace sjvp

@@ -35,8 +35,6 @@
 
 namespace sjvp {
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
 constexpr int kF32Waves = 4;
 constexpr int kF32Threads = 64 * kF32Waves;
 constexpr int kF32Rows = 16;  // rows of one wave's tile, owned and streamed
@@ -101,22 +99,44 @@ __device__ __forceinline__ F32Place f32_place(int blocks, int H) {
     return w;
 }
 
-// W consecutive elements from column `col` of a row.  VEC: 16-byte aligned rows and D % 4 == 0.  MASK (D < HD):
-// zero where the column is >= D (such lanes read column 0).
+// How the columns of a row fill the head dimension HD that a kernel is compiled for.  An instance each: with the forms in
+// one kernel the registers of the cutting one spill into the loop of the one that has nothing to cut (backward at D = 128
+// 8 % longer).  Forward + backward at B=64 H=12 L=128, with single loads and the selects at the load / as here: D = 65 3396 /
+// 1072 us, 127 4675 / 1138, 68 1567 / 977, 64 off the 16-byte grid 722 / 511.
+enum F32Columns {
+    kColumnsAll,    // D == HD
+    kColumnsWhole,  // HD / 2 <= D < HD, D % 4 == 0: a piece of W columns exists or does not
+    kColumnsCut,    // HD / 2 <= D < HD
+};
+
+// W consecutive elements from column `col` of a row, as one load (fp32 needs no more than 4-byte alignment for it).
+// MASK: columns >= D become zero in two steps, so that the second one can be put where the load has arrived
+// anyway.  f32_ld reads W elements of the row in any case: a piece beyond D stands at column 0 (VEC: D % 4 == 0), or
+// every piece that does not lie below D whole is read as the row's last W elements.  f32_cut moves what
+// exists of the piece to its place and zeroes the rest.
+template <int W>
+struct F32Vec {
+    typedef float type __attribute__((ext_vector_type(W), aligned(4)));
+};
 template <int W, bool VEC, bool MASK>
 __device__ __forceinline__ void f32_ld(float* x, const float* row, int col, int D) {
-    typedef float vec_t __attribute__((ext_vector_type(W)));
-    if constexpr (VEC) {
-        const bool ok = !MASK || col < D;
-        const vec_t v = *reinterpret_cast<const vec_t*>(row + (ok ? col : 0));
+    const int at = !MASK ? col : VEC ? (col < D ? col : 0) : min(col, D - W);  // D >= 16
+    const typename F32Vec<W>::type v = *reinterpret_cast<const typename F32Vec<W>::type*>(row + at);
 #pragma unroll
-        for (int e = 0; e < W; ++e) x[e] = ok ? v[e] : 0.f;
-    } else {
+    for (int e = 0; e < W; ++e) x[e] = v[e];
+}
+template <int W, bool VEC>
+__device__ __forceinline__ void f32_cut(float* x, int col, int D) {
+    const int n = D - col;  // columns of the piece that exist, W or more: all
 #pragma unroll
-        for (int e = 0; e < W; ++e) {
-            const bool ok = !MASK || col + e < D;
-            const float v = row[ok ? col + e : 0];
-            x[e] = ok ? v : 0.f;
+    for (int e = 0; e < W; ++e) {
+        if constexpr (VEC) {
+            x[e] = n > 0 ? x[e] : 0.f;
+        } else {
+            float y = n >= W ? x[e] : 0.f;  // column col + e was read into x[e + W - n]
+#pragma unroll
+            for (int t = e + 1; t < W; ++t) y = n == W - (t - e) ? x[t] : y;
+            x[e] = y;
         }
     }
 }
@@ -124,7 +144,7 @@ __device__ __forceinline__ const float* f32_row(const float* base, int64_t sl, i
     return base + (int64_t)(row < L ? row : L - 1) * sl;  // rows beyond L stand for the last one: the caller masks
 }
 
-// Score-side operand of 16 rows: element (m, e) of lane l = X[row][16 m + 4 (l/16) + e].
+// Score-side operand of 16 rows: element (m, e) of lane l = X[row][16 m + 4 (l/16) + e], to be cut where MASK.
 template <int HD, bool VEC, bool MASK>
 __device__ __forceinline__ void f32_load_rows(f32x4* x, const float* base, int64_t sl, int row, int L, int D, int g) {
     const float* p = f32_row(base, sl, row, L);
@@ -135,10 +155,24 @@ __device__ __forceinline__ void f32_load_rows(f32x4* x, const float* base, int64
         x[m] = f32x4{v[0], v[1], v[2], v[3]};
     }
 }
-// The same for owned rows, zero beyond L.
-template <int HD, bool VEC>
+template <int HD, bool VEC, bool MASK>
+__device__ __forceinline__ void f32_cut_rows(f32x4* x, int D, int g) {
+    if constexpr (MASK) {
+        // (a class holds the head dimensions above half of HD: those pieces are whole)
+#pragma unroll
+        for (int m = HD / 32; m < HD / 16; ++m) {
+            if (!VEC && 16 * m + 16 <= D) continue;  // wave-uniform; the few selects of VEC cost less than a branch
+            float v[4] = {x[m][0], x[m][1], x[m][2], x[m][3]};
+            f32_cut<4, VEC>(v, 16 * m + 4 * g, D);
+            x[m] = f32x4{v[0], v[1], v[2], v[3]};
+        }
+    }
+}
+// The same for owned rows, cut, and zero beyond L.
+template <int HD, bool VEC, bool MASK>
 __device__ __forceinline__ void f32_load_own(f32x4* x, const float* base, int64_t sl, int row, int L, int D, int g) {
-    f32_load_rows<HD, VEC, true>(x, base, sl, row, L, D, g);
+    f32_load_rows<HD, VEC, MASK>(x, base, sl, row, L, D, g);
+    f32_cut_rows<HD, VEC, MASK>(x, D, g);
 #pragma unroll
     for (int m = 0; m < HD / 16; ++m)
         if (row >= L) x[m] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -159,6 +193,13 @@ __device__ __forceinline__ void f32_load_cols(float* x, const float* base, int64
 #pragma unroll
     for (int mm = 0; mm < F32Cols<HD>::MM; ++mm) f32_ld<W, VEC, MASK>(x + W * mm, p, 16 * W * mm + W * c, D);
 }
+template <int HD, bool VEC, bool MASK>
+__device__ __forceinline__ void f32_cut_cols(float* x, int D, int c) {
+    if constexpr (MASK) {
+        constexpr int W = F32Cols<HD>::W, mm = F32Cols<HD>::MM - 1;  // the others lie below half of HD
+        f32_cut<W, VEC>(x + W * mm, 16 * W * mm + W * c, D);
+    }
+}
 // Zero the operand of a row that does not exist (its tile entries are zero, but 0 * inf is not).
 template <int T>
 __device__ __forceinline__ void f32_zero_unless(float* x, bool valid) {
@@ -173,11 +214,12 @@ __device__ __forceinline__ void f32_store_cols(float* row, const float* x, int m
     constexpr int W = F32Cols<HD>::W;
     const int col = 16 * W * mm + 4 * W * g + W * j;
     if (!valid) return;
-    if constexpr (VEC && W == 4) {
-        if (col < D) *reinterpret_cast<f32x4*>(row + col) = f32x4{x[0], x[1], x[2], x[3]};
-    } else if constexpr (VEC) {
-        if (col < D) *reinterpret_cast<f32x2*>(row + col) = f32x2{x[0], x[1]};
-    } else {
+    if (col + W <= D) {
+        typename F32Vec<W>::type v;
+#pragma unroll
+        for (int e = 0; e < W; ++e) v[e] = x[e];
+        *reinterpret_cast<typename F32Vec<W>::type*>(row + col) = v;
+    } else if constexpr (!VEC) {
 #pragma unroll
         for (int e = 0; e < W; ++e)
             if (col + e < D) row[col + e] = x[e];
@@ -241,11 +283,12 @@ constexpr int f32_red_floats() { return SPLIT > 1 ? SPLIT * HD / 16 * 4 * 64 : 1
 
 // ---------------------------------------------------------------------------------------------
 // Forward (ryu_triton.py:188-291 in fp32): O, TO, lse, mu, li.
-template <int HD, bool JVP, int SPLIT, bool VEC>
+template <int HD, bool JVP, int SPLIT, F32Columns COLS>
 __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel(const FwdParamsF32 p) {
     __shared__ float red[f32_red_floats<HD, SPLIT>()];
     __shared__ float stat[SPLIT > 1 ? SPLIT * 3 * kF32Rows : 1];
     constexpr int M = HD / 16, T = HD / 16;
+    constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
     const F32Place w = f32_place<SPLIT>(p.blocks, p.H);
     const int qrow = w.row0 + w.n;
     const bool qvalid = qrow < p.Lq;
@@ -260,8 +303,8 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
         return;
     }
     f32x4 q[M], tq[M];
-    f32_load_own<HD, VEC>(q, p.q.head(w.b, w.h), p.q.sl, qrow, p.Lq, p.D, w.g);
-    if constexpr (JVP) f32_load_own<HD, VEC>(tq, p.tq.head(w.b, w.h), p.tq.sl, qrow, p.Lq, p.D, w.g);
+    f32_load_own<HD, VEC, MASK>(q, p.q.head(w.b, w.h), p.q.sl, qrow, p.Lq, p.D, w.g);
+    if constexpr (JVP) f32_load_own<HD, VEC, MASK>(tq, p.tq.head(w.b, w.h), p.tq.sl, qrow, p.Lq, p.D, w.g);
     f32x4 acc[T], tacc[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -275,83 +318,85 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
     const float sl2 = p.scale * kLog2e;
     float m_i = -INFINITY, l_i = 0.f, mu_i = 0.f;  // maximum (log2 units), exp-sum, sum p * S_dot of the lane's keys
 
-    auto walk = [&](auto mask_tag) {
-        constexpr bool MASK = decltype(mask_tag)::value;
-        f32x4 kr[M], tkr[M];
-        auto load = [&](int k0) {
-            f32_load_rows<HD, VEC, MASK>(kr, kb, p.k.sl, k0 + w.n, p.Lk, p.D, w.g);
-            if constexpr (JVP) f32_load_rows<HD, VEC, MASK>(tkr, tkb, p.tk.sl, k0 + w.n, p.Lk, p.D, w.g);
-        };
-        f32_walk<SPLIT>(w, p.Lk, load, [&](int k0, int next) {
-            const bool ragged = k0 + kF32Rows > p.Lk;  // wave-uniform
-            float v[4][T], tv[4][T];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32_load_cols<HD, VEC, MASK>(v[j], vb, p.v.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
-                if constexpr (JVP) f32_load_cols<HD, VEC, MASK>(tv[j], tvb, p.tv.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            f32x4 s = {0.f, 0.f, 0.f, 0.f}, ts = s, ts2 = s;
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s = mfma_f32(kr[m][e], q[m][e], s);
-                    if constexpr (JVP) {
-                        ts = mfma_f32(kr[m][e], tq[m][e], ts);
-                        ts2 = mfma_f32(tkr[m][e], q[m][e], ts2);
-                    }
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            if (next < p.Lk) load(next);
-            s *= sl2;
-            if (ragged) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool kvalid = k0 + 4 * w.g + j < p.Lk;
-                    s[j] = kvalid ? s[j] : -INFINITY;
-                    f32_zero_unless<T>(v[j], kvalid);
-                    if constexpr (JVP) f32_zero_unless<T>(tv[j], kvalid);
-                }
-            }
-            const float mloc = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-            if (__builtin_amdgcn_ballot_w64(mloc > m_i) != 0) {  // wave-uniform
-                const float m_new = fmaxf(m_i, group_max(mloc));  // finite: every tile holds at least one key
-                const float alpha = fast_exp2(m_i - m_new);
-                m_i = m_new;
-                l_i *= alpha;
-                mu_i *= alpha;
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    acc[t] *= alpha;
-                    if constexpr (JVP) tacc[t] *= alpha;
-                }
-            }
-            f32x4 pt = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s[j] = fast_exp2(s[j] - m_i);
-                l_i += s[j];
-                if constexpr (JVP) {
-                    pt[j] = s[j] * ((ts[j] + ts2[j]) * p.scale);
-                    mu_i += pt[j];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    acc[t] = mfma_f32(v[j][t], s[j], acc[t]);
-                    if constexpr (JVP) tacc[t] = mfma_f32(v[j][t], pt[j], tacc[t]);
-                }
-                if constexpr (JVP)
-#pragma unroll
-                    for (int t = 0; t < T; ++t) tacc[t] = mfma_f32(tv[j][t], s[j], tacc[t]);
-            }
-        });
+    f32x4 kr[M], tkr[M];
+    auto load = [&](int k0) {
+        f32_load_rows<HD, VEC, MASK>(kr, kb, p.k.sl, k0 + w.n, p.Lk, p.D, w.g);
+        if constexpr (JVP) f32_load_rows<HD, VEC, MASK>(tkr, tkb, p.tk.sl, k0 + w.n, p.Lk, p.D, w.g);
     };
-    if (p.D == HD) walk(std::false_type{});
-    else walk(std::true_type{});
+    f32_walk<SPLIT>(w, p.Lk, load, [&](int k0, int next) {
+        const bool ragged = k0 + kF32Rows > p.Lk;  // wave-uniform
+        float v[4][T], tv[4][T];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32_load_cols<HD, VEC, MASK>(v[j], vb, p.v.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
+            if constexpr (JVP) f32_load_cols<HD, VEC, MASK>(tv[j], tvb, p.tv.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        f32_cut_rows<HD, VEC, MASK>(kr, p.D, w.g);
+        if constexpr (JVP) f32_cut_rows<HD, VEC, MASK>(tkr, p.D, w.g);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f}, ts = s, ts2 = s;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s = mfma_f32(kr[m][e], q[m][e], s);
+                if constexpr (JVP) {
+                    ts = mfma_f32(kr[m][e], tq[m][e], ts);
+                    ts2 = mfma_f32(tkr[m][e], q[m][e], ts2);
+                }
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        if (next < p.Lk) load(next);
+        s *= sl2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32_cut_cols<HD, VEC, MASK>(v[j], p.D, w.n);
+            if constexpr (JVP) f32_cut_cols<HD, VEC, MASK>(tv[j], p.D, w.n);
+        }
+        if (ragged) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool kvalid = k0 + 4 * w.g + j < p.Lk;
+                s[j] = kvalid ? s[j] : -INFINITY;
+                f32_zero_unless<T>(v[j], kvalid);
+                if constexpr (JVP) f32_zero_unless<T>(tv[j], kvalid);
+            }
+        }
+        const float mloc = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        if (__builtin_amdgcn_ballot_w64(mloc > m_i) != 0) {  // wave-uniform
+            const float m_new = fmaxf(m_i, group_max(mloc));  // finite: every tile holds at least one key
+            const float alpha = fast_exp2(m_i - m_new);
+            m_i = m_new;
+            l_i *= alpha;
+            mu_i *= alpha;
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                acc[t] *= alpha;
+                if constexpr (JVP) tacc[t] *= alpha;
+            }
+        }
+        f32x4 pt = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s[j] = fast_exp2(s[j] - m_i);
+            l_i += s[j];
+            if constexpr (JVP) {
+                pt[j] = s[j] * ((ts[j] + ts2[j]) * p.scale);
+                mu_i += pt[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                acc[t] = mfma_f32(v[j][t], s[j], acc[t]);
+                if constexpr (JVP) tacc[t] = mfma_f32(v[j][t], pt[j], tacc[t]);
+            }
+            if constexpr (JVP)
+#pragma unroll
+                for (int t = 0; t < T; ++t) tacc[t] = mfma_f32(tv[j][t], s[j], tacc[t]);
+        }
+    });
     float l = group_sum(l_i), mu_un = group_sum(mu_i);
     if constexpr (SPLIT > 1) {
         // bring the waves' sums to one maximum (a wave without keys has m = -inf, factor 0)
@@ -399,10 +444,11 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
 
 // ---------------------------------------------------------------------------------------------
 // Row-owned backward: dQ (, dQ_dot) and the row sums for the column-owned kernel.
-template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, bool VEC>
+template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
 __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_row_f32_kernel(const BwdParamsF32 p) {
     __shared__ float red[f32_red_floats<HD, SPLIT>()];
     constexpr int M = HD / 16, T = HD / 16;
+    constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
     const F32Place w = f32_place<SPLIT>(p.q_blocks, p.H);
     if (w.row0 >= p.Lq) return;
     const int qrow = w.row0 + w.n;
@@ -410,16 +456,16 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
 
     f32x4 q[M], tq[M], g[M], dO[M], dq[T], dtq[T];
     float s4 = 0.f, s7d = 0.f;
-    f32_load_own<HD, VEC>(q, p.q.head(w.b, w.h), p.q.sl, qrow, p.Lq, p.D, w.g);
+    f32_load_own<HD, VEC, MASK>(q, p.q.head(w.b, w.h), p.q.sl, qrow, p.Lq, p.D, w.g);
     if constexpr (HAS_G) {
-        f32_load_own<HD, VEC>(tq, p.tq.head(w.b, w.h), p.tq.sl, qrow, p.Lq, p.D, w.g);
-        f32_load_own<HD, VEC>(g, p.dTO.head(w.b, w.h), p.dTO.sl, qrow, p.Lq, p.D, w.g);
+        f32_load_own<HD, VEC, MASK>(tq, p.tq.head(w.b, w.h), p.tq.sl, qrow, p.Lq, p.D, w.g);
+        f32_load_own<HD, VEC, MASK>(g, p.dTO.head(w.b, w.h), p.dTO.sl, qrow, p.Lq, p.D, w.g);
     }
-    if constexpr (HAS_DO) f32_load_own<HD, VEC>(dO, p.dO.head(w.b, w.h), p.dO.sl, qrow, p.Lq, p.D, w.g);
+    if constexpr (HAS_DO) f32_load_own<HD, VEC, MASK>(dO, p.dO.head(w.b, w.h), p.dO.sl, qrow, p.Lq, p.D, w.g);
     {
         f32x4 o[M], to[M];
-        f32_load_own<HD, VEC>(o, p.o.head(w.b, w.h), p.o.sl, qrow, p.Lq, p.D, w.g);
-        if constexpr (HAS_G) f32_load_own<HD, VEC>(to, p.to.head(w.b, w.h), p.to.sl, qrow, p.Lq, p.D, w.g);
+        f32_load_own<HD, VEC, MASK>(o, p.o.head(w.b, w.h), p.o.sl, qrow, p.Lq, p.D, w.g);
+        if constexpr (HAS_G) f32_load_own<HD, VEC, MASK>(to, p.to.head(w.b, w.h), p.to.sl, qrow, p.Lq, p.D, w.g);
 #pragma unroll
         for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -452,86 +498,92 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
     const float* tvb = HAS_G ? p.tv.head(w.b, w.h) : nullptr;
     const float sl2 = p.scale * kLog2e;
 
-    auto walk = [&](auto mask_tag) {
-        constexpr bool MASK = decltype(mask_tag)::value;
-        f32x4 kr[M], tkr[M], vr[M], tvr[M];
-        auto load = [&](int k0) {
-            f32_load_rows<HD, VEC, MASK>(kr, kb, p.k.sl, k0 + w.n, p.Lk, p.D, w.g);
-            if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tkr, tkb, p.tk.sl, k0 + w.n, p.Lk, p.D, w.g);
-            f32_load_rows<HD, VEC, MASK>(vr, vb, p.v.sl, k0 + w.n, p.Lk, p.D, w.g);
-            if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tvr, tvb, p.tv.sl, k0 + w.n, p.Lk, p.D, w.g);
-        };
-        f32_walk<SPLIT>(w, p.Lk, load, [&](int k0, int next) {
-            const bool ragged = k0 + kF32Rows > p.Lk;  // wave-uniform
-            float kc[4][T], tkc[4][T];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32_load_cols<HD, VEC, MASK>(kc[j], kb, p.k.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
-                if constexpr (HAS_G)
-                    f32_load_cols<HD, VEC, MASK>(tkc[j], tkb, p.tk.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            f32x4 s = zero, ts = zero, ts2 = zero, wt = zero, xy = zero, xy2 = zero;
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s = mfma_f32(kr[m][e], q[m][e], s);
-                    if constexpr (HAS_G) {
-                        ts = mfma_f32(kr[m][e], tq[m][e], ts);
-                        ts2 = mfma_f32(tkr[m][e], q[m][e], ts2);
-                    }
-                }
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if constexpr (HAS_DO) xy = mfma_f32(vr[m][e], dO[m][e], xy);
-                    if constexpr (HAS_G) {
-                        wt = mfma_f32(vr[m][e], g[m][e], wt);
-                        xy2 = mfma_f32(tvr[m][e], g[m][e], xy2);
-                    }
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            if (next < p.Lk) load(next);
-            f32x4 ds, dts = zero;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pj = fast_exp2(fmaf(s[j], sl2, -lse2));
-                if constexpr (HAS_G) {
-                    const float nn = fmaf(ts[j] + ts2[j], p.scale, -mu);
-                    dts[j] = pj * (wt[j] - s4);
-                    ds[j] = fmaf(dts[j], nn, pj * (xy[j] + xy2[j] - s7d));
-                } else {
-                    ds[j] = pj * (xy[j] - s7d);
-                }
-            }
-            if (ragged) {  // keys that do not exist contribute nothing
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool kvalid = k0 + 4 * w.g + j < p.Lk;
-                    ds[j] = kvalid ? ds[j] : 0.f;
-                    dts[j] = kvalid ? dts[j] : 0.f;
-                    f32_zero_unless<T>(kc[j], kvalid);
-                    if constexpr (HAS_G) f32_zero_unless<T>(tkc[j], kvalid);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    dq[t] = mfma_f32(kc[j][t], ds[j], dq[t]);
-                    if constexpr (HAS_G) dtq[t] = mfma_f32(kc[j][t], dts[j], dtq[t]);
-                }
-                if constexpr (HAS_G)
-#pragma unroll
-                    for (int t = 0; t < T; ++t) dq[t] = mfma_f32(tkc[j][t], dts[j], dq[t]);
-            }
-        });
+    f32x4 kr[M], tkr[M], vr[M], tvr[M];
+    auto load = [&](int k0) {
+        f32_load_rows<HD, VEC, MASK>(kr, kb, p.k.sl, k0 + w.n, p.Lk, p.D, w.g);
+        if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tkr, tkb, p.tk.sl, k0 + w.n, p.Lk, p.D, w.g);
+        f32_load_rows<HD, VEC, MASK>(vr, vb, p.v.sl, k0 + w.n, p.Lk, p.D, w.g);
+        if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tvr, tvb, p.tv.sl, k0 + w.n, p.Lk, p.D, w.g);
     };
-    if (p.D == HD) walk(std::false_type{});
-    else walk(std::true_type{});
+    f32_walk<SPLIT>(w, p.Lk, load, [&](int k0, int next) {
+        const bool ragged = k0 + kF32Rows > p.Lk;  // wave-uniform
+        float kc[4][T], tkc[4][T];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32_load_cols<HD, VEC, MASK>(kc[j], kb, p.k.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
+            if constexpr (HAS_G)
+                f32_load_cols<HD, VEC, MASK>(tkc[j], tkb, p.tk.sl, k0 + 4 * w.g + j, p.Lk, p.D, w.n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        f32_cut_rows<HD, VEC, MASK>(kr, p.D, w.g);
+        f32_cut_rows<HD, VEC, MASK>(vr, p.D, w.g);
+        if constexpr (HAS_G) {
+            f32_cut_rows<HD, VEC, MASK>(tkr, p.D, w.g);
+            f32_cut_rows<HD, VEC, MASK>(tvr, p.D, w.g);
+        }
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 s = zero, ts = zero, ts2 = zero, wt = zero, xy = zero, xy2 = zero;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s = mfma_f32(kr[m][e], q[m][e], s);
+                if constexpr (HAS_G) {
+                    ts = mfma_f32(kr[m][e], tq[m][e], ts);
+                    ts2 = mfma_f32(tkr[m][e], q[m][e], ts2);
+                }
+            }
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (HAS_DO) xy = mfma_f32(vr[m][e], dO[m][e], xy);
+                if constexpr (HAS_G) {
+                    wt = mfma_f32(vr[m][e], g[m][e], wt);
+                    xy2 = mfma_f32(tvr[m][e], g[m][e], xy2);
+                }
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        if (next < p.Lk) load(next);
+        f32x4 ds, dts = zero;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float pj = fast_exp2(fmaf(s[j], sl2, -lse2));
+            if constexpr (HAS_G) {
+                const float nn = fmaf(ts[j] + ts2[j], p.scale, -mu);
+                dts[j] = pj * (wt[j] - s4);
+                ds[j] = fmaf(dts[j], nn, pj * (xy[j] + xy2[j] - s7d));
+            } else {
+                ds[j] = pj * (xy[j] - s7d);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32_cut_cols<HD, VEC, MASK>(kc[j], p.D, w.n);
+            if constexpr (HAS_G) f32_cut_cols<HD, VEC, MASK>(tkc[j], p.D, w.n);
+        }
+        if (ragged) {  // keys that do not exist contribute nothing
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool kvalid = k0 + 4 * w.g + j < p.Lk;
+                ds[j] = kvalid ? ds[j] : 0.f;
+                dts[j] = kvalid ? dts[j] : 0.f;
+                f32_zero_unless<T>(kc[j], kvalid);
+                if constexpr (HAS_G) f32_zero_unless<T>(tkc[j], kvalid);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                dq[t] = mfma_f32(kc[j][t], ds[j], dq[t]);
+                if constexpr (HAS_G) dtq[t] = mfma_f32(kc[j][t], dts[j], dtq[t]);
+            }
+            if constexpr (HAS_G)
+#pragma unroll
+                for (int t = 0; t < T; ++t) dq[t] = mfma_f32(tkc[j][t], dts[j], dq[t]);
+        }
+    });
     f32_store<HD, VEC, SPLIT>(red, p.dq.head(w.b, w.h) + (int64_t)qrow * p.dq.sl, dq, p.scale, w, p.D, qvalid);
     if constexpr (HAS_G)
         f32_store<HD, VEC, SPLIT>(red, p.dtq.head(w.b, w.h) + (int64_t)qrow * p.dtq.sl, dtq, p.scale, w, p.D, qvalid);
@@ -539,21 +591,22 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
 
 // ---------------------------------------------------------------------------------------------
 // Column-owned backward: dK, dV (, dK_dot, dV_dot).
-template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, bool VEC>
+template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
 __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_col_f32_kernel(const BwdParamsF32 p) {
     __shared__ float red[f32_red_floats<HD, SPLIT>()];
     constexpr int M = HD / 16, T = HD / 16;
+    constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
     const F32Place w = f32_place<SPLIT>(p.k_blocks, p.H);
     if (w.row0 >= p.Lk) return;
     const int krow = w.row0 + w.n;
     const bool kvalid = krow < p.Lk;
 
     f32x4 k[M], v[M], tk[M], tv[M], dk[T], dv[T], dtk[T], dtv[T];
-    f32_load_own<HD, VEC>(k, p.k.head(w.b, w.h), p.k.sl, krow, p.Lk, p.D, w.g);
-    f32_load_own<HD, VEC>(v, p.v.head(w.b, w.h), p.v.sl, krow, p.Lk, p.D, w.g);
+    f32_load_own<HD, VEC, MASK>(k, p.k.head(w.b, w.h), p.k.sl, krow, p.Lk, p.D, w.g);
+    f32_load_own<HD, VEC, MASK>(v, p.v.head(w.b, w.h), p.v.sl, krow, p.Lk, p.D, w.g);
     if constexpr (HAS_G) {
-        f32_load_own<HD, VEC>(tk, p.tk.head(w.b, w.h), p.tk.sl, krow, p.Lk, p.D, w.g);
-        f32_load_own<HD, VEC>(tv, p.tv.head(w.b, w.h), p.tv.sl, krow, p.Lk, p.D, w.g);
+        f32_load_own<HD, VEC, MASK>(tk, p.tk.head(w.b, w.h), p.tk.sl, krow, p.Lk, p.D, w.g);
+        f32_load_own<HD, VEC, MASK>(tv, p.tv.head(w.b, w.h), p.tv.sl, krow, p.Lk, p.D, w.g);
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -569,120 +622,125 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
     const int64_t so = (int64_t)w.bh * p.Lr + 4 * w.g;  // rows below Lr exist in every statistic
     const float sl2 = p.scale * kLog2e;
 
-    auto walk = [&](auto mask_tag) {
-        constexpr bool MASK = decltype(mask_tag)::value;
-        f32x4 qr[M], tqr[M], gr[M], dor[M];
-        auto load = [&](int q0) {
-            f32_load_rows<HD, VEC, MASK>(qr, qb, p.q.sl, q0 + w.n, p.Lq, p.D, w.g);
-            if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tqr, tqb, p.tq.sl, q0 + w.n, p.Lq, p.D, w.g);
-        };
-        f32_walk<SPLIT>(w, p.Lq, load, [&](int q0, int next) {
-            const bool ragged = q0 + kF32Rows > p.Lq;  // wave-uniform
-            const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            const f32x4 lse2 = *reinterpret_cast<const f32x4*>(p.lse2 + so + q0);
-            const f32x4 s7d = *reinterpret_cast<const f32x4*>(p.s7d + so + q0);
-            f32x4 mu = zero, s4 = zero;
-            if constexpr (HAS_G) {
-                s4 = *reinterpret_cast<const f32x4*>(p.s4 + so + q0);
-                mu = *reinterpret_cast<const f32x4*>(p.mu + so + q0);
-            }
-            // output-side operands of row 4 g + j: Q, [G, Q_dot], [dO]; those of j + 1 are requested ahead of j's
-            // contractions (all four at once do not fit the registers)
-            float cq[2][T], cg[2][T], ctq[2][T], cdo[2][T];
-            auto load_cols = [&](int j, int u) {
-                const int row = q0 + 4 * w.g + j;
-                f32_load_cols<HD, VEC, MASK>(cq[u], qb, p.q.sl, row, p.Lq, p.D, w.n);
-                if constexpr (HAS_G) {
-                    f32_load_cols<HD, VEC, MASK>(cg[u], gb, p.dTO.sl, row, p.Lq, p.D, w.n);
-                    f32_load_cols<HD, VEC, MASK>(ctq[u], tqb, p.tq.sl, row, p.Lq, p.D, w.n);
-                }
-                if constexpr (HAS_DO) f32_load_cols<HD, VEC, MASK>(cdo[u], dob, p.dO.sl, row, p.Lq, p.D, w.n);
-            };
-            // G and dO rows are first used behind the Q, Q_dot contractions: no need to hold them from the last tile
-            if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(gr, gb, p.dTO.sl, q0 + w.n, p.Lq, p.D, w.g);
-            if constexpr (HAS_DO) f32_load_rows<HD, VEC, MASK>(dor, dob, p.dO.sl, q0 + w.n, p.Lq, p.D, w.g);
-            load_cols(0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            f32x4 s = zero, ts = zero, ts2 = zero, wt = zero, xy = zero, xy2 = zero;
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s = mfma_f32(qr[m][e], k[m][e], s);
-                    if constexpr (HAS_G) {
-                        ts = mfma_f32(tqr[m][e], k[m][e], ts);
-                        ts2 = mfma_f32(qr[m][e], tk[m][e], ts2);
-                    }
-                }
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if constexpr (HAS_G) {
-                        wt = mfma_f32(gr[m][e], v[m][e], wt);
-                        xy2 = mfma_f32(gr[m][e], tv[m][e], xy2);
-                    }
-                    if constexpr (HAS_DO) xy = mfma_f32(dor[m][e], v[m][e], xy);
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            load_cols(1, 1);
-            if (next < p.Lq) load(next);
-            f32x4 pr, pn = zero, ds, dts = zero;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pj = kvalid ? fast_exp2(fmaf(s[j], sl2, -lse2[j])) : 0.f;  // a padded key contributes nothing
-                pr[j] = pj;
-                if constexpr (HAS_G) {
-                    const float nn = fmaf(ts[j] + ts2[j], p.scale, -mu[j]);
-                    dts[j] = pj * (wt[j] - s4[j]);
-                    ds[j] = fmaf(dts[j], nn, pj * (xy[j] + xy2[j] - s7d[j]));
-                    pn[j] = pj * nn;
-                } else {
-                    ds[j] = pj * (xy[j] - s7d[j]);
-                }
-            }
-            if (ragged) {  // nor does a query that does not exist
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool qvalid = q0 + 4 * w.g + j < p.Lq;
-                    pr[j] = qvalid ? pr[j] : 0.f;
-                    pn[j] = qvalid ? pn[j] : 0.f;
-                    ds[j] = qvalid ? ds[j] : 0.f;
-                    dts[j] = qvalid ? dts[j] : 0.f;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int u = j & 1;
-                if (ragged) {
-                    const bool qvalid = q0 + 4 * w.g + j < p.Lq;
-                    f32_zero_unless<T>(cq[u], qvalid);
-                    if constexpr (HAS_G) {
-                        f32_zero_unless<T>(cg[u], qvalid);
-                        f32_zero_unless<T>(ctq[u], qvalid);
-                    }
-                    if constexpr (HAS_DO) f32_zero_unless<T>(cdo[u], qvalid);
-                }
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    dk[t] = mfma_f32(cq[u][t], ds[j], dk[t]);
-                    if constexpr (HAS_G) {
-                        dtk[t] = mfma_f32(cq[u][t], dts[j], dtk[t]);
-                        dv[t] = mfma_f32(cg[u][t], pn[j], dv[t]);
-                        dtv[t] = mfma_f32(cg[u][t], pr[j], dtv[t]);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    if constexpr (HAS_G) dk[t] = mfma_f32(ctq[u][t], dts[j], dk[t]);
-                    if constexpr (HAS_DO) dv[t] = mfma_f32(cdo[u][t], pr[j], dv[t]);
-                }
-                if (j < 2) load_cols(j + 2, u);
-            }
-        });
+    f32x4 qr[M], tqr[M], gr[M], dor[M];
+    auto load = [&](int q0) {
+        f32_load_rows<HD, VEC, MASK>(qr, qb, p.q.sl, q0 + w.n, p.Lq, p.D, w.g);
+        if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(tqr, tqb, p.tq.sl, q0 + w.n, p.Lq, p.D, w.g);
     };
-    if (p.D == HD) walk(std::false_type{});
-    else walk(std::true_type{});
+    f32_walk<SPLIT>(w, p.Lq, load, [&](int q0, int next) {
+        const bool ragged = q0 + kF32Rows > p.Lq;  // wave-uniform
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        const f32x4 lse2 = *reinterpret_cast<const f32x4*>(p.lse2 + so + q0);
+        const f32x4 s7d = *reinterpret_cast<const f32x4*>(p.s7d + so + q0);
+        f32x4 mu = zero, s4 = zero;
+        if constexpr (HAS_G) {
+            s4 = *reinterpret_cast<const f32x4*>(p.s4 + so + q0);
+            mu = *reinterpret_cast<const f32x4*>(p.mu + so + q0);
+        }
+        // output-side operands of row 4 g + j: Q, [G, Q_dot], [dO]; those of j + 1 are requested ahead of j's
+        // contractions (all four at once do not fit the registers)
+        float cq[2][T], cg[2][T], ctq[2][T], cdo[2][T];
+        auto load_cols = [&](int j, int u) {
+            const int row = q0 + 4 * w.g + j;
+            f32_load_cols<HD, VEC, MASK>(cq[u], qb, p.q.sl, row, p.Lq, p.D, w.n);
+            if constexpr (HAS_G) {
+                f32_load_cols<HD, VEC, MASK>(cg[u], gb, p.dTO.sl, row, p.Lq, p.D, w.n);
+                f32_load_cols<HD, VEC, MASK>(ctq[u], tqb, p.tq.sl, row, p.Lq, p.D, w.n);
+            }
+            if constexpr (HAS_DO) f32_load_cols<HD, VEC, MASK>(cdo[u], dob, p.dO.sl, row, p.Lq, p.D, w.n);
+        };
+        // G and dO rows are first used behind the Q, Q_dot contractions: no need to hold them from the last tile
+        if constexpr (HAS_G) f32_load_rows<HD, VEC, MASK>(gr, gb, p.dTO.sl, q0 + w.n, p.Lq, p.D, w.g);
+        if constexpr (HAS_DO) f32_load_rows<HD, VEC, MASK>(dor, dob, p.dO.sl, q0 + w.n, p.Lq, p.D, w.g);
+        load_cols(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        f32_cut_rows<HD, VEC, MASK>(qr, p.D, w.g);
+        if constexpr (HAS_G) f32_cut_rows<HD, VEC, MASK>(tqr, p.D, w.g);
+        f32x4 s = zero, ts = zero, ts2 = zero, wt = zero, xy = zero, xy2 = zero;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s = mfma_f32(qr[m][e], k[m][e], s);
+                if constexpr (HAS_G) {
+                    ts = mfma_f32(tqr[m][e], k[m][e], ts);
+                    ts2 = mfma_f32(qr[m][e], tk[m][e], ts2);
+                }
+            }
+        if constexpr (HAS_G) f32_cut_rows<HD, VEC, MASK>(gr, p.D, w.g);
+        if constexpr (HAS_DO) f32_cut_rows<HD, VEC, MASK>(dor, p.D, w.g);
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (HAS_G) {
+                    wt = mfma_f32(gr[m][e], v[m][e], wt);
+                    xy2 = mfma_f32(gr[m][e], tv[m][e], xy2);
+                }
+                if constexpr (HAS_DO) xy = mfma_f32(dor[m][e], v[m][e], xy);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        load_cols(1, 1);
+        if (next < p.Lq) load(next);
+        f32x4 pr, pn = zero, ds, dts = zero;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float pj = kvalid ? fast_exp2(fmaf(s[j], sl2, -lse2[j])) : 0.f;  // a padded key contributes nothing
+            pr[j] = pj;
+            if constexpr (HAS_G) {
+                const float nn = fmaf(ts[j] + ts2[j], p.scale, -mu[j]);
+                dts[j] = pj * (wt[j] - s4[j]);
+                ds[j] = fmaf(dts[j], nn, pj * (xy[j] + xy2[j] - s7d[j]));
+                pn[j] = pj * nn;
+            } else {
+                ds[j] = pj * (xy[j] - s7d[j]);
+            }
+        }
+        if (ragged) {  // nor does a query that does not exist
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool qvalid = q0 + 4 * w.g + j < p.Lq;
+                pr[j] = qvalid ? pr[j] : 0.f;
+                pn[j] = qvalid ? pn[j] : 0.f;
+                ds[j] = qvalid ? ds[j] : 0.f;
+                dts[j] = qvalid ? dts[j] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int u = j & 1;
+            f32_cut_cols<HD, VEC, MASK>(cq[u], p.D, w.n);
+            if constexpr (HAS_G) {
+                f32_cut_cols<HD, VEC, MASK>(cg[u], p.D, w.n);
+                f32_cut_cols<HD, VEC, MASK>(ctq[u], p.D, w.n);
+            }
+            if constexpr (HAS_DO) f32_cut_cols<HD, VEC, MASK>(cdo[u], p.D, w.n);
+            if (ragged) {
+                const bool qvalid = q0 + 4 * w.g + j < p.Lq;
+                f32_zero_unless<T>(cq[u], qvalid);
+                if constexpr (HAS_G) {
+                    f32_zero_unless<T>(cg[u], qvalid);
+                    f32_zero_unless<T>(ctq[u], qvalid);
+                }
+                if constexpr (HAS_DO) f32_zero_unless<T>(cdo[u], qvalid);
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                dk[t] = mfma_f32(cq[u][t], ds[j], dk[t]);
+                if constexpr (HAS_G) {
+                    dtk[t] = mfma_f32(cq[u][t], dts[j], dtk[t]);
+                    dv[t] = mfma_f32(cg[u][t], pn[j], dv[t]);
+                    dtv[t] = mfma_f32(cg[u][t], pr[j], dtv[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if constexpr (HAS_G) dk[t] = mfma_f32(ctq[u][t], dts[j], dk[t]);
+                if constexpr (HAS_DO) dv[t] = mfma_f32(cdo[u][t], pr[j], dv[t]);
+            }
+            if (j < 2) load_cols(j + 2, u);
+        }
+    });
     f32_store<HD, VEC, SPLIT>(red, p.dk.head(w.b, w.h) + (int64_t)krow * p.dk.sl, dk, p.scale, w, p.D, kvalid);
     f32_store<HD, VEC, SPLIT>(red, p.dv.head(w.b, w.h) + (int64_t)krow * p.dv.sl, dv, 1.0f, w, p.D, kvalid);
     if constexpr (HAS_G) {

@@ -78,9 +78,8 @@ int fwd_f32io(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 int bwd_fused_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, hipStream_t stream);
 int bwd_pair_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 
-// fp32 correctness mode: forward, and the row-owned + column-owned backward pair.  `vec`: every row of every
-// tensor starts on a 16-byte boundary and D % 4 == 0.
-int fwd_f32(const FwdParamsF32& p, int BH, bool jvp, bool vec, hipStream_t stream);
-int bwd_f32(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, bool vec, hipStream_t stream);
+// fp32 correctness mode: forward, and the row-owned + column-owned backward pair.
+int fwd_f32(const FwdParamsF32& p, int BH, bool jvp, hipStream_t stream);
+int bwd_f32(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 
 }  // namespace sjvp
