@@ -49,8 +49,10 @@ int check_common(int B, int H, int Lq, int Lk, int D, int dtype, float scale) {
     if (dtype < SJVP_BF16 || dtype > SJVP_FP32_BF16) return SJVP_ERR_DTYPE;
     if (B < 1 || H < 1 || Lq < 1 || Lk < 1) return SJVP_ERR_SHAPE;
     if (D < 16 || D > 128) return SJVP_ERR_HEAD_DIM;
-    // the finest launch takes one workgroup per 32 rows of the longer axis rounded up to 128 (the
-    // statistic rows): that grid, in 64 bits, has to fit the 31 bits of a launch dimension
+    // the finest launch whose grid grows with the problem takes one workgroup per 64 rows of the longer axis rounded up
+    // to 128 (the statistic rows); one per 32 is what has always been refused: in 64 bits, that grid has to fit the 31 bits
+    // of a launch dimension.  (The split fp32 launches take one per 16 rows, but only up to 2304 groups of 16
+    // rows, see split() in sjvp_f32.hip, and with the statistic rows at most 8 workgroups for each group.)
     const int64_t longer = Lq > Lk ? Lq : Lk;
     if (longer > (1LL << 30)) return SJVP_ERR_SHAPE;  // keeps the 32-bit round-ups below exact
     const int64_t blocks = (int64_t)B * H * ((longer + 127) / 128 * 4);

@@ -351,9 +351,8 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_row16_kernel(const BwdPa
 }
 
 // ---------------------------------------------------------------------------------------------
-// Column-owned kernel: a workgroup of four waves owns 64 keys.  PART selects the gradients that are
-// accumulated: 3 all four (HD <= 64), 1 dK (, dK_dot), 2 dV (, dV_dot) (HD = 128 runs as two launches
-// to stay inside the register file).  LDS: [ring of Q | [Q_dot | G] | [dO] | lse2, mu, s4, s7d stages]
+// Column-owned kernel: a workgroup of four waves owns 64 keys and accumulates all their gradients (HD <= 64; the
+// paired form below serves HD = 128).  LDS: [ring of Q | [Q_dot | G] | [dO] | lse2, mu, s4, s7d stages]
 // [sink]; the ring doubles as store staging after the last stage.
 template <int HD, int R, bool HAS_DO, bool HAS_G>
 struct Col16Smem {
@@ -365,12 +364,11 @@ struct Col16Smem {
     static_assert(R * slot >= kXWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART, int IO>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO>
 __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     using SM = Col16Smem<HD, R, HAS_DO, HAS_G>;
-    constexpr bool DO_K = (PART & 1) != 0, DO_V = (PART & 2) != 0;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
     constexpr int oTQ = SE, oG = 2 * SE, oDO = (HAS_G ? 3 : 1) * SE, oST = SM::nt * SE;
@@ -435,28 +433,28 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         const int64_t slice = b * p.k.sb + h * p.k.sh;
         const uint32_t at = ((uint32_t)krow * (uint32_t)p.k.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
         load_b_operands16_at<HD>(kB, p.k.ptr + slice, at);
-        if constexpr (DO_K) load_b_operands16_at<HD>(vB, p.v.ptr + slice, at);
+        load_b_operands16_at<HD>(vB, p.v.ptr + slice, at);
         if constexpr (HAS_G) {
             load_b_operands16_at<HD>(tkB, p.tk.ptr + slice, at);
-            if constexpr (DO_K) load_b_operands16_at<HD>(tvB, p.tv.ptr + slice, at);
+            load_b_operands16_at<HD>(tvB, p.tv.ptr + slice, at);
         }
         begin_copies();
     } else {
         load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
-        if constexpr (DO_K) load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
+        load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
         if constexpr (HAS_G) {
             load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
-            if constexpr (DO_K) load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
         }
         begin_copies();
     }
 #pragma unroll
     for (int c = 0; c < KC; ++c) {  // the own rows are awaited here
         asm volatile("" : "+v"(kB[c]));
-        if constexpr (DO_K) asm volatile("" : "+v"(vB[c]));
+        asm volatile("" : "+v"(vB[c]));
         if constexpr (HAS_G) {
             asm volatile("" : "+v"(tkB[c]));
-            if constexpr (DO_K) asm volatile("" : "+v"(tvB[c]));
+            asm volatile("" : "+v"(tvB[c]));
         }
     }
     if constexpr (DMA) {
@@ -493,21 +491,17 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             a.q = lds_a_rows16<HD>(sQ, t, c, n, g);
             if constexpr (HAS_G) {
                 a.tq = lds_a_rows16<HD>(sTQ, t, c, n, g);
-                if constexpr (DO_K) a.g = lds_a_rows16<HD>(sG, t, c, n, g);
+                a.g = lds_a_rows16<HD>(sG, t, c, n, g);
             }
-            if constexpr (HAS_DO && DO_K) a.d = lds_a_rows16<HD>(sDO, t, c, n, g);
+            if constexpr (HAS_DO) a.d = lds_a_rows16<HD>(sDO, t, c, n, g);
             return a;
         };
         auto load_grad = [&](int d) {
             AOps a;
-            if constexpr (DO_K) {
-                a.q = lds_a_tr16<HD>(sQ, 16 * d, lane);
-                if constexpr (HAS_G) a.tq = lds_a_tr16<HD>(sTQ, 16 * d, lane);
-            }
-            if constexpr (DO_V) {
-                if constexpr (HAS_G) a.g = lds_a_tr16<HD>(sG, 16 * d, lane);
-                if constexpr (HAS_DO) a.d = lds_a_tr16<HD>(sDO, 16 * d, lane);
-            }
+            a.q = lds_a_tr16<HD>(sQ, 16 * d, lane);
+            if constexpr (HAS_G) a.tq = lds_a_tr16<HD>(sTQ, 16 * d, lane);
+            if constexpr (HAS_G) a.g = lds_a_tr16<HD>(sG, 16 * d, lane);
+            if constexpr (HAS_DO) a.d = lds_a_tr16<HD>(sDO, 16 * d, lane);
             return a;
         };
         f32x4 s[2], ts[2], w[2], xy[2];
@@ -521,8 +515,8 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         // XY - s7d leave the matrix cores ready for use.
         auto load_sums = [&](int u) __attribute__((always_inline)) {
             const int r0 = 16 * u + 4 * g;  // register j of tile u is query 16 u + 4 g + j
-            if constexpr (HAS_G && DO_K) w[u] = *reinterpret_cast<const f32x4*>(sStat + 2 * kStageRows + r0);
-            if constexpr (DO_K) xy[u] = *reinterpret_cast<const f32x4*>(sStat + 3 * kStageRows + r0);
+            if constexpr (HAS_G) w[u] = *reinterpret_cast<const f32x4*>(sStat + 2 * kStageRows + r0);
+            xy[u] = *reinterpret_cast<const f32x4*>(sStat + 3 * kStageRows + r0);
         };
         auto load_stats = [&](int u) __attribute__((always_inline)) {
             const int r0 = 16 * u + 4 * g;
@@ -534,12 +528,10 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             if constexpr (HAS_G) {
                 ts[t] = T::mfma16(a.q, tkB[c], ts[t]);
                 ts[t] = T::mfma16(a.tq, kB[c], ts[t]);
-                if constexpr (DO_K) {
-                    w[t] = T::mfma16(a.g, vB[c], w[t]);
-                    xy[t] = T::mfma16(a.g, tvB[c], xy[t]);
-                }
+                w[t] = T::mfma16(a.g, vB[c], w[t]);
+                xy[t] = T::mfma16(a.g, tvB[c], xy[t]);
             }
-            if constexpr (HAS_DO && DO_K) xy[t] = T::mfma16(a.d, vB[c], xy[t]);
+            if constexpr (HAS_DO) xy[t] = T::mfma16(a.d, vB[c], xy[t]);
         };
         // in place: s -> P, ts -> P_dot, w -> dS_dot, xy -> dS  (rows beyond Lq are zero rows of Q,
         // Q_dot, G, dO with finite statistics: they contribute nothing)
@@ -550,13 +542,11 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
                 s[t][j] = pj;
                 if constexpr (HAS_G) {
                     const float nn = fmaf(ts[t][j], p.scale, -mu4[t][j]);
-                    if constexpr (DO_K) {
-                        const float dts = pj * w[t][j];
-                        w[t][j] = dts;
-                        xy[t][j] = fmaf(dts, nn, pj * xy[t][j]);
-                    }
-                    if constexpr (DO_V) ts[t][j] = pj * nn;
-                } else if constexpr (DO_K) {
+                    const float dts = pj * w[t][j];
+                    w[t][j] = dts;
+                    xy[t][j] = fmaf(dts, nn, pj * xy[t][j]);
+                    ts[t][j] = pj * nn;
+                } else {
                     xy[t][j] = pj * xy[t][j];
                 }
             }
@@ -595,31 +585,27 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         __builtin_amdgcn_sched_barrier(0);
         pointwise(1);
         u32x4 pB, dsB, pdB, dtsB;
-        if constexpr (DO_V) pB = pack_b16<T>(s[0], s[1]);
-        if constexpr (DO_K) dsB = pack_b16<T>(xy[0], xy[1]);
+        pB = pack_b16<T>(s[0], s[1]);
+        dsB = pack_b16<T>(xy[0], xy[1]);
         if constexpr (HAS_G) {
-            if constexpr (DO_V) pdB = pack_b16<T>(ts[0], ts[1]);
-            if constexpr (DO_K) dtsB = pack_b16<T>(w[0], w[1]);
+            pdB = pack_b16<T>(ts[0], ts[1]);
+            dtsB = pack_b16<T>(w[0], w[1]);
         }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             AOps nxt;
             if (d + 1 < DT) nxt = load_grad(d + 1);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (DO_K) {
-                dk[d] = T::mfma16(cur.q, dsB, dk[d]);
-                if constexpr (HAS_G) {
-                    dtk[d] = T::mfma16(cur.q, dtsB, dtk[d]);
-                    dk[d] = T::mfma16(cur.tq, dtsB, dk[d]);
-                }
+            dk[d] = T::mfma16(cur.q, dsB, dk[d]);
+            if constexpr (HAS_G) {
+                dtk[d] = T::mfma16(cur.q, dtsB, dtk[d]);
+                dk[d] = T::mfma16(cur.tq, dtsB, dk[d]);
             }
-            if constexpr (DO_V) {
-                if constexpr (HAS_G) {
-                    dtv[d] = T::mfma16(cur.g, pB, dtv[d]);
-                    dv[d] = T::mfma16(cur.g, pdB, dv[d]);
-                }
-                if constexpr (HAS_DO) dv[d] = T::mfma16(cur.d, pB, dv[d]);
+            if constexpr (HAS_G) {
+                dtv[d] = T::mfma16(cur.g, pB, dtv[d]);
+                dv[d] = T::mfma16(cur.g, pdB, dv[d]);
             }
+            if constexpr (HAS_DO) dv[d] = T::mfma16(cur.d, pB, dv[d]);
             __builtin_amdgcn_sched_barrier(0);
             cur = nxt;
         }
@@ -636,21 +622,17 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     if (!wave_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
     const int row0 = key0 + wave * 16;
-    if constexpr (DO_K) {
-        store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane);
-        if constexpr (HAS_G)
-            store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane);
-    }
-    if constexpr (DO_V) {
-        store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
-        if constexpr (HAS_G)
-            store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
-    }
+    store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane);
+    if constexpr (HAS_G)
+        store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane);
+    store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
+    if constexpr (HAS_G)
+        store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PART, int OCC, int IO = kIoDma>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdParams p) {
-    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, PART, IO>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The column-owned launch with the second launch of the row-owned kernel at its end: workgroups
@@ -662,7 +644,7 @@ template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = 
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks)
-        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, 3, IO>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, col_blocks);
     else
         bwd_row16_body<T, HD, R, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
 }

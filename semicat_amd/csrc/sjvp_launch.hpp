@@ -66,13 +66,13 @@ int launch(K kernel, int grid, int smem_bytes, hipStream_t stream, const P& para
 template <typename T> int fwd_vec(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 template <typename T> int fwd_any(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 
-// Backward: the single launch (short key axes, D <= 64; rows of any alignment), and the row + column pair on rows
-// as above.
+// Backward: the single launch (short key axes, D <= 64; 16-byte aligned 16-bit rows: bwd_select keeps others away from it),
+// and the row + column pair on rows as above.
 template <typename T> int bwd_fused(const BwdParams& p, int BH, bool has_do, bool has_g, hipStream_t stream);
 template <typename T> int bwd_pair_vec(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 template <typename T> int bwd_pair_any(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
 
-// fp32 tensors with bf16 arithmetic (the cast folded into the loads and stores).
+// fp32 tensors with bf16 arithmetic (the cast folded into the loads and stores; rows of any alignment).
 // The views carry fp32 pointers cast to elem_t* and strides counted in 2-byte units.
 int fwd_f32io(const FwdParams& p, int grid, bool jvp, hipStream_t stream);
 int bwd_fused_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, hipStream_t stream);

@@ -56,7 +56,7 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
             return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO>, grid + BH * (p.Lr / kXOwned16), smem,
                           stream, pr, kXThreads16);
         }
-        return launch(bwd_col16_kernel<T, HD, XR, HAS_DO, HAS_G, 3, 2, IO>, grid, CS::bytes, stream, p, kXThreads16);
+        return launch(bwd_col16_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO>, grid, CS::bytes, stream, p, kXThreads16);
     }
 }
 

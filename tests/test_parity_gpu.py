@@ -213,7 +213,7 @@ def test_unaligned_and_odd_head_dim_take_the_scalar_path(K):
     (200, 300, 64, 1), (129, 130, 128, 3), (64, 70, 80, 1)])                        # misaligned base pointers
 def test_register_staged_kernels_beyond_one_block(K, mode, Lq, Lk, D, offset):
     """Inputs the LDS-DMA kernels cannot take (head dimension not a multiple of 8, or base pointers
-    off the 16-byte grid) run on the 32-wide register-staged kernels: several blocks each way, ragged
+    off the 16-byte grid) run on the kernels that stage their copies through registers: several blocks each way, ragged
     ends, every head-dimension class (32, 64, 128 incl. the split column launches), all three
     cotangent modes, against the fp64 oracle."""
     dtype = torch.bfloat16 if (Lq + D) % 2 else torch.float16
@@ -951,7 +951,7 @@ def test_saturated_rows_on_the_row_and_column_pair(K, dtype, D, Lk, only_dto):
 @pytest.mark.parametrize("D,Lk,dtype,mode", [(80, 133, torch.float16, "auto"), (36, 70, torch.bfloat16, "auto"),
                                              (128, 133, torch.bfloat16, "always"), (64, 100, torch.bfloat16, "auto")])
 def test_saturated_rows_on_the_register_staged_pair(K, repair_mode, D, Lk, dtype, mode):
-    """The same repair in the 32-wide register-staged kernels (base pointers off the 16-byte grid, or a
+    """The same repair in the kernels that stage their copies through registers (base pointers off the 16-byte grid, or a
     head dimension that is not a multiple of 8): saturated rows, up to 0.999998 of the probability on one
     key, keep the gate for every output."""
     repair_mode(mode)
