@@ -364,8 +364,8 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
         }
         const float mloc = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
         if (__builtin_amdgcn_ballot_w64(mloc > m_i) != 0) {  // wave-uniform
-            const float m_new = fmaxf(m_i, group_max(mloc));  // finite: every tile holds at least one key
-            const float alpha = fast_exp2(m_i - m_new);
+            const float m_new = fmaxf(m_i, group_max(mloc));
+            const float alpha = m_i < m_new ? fast_exp2(m_i - m_new) : 1.f;  // (both may be -inf, see below)
             m_i = m_new;
             l_i *= alpha;
             mu_i *= alpha;
@@ -375,10 +375,13 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
                 if constexpr (JVP) tacc[t] *= alpha;
             }
         }
+        // A row whose keys so far all score -inf (products that overflow) has no maximum yet, and no probability: a
+        // wave of a split group may hold nothing but such keys.
+        const float base = m_i == -INFINITY ? 0.f : m_i;
         f32x4 pt = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            s[j] = fast_exp2(s[j] - m_i);
+            s[j] = fast_exp2(s[j] - base);
             l_i += s[j];
             if constexpr (JVP) {
                 pt[j] = s[j] * ((ts[j] + ts2[j]) * p.scale);
