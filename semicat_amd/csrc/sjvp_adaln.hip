@@ -363,7 +363,8 @@ __device__ __forceinline__ Gelu gelu(float u) {
     const float k = 0.7978845608028654f, c = 0.044715f;
     const float z1 = k * (1.f + 3.f * c * u * u), z2 = 6.f * k * c * u;
     const float T = 1.f - 2.f / (__expf(2.f * k * (u + c * u * u * u)) + 1.f), d = 1.f - T * T;
-    return {0.5f * u * (1.f + T), 0.5f * (1.f + T) + 0.5f * u * d * z1, d * z1 + 0.5f * u * d * (z2 - 2.f * T * z1 * z1)};
+    // (z1^2 alone overflows from 1e10 on, where d is 0)
+    return {0.5f * u * (1.f + T), 0.5f * (1.f + T) + 0.5f * u * d * z1, d * (z1 + 0.5f * u * z2) - u * T * (d * z1) * z1};
 }
 
 __device__ __forceinline__ void load8(const void* base, int64_t at, float* v) {
