@@ -8,6 +8,7 @@ whole network and then back-propagates through that derivative (semicat.py:152-1
 """
 from __future__ import annotations
 
+import contextlib
 from typing import Optional
 
 import torch
@@ -65,6 +66,14 @@ def vfm_loss(net: nn.Module, x0: Tensor, x1: Tensor, label_smoothing: float = 0.
                            label_smoothing=label_smoothing)
 
 
+def _uncached_autocast(kind: str):
+    """The caller's autocast context, where there is one, without its cache: casts of the weights made without gradients
+    must not enter it, a network call behind would take them from there and lose its weights' gradients."""
+    if not torch.amp.is_autocast_available(kind) or not torch.is_autocast_enabled(kind):
+        return contextlib.nullcontext()
+    return torch.autocast(kind, dtype=torch.get_autocast_dtype(kind), cache_enabled=False)
+
+
 def lag_self_distillation_loss(net: nn.Module, x0: Tensor, x1: Tensor, t: Optional[Tensor] = None,
                                s: Optional[Tensor] = None) -> Tensor:
     """``mean_{b,s} sum_v ((1 - t) d/dt x_{s,t} - softmax(net(x_{s,t}, t, t)) + x_{s,t})^2`` with the
@@ -79,11 +88,7 @@ def lag_self_distillation_loss(net: nn.Module, x0: Tensor, x1: Tensor, t: Option
     xst, dv = torch.func.jvp(lambda end: flow_map(net, xs, s, end, jvp_attention=True),
                              (t,), (torch.ones_like(t),))
     xst = xst.detach()
-    # Casts of the weights made without gradients must not enter the cache of the caller's autocast context: a network
-    # call behind this one would take them from there and lose its weights' gradients.
-    kind = xst.device.type
-    with torch.no_grad(), torch.autocast(kind, dtype=torch.get_autocast_dtype(kind),
-                                         enabled=torch.is_autocast_enabled(kind), cache_enabled=False):
+    with torch.no_grad(), _uncached_autocast(xst.device.type):
         target = net(xst, t, t).softmax(dim=-1)
     return ((1.0 - _per_sample(t, xst)) * dv - target + xst).pow(2).sum(dim=-1).mean()
 

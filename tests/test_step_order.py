@@ -26,3 +26,14 @@ def test_order_of_the_two_losses_under_autocast():
     a, b = grads(("vfm", "sd")), grads(("sd", "vfm"))
     for n in a:
         assert (a[n] - b[n]).norm() <= 2e-2 * a[n].norm(), n  # bf16: sums in another order
+
+
+def test_losses_on_a_device_without_autocast():
+    """Shapes and operation counts are taken on the meta device, which has no autocast at all."""
+    with torch.device("meta"):
+        net = DIT(vocab_size=20, hidden_size=32, cond_dim=16, n_blocks=1, n_heads=2, dropout=0.0, length=8,
+                  attention_override=math_attention, rotary="torch")
+        x0, x1, t = torch.randn(4, 8, 20), torch.zeros(4, 8, dtype=torch.long), torch.rand(4)
+        loss = ts.lag_self_distillation_loss(net, x0, x1, t=t, s=t * torch.rand(4)) + ts.vfm_loss(net, x0, x1, t=t)
+    loss.backward()
+    assert all(p.grad is not None and p.grad.shape == p.shape for p in net.parameters())
