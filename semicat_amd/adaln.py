@@ -19,19 +19,20 @@ not the full derivative of the tangent."""
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional
 
 import torch
 import torch.autograd.forward_ad as fwAD
 from torch import Tensor, nn
 from torch._C import _functorch
-from torch.autograd.function import once_differentiable
 from torch.nn.modules import module as _module
 
 from . import _lib, functional, kernels
 from .functional import _below_jvp, _dual_above
 
 _MOD = ("gate", "tgate", "scale", "tscale", "shift", "tshift")
+_ARGUMENTS = ("x", "a", "gate", "scale", "shift", "w", "b", "tx", "ta", "tgate", "tscale", "tshift")
 
 
 def _aligned(t: Optional[Tensor], bytes_: int = 16) -> Optional[Tensor]:
@@ -52,6 +53,11 @@ def _mod_rows(t: Optional[Tensor]) -> Optional[Tensor]:
     return t.contiguous().clone()
 
 
+def _laid_out(tensors: dict) -> dict:
+    """The named tensors as the launches read them; those that are so already are handed back themselves."""
+    return {n: _mod_rows(t) if n in _MOD else _aligned(t) for n, t in tensors.items()}
+
+
 def _outputs(like: Tensor, first: bool = True, second: bool = True, shape=None):
     """Uninitialised memory for an output and its tangent (or either), each with a storage of its own: of a tangent whose
     storage offset or size differs from its primal's, ``make_dual`` keeps a copy in zeroed memory of the whole
@@ -70,8 +76,10 @@ def _pair(like: Tensor, first: bool = True, second: bool = True):
 
 def _stacked(p: Tensor, t: Tensor) -> Tensor:
     """The rows of both tensors as one matrix, without a copy where they lie side by side."""
-    p, t = p.detach().contiguous(), t.detach().contiguous()
     rows, W = p.numel() // p.shape[-1], p.shape[-1]
+    if torch.is_grad_enabled():  # a recorded backward
+        return torch.cat((p.reshape(rows, W), t.reshape(rows, W)))
+    p, t = p.detach().contiguous(), t.detach().contiguous()
     if t.data_ptr() == p.data_ptr() + p.numel() * p.element_size() \
             and t.untyped_storage().data_ptr() == p.untyped_storage().data_ptr():
         return p.as_strided((2 * rows, W), (W, 1))
@@ -101,6 +109,61 @@ def _launch(fn, jvp: bool, shape, eps: float, tensors: dict) -> None:
         _lib.check(getattr(_lib.load(), fn)(ctypes.byref(p), int(jvp), stream))
 
 
+def _recorded(outputs, inputs, cotangents):
+    """Gradients of ``outputs`` as operations that autograd records: what a backward with ``create_graph`` takes in the
+    place of a launch, which has no derivative.  None for an input that needs none."""
+    at = [i for i, z in enumerate(inputs) if z is not None and z.requires_grad]
+    pairs = [(o, c.to(o.dtype)) for o, c in zip(outputs, cotangents) if c is not None and o.requires_grad]
+    grads = [None] * len(inputs)
+    if at and pairs:
+        found = torch.autograd.grad([o for o, _ in pairs], [inputs[i] for i in at], [c for _, c in pairs],
+                                    create_graph=True, allow_unused=True)
+        for i, g in zip(at, found):
+            grads[i] = g
+    return grads
+
+
+def _plus(*terms):
+    """Sum of the terms that are there."""
+    terms = [z for z in terms if z is not None]
+    return sum(terms[1:], terms[0]) if terms else None
+
+
+def _times(p, q):
+    return None if p is None or q is None else p * q
+
+
+def _gated_norm_recorded(t: dict, jvp: bool, eps: float, dy, dh, dty, dth) -> dict:
+    """The reverse mode of :class:`GatedNormFunction` in recorded PyTorch operations."""
+    out = {}
+    if t["w"] is not None:
+        gated = t["a"] is not None
+        y, ty = (t["y"], t["ty"]) if gated else (t["x"], t["tx"])
+        w, b, scale, shift, tscale, tshift = (t[n] for n in ("w", "b", "scale", "shift", "tscale", "tshift"))
+        y32, scale32 = y.float(), 1.0 + scale.float()
+        mean = y32.mean(-1, keepdim=True)
+        r = (y32.var(-1, unbiased=False, keepdim=True) + eps).rsqrt()
+        normed = (y32 - mean) * r * w + b
+        outputs, cotangents = [normed * scale32 + shift.float()], [dh]
+        if jvp:
+            mean, r = mean.detach(), r.detach()  # constants of the tangent, see the module's docstring
+            xhat = (y32 - mean) * r
+            centred = 0.0 * y32 if ty is None else ty.float() - ty.float().mean(-1, keepdim=True)
+            th = r * (centred - xhat * (centred * xhat).mean(-1, keepdim=True)) * w * scale32
+            outputs.append(_plus(th, _times(normed, tscale), tshift))
+            cotangents.append(dth)
+        g_y, g_ty, *rest = _recorded(outputs, (y, ty, scale, shift, w, b, tscale, tshift), cotangents)
+        out.update(zip(("scale", "shift", "w", "b", "tscale", "tshift"), rest))
+        dy, dty = _plus(dy, g_y), _plus(dty, g_ty)
+    out["x"], out["tx"] = dy, dty
+    if t["a"] is not None:
+        out["a"] = _plus(_times(dy, t["gate"]), _times(dty, t["tgate"]))
+        out["ta"] = _times(dty, t["gate"])
+        rows = _plus(_times(dy, t["a"]), _times(dty, t["ta"])), _times(dty, t["a"])
+        out["gate"], out["tgate"] = (None if z is None else z.float().sum(1, keepdim=True).to(z.dtype) for z in rows)
+    return out
+
+
 class GatedNormFunction(torch.autograd.Function):
     """``y = a gate + x`` and ``h = norm(y) (1 + scale) + shift`` with their tangents ``ty, th``.  Without ``a`` the
     norm reads ``x`` and ``y`` is None; without ``w`` there is no ``h``."""
@@ -109,31 +172,36 @@ class GatedNormFunction(torch.autograd.Function):
     def forward(ctx, eps, jvp, x, a, gate, scale, shift, w, b, tx, ta, tgate, tscale, tshift):
         ctx.set_materialize_grads(False)
         ctx.eps, ctx.jvp = eps, jvp
-        names = dict(x=_aligned(x), a=_aligned(a), tx=_aligned(tx), ta=_aligned(ta), w=_aligned(w), b=_aligned(b),
-                     gate=_mod_rows(gate), tgate=_mod_rows(tgate), scale=_mod_rows(scale), tscale=_mod_rows(tscale),
-                     shift=_mod_rows(shift), tshift=_mod_rows(tshift))
+        given = dict(x=x, a=a, tx=tx, ta=ta, w=w, b=b, gate=gate, tgate=tgate, scale=scale, tscale=tscale, shift=shift,
+                     tshift=tshift)
+        names = _laid_out(given)
+        # (copies made here are not part of the graph that a recorded backward continues)
+        ctx.as_given = all(names[n] is t for n, t in given.items())
 
         y, ty = _outputs(x, a is not None, a is not None and jvp)
         h, th = _outputs(x, w is not None, w is not None and jvp)
         _launch("sjvp_adaln_fwd", jvp, x.shape, eps, dict(names, y=y, ty=ty, h=h, th=th))
         if a is not None:  # the reverse mode reads y in the place of x, and without a norm neither
-            names["x"] = names["tx"] = None
-        ctx.names = list(names) + ["y", "ty"]
-        ctx.save_for_backward(*names.values(), *((None, None) if w is None else (y, ty)))
+            given["x"] = given["tx"] = None
+        ctx.names = list(given) + ["y", "ty"]
+        ctx.save_for_backward(*given.values(), *((None, None) if w is None else (y, ty)))
         return y, h, ty, th
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy, dh, dty, dth):
         if dy is None and dh is None and dty is None and dth is None:
             return (None,) * 14
         t = dict(zip(ctx.names, ctx.saved_tensors))
+        if torch.is_grad_enabled():
+            out = _gated_norm_recorded(t, ctx.jvp, ctx.eps, dy, dh, dty, dth)
+            return (None, None, *(out.get(n) if need else None for n, need in zip(_ARGUMENTS, ctx.needs_input_grad[2:])))
+        if not ctx.as_given:
+            t.update(_laid_out({n: z for n, z in t.items() if n not in ("y", "ty")}))
         if t["x"] is None:
             t["x"] = t["a"]  # not read, but the call names its shape, dtype and device by x
         x, jvp = t["x"], ctx.jvp
         B, S, W = x.shape
-        need = dict(zip(("x", "a", "gate", "scale", "shift", "w", "b", "tx", "ta", "tgate", "tscale", "tshift"),
-                        ctx.needs_input_grad[2:]))
+        need = dict(zip(_ARGUMENTS, ctx.needs_input_grad[2:]))
         out = {}
         for n in ("x", "a"):
             out["d" + n], out["dt" + n] = _pair(x, need[n], need["t" + n])
@@ -152,18 +220,25 @@ class GeluFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, tu):
         ctx.set_materialize_grads(False)
+        ctx.save_for_backward(u, tu)
         u, tu = _aligned(u), _aligned(tu)
         y, ty = _outputs(u, True, tu is not None)
         _gelu(u, tu, None, None, y, ty, 0)
-        ctx.save_for_backward(u, tu)
         return y, ty
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy, dty):
         if dy is None and dty is None:
             return None, None
         u, tu = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            x, k, c = u.float(), math.sqrt(2.0 / math.pi), 0.044715
+            T = torch.tanh(k * (x + c * x ** 3))
+            y = 0.5 * x * (1.0 + T)
+            slope = 0.5 * (1.0 + T) + 0.5 * x * (1.0 - T * T) * k * (1.0 + 3.0 * c * x * x)
+            outputs = (y,) if tu is None else (y, slope * tu.float())
+            return tuple(_recorded(outputs, (u, tu), (dy, dty)))
+        u, tu = _aligned(u), _aligned(tu)
         du, dtu = _pair(u, True, tu is not None and dty is not None)
         _gelu(u, tu, _aligned(dy), _aligned(dty), du, dtu, 1)
         return du, dtu
@@ -180,7 +255,6 @@ class ChunkFunction(torch.autograd.Function):
         return tuple(x.detach()[:, None].chunk(n, dim=2))
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, *grads):
         some = next((g for g in grads if g is not None), None)
         if some is None:
@@ -210,19 +284,48 @@ class PackedAttentionFunction(torch.autograd.Function):
         return out
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, d_y, d_ty):
-        qkv, t_qkv, cos, sin, y, ty, lse, mu = ctx.saved_tensors
         if d_y is None and d_ty is None:
             return (None,) * 4
-        d_qkv, d_t_qkv = _pair(qkv, True, d_ty is not None)
-        o, to, d_o, d_to = (None if t is None else t.transpose(1, 2) for t in (y, ty, d_y, d_ty))
-        tangents = (None,) * 3 if d_ty is None else _heads(t_qkv)
-        if d_ty is None:
-            to = mu = None
-        kernels.attention_jvp_backward(*_heads(qkv), *tangents, o, to, lse, mu, dO=d_o, dTO=d_to, rope=(cos, sin),
-                                       grads=(*_heads(d_qkv), *((None,) * 3 if d_ty is None else _heads(d_t_qkv))))
-        return d_qkv, d_t_qkv, None, None
+        run = PackedAttentionBackwardFunction.apply if torch.is_grad_enabled() else _packed_attention_backward
+        return *run(d_y, d_ty, *ctx.saved_tensors), None, None
+
+
+def _packed_attention_backward(d_y, d_ty, qkv, t_qkv, cos, sin, y, ty, lse, mu):
+    """Gradients for the cotangents of both outputs in one launch (either may be None)."""
+    d_qkv, d_t_qkv = _pair(qkv, True, d_ty is not None)
+    o, to, d_o, d_to = (None if t is None else t.transpose(1, 2) for t in (y, ty, d_y, d_ty))
+    tangents = (None,) * 3 if d_ty is None else _heads(t_qkv)
+    if d_ty is None:
+        to = mu = None
+    kernels.attention_jvp_backward(*_heads(qkv), *tangents, o, to, lse, mu, dO=d_o, dTO=d_to, rope=(cos, sin),
+                                   grads=(*_heads(d_qkv), *((None,) * 3 if d_ty is None else _heads(d_t_qkv))))
+    return d_qkv, d_t_qkv
+
+
+class PackedAttentionBackwardFunction(torch.autograd.Function):
+    """The same where a graph of the backward is asked for."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        return _packed_attention_backward(*args)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise NotImplementedError("double backward of the attention-JVP op is not implemented")
+
+
+class _CastOf(torch.autograd.Function):
+    """``w16``, the values that were cast from ``w``, as part of the graph of ``w``."""
+
+    @staticmethod
+    def forward(ctx, w, w16):
+        ctx.dtype = w.dtype
+        return w16.view_as(w16)
+
+    @staticmethod
+    def backward(ctx, g):
+        return g.to(ctx.dtype), None
 
 
 class LinearFunction(torch.autograd.Function):
@@ -246,14 +349,16 @@ class LinearFunction(torch.autograd.Function):
         torch.mm(t_rows, w16.t(), out=ty.view(-1, w.shape[0]))
         ctx.save_for_backward(x, tx, w16)
         ctx.w_dtype = w.dtype
+        ctx.weight = w  # for its place in the graph; its values may have changed since
         return y, ty
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dy, dty):
         x, tx, w16 = ctx.saved_tensors
         if dy is None and dty is None:
             return (None,) * 4
+        if torch.is_grad_enabled():
+            w16 = _CastOf.apply(ctx.weight, w16)
         dx = dtx = dw = db = None
         need_x, need_tx, need_w, need_b = ctx.needs_input_grad
         if dy is not None and dty is not None:
