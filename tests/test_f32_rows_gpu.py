@@ -45,15 +45,18 @@ def test_every_head_dimension_among_nan(first):
 def test_unaligned_rows_cost_what_aligned_rows_cost(D, offset, like):
     from semicat_amd import kernels as K
 
-    def us(D, offset):
+    def launches(D, offset):
         B, H, L = 64, 12, 128
         make = lambda: torch.randn(B * H * L * D + offset, device="cuda")[offset:].view(B, H, L, D)
         x = [make() for _ in range(8)]
         fwd, (o, to, lse, mu, _) = K.plan_forward(*x[:6], with_li=False)
         fwd()
         bwd, _ = K.plan_backward(*x[:6], o, to, lse, mu, dO=x[6], dTO=x[7])
-        best = float("inf")
-        for _ in range(5):
+        return fwd, bwd
+
+    both, best = [launches(D, offset), launches(like, 0)], [float("inf")] * 2
+    for _ in range(8):  # in turn, so that clocks and neighbours meet both
+        for i, (fwd, bwd) in enumerate(both):
             e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
             e[0].record()
             for _ in range(4):
@@ -61,9 +64,6 @@ def test_unaligned_rows_cost_what_aligned_rows_cost(D, offset, like):
                 bwd()
             e[1].record()
             torch.cuda.synchronize()
-            best = min(best, e[0].elapsed_time(e[1]) * 250)
-        return best
-
-    a, b = us(D, offset), us(like, 0)
-    print(f"[f32 rows] D={D}+{offset} {a:.0f} us, D={like} {b:.0f} us")
-    assert a < 1.25 * b
+            best[i] = min(best[i], e[0].elapsed_time(e[1]) * 250)
+    print(f"[f32 rows] D={D}+{offset} {best[0]:.0f} us, D={like} {best[1]:.0f} us")
+    assert best[0] < 1.25 * best[1]
