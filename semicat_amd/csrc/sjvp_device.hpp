@@ -104,6 +104,16 @@ __device__ __forceinline__ bool workgroup_barrier_or(bool pred) {
     return __syncthreads_or(pred) != 0;
 }
 
+// Exchange through LDS among the lanes of ONE wave: the wave's LDS instructions run in order, but the compiler sees
+// lanes one by one, and where the reads stand under a condition it may send the lanes outside it ahead, to
+// writes that come behind the reads (seen: the next tensor's tile of the row stores written by the lanes
+// without a row before the others had read the last one).  No instruction.
+__device__ __forceinline__ void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 

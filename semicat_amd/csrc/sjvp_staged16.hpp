@@ -208,11 +208,13 @@ __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, i
         for (int dt = 0; dt < HD / 16; ++dt) store_f32x4(row, acc[dt] * mul, 16 * dt + 4 * g, D);
     } else {
         constexpr int P = StoreStage16<HD>::pitch;
+        wave_exchange();  // the tile's last readers are done
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             u32x2 val = {T::pack2(acc[dt][0] * mul, acc[dt][1] * mul), T::pack2(acc[dt][2] * mul, acc[dt][3] * mul)};
             *reinterpret_cast<u32x2*>(stage + n * P + 16 * dt + 4 * g) = val;
         }
+        wave_exchange();
         constexpr int CH = HD / 8;
         constexpr int RPI = 64 / CH;
 #pragma unroll
