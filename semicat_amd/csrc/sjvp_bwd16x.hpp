@@ -4,6 +4,10 @@
 //   bwd_row16_kernel   4 waves x 16 queries; streams K, V (, K_dot, V_dot)        -> dQ (, dQ_dot)
 //   bwd_col16_kernel   4 waves x 16 keys;    streams Q (, Q_dot, G) (, dO) + stats -> dK, dV (, dK_dot, dV_dot)
 // (workgroups of four waves: at 160-200 registers two or three of them share a CU)
+// NC = 2: a wave owns 2 x 16 positions and every operand that it reads from LDS feeds twice as many matrix instructions
+// (the transposing reads deliver 128 bytes per clock and CU, one operand of 1 KB in the time of half a matrix
+// instruction of each of its four SIMDs: with 16 positions and no tangents every operand feeds one instruction, and the
+// LDS is what such a kernel waits for).  Only where 256 registers hold it: measured beside the dispatch.
 // The owned rows are loaded straight into registers (each lane its own 16-byte pieces), the streamed
 // side goes through an LDS ring filled by LDS-DMA (IO = kIoDma), or, where the rows do not start on 16-byte boundaries
 // or hold fp32 elements, through registers one stage ahead (sjvp_staged16.hpp).  Each gradient is accumulated in fp32 registers by
@@ -78,7 +82,7 @@ struct Row16Smem {
 
 // (the body of the kernel as a function of the workgroup's index and the number of workgroups, so that the
 // second launch can also ride at the end of the column-owned launch, see bwd_col16_repair_kernel)
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO, int NC = 1>
 __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     constexpr bool SECOND = PASS == 2;   // second launch: sums from the workspace, flagged workgroups only
@@ -94,7 +98,9 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15;
     const int g = lane >> 4;
-    const int q_blocks = p.Lr / kXOwned16;  // statistic rows up to Lr are all covered
+    static_assert(NC == 1 || PASS == 0, "the passes of the repair go by blocks of 64 rows");
+    constexpr int OWNED = NC * kXOwned16;
+    const int q_blocks = p.Lr / OWNED;  // statistic rows up to Lr are all covered
     // Workgroups run through the heads in descending order: this launch follows the forward, which
     // ran through them in ascending order, so it starts on what the caches still hold (the
     // column-owned launch after it ascends again).
@@ -102,43 +108,53 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     const int bh = bid / q_blocks;
     const int qb = bid % q_blocks;
     const int b = bh / p.H, h = bh % p.H;
-    const int q0 = qb * kXOwned16;
-    const int qrow = q0 + wave * 16 + n;
-    const bool qvalid = qrow < p.Lq;
-    const bool wave_active = (q0 + wave * 16) < p.Lq;
+    const int q0 = qb * OWNED;
+    const int wrow = q0 + wave * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
+    const bool wave_active = wrow < p.Lq;
     if constexpr (SECOND) {
         if (p.rowfix == 1 && p.flags[bid] == 0) return;  // nothing to repair in this workgroup's rows
     }
 
     // The own rows are requested first, as B operands; the set-up of the stage copies runs while they travel.
-    u32x4 qB[KC], tqB[KC], gB[KC], doB[KC];
-    u32x4 oR[KC], toR[KC];
-    float s4 = 0.f, s7d = 0.f;
-    const int64_t so = (int64_t)bh * p.Lr + qrow;  // rows below Lr exist in every statistic
-    if (DMA && p.q_side_uniform && p.D == HD && q0 + kXOwned16 <= p.Lq) {
+    u32x4 qB[NC][KC], tqB[NC][KC], gB[NC][KC], doB[NC][KC];
+    u32x4 oR[NC][KC], toR[NC][KC];
+    float lse_in[NC], mu_in[NC];
+    const int64_t so = (int64_t)bh * p.Lr + wrow + n;  // rows below Lr exist in every statistic
+    if (DMA && p.q_side_uniform && p.D == HD && q0 + OWNED <= p.Lq) {
         // the common case: whole rows that all exist, every tensor with q's strides
         const int64_t slice = b * p.q.sb + h * p.q.sh;
-        const uint32_t at = ((uint32_t)qrow * (uint32_t)p.q.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
-        load_b_operands16_at<HD>(qB, p.q.ptr + slice, at);
-        if constexpr (!SECOND) load_b_operands16_at<HD>(oR, p.o.ptr + slice, at);
-        if constexpr (HAS_G) {
-            load_b_operands16_at<HD>(tqB, p.tq.ptr + slice, at);
-            load_b_operands16_at<HD>(gB, p.dTO.ptr + slice, at);
-            if constexpr (!SECOND) load_b_operands16_at<HD>(toR, p.to.ptr + slice, at);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const uint32_t at = ((uint32_t)(wrow + 16 * u + n) * (uint32_t)p.q.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
+            load_b_operands16_at<HD>(qB[u], p.q.ptr + slice, at);
+            if constexpr (!SECOND) load_b_operands16_at<HD>(oR[u], p.o.ptr + slice, at);
+            if constexpr (HAS_G) {
+                load_b_operands16_at<HD>(tqB[u], p.tq.ptr + slice, at);
+                load_b_operands16_at<HD>(gB[u], p.dTO.ptr + slice, at);
+                if constexpr (!SECOND) load_b_operands16_at<HD>(toR[u], p.to.ptr + slice, at);
+            }
+            if constexpr (HAS_DO) load_b_operands16_at<HD>(doB[u], p.dO.ptr + slice, at);
         }
-        if constexpr (HAS_DO) load_b_operands16_at<HD>(doB, p.dO.ptr + slice, at);
     } else {
-        load_b_operands16<T, HD, IO>(qB, p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qvalid);
-        if constexpr (!SECOND) load_b_operands16<T, HD, IO>(oR, p.o.head(b, h) + (int64_t)qrow * p.o.sl, g, p.D, qvalid);
-        if constexpr (HAS_G) {
-            load_b_operands16<T, HD, IO>(tqB, p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qvalid);
-            load_b_operands16<T, HD, IO>(gB, p.dTO.head(b, h) + (int64_t)qrow * p.dTO.sl, g, p.D, qvalid);
-            if constexpr (!SECOND) load_b_operands16<T, HD, IO>(toR, p.to.head(b, h) + (int64_t)qrow * p.to.sl, g, p.D, qvalid);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int64_t qrow = wrow + 16 * u + n;
+            const bool qvalid = qrow < p.Lq;
+            load_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + qrow * p.q.sl, g, p.D, qvalid);
+            if constexpr (!SECOND) load_b_operands16<T, HD, IO>(oR[u], p.o.head(b, h) + qrow * p.o.sl, g, p.D, qvalid);
+            if constexpr (HAS_G) {
+                load_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + qrow * p.tq.sl, g, p.D, qvalid);
+                load_b_operands16<T, HD, IO>(gB[u], p.dTO.head(b, h) + qrow * p.dTO.sl, g, p.D, qvalid);
+                if constexpr (!SECOND) load_b_operands16<T, HD, IO>(toR[u], p.to.head(b, h) + qrow * p.to.sl, g, p.D, qvalid);
+            }
+            if constexpr (HAS_DO) load_b_operands16<T, HD, IO>(doB[u], p.dO.head(b, h) + qrow * p.dO.sl, g, p.D, qvalid);
         }
-        if constexpr (HAS_DO) load_b_operands16<T, HD, IO>(doB, p.dO.head(b, h) + (int64_t)qrow * p.dO.sl, g, p.D, qvalid);
     }
-    float lse_in = p.lse[so];  // requested with the rows: they are awaited together
-    float mu_in = HAS_G ? p.mu[so] : 0.f;
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {  // requested with the rows: they are awaited together
+        lse_in[u] = p.lse[so + 16 * u];
+        mu_in[u] = HAS_G ? p.mu[so + 16 * u] : 0.f;
+    }
 
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
                                          StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
@@ -162,32 +178,33 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     issue_next();
 
     // row sums s4 = rowsum(G*O), s7d = rowsum(G*TO) + rowsum(dO*O) from the lane's 16-byte pieces, combined
-    // over the four lanes of a query
-    {
+    // over the four lanes of a query.  The tiles W and XY are accumulated on top of -s4 and -s7d, so that W - s4 and
+    // XY - s7d leave the matrix cores ready for use.
+    float n4[NC], n7[NC], lse2[NC], mu[NC];
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
         if constexpr (SECOND) {
             // the corrected sums the first launch left in the workspace (negated there)
-            s4 = -p.s4[so];
-            s7d = -p.s7d[so];
+            n4[u] = p.s4[so + 16 * u];
+            n7[u] = p.s7d[so + 16 * u];
         } else {
+            float s4 = 0.f, s7d = 0.f;
 #pragma unroll
             for (int c = 0; c < KC; ++c) {
                 if constexpr (HAS_G) {
-                    s4 += dot8<T>(gB[c], oR[c]);
-                    s7d += dot8<T>(gB[c], toR[c]);
+                    s4 += dot8<T>(gB[u][c], oR[u][c]);
+                    s7d += dot8<T>(gB[u][c], toR[u][c]);
                 }
-                if constexpr (HAS_DO) s7d += dot8<T>(doB[c], oR[c]);
+                if constexpr (HAS_DO) s7d += dot8<T>(doB[u][c], oR[u][c]);
             }
-            s4 = group_sum(s4);
-            s7d = group_sum(s7d);
+            n4[u] = -group_sum(s4);
+            n7[u] = -group_sum(s7d);
         }
+        asm volatile("" : "+v"(lse_in[u]), "+v"(mu_in[u]));  // not before the copies of stage 0 are under way
+        lse2[u] = lse_in[u] * kLog2e;
+        mu[u] = HAS_G ? mu_in[u] : 0.f;
+        asm volatile("" : "+v"(lse2[u]), "+v"(mu[u]), "+v"(n4[u]), "+v"(n7[u]));  // every load so far is awaited here
     }
-    asm volatile("" : "+v"(lse_in), "+v"(mu_in));  // not before the copies of stage 0 are under way
-    float lse2 = lse_in * kLog2e;
-    float mu = HAS_G ? mu_in : 0.f;
-    // The tiles W and XY are accumulated on top of -s4 and -s7d, so that W - s4 and XY - s7d leave the matrix
-    // cores ready for use.
-    float n4 = -s4, n7 = -s7d;
-    asm volatile("" : "+v"(lse2), "+v"(mu), "+v"(n4), "+v"(n7));  // every load so far is awaited here
     if constexpr (DMA) {
         while (issued < R && issued < ns) issue_next();
     } else {
@@ -196,18 +213,22 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     // every row below Lr gets its workspace entries (zeros beyond Lq except lse2, which is finite): the
     // column-owned kernel, which runs after this one, stages 32-row groups
     if constexpr (!SECOND) {
-        if (g == 0) p.lse2[so] = lse2;
+#pragma unroll
+        for (int u = 0; u < NC; ++u)
+            if (g == 0) p.lse2[so + 16 * u] = lse2[u];
     }
     const float sl2 = p.scale * kLog2e;
-    f32x4 dq[DT], dtq[DT];
+    f32x4 dq[NC][DT], dtq[NC][DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-        dq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dtq[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int u = 0; u < NC; ++u)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            dq[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dtq[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     // First launch: this lane's part of sum_j dS_dot_ij, sum_j dS_ij (zero in exact arithmetic), and of
     // their absolute sums, which only set the scale of a threshold and are sampled on every fourth key.
-    float r4 = 0.f, r7 = 0.f, a4 = 0.f, a7 = 0.f;
+    float r4[NC] = {}, r7[NC] = {}, a4[NC] = {}, a7[NC] = {};
 
     auto compute = [&](const elem_t* slot, int k0, auto ragged_tag) {
         const elem_t* sK = slot;
@@ -215,56 +236,71 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         const elem_t* sTK = slot + 2 * SE;
         const elem_t* sTV = slot + 3 * SE;
         // tiles: rows = keys (registers), columns = this wave's queries (lanes)
-        f32x4 s[2], ts[2], w[2], xy[2];
+        f32x4 s[NC][2], ts[NC][2], w[NC][2], xy[NC][2];
         auto scores = [&](int t) __attribute__((always_inline)) {
-            s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            ts[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            w[t] = f32x4{n4, n4, n4, n4};
-            xy[t] = f32x4{n7, n7, n7, n7};
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                s[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                ts[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                w[u][t] = f32x4{n4[u], n4[u], n4[u], n4[u]};
+                xy[u][t] = f32x4{n7[u], n7[u], n7[u], n7[u]};
+            }
 #pragma unroll
             for (int c = 0; c < KC; ++c) {
                 const u32x4 ak = lds_a_rows16<HD>(sK, t, c, n, g);
                 const u32x4 av = lds_a_rows16<HD>(sV, t, c, n, g);
-                s[t] = T::mfma16(ak, qB[c], s[t]);
-                if constexpr (HAS_G) {
-                    ts[t] = T::mfma16(ak, tqB[c], ts[t]);
-                    const u32x4 atk = lds_a_rows16<HD>(sTK, t, c, n, g);
-                    ts[t] = T::mfma16(atk, qB[c], ts[t]);
-                    w[t] = T::mfma16(av, gB[c], w[t]);
-                    const u32x4 atv = lds_a_rows16<HD>(sTV, t, c, n, g);
-                    xy[t] = T::mfma16(atv, gB[c], xy[t]);
+#pragma unroll
+                for (int u = 0; u < NC; ++u) {
+                    s[u][t] = T::mfma16(ak, qB[u][c], s[u][t]);
+                    if constexpr (HAS_G) ts[u][t] = T::mfma16(ak, tqB[u][c], ts[u][t]);
                 }
-                if constexpr (HAS_DO) xy[t] = T::mfma16(av, doB[c], xy[t]);
+                if constexpr (HAS_G) {
+                    const u32x4 atk = lds_a_rows16<HD>(sTK, t, c, n, g);
+#pragma unroll
+                    for (int u = 0; u < NC; ++u) {
+                        ts[u][t] = T::mfma16(atk, qB[u][c], ts[u][t]);
+                        w[u][t] = T::mfma16(av, gB[u][c], w[u][t]);
+                    }
+                    const u32x4 atv = lds_a_rows16<HD>(sTV, t, c, n, g);
+#pragma unroll
+                    for (int u = 0; u < NC; ++u) xy[u][t] = T::mfma16(atv, gB[u][c], xy[u][t]);
+                }
+                if constexpr (HAS_DO) {
+#pragma unroll
+                    for (int u = 0; u < NC; ++u) xy[u][t] = T::mfma16(av, doB[u][c], xy[u][t]);
+                }
             }
         };
         constexpr bool ragged = decltype(ragged_tag)::value;  // the stage reaches beyond Lk (only the last one can)
         // in place: w -> dS_dot, xy -> dS
         auto pointwise = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float pj = fast_exp2(fmaf(s[t][j], sl2, -lse2));
-                // keys beyond Lk are zero rows; exp(-lse) may overflow when every real score is very
-                // negative, so their P is forced to zero
-                if constexpr (ragged) {
-                    if (k0 + 16 * t + 4 * g + j >= p.Lk) pj = 0.f;
-                }
-                if constexpr (HAS_G) {
-                    const float nn = fmaf(ts[t][j], p.scale, -mu);
-                    const float dts = pj * w[t][j];
-                    w[t][j] = dts;
-                    xy[t][j] = fmaf(dts, nn, pj * xy[t][j]);
-                    if constexpr (!SECOND) {
-                        r4 += dts;
-                        if (j == 0) a4 += fabsf(dts);
+            for (int u = 0; u < NC; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float pj = fast_exp2(fmaf(s[u][t][j], sl2, -lse2[u]));
+                    // keys beyond Lk are zero rows; exp(-lse) may overflow when every real score is very
+                    // negative, so their P is forced to zero
+                    if constexpr (ragged) {
+                        if (k0 + 16 * t + 4 * g + j >= p.Lk) pj = 0.f;
                     }
-                } else {
-                    xy[t][j] = pj * xy[t][j];
+                    if constexpr (HAS_G) {
+                        const float nn = fmaf(ts[u][t][j], p.scale, -mu[u]);
+                        const float dts = pj * w[u][t][j];
+                        w[u][t][j] = dts;
+                        xy[u][t][j] = fmaf(dts, nn, pj * xy[u][t][j]);
+                        if constexpr (!SECOND) {
+                            r4[u] += dts;
+                            if (j == 0) a4[u] += fabsf(dts);
+                        }
+                    } else {
+                        xy[u][t][j] = pj * xy[u][t][j];
+                    }
+                    if constexpr (!SECOND) {
+                        r7[u] += xy[u][t][j];
+                        if (j == 0) a7[u] += fabsf(xy[u][t][j]);
+                    }
                 }
-                if constexpr (!SECOND) {
-                    r7 += xy[t][j];
-                    if (j == 0) a7 += fabsf(xy[t][j]);
-                }
-            }
         };
         // the second key tile's MFMA chains run under the first tile's element-wise arithmetic
         scores(0);
@@ -282,9 +318,12 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         if constexpr (HAS_G) atk = lds_a_tr16<HD>(sTK, 0, lane);
         __builtin_amdgcn_sched_barrier(0);
         pointwise(1);
-        const u32x4 dsB = pack_b16<T>(xy[0], xy[1]);
-        u32x4 dtsB;
-        if constexpr (HAS_G) dtsB = pack_b16<T>(w[0], w[1]);
+        u32x4 dsB[NC], dtsB[NC];
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            dsB[u] = pack_b16<T>(xy[u][0], xy[u][1]);
+            if constexpr (HAS_G) dtsB[u] = pack_b16<T>(w[u][0], w[u][1]);
+        }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             u32x4 nk, ntk;
@@ -293,10 +332,13 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
                 if constexpr (HAS_G) ntk = lds_a_tr16<HD>(sTK, 16 * (d + 1), lane);
             }
             __builtin_amdgcn_sched_barrier(0);
-            dq[d] = T::mfma16(ak, dsB, dq[d]);
-            if constexpr (HAS_G) {
-                dtq[d] = T::mfma16(ak, dtsB, dtq[d]);
-                dq[d] = T::mfma16(atk, dtsB, dq[d]);
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                dq[u][d] = T::mfma16(ak, dsB[u], dq[u][d]);
+                if constexpr (HAS_G) {
+                    dtq[u][d] = T::mfma16(ak, dtsB[u], dtq[u][d]);
+                    dq[u][d] = T::mfma16(atk, dtsB[u], dq[u][d]);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
             ak = nk;
@@ -319,35 +361,49 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     stage(ns - 1, std::true_type{});
     if constexpr (!SECOND) {
         // the residues of the row sums (see the top of the file); the four lanes of a query hold its keys
-        r4 = group_sum(r4);
-        r7 = group_sum(r7);
-        a4 = 4.0f * group_sum(a4);
-        a7 = 4.0f * group_sum(a7);
-        if (g == 0) {
-            p.s4[so] = n4 - r4;  // minus the corrected sums: the column-owned kernel starts its tiles from them
-            p.s7d[so] = n7 - r7;
+        bool wanted = false;
+        int own = n;
+        asm volatile("" : "+v"(own));  // (formed anew: nothing of the address is held through the loop)
+        const int64_t so = (int64_t)bh * p.Lr + wrow + own;
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            r4[u] = group_sum(r4[u]);
+            r7[u] = group_sum(r7[u]);
+            a4[u] = 4.0f * group_sum(a4[u]);
+            a7[u] = 4.0f * group_sum(a7[u]);
+            if (g == 0) {
+                p.s4[so + 16 * u] = n4[u] - r4[u];  // minus the corrected sums: the column-owned kernel starts its tiles from them
+                p.s7d[so + 16 * u] = n7[u] - r7[u];
+            }
+            // A residue matters where it is not small against the rounding of the tiles it is spread over:
+            // |rho| against tau * sum_j |tile_ij|, tau = the unit roundoff of the 16-bit format.  NaN compares false.
+            wanted = wanted || (wrow + 16 * u + n < p.Lq && (fabsf(r4[u]) > p.rowfix_tau * a4[u] || fabsf(r7[u]) > p.rowfix_tau * a7[u]));
         }
-        // A residue matters where it is not small against the rounding of the tiles it is spread over:
-        // |rho| against tau * sum_j |tile_ij|, tau = the unit roundoff of the 16-bit format.  NaN compares false.
-        const bool wanted = qvalid && (fabsf(r4) > p.rowfix_tau * a4 || fabsf(r7) > p.rowfix_tau * a7);
         if (p.rowfix == 1) {
-            const bool any = workgroup_barrier_or(wanted);
-            if (tid == 0) p.flags[bid] = any ? 1 : 0;
+            // one flag per 64 rows, which is what a workgroup of the second launch owns
+#pragma unroll
+            for (int f = 0; f < NC; ++f) {
+                const bool any = workgroup_barrier_or(wanted && wave / (kXWaves16 / NC) == f);
+                if (tid == 0) p.flags[NC * bid + f] = any ? 1 : 0;
+            }
         }
         if constexpr (MEASURE) return;  // the second launch writes dQ, dQ_dot
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!wave_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
-    const int row0 = q0 + wave * 16;
-    store_rows16<T, HD, IO>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq, p.scale, lane);
-    if constexpr (HAS_G)
-        store_rows16<T, HD, IO>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq, p.scale, lane);
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int row0 = wrow + 16 * u;
+        store_rows16<T, HD, IO>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq[u], p.scale, lane);
+        if constexpr (HAS_G)
+            store_rows16<T, HD, IO>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq[u], p.scale, lane);
+    }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma, int NC = 1>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_row16_kernel(const BwdParams p) {
-    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO, NC>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -364,7 +420,7 @@ struct Col16Smem {
     static_assert(R * slot >= kXWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int NC = 1>
 __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -379,15 +435,15 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15;
     const int g = lane >> 4;
-    const int k_blocks = (p.Lk + kXOwned16 - 1) / kXOwned16;
+    constexpr int OWNED = NC * kXOwned16;
+    const int k_blocks = (p.Lk + OWNED - 1) / OWNED;
     const int bid = xcd_linear_id(block, blocks);
     const int bh = bid / k_blocks;
     const int kb = bid % k_blocks;
     const int b = bh / p.H, h = bh % p.H;
-    const int key0 = kb * kXOwned16;
-    const int krow = key0 + wave * 16 + n;
-    const bool kvalid = krow < p.Lk;
-    const bool wave_active = (key0 + wave * 16) < p.Lk;
+    const int key0 = kb * OWNED;
+    const int wrow = key0 + wave * 16 * NC;  // the wave's first key; the lane's are wrow + 16 u + n
+    const bool wave_active = wrow < p.Lk;
 
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
                                          StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
@@ -427,50 +483,62 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         issue_next();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
-    u32x4 kB[KC], vB[KC], tkB[KC], tvB[KC];
-    if (DMA && p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
+    u32x4 kB[NC][KC], vB[NC][KC], tkB[NC][KC], tvB[NC][KC];
+    if (DMA && p.k_side_uniform && p.D == HD && key0 + OWNED <= p.Lk) {
         // the common case: whole rows that all exist, every tensor with k's strides
         const int64_t slice = b * p.k.sb + h * p.k.sh;
-        const uint32_t at = ((uint32_t)krow * (uint32_t)p.k.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
-        load_b_operands16_at<HD>(kB, p.k.ptr + slice, at);
-        load_b_operands16_at<HD>(vB, p.v.ptr + slice, at);
-        if constexpr (HAS_G) {
-            load_b_operands16_at<HD>(tkB, p.tk.ptr + slice, at);
-            load_b_operands16_at<HD>(tvB, p.tv.ptr + slice, at);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const uint32_t at = ((uint32_t)(wrow + 16 * u + n) * (uint32_t)p.k.sl + 8u * (uint32_t)g) * (uint32_t)sizeof(elem_t);
+            load_b_operands16_at<HD>(kB[u], p.k.ptr + slice, at);
+            load_b_operands16_at<HD>(vB[u], p.v.ptr + slice, at);
+            if constexpr (HAS_G) {
+                load_b_operands16_at<HD>(tkB[u], p.tk.ptr + slice, at);
+                load_b_operands16_at<HD>(tvB[u], p.tv.ptr + slice, at);
+            }
         }
         begin_copies();
     } else {
-        load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
-        load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
-        if constexpr (HAS_G) {
-            load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
-            load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int64_t krow = wrow + 16 * u + n;
+            const bool kvalid = krow < p.Lk;
+            load_b_operands16<T, HD, IO>(kB[u], p.k.head(b, h) + krow * p.k.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(vB[u], p.v.head(b, h) + krow * p.v.sl, g, p.D, kvalid);
+            if constexpr (HAS_G) {
+                load_b_operands16<T, HD, IO>(tkB[u], p.tk.head(b, h) + krow * p.tk.sl, g, p.D, kvalid);
+                load_b_operands16<T, HD, IO>(tvB[u], p.tv.head(b, h) + krow * p.tv.sl, g, p.D, kvalid);
+            }
         }
         begin_copies();
     }
 #pragma unroll
-    for (int c = 0; c < KC; ++c) {  // the own rows are awaited here
-        asm volatile("" : "+v"(kB[c]));
-        asm volatile("" : "+v"(vB[c]));
-        if constexpr (HAS_G) {
-            asm volatile("" : "+v"(tkB[c]));
-            asm volatile("" : "+v"(tvB[c]));
+    for (int u = 0; u < NC; ++u)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {  // the own rows are awaited here
+            asm volatile("" : "+v"(kB[u][c]));
+            asm volatile("" : "+v"(vB[u][c]));
+            if constexpr (HAS_G) {
+                asm volatile("" : "+v"(tkB[u][c]));
+                asm volatile("" : "+v"(tvB[u][c]));
+            }
         }
-    }
     if constexpr (DMA) {
         while (issued < R && issued < ns) issue_next();
     } else {
         plan.commit();
     }
     const float sl2 = p.scale * kLog2e;
-    f32x4 dk[DT], dv[DT], dtk[DT], dtv[DT];
+    f32x4 dk[NC][DT], dv[NC][DT], dtk[NC][DT], dtv[NC][DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-        dk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dtk[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dtv[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int u = 0; u < NC; ++u)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            dk[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dv[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dtk[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            dtv[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 
     auto compute = [&](const elem_t* slot) {
         const elem_t* sQ = slot;
@@ -504,52 +572,64 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             if constexpr (HAS_DO) a.d = lds_a_tr16<HD>(sDO, 16 * d, lane);
             return a;
         };
-        f32x4 s[2], ts[2], w[2], xy[2];
+        f32x4 s[NC][2], ts[NC][2], w[NC][2], xy[NC][2];
         f32x4 lse4[2], mu4[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            ts[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int u = 0; u < NC; ++u)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                s[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                ts[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
         // The workspace holds -s4 and -s7d: W and XY are accumulated on top of them, so that W - s4 and
         // XY - s7d leave the matrix cores ready for use.
-        auto load_sums = [&](int u) __attribute__((always_inline)) {
-            const int r0 = 16 * u + 4 * g;  // register j of tile u is query 16 u + 4 g + j
-            if constexpr (HAS_G) w[u] = *reinterpret_cast<const f32x4*>(sStat + 2 * kStageRows + r0);
-            xy[u] = *reinterpret_cast<const f32x4*>(sStat + 3 * kStageRows + r0);
+        auto load_sums = [&](int t) __attribute__((always_inline)) {
+            const int r0 = 16 * t + 4 * g;  // register j of tile t is query 16 t + 4 g + j
+            if constexpr (HAS_G) w[0][t] = *reinterpret_cast<const f32x4*>(sStat + 2 * kStageRows + r0);
+            xy[0][t] = *reinterpret_cast<const f32x4*>(sStat + 3 * kStageRows + r0);
+#pragma unroll
+            for (int u = 1; u < NC; ++u) {
+                if constexpr (HAS_G) w[u][t] = w[0][t];
+                xy[u][t] = xy[0][t];
+            }
         };
-        auto load_stats = [&](int u) __attribute__((always_inline)) {
-            const int r0 = 16 * u + 4 * g;
-            lse4[u] = *reinterpret_cast<const f32x4*>(sStat + 0 * kStageRows + r0);
-            if constexpr (HAS_G) mu4[u] = *reinterpret_cast<const f32x4*>(sStat + 1 * kStageRows + r0);
+        auto load_stats = [&](int t) __attribute__((always_inline)) {
+            const int r0 = 16 * t + 4 * g;
+            lse4[t] = *reinterpret_cast<const f32x4*>(sStat + 0 * kStageRows + r0);
+            if constexpr (HAS_G) mu4[t] = *reinterpret_cast<const f32x4*>(sStat + 1 * kStageRows + r0);
         };
         auto score_step = [&](int t, int c, const AOps& a) __attribute__((always_inline)) {
-            s[t] = T::mfma16(a.q, kB[c], s[t]);
-            if constexpr (HAS_G) {
-                ts[t] = T::mfma16(a.q, tkB[c], ts[t]);
-                ts[t] = T::mfma16(a.tq, kB[c], ts[t]);
-                w[t] = T::mfma16(a.g, vB[c], w[t]);
-                xy[t] = T::mfma16(a.g, tvB[c], xy[t]);
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                s[u][t] = T::mfma16(a.q, kB[u][c], s[u][t]);
+                if constexpr (HAS_G) {
+                    ts[u][t] = T::mfma16(a.q, tkB[u][c], ts[u][t]);
+                    ts[u][t] = T::mfma16(a.tq, kB[u][c], ts[u][t]);
+                    w[u][t] = T::mfma16(a.g, vB[u][c], w[u][t]);
+                    xy[u][t] = T::mfma16(a.g, tvB[u][c], xy[u][t]);
+                }
+                if constexpr (HAS_DO) xy[u][t] = T::mfma16(a.d, vB[u][c], xy[u][t]);
             }
-            if constexpr (HAS_DO) xy[t] = T::mfma16(a.d, vB[c], xy[t]);
         };
         // in place: s -> P, ts -> P_dot, w -> dS_dot, xy -> dS  (rows beyond Lq are zero rows of Q,
         // Q_dot, G, dO with finite statistics: they contribute nothing)
         auto pointwise = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pj = fast_exp2(fmaf(s[t][j], sl2, -lse4[t][j]));
-                s[t][j] = pj;
-                if constexpr (HAS_G) {
-                    const float nn = fmaf(ts[t][j], p.scale, -mu4[t][j]);
-                    const float dts = pj * w[t][j];
-                    w[t][j] = dts;
-                    xy[t][j] = fmaf(dts, nn, pj * xy[t][j]);
-                    ts[t][j] = pj * nn;
-                } else {
-                    xy[t][j] = pj * xy[t][j];
+            for (int u = 0; u < NC; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float pj = fast_exp2(fmaf(s[u][t][j], sl2, -lse4[t][j]));
+                    s[u][t][j] = pj;
+                    if constexpr (HAS_G) {
+                        const float nn = fmaf(ts[u][t][j], p.scale, -mu4[t][j]);
+                        const float dts = pj * w[u][t][j];
+                        w[u][t][j] = dts;
+                        xy[u][t][j] = fmaf(dts, nn, pj * xy[u][t][j]);
+                        ts[u][t][j] = pj * nn;
+                    } else {
+                        xy[u][t][j] = pj * xy[u][t][j];
+                    }
                 }
-            }
         };
         load_sums(0);
         AOps cur = load_score(0, 0);
@@ -584,28 +664,32 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         pointwise(0);
         __builtin_amdgcn_sched_barrier(0);
         pointwise(1);
-        u32x4 pB, dsB, pdB, dtsB;
-        pB = pack_b16<T>(s[0], s[1]);
-        dsB = pack_b16<T>(xy[0], xy[1]);
-        if constexpr (HAS_G) {
-            pdB = pack_b16<T>(ts[0], ts[1]);
-            dtsB = pack_b16<T>(w[0], w[1]);
+        u32x4 pB[NC], dsB[NC], pdB[NC], dtsB[NC];
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            pB[u] = pack_b16<T>(s[u][0], s[u][1]);
+            dsB[u] = pack_b16<T>(xy[u][0], xy[u][1]);
+            if constexpr (HAS_G) {
+                pdB[u] = pack_b16<T>(ts[u][0], ts[u][1]);
+                dtsB[u] = pack_b16<T>(w[u][0], w[u][1]);
+            }
         }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             AOps nxt;
             if (d + 1 < DT) nxt = load_grad(d + 1);
             __builtin_amdgcn_sched_barrier(0);
-            dk[d] = T::mfma16(cur.q, dsB, dk[d]);
-            if constexpr (HAS_G) {
-                dtk[d] = T::mfma16(cur.q, dtsB, dtk[d]);
-                dk[d] = T::mfma16(cur.tq, dtsB, dk[d]);
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                dk[u][d] = T::mfma16(cur.q, dsB[u], dk[u][d]);
+                if constexpr (HAS_G) {
+                    dtk[u][d] = T::mfma16(cur.q, dtsB[u], dtk[u][d]);
+                    dk[u][d] = T::mfma16(cur.tq, dtsB[u], dk[u][d]);
+                    dtv[u][d] = T::mfma16(cur.g, pB[u], dtv[u][d]);
+                    dv[u][d] = T::mfma16(cur.g, pdB[u], dv[u][d]);
+                }
+                if constexpr (HAS_DO) dv[u][d] = T::mfma16(cur.d, pB[u], dv[u][d]);
             }
-            if constexpr (HAS_G) {
-                dtv[d] = T::mfma16(cur.g, pB, dtv[d]);
-                dv[d] = T::mfma16(cur.g, pdB, dv[d]);
-            }
-            if constexpr (HAS_DO) dv[d] = T::mfma16(cur.d, pB, dv[d]);
             __builtin_amdgcn_sched_barrier(0);
             cur = nxt;
         }
@@ -621,18 +705,21 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!wave_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
-    const int row0 = key0 + wave * 16;
-    store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk, p.scale, lane);
-    if constexpr (HAS_G)
-        store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk, p.scale, lane);
-    store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv, 1.0f, lane);
-    if constexpr (HAS_G)
-        store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv, 1.0f, lane);
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int row0 = wrow + 16 * u;
+        store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk[u], p.scale, lane);
+        if constexpr (HAS_G)
+            store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk[u], p.scale, lane);
+        store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv[u], 1.0f, lane);
+        if constexpr (HAS_G)
+            store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv[u], 1.0f, lane);
+    }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdParams p) {
-    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The column-owned launch with the second launch of the row-owned kernel at its end: workgroups
@@ -640,11 +727,11 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdPa
 // not depend on the column pass (it rewrites dQ, dQ_dot of flagged workgroups from the sums the first pass
 // left).  Nearly all of those workgroups leave at once; dealt out behind the column pass they fill the time in
 // which its last workgroups run alone, where a launch of their own costs a few microseconds.
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks)
-        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC>(p, (int)blockIdx.x, col_blocks);
     else
         bwd_row16_body<T, HD, R, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
 }

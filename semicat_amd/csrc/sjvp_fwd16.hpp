@@ -37,8 +37,11 @@ struct Fwd16Smem {
 // streams).
 // IO: how the tensors lie in memory (sjvp_staged16.hpp); anything but kIoDma copies its stages through registers,
 // one stage ahead, and loads its own rows straight into registers.
-template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma>
-__global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams p) {
+// NC: sets of 16 queries per wavefront (NC = 2: four wavefronts, every operand read from LDS feeds both sets; with tangents
+// 202 registers and no gain: 96.6 us against 97.6 at B=8 H=16 L=1024 D=64, 105 against 101 at B=128 H=12 L=256).
+template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1>
+__global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdParams p) {
+    constexpr int NT = kThreads16 / NC;  // threads of the workgroup
     static_assert(!ROPE || (HD == 64 && SPB == 1), "the folded rotation covers HD = 64, one stage per barrier");
     constexpr bool DMA = IO == kIoDma;
     static_assert(DMA || (SPB == 1 && !ROPE), "staged copies run one stage ahead, unrotated");
@@ -62,11 +65,11 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     const int qb = bid % p.q_blocks;
     const int b = bh / p.H, h = bh % p.H;
     const int q0 = qb * kOwned16;
-    const int qrow = q0 + wave * 16 + n;
-    const bool wave_active = (q0 + wave * 16) < p.Lq;
+    const int wrow = q0 + wave * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
+    const bool wave_active = wrow < p.Lq;
 
-    u32x4 qB[KC], tqB[KC];
-    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1>, StagedPlan<T, HD, SM::nt, kThreads16, IO>>;
+    u32x4 qB[NC][KC], tqB[NC][KC];
+    using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, NT>, StagedPlan<T, HD, SM::nt, NT, IO>>;
     constexpr int SPT = StagePlan::N;
     StagePlan plan;
     // slot layout K | V | K_dot | V_dot (primal only: K | V)
@@ -74,7 +77,7 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     if constexpr (DMA) {
         // own rows first (issued before the stages, so they land first), then the ring
         {
-            CopyPlan<HD, JVP ? 8 : 4, 4> own_plan;
+            CopyPlan<HD, JVP ? 8 : 4, 4, NT> own_plan;
             if constexpr (JVP)
                 own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl},
                               Src{p.tq.head(b, h), p.tq.sl});
@@ -88,9 +91,14 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
         else
             plan.init(tid, 0, p.D, smem_raw + SM::sink, sk, sv);
     } else {
-        staged_b_operands16<T, HD, IO>(qB, p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int qrow = wrow + 16 * u + n;
+            staged_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
+            if constexpr (JVP)
+                staged_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
+        }
         if constexpr (JVP) {
-            staged_b_operands16<T, HD, IO>(tqB, p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
             plan.init(tid, p.D, sk, sv, Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
         } else {
             plan.init(tid, p.D, sk, sv);
@@ -114,30 +122,40 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
     }
 
     const float sl2 = p.scale * kLog2e;
-    float m_i = -INFINITY;     // reference maximum (same in the four lanes of a query)
-    float m_true = -INFINITY;  // maximum over the keys this lane has seen (for LI)
-    float l_i = 0.f;           // exp-sum over the keys this lane has seen
-    float mu_i = 0.f;          // sum of p * S_dot over the same keys
+    // per set of queries
+    float m_i[NC];     // reference maximum (same in the four lanes of a query)
+    float m_true[NC];  // maximum over the keys this lane has seen (for LI)
+    float l_i[NC];     // exp-sum over the keys this lane has seen
+    float mu_i[NC];    // sum of p * S_dot over the same keys
     // acc = sum P~ V;  tacc = sum (P~ * S_dot) V + P~ V_dot  (the reference's g_acc + p_tv_acc, which
     // only ever appear added together, ryu_triton.py:274-275)
-    f32x4 acc[DT], tacc[DT];
+    f32x4 acc[NC][DT], tacc[NC][DT];
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        tacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < NC; ++u) {
+        m_i[u] = m_true[u] = -INFINITY;
+        l_i[u] = mu_i[u] = 0.f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            tacc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     }
 
     // SPB = 1: the own rows and stage 0 were issued before the other stages; SPB = 2: everything
     if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1);
     workgroup_barrier();
     if constexpr (DMA) {
-        const int r = 16 * (wave & 1) + n;
-        read_b_operands16<HD>(qB, own + (wave >> 1) * SE, r, g);
-        if constexpr (JVP) read_b_operands16<HD>(tqB, own + (4 + (wave >> 1)) * SE, r, g);
-        if constexpr (ROPE) {
-            // the lane's two operands are columns 8g.. and 32 + 8g.. of its query: a rotation pair
-            rope8<T>(qB[0], qB[1], p.rope, qrow, g, 1.0f);
-            if constexpr (JVP) rope8<T>(tqB[0], tqB[1], p.rope, qrow, g, 1.0f);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int r0 = wave * 16 * NC + 16 * u;  // of the workgroup's 128 rows, 32 to a slab
+            const int r = (r0 & 31) + n;
+            read_b_operands16<HD>(qB[u], own + (r0 >> 5) * SE, r, g);
+            if constexpr (JVP) read_b_operands16<HD>(tqB[u], own + (4 + (r0 >> 5)) * SE, r, g);
+            if constexpr (ROPE) {
+                // the lane's two operands are columns 8g.. and 32 + 8g.. of its query: a rotation pair
+                rope8<T>(qB[u][0], qB[u][1], p.rope, q0 + r0 + n, g, 1.0f);
+                if constexpr (JVP) rope8<T>(tqB[u][0], tqB[u][1], p.rope, q0 + r0 + n, g, 1.0f);
+            }
         }
     }
     // ROPE: rotate the K (, K_dot) slab of a landed stage in place; 128 items per slab
@@ -161,70 +179,94 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
         const elem_t* sV = slot + SE;
         const elem_t* sTK = slot + 2 * SE;
         const elem_t* sTV = slot + 3 * SE;
-        f32x4 s[2], ts[2];
+        f32x4 s[NC][2], ts[NC][2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-            ts[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                s[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                ts[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
 #pragma unroll
             for (int c = 0; c < KC; ++c) {
                 const u32x4 a = lds_a_rows16<HD>(sK, t, c, n, g);
-                s[t] = T::mfma16(a, qB[c], s[t]);
+#pragma unroll
+                for (int u = 0; u < NC; ++u) {
+                    s[u][t] = T::mfma16(a, qB[u][c], s[u][t]);
+                    if constexpr (JVP) ts[u][t] = T::mfma16(a, tqB[u][c], ts[u][t]);
+                }
                 if constexpr (JVP) {
-                    ts[t] = T::mfma16(a, tqB[c], ts[t]);
                     const u32x4 at = lds_a_rows16<HD>(sTK, t, c, n, g);
-                    ts[t] = T::mfma16(at, qB[c], ts[t]);
+#pragma unroll
+                    for (int u = 0; u < NC; ++u) ts[u][t] = T::mfma16(at, qB[u][c], ts[u][t]);
                 }
             }
         }
         if (k0 + kStageRows > p.Lk) {  // wave-uniform: only the last stage can be ragged
             // keys beyond Lk are zero rows in LDS (their S_dot is already 0)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int u = 0; u < NC; ++u)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (k0 + 16 * t + 4 * g + j >= p.Lk) s[t][j] = -INFINITY;
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (k0 + 16 * t + 4 * g + j >= p.Lk) s[u][t][j] = -INFINITY;
         }
-        float mloc = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                           fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3]))) * sl2;
-        m_true = fmaxf(m_true, mloc);
-        if (__builtin_amdgcn_ballot_w64(mloc > m_i + kMaxSlack) != 0) {  // wave-uniform branch
-            const float m_new = fmaxf(m_i, group_max(mloc));
-            const float alpha = fast_exp2(m_i - m_new);  // 0 on the first tile
-            m_i = m_new;
-            l_i *= alpha;
-            if constexpr (JVP) mu_i *= alpha;
+        float mloc[NC];
+        bool raise = false;
 #pragma unroll
-            for (int d = 0; d < DT; ++d) {
-                acc[d] *= alpha;
-                if constexpr (JVP) tacc[d] *= alpha;
-            }
+        for (int u = 0; u < NC; ++u) {
+            mloc[u] = fmaxf(fmaxf(fmaxf(s[u][0][0], s[u][0][1]), fmaxf(s[u][0][2], s[u][0][3])),
+                            fmaxf(fmaxf(s[u][1][0], s[u][1][1]), fmaxf(s[u][1][2], s[u][1][3]))) * sl2;
+            m_true[u] = fmaxf(m_true[u], mloc[u]);
+            raise = raise || mloc[u] > m_i[u] + kMaxSlack;
         }
+        if (__builtin_amdgcn_ballot_w64(raise) != 0) {  // wave-uniform branch
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+            for (int u = 0; u < NC; ++u) {
+                const float m_new = fmaxf(m_i[u], group_max(mloc[u]));
+                const float alpha = fast_exp2(m_i[u] - m_new);  // 0 on the first tile
+                m_i[u] = m_new;
+                l_i[u] *= alpha;
+                if constexpr (JVP) mu_i[u] *= alpha;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float pj = fast_exp2(fmaf(s[t][j], sl2, -m_i));
-                s[t][j] = pj;
-                l_i += pj;
-                if constexpr (JVP) {
-                    const float pt = pj * (ts[t][j] * p.scale);
-                    ts[t][j] = pt;
-                    mu_i += pt;
+                for (int d = 0; d < DT; ++d) {
+                    acc[u][d] *= alpha;
+                    if constexpr (JVP) tacc[u][d] *= alpha;
                 }
             }
         }
-        const u32x4 pb = pack_b16<T>(s[0], s[1]);
-        u32x4 ptb;
-        if constexpr (JVP) ptb = pack_b16<T>(ts[0], ts[1]);
+        u32x4 pb[NC], ptb[NC];
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float pj = fast_exp2(fmaf(s[u][t][j], sl2, -m_i[u]));
+                    s[u][t][j] = pj;
+                    l_i[u] += pj;
+                    if constexpr (JVP) {
+                        const float pt = pj * (ts[u][t][j] * p.scale);
+                        ts[u][t][j] = pt;
+                        mu_i[u] += pt;
+                    }
+                }
+            pb[u] = pack_b16<T>(s[u][0], s[u][1]);
+            if constexpr (JVP) ptb[u] = pack_b16<T>(ts[u][0], ts[u][1]);
+        }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             const u32x4 av = lds_a_tr16<HD>(sV, 16 * d, lane);
-            acc[d] = T::mfma16(av, pb, acc[d]);
+#pragma unroll
+            for (int u = 0; u < NC; ++u) {
+                acc[u][d] = T::mfma16(av, pb[u], acc[u][d]);
+                if constexpr (JVP) tacc[u][d] = T::mfma16(av, ptb[u], tacc[u][d]);
+            }
             if constexpr (JVP) {
-                tacc[d] = T::mfma16(av, ptb, tacc[d]);
                 const u32x4 atv = lds_a_tr16<HD>(sTV, 16 * d, lane);
-                tacc[d] = T::mfma16(atv, pb, tacc[d]);
+#pragma unroll
+                for (int u = 0; u < NC; ++u) tacc[u][d] = T::mfma16(atv, pb[u], tacc[u][d]);
             }
         }
     };
@@ -257,43 +299,46 @@ __global__ __launch_bounds__(kThreads16, OCC) void fwd16_kernel(const FwdParams 
         }
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
-    const int64_t so = (int64_t)bh * p.Lr + qrow;
-    if (!wave_active) {
-        // All 16 rows of this wave lie beyond Lq: their statistic rows get the values a zero query
-        // row produces (and the reference initialises them with): log(Lk), 0, Lk.
-        if (g == 0) {
-            p.lse[so] = fast_log2((float)p.Lk) * kLn2;
-            if constexpr (JVP) p.mu[so] = 0.f;
-            if (p.li) p.li[so] = (float)p.Lk;
-        }
-        return;
-    }
-    // Combine the four lanes' partial sums (they cover disjoint keys of the same query).
-    const float l = group_sum(l_i);
-    const float inv_l = 1.0f / l;
-    float mu_un = 0.f;
-    if constexpr (JVP) mu_un = group_sum(mu_i);
-    if (p.li) m_true = group_max(m_true);
-    if (g == 0) {
-        // Statistic rows up to Lr are all written: a padded query row (all-zero q, q_dot) yields
-        // exactly the values the reference initialises them with: log(Lk), 0, Lk.
-        p.lse[so] = (m_i + fast_log2(l)) * kLn2;
-        if constexpr (JVP) p.mu[so] = mu_un * inv_l;
-        // LI is the exp-sum relative to the true row maximum (ryu_triton.py:291); l is relative
-        // to m_i, which may lag behind it by up to kMaxSlack.
-        if (p.li) p.li[so] = l * fast_exp2(m_i - m_true);
-    }
-    const float cmu = mu_un * inv_l;
-    if constexpr (JVP) {
-        // TO = (g_acc + p_tv_acc - mu_un * O) / l     (ryu_triton.py:274-275)
-#pragma unroll
-        for (int d = 0; d < DT; ++d) tacc[d] -= cmu * acc[d];
-    }
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
-    const int row0 = q0 + wave * 16;
-    store_rows16<T, HD, IO>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc, inv_l, lane);
-    if constexpr (JVP)
-        store_rows16<T, HD, IO>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc, inv_l, lane);
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const int row0 = wrow + 16 * u;
+        const int64_t so = (int64_t)bh * p.Lr + row0 + n;
+        if (row0 >= p.Lq) {
+            // All 16 rows lie beyond Lq: their statistic rows get the values a zero query row produces (and the
+            // reference initialises them with): log(Lk), 0, Lk.
+            if (g == 0) {
+                p.lse[so] = fast_log2((float)p.Lk) * kLn2;
+                if constexpr (JVP) p.mu[so] = 0.f;
+                if (p.li) p.li[so] = (float)p.Lk;
+            }
+            continue;
+        }
+        // Combine the four lanes' partial sums (they cover disjoint keys of the same query).
+        const float l = group_sum(l_i[u]);
+        const float inv_l = 1.0f / l;
+        float mu_un = 0.f;
+        if constexpr (JVP) mu_un = group_sum(mu_i[u]);
+        if (p.li) m_true[u] = group_max(m_true[u]);
+        if (g == 0) {
+            // Statistic rows up to Lr are all written: a padded query row (all-zero q, q_dot) yields
+            // exactly the values the reference initialises them with: log(Lk), 0, Lk.
+            p.lse[so] = (m_i[u] + fast_log2(l)) * kLn2;
+            if constexpr (JVP) p.mu[so] = mu_un * inv_l;
+            // LI is the exp-sum relative to the true row maximum (ryu_triton.py:291); l is relative
+            // to m_i, which may lag behind it by up to kMaxSlack.
+            if (p.li) p.li[so] = l * fast_exp2(m_i[u] - m_true[u]);
+        }
+        const float cmu = mu_un * inv_l;
+        if constexpr (JVP) {
+            // TO = (g_acc + p_tv_acc - mu_un * O) / l     (ryu_triton.py:274-275)
+#pragma unroll
+            for (int d = 0; d < DT; ++d) tacc[u][d] -= cmu * acc[u][d];
+        }
+        store_rows16<T, HD, IO>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc[u], inv_l, lane);
+        if constexpr (JVP)
+            store_rows16<T, HD, IO>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc[u], inv_l, lane);
+    }
 }
 
 }  // namespace sjvp

@@ -21,7 +21,17 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         // "always": a launch that measures the row-sum residues, then one that computes with the corrected
         // sums; otherwise the pass itself and, unless switched off, a second launch in which the workgroups
         // whose residues call for it run again
-        if (p.rowfix == 2) rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 1, IO>, grid, smem, stream, p, kXThreads16);
+        // Without the cotangent on TO a wave has registers for 32 queries, which every operand read from LDS then
+        // serves: 78 -> 68 us at B=8 H=16 L=1024 D=64, 120 -> 105 at D=128.  Half as many waves: from four workgroups
+        // of 64 queries per compute unit on (1024 of them 0.76 to 1.01 of the time, 512 1.03 to 1.13), and from 256
+        // keys on (128 of them 1.02).
+        bool wide = false;
+        if constexpr (!HAS_G && IO == kIoDma) wide = p.rowfix != 2 && grid >= 1024 && p.Lk >= 256;
+        if (wide) {
+            if constexpr (!HAS_G && IO == kIoDma)
+                rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, HD == 128 ? 2 : 3, 0, IO, 2>, grid / 2, smem, stream, p,
+                            kXThreads16);
+        } else if (p.rowfix == 2) rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 1, IO>, grid, smem, stream, p, kXThreads16);
         else rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 0, IO>, grid, smem, stream, p, kXThreads16);
         // The second launch does not depend on the column-owned pass.  Where nearly all of its workgroups leave
         // at once (repair of flagged workgroups only), they ride at the end of that launch instead of paying for
@@ -49,6 +59,19 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         }
         return launch(bwd_col16p_kernel<T, HD, PR, HAS_DO, HAS_G, IO>, grid, PS::bytes, stream, p, kThreads16);
     } else {
+        // 32 keys per wave where the accumulators leave room for them (as in the row-owned launch): 92 -> 80 us at B=8
+        // H=16 L=1024 D=64, cotangent on O only, from two workgroups of 64 keys per compute unit on (512 of them 0.96 to
+        // 1.01 of the time, 256 1.16 to 1.23); at D = 32 with both cotangents 129 -> 112 us, from 1024 workgroups and
+        // 512 queries on (1024 and 256: 0.97 to 1.04).
+        if constexpr (IO == kIoDma && (!HAS_G || HD == 32)) {
+            if (rides && (HAS_G ? grid >= 1024 && p.Lq >= 512 : grid >= 512 && p.Lq >= 256)) {
+                BwdParams pr = p;
+                pr.col_workgroups = BH * ((p.Lk + 2 * kXOwned16 - 1) / (2 * kXOwned16));
+                constexpr int smem = CS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? CS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
+                return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO, 2>,
+                              pr.col_workgroups + BH * (p.Lr / kXOwned16), smem, stream, pr, kXThreads16);
+            }
+        }
         if (rides) {
             BwdParams pr = p;
             pr.col_workgroups = grid;

@@ -12,33 +12,36 @@ constexpr int kRingPrimal = 4;  // primal only (two slabs per stage)
 // key-axis length from which the forward takes two stages per barrier
 constexpr int kFwdPairedFrom = 256;
 
+template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false>
+int fwd16_one(const FwdParams& p, int grid, hipStream_t stream) {
+    constexpr int smem = Fwd16Smem<HD, R, JVP, SPB>::bytes;
+    // Without tangents a wave has registers for 32 queries, which every operand read from LDS then serves: 53 -> 48 us at
+    // B=8 H=16 L=1024 D=64, 141 -> 134 at B=8 H=8 L=2048 D=128.  Half as many waves: from as many workgroups on as the
+    // chip holds (D <= 64: 1024 of them 0.90 to 1.01 of the time, 512 0.97 to 1.08; D = 128: 512 of them from 1024 keys
+    // on 0.95 to 0.98, with 256 to 512 keys 1.01 to 1.07).
+    if constexpr (!JVP && SPB == 2) {
+        if (HD == 128 ? grid >= 512 && p.Lk >= 1024 : grid >= 1024)
+            return launch(fwd16_kernel<T, HD, R, JVP, HD == 128 ? 2 : 4, SPB, ROPE, kIoDma, 2>, grid, smem, stream, p,
+                          kThreads16 / 2);
+    }
+    return launch(fwd16_kernel<T, HD, R, JVP, OCC, SPB, ROPE>, grid, smem, stream, p, kThreads16);
+}
+
 template <typename T, int HD>
 int fwd16_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
     // two stages in flight and at most 128 registers: two workgroups (sixteen waves) share a CU, which
     // overlaps one's copies with the other's arithmetic; HD = 128 needs the whole register budget
     constexpr int OCC = HD == 128 ? 2 : 4;
     if constexpr (HD == 64) {
-        if (p.rope.cos) {  // rotary embedding folded in (short key axes only, checked by the caller)
-            if (jvp)
-                return launch(fwd16_kernel<T, HD, kRingJvp, true, OCC, 1, true>, grid,
-                              Fwd16Smem<HD, kRingJvp, true>::bytes, stream, p, kThreads16);
-            return launch(fwd16_kernel<T, HD, kRingPrimal, false, OCC, 1, true>, grid,
-                          Fwd16Smem<HD, kRingPrimal, false>::bytes, stream, p, kThreads16);
-        }
+        if (p.rope.cos)  // rotary embedding folded in (short key axes only, checked by the caller)
+            return jvp ? fwd16_one<T, HD, kRingJvp, true, OCC, 1, true>(p, grid, stream)
+                       : fwd16_one<T, HD, kRingPrimal, false, OCC, 1, true>(p, grid, stream);
     }
-    if (p.Lk >= kFwdPairedFrom) {
-        // long key axes: two stages per barrier over a ring of four slots in the same LDS footprint
-        if (jvp)
-            return launch(fwd16_kernel<T, HD, 4, true, OCC, 2>, grid, Fwd16Smem<HD, 4, true, 2>::bytes, stream,
-                          p, kThreads16);
-        return launch(fwd16_kernel<T, HD, 4, false, OCC, 2>, grid, Fwd16Smem<HD, 4, false, 2>::bytes, stream,
-                      p, kThreads16);
-    }
-    if (jvp)
-        return launch(fwd16_kernel<T, HD, kRingJvp, true, OCC>, grid, Fwd16Smem<HD, kRingJvp, true>::bytes,
-                      stream, p, kThreads16);
-    return launch(fwd16_kernel<T, HD, kRingPrimal, false, OCC>, grid, Fwd16Smem<HD, kRingPrimal, false>::bytes,
-                  stream, p, kThreads16);
+    // long key axes: two stages per barrier over a ring of four slots in the same LDS footprint
+    if (p.Lk >= kFwdPairedFrom)
+        return jvp ? fwd16_one<T, HD, 4, true, OCC, 2>(p, grid, stream) : fwd16_one<T, HD, 4, false, OCC, 2>(p, grid, stream);
+    return jvp ? fwd16_one<T, HD, kRingJvp, true, OCC>(p, grid, stream)
+               : fwd16_one<T, HD, kRingPrimal, false, OCC>(p, grid, stream);
 }
 
 }  // namespace
