@@ -52,7 +52,8 @@ int check_common(int B, int H, int Lq, int Lk, int D, int dtype, float scale) {
     // the finest launch whose grid grows with the problem takes one workgroup per 64 rows of the longer axis rounded up
     // to 128 (the statistic rows); one per 32 is what has always been refused: in 64 bits, that grid has to fit the 31 bits
     // of a launch dimension.  (The split fp32 launches take one per 16 rows, but only up to 2304 groups of 16
-    // rows, see split() in sjvp_f32.hip, and with the statistic rows at most 8 workgroups for each group.)
+    // rows, see split() in sjvp_f32.hip, and with the statistic rows at most 8 workgroups for each group; the split 16-bit
+    // ones, split_rows() in sjvp_launch.hpp, have at most two workgroups per compute unit.)
     const int64_t longer = Lq > Lk ? Lq : Lk;
     if (longer > (1LL << 30)) return SJVP_ERR_SHAPE;  // keeps the 32-bit round-ups below exact
     const int64_t blocks = (int64_t)B * H * ((longer + 127) / 128 * 4);

@@ -39,26 +39,6 @@ constexpr int kXWaves16 = 4;
 constexpr int kXThreads16 = 64 * kXWaves16;
 constexpr int kXOwned16 = 16 * kXWaves16;  // owned positions per workgroup
 
-// B operands (all head-dimension chunks of 32) of one owned row, straight from global memory.
-template <typename T, int HD, int IO>
-__device__ __forceinline__ void load_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
-    if constexpr (IO != kIoDma) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
-#pragma unroll
-    for (int c = 0; c < HD / 32; ++c) {
-        out[c] = u32x4{0u, 0u, 0u, 0u};
-        if (valid && 32 * c + 8 * g < D) out[c] = *reinterpret_cast<const u32x4*>(row + 32 * c + 8 * g);
-    }
-}
-
-// The same from a uniform slice pointer and the lane's byte offset in the slice: whole rows of HD elements
-// that all exist, no predicates, one 32-bit offset for every tensor of equal strides.
-template <int HD>
-__device__ __forceinline__ void load_b_operands16_at(u32x4* out, const elem_t* slice, uint32_t lane_bytes) {
-    const char* base = reinterpret_cast<const char*>(slice);
-#pragma unroll
-    for (int c = 0; c < HD / 32; ++c) out[c] = *reinterpret_cast<const u32x4*>(base + lane_bytes + 64 * c);
-}
-
 // sum over the 16-bit pairs of a[i]*b[i]
 template <typename T>
 __device__ __forceinline__ float dot8(const u32x4& a, const u32x4& b) {
@@ -71,24 +51,28 @@ __device__ __forceinline__ float dot8(const u32x4& a, const u32x4& b) {
 // ---------------------------------------------------------------------------------------------
 // Row-owned kernel.  LDS: [ring of K | V (| K_dot | V_dot) stages][sink]; the ring doubles as store
 // staging after the last stage.
-template <int HD, int R, bool HAS_G>
+template <int HD, int R, bool HAS_G, int SPLIT = 1>
 struct Row16Smem {
     static constexpr int nt = HAS_G ? 4 : 2;
     static constexpr int slot = nt * Slab<HD>::elems;
-    static constexpr int sink = R * slot * (int)sizeof(elem_t);
+    static constexpr int loop = R * slot * (int)sizeof(elem_t);
+    static constexpr int after = SPLIT > 1 ? Split16Smem<HD, kXWaves16, HAS_G ? 2 : 1>::bytes : 0;
+    static constexpr int sink = loop > after ? loop : after;
     static constexpr int bytes = sink + kSink16;
     static_assert(R * slot >= kXWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
 
 // (the body of the kernel as a function of the workgroup's index and the number of workgroups, so that the
 // second launch can also ride at the end of the column-owned launch, see bwd_col16_repair_kernel)
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO, int NC = 1>
+// SPLIT > 1 (launches of few workgroups): the SPLIT waves of a group share 16 queries and take every SPLIT-th stage each, SPLIT
+// stages to a barrier (ring of 2 SPLIT); their sums meet in LDS at the end, in a fixed order.
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO, int NC = 1, int SPLIT = 1>
 __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     constexpr bool SECOND = PASS == 2;   // second launch: sums from the workspace, flagged workgroups only
     constexpr bool MEASURE = PASS == 1;  // first launch of "always": residues and sums only, no gradients
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    using SM = Row16Smem<HD, R, HAS_G>;
+    using SM = Row16Smem<HD, R, HAS_G, SPLIT>;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
     constexpr int KC = HD / 32;
@@ -99,7 +83,9 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     const int n = lane & 15;
     const int g = lane >> 4;
     static_assert(NC == 1 || PASS == 0, "the passes of the repair go by blocks of 64 rows");
-    constexpr int OWNED = NC * kXOwned16;
+    static_assert(SPLIT == 1 || (PASS == 0 && NC == 1 && R == 2 * SPLIT), "a step is a stage for every part");
+    const int part = SPLIT > 1 ? wave % SPLIT : 0, group = wave / SPLIT;
+    constexpr int OWNED = NC * kXOwned16 / SPLIT;
     const int q_blocks = p.Lr / OWNED;  // statistic rows up to Lr are all covered
     // Workgroups run through the heads in descending order: this launch follows the forward, which
     // ran through them in ascending order, so it starts on what the caches still hold (the
@@ -109,7 +95,7 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     const int qb = bid % q_blocks;
     const int b = bh / p.H, h = bh % p.H;
     const int q0 = qb * OWNED;
-    const int wrow = q0 + wave * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
+    const int wrow = q0 + group * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
     const bool wave_active = wrow < p.Lq;
     if constexpr (SECOND) {
         if (p.rowfix == 1 && p.flags[bid] == 0) return;  // nothing to repair in this workgroup's rows
@@ -159,23 +145,38 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
                                          StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
     constexpr int SPT = StagePlan::N;
-    StagePlan plan;
-    if constexpr (HAS_G)
-        init_plan(plan, tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl},
-                  Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
-    else
-        init_plan(plan, tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
+    StagePlan plan[DMA ? 1 : SPLIT];
+#pragma unroll
+    for (int u = 0; u < (DMA ? 1 : SPLIT); ++u) {
+        if constexpr (HAS_G)
+            init_plan(plan[u], tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl},
+                      Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
+        else
+            init_plan(plan[u], tid, p.D, smem_raw + SM::sink, Src{p.k.head(b, h), p.k.sl}, Src{p.v.head(b, h), p.v.sl});
+        if constexpr (!DMA && SPLIT > 1) plan[u].take(u, SPLIT);
+    }
     const int ns = (p.Lk + kStageRows - 1) / kStageRows;
     int issued = 0;
-    auto issue_next = [&]() {
-        issue_plan(plan, ring + (issued % R) * SM::slot, p.Lk - issued * kStageRows,
+    auto issue_next = [&](int u = 0) {  // u: place of the stage in its step
+        issue_plan(plan[DMA ? 0 : u], ring + (issued % R) * SM::slot, p.Lk - issued * kStageRows,
                    p.D == HD && (issued + 1) * kStageRows <= p.Lk);
         ++issued;
     };
-    // Stage 0 only for now: the loads of the own rows are awaited by a wait for everything this wave has
+    auto issue_step = [&]() {
+#pragma unroll
+        for (int u = 0; u < SPLIT; ++u)
+            if (SPLIT == 1 || issued < ns) issue_next(u);
+    };
+    auto commit_step = [&]() {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int u = 0; u < SPLIT; ++u) plan[u].commit();
+        }
+    };
+    // The first step (stage 0) only for now: the loads of the own rows are awaited by a wait for everything this wave has
     // outstanding (the compiler cannot tell them from the stage copies), so the later stages are issued once
     // the own rows are in registers and land under the first stage's arithmetic.
-    issue_next();
+    issue_step();
 
     // row sums s4 = rowsum(G*O), s7d = rowsum(G*TO) + rowsum(dO*O) from the lane's 16-byte pieces, combined
     // over the four lanes of a query.  The tiles W and XY are accumulated on top of -s4 and -s7d, so that W - s4 and
@@ -208,14 +209,14 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     if constexpr (DMA) {
         while (issued < R && issued < ns) issue_next();
     } else {
-        plan.commit();
+        commit_step();
     }
     // every row below Lr gets its workspace entries (zeros beyond Lq except lse2, which is finite): the
     // column-owned kernel, which runs after this one, stages 32-row groups
     if constexpr (!SECOND) {
 #pragma unroll
         for (int u = 0; u < NC; ++u)
-            if (g == 0) p.lse2[so + 16 * u] = lse2[u];
+            if (g == 0 && part == 0) p.lse2[so + 16 * u] = lse2[u];
     }
     const float sl2 = p.scale * kLog2e;
     f32x4 dq[NC][DT], dtq[NC][DT];
@@ -355,10 +356,26 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         workgroup_barrier();  // stage i has landed for every wave; stage i-1 is fully consumed
         if ((i > 0 || !DMA) && issued < ns) issue_next();
         if (wave_active) compute(ring + (i % R) * SM::slot, i * kStageRows, ragged_tag);
-        if constexpr (!DMA) plan.commit();
+        commit_step();
     };
-    for (int i = 0; i < ns - 1; ++i) stage(i, std::false_type{});
-    stage(ns - 1, std::true_type{});
+    if constexpr (SPLIT > 1) {
+        const elem_t* part_ring = ring + part * SM::slot;
+        for (int i = 0; i < ns; i += SPLIT) {
+            if constexpr (DMA) wait_stages<SPT>(issued - SPLIT - i > 0 ? issued - SPLIT - i : 0);
+            workgroup_barrier();  // as above, of a step
+            if (i > 0 || !DMA) issue_step();
+            const int mine = i + part;
+            if (wave_active && mine < ns) {
+                const elem_t* slot = part_ring + (i % R) * SM::slot;
+                if (mine == ns - 1) compute(slot, mine * kStageRows, std::true_type{});
+                else compute(slot, mine * kStageRows, std::false_type{});
+            }
+            commit_step();
+        }
+    } else {
+        for (int i = 0; i < ns - 1; ++i) stage(i, std::false_type{});
+        stage(ns - 1, std::true_type{});
+    }
     if constexpr (!SECOND) {
         // the residues of the row sums (see the top of the file); the four lanes of a query hold its keys
         bool wanted = false;
@@ -369,9 +386,33 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         for (int u = 0; u < NC; ++u) {
             r4[u] = group_sum(r4[u]);
             r7[u] = group_sum(r7[u]);
-            a4[u] = 4.0f * group_sum(a4[u]);
-            a7[u] = 4.0f * group_sum(a7[u]);
-            if (g == 0) {
+            a4[u] = group_sum(a4[u]);
+            a7[u] = group_sum(a7[u]);
+            if constexpr (SPLIT > 1) {
+                using SP = Split16Smem<HD, kXWaves16, HAS_G ? 2 : 1>;
+                float* stat = reinterpret_cast<float*>(smem_raw + SP::red);
+                workgroup_barrier();  // the ring has been read
+                float* mine = stat + wave * 64 + n;
+                if (g == 0) {
+                    mine[0] = r4[u];
+                    mine[16] = r7[u];
+                    mine[32] = a4[u];
+                    mine[48] = a7[u];
+                }
+                workgroup_barrier();
+                const float* all = stat + SPLIT * group * 64 + n;
+                r4[u] = r7[u] = a4[u] = a7[u] = 0.f;
+#pragma unroll
+                for (int s = 0; s < SPLIT; ++s) {
+                    r4[u] += all[64 * s];
+                    r7[u] += all[64 * s + 16];
+                    a4[u] += all[64 * s + 32];
+                    a7[u] += all[64 * s + 48];
+                }
+            }
+            a4[u] *= 4.0f;
+            a7[u] *= 4.0f;
+            if (g == 0 && part == 0) {
                 p.s4[so + 16 * u] = n4[u] - r4[u];  // minus the corrected sums: the column-owned kernel starts its tiles from them
                 p.s7d[so + 16 * u] = n7[u] - r7[u];
             }
@@ -380,14 +421,39 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
             wanted = wanted || (wrow + 16 * u + n < p.Lq && (fabsf(r4[u]) > p.rowfix_tau * a4[u] || fabsf(r7[u]) > p.rowfix_tau * a7[u]));
         }
         if (p.rowfix == 1) {
-            // one flag per 64 rows, which is what a workgroup of the second launch owns
+            // one flag per 64 rows, which is what a workgroup of the second launch owns; the workgroups that share them
+            // write a byte or two each
 #pragma unroll
             for (int f = 0; f < NC; ++f) {
                 const bool any = workgroup_barrier_or(wanted && wave / (kXWaves16 / NC) == f);
-                if (tid == 0) p.flags[NC * bid + f] = any ? 1 : 0;
+                if (tid != 0) continue;
+                if constexpr (SPLIT == 1) p.flags[NC * bid + f] = any ? 1 : 0;
+                else if constexpr (SPLIT == 2) reinterpret_cast<uint16_t*>(p.flags)[bid] = any ? 1 : 0;
+                else reinterpret_cast<uint8_t*>(p.flags)[bid] = any ? 1 : 0;
             }
         }
         if constexpr (MEASURE) return;  // the second launch writes dQ, dQ_dot
+    }
+    if constexpr (SPLIT > 1) {
+        static_assert(SPLIT <= 4, "flags are bytes of 16 rows");
+        using SP = Split16Smem<HD, kXWaves16, HAS_G ? 2 : 1>;
+        f32x4* red = reinterpret_cast<f32x4*>(smem_raw);
+        elem_t* tile = reinterpret_cast<elem_t*>(smem_raw + SP::red + SP::stat) + wave * StoreStage16<HD>::elems;
+        split_put<DT, kXWaves16>(red, 0, wave, lane, dq[0]);  // (the ring was given up in front of the residues)
+        if constexpr (HAS_G) split_put<DT, kXWaves16>(red, 1, wave, lane, dtq[0]);
+        workgroup_barrier();
+        if (!wave_active) return;
+        if (part == 0) {
+            split_sum<DT, kXWaves16, SPLIT>(dq[0], red, 0, group, lane);
+            store_rows16<T, HD, IO>(tile, p.dq.head(b, h), p.dq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
+        }
+        if constexpr (HAS_G) {
+            if (part == 1) {
+                split_sum<DT, kXWaves16, SPLIT>(dq[0], red, 1, group, lane);
+                store_rows16<T, HD, IO>(tile, p.dtq.head(b, h), p.dtq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
+            }
+        }
+        return;
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!wave_active) return;
@@ -401,30 +467,34 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma, int NC = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma, int NC = 1,
+          int SPLIT = 1>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_row16_kernel(const BwdParams p) {
-    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO, NC>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO, NC, SPLIT>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------
 // Column-owned kernel: a workgroup of four waves owns 64 keys and accumulates all their gradients (HD <= 64; the
 // paired form below serves HD = 128).  LDS: [ring of Q | [Q_dot | G] | [dO] | lse2, mu, s4, s7d stages]
 // [sink]; the ring doubles as store staging after the last stage.
-template <int HD, int R, bool HAS_DO, bool HAS_G>
+template <int HD, int R, bool HAS_DO, bool HAS_G, int SPLIT = 1>
 struct Col16Smem {
     static constexpr int nt = 1 + (HAS_G ? 2 : 0) + (HAS_DO ? 1 : 0);
     static constexpr int stat_elems = 4 * kStageRows * 2;  // 4 float arrays of 32, in elem_t units
     static constexpr int slot = nt * Slab<HD>::elems + stat_elems;
-    static constexpr int sink = R * slot * (int)sizeof(elem_t);
+    static constexpr int loop = R * slot * (int)sizeof(elem_t);
+    static constexpr int after = SPLIT > 1 ? Split16Smem<HD, kXWaves16, HAS_G ? 4 : 2>::bytes : 0;
+    static constexpr int sink = loop > after ? loop : after;
     static constexpr int bytes = sink + kSink16;
     static_assert(R * slot >= kXWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int NC = 1>
+// (SPLIT: as in the row-owned kernel)
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int NC = 1, int SPLIT = 1>
 __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    using SM = Col16Smem<HD, R, HAS_DO, HAS_G>;
+    using SM = Col16Smem<HD, R, HAS_DO, HAS_G, SPLIT>;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
     constexpr int oTQ = SE, oG = 2 * SE, oDO = (HAS_G ? 3 : 1) * SE, oST = SM::nt * SE;
@@ -435,26 +505,28 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15;
     const int g = lane >> 4;
-    constexpr int OWNED = NC * kXOwned16;
+    static_assert(SPLIT == 1 || (NC == 1 && R == 2 * SPLIT), "a step is a stage for every part");
+    const int part = SPLIT > 1 ? wave % SPLIT : 0, group = wave / SPLIT;
+    constexpr int OWNED = NC * kXOwned16 / SPLIT;
     const int k_blocks = (p.Lk + OWNED - 1) / OWNED;
     const int bid = xcd_linear_id(block, blocks);
     const int bh = bid / k_blocks;
     const int kb = bid % k_blocks;
     const int b = bh / p.H, h = bh % p.H;
     const int key0 = kb * OWNED;
-    const int wrow = key0 + wave * 16 * NC;  // the wave's first key; the lane's are wrow + 16 u + n
+    const int wrow = key0 + group * 16 * NC;  // the wave's first key; the lane's are wrow + 16 u + n
     const bool wave_active = wrow < p.Lk;
 
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, kXThreads16>,
                                          StagedPlan<T, HD, SM::nt, kXThreads16, IO>>;
     constexpr int SPT = StagePlan::N + 1;  // plus one 4-byte copy of statistics
-    StagePlan plan;
+    StagePlan plan[DMA ? 1 : SPLIT];
     const int ns = (p.Lq + kStageRows - 1) / kStageRows;
     int issued = 0;
-    auto issue_next = [&]() {
+    auto issue_next = [&](int u = 0) {  // u: place of the stage in its step
         elem_t* slot = ring + (issued % R) * SM::slot;
         const int row0 = issued * kStageRows;
-        issue_plan(plan, slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
+        issue_plan(plan[DMA ? 0 : u], slot, p.Lq - row0, p.D == HD && row0 + kStageRows <= p.Lq);
         // the four statistic arrays (lse2, mu, s4, s7d) of the stage's rows, one per wave, 32 lanes
         // each (rows < Lr exist in all of them); every wave issues exactly one 4-byte LDS-DMA
         // (the three workspace arrays lie one behind the other: chosen by arithmetic, which stays in scalar
@@ -466,21 +538,34 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         if (lane < 32) dma4(src + (int64_t)bh * p.Lr + row0 + lane, lds_addr(st) + (uint32_t)(wave * 32 * 4));
         ++issued;
     };
+    auto issue_step = [&]() {
+#pragma unroll
+        for (int u = 0; u < SPLIT; ++u)
+            if (SPLIT == 1 || issued < ns) issue_next(u);
+    };
+    auto commit_step = [&]() {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int u = 0; u < SPLIT; ++u) plan[u].commit();
+        }
+    };
     // called behind the requests for the own rows on both paths below (see bwd_row16_kernel): set-up of the
-    // stage copies, and stage 0 only for now
+    // stage copies, and the first step (stage 0) only for now
     auto begin_copies = [&]() __attribute__((always_inline)) {
-        {
-            const Src q{p.q.head(b, h), p.q.sl};
+        const Src q{p.q.head(b, h), p.q.sl};
+#pragma unroll
+        for (int u = 0; u < (DMA ? 1 : SPLIT); ++u) {
             if constexpr (HAS_G && HAS_DO)
-                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+                init_plan(plan[u], tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                           Src{p.dTO.head(b, h), p.dTO.sl}, Src{p.dO.head(b, h), p.dO.sl});
             else if constexpr (HAS_G)
-                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
+                init_plan(plan[u], tid, p.D, smem_raw + SM::sink, q, Src{p.tq.head(b, h), p.tq.sl},
                           Src{p.dTO.head(b, h), p.dTO.sl});
             else
-                init_plan(plan, tid, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
+                init_plan(plan[u], tid, p.D, smem_raw + SM::sink, q, Src{p.dO.head(b, h), p.dO.sl});
+            if constexpr (!DMA && SPLIT > 1) plan[u].take(u, SPLIT);
         }
-        issue_next();
+        issue_step();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
     u32x4 kB[NC][KC], vB[NC][KC], tkB[NC][KC], tvB[NC][KC];
@@ -526,7 +611,7 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     if constexpr (DMA) {
         while (issued < R && issued < ns) issue_next();
     } else {
-        plan.commit();
+        commit_step();
     }
     const float sl2 = p.scale * kLog2e;
     f32x4 dk[NC][DT], dv[NC][DT], dtk[NC][DT], dtv[NC][DT];
@@ -695,12 +780,42 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         }
     };
 
+    if constexpr (SPLIT > 1) {
+        const elem_t* part_ring = ring + part * SM::slot;
+        for (int i = 0; i < ns; i += SPLIT) {
+            wait_stages<SPT>(DMA && issued - SPLIT - i > 0 ? issued - SPLIT - i : 0);
+            workgroup_barrier();  // as below, of a step
+            if (i > 0 || !DMA) issue_step();
+            if (wave_active && i + part < ns) compute(part_ring + (i % R) * SM::slot);
+            commit_step();
+        }
+        using SP = Split16Smem<HD, kXWaves16, HAS_G ? 4 : 2>;
+        f32x4* red = reinterpret_cast<f32x4*>(smem_raw);
+        elem_t* tile = reinterpret_cast<elem_t*>(smem_raw + SP::red + SP::stat) + wave * StoreStage16<HD>::elems;
+        workgroup_barrier();  // every wave is done reading the ring
+        split_put<DT, kXWaves16>(red, 0, wave, lane, dk[0]);
+        split_put<DT, kXWaves16>(red, 1, wave, lane, dv[0]);
+        if constexpr (HAS_G) {
+            split_put<DT, kXWaves16>(red, 2, wave, lane, dtk[0]);
+            split_put<DT, kXWaves16>(red, 3, wave, lane, dtv[0]);
+        }
+        workgroup_barrier();
+        if (!wave_active) return;
+#pragma unroll
+        for (int k = 0; k < (HAS_G ? 4 : 2); ++k) {
+            if (k % SPLIT != part) continue;  // wave-uniform
+            const OutView out = k == 0 ? p.dk : k == 1 ? p.dv : k == 2 ? p.dtk : p.dtv;
+            split_sum<DT, kXWaves16, SPLIT>(dk[0], red, k, group, lane);
+            store_rows16<T, HD, IO>(tile, out.head(b, h), out.sl, wrow, p.Lk, p.D, dk[0], k % 2 == 0 ? p.scale : 1.0f, lane);
+        }
+        return;
+    }
     for (int i = 0; i < ns; ++i) {
         wait_stages<SPT>(DMA ? issued - 1 - i : 0);  // staged: the statistics still come by LDS-DMA
         workgroup_barrier();  // stage i has landed for every wave; stage i-1 is fully consumed
         if ((i > 0 || !DMA) && issued < ns) issue_next();
         if (wave_active) compute(ring + (i % R) * SM::slot);
-        if constexpr (!DMA) plan.commit();
+        commit_step();
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
     if (!wave_active) return;
@@ -717,9 +832,9 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1, int SPLIT = 1>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdParams p) {
-    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The column-owned launch with the second launch of the row-owned kernel at its end: workgroups
@@ -727,13 +842,14 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdPa
 // not depend on the column pass (it rewrites dQ, dQ_dot of flagged workgroups from the sums the first pass
 // left).  Nearly all of those workgroups leave at once; dealt out behind the column pass they fill the time in
 // which its last workgroups run alone, where a launch of their own costs a few microseconds.
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1, int SPLIT = 1,
+          int RROW = R>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks)
-        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT>(p, (int)blockIdx.x, col_blocks);
     else
-        bwd_row16_body<T, HD, R, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
+        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
 }
 
 // ---------------------------------------------------------------------------------------------

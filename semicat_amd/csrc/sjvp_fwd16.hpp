@@ -18,15 +18,17 @@ namespace sjvp {
 // moves into registers before the first stage is consumed, land in slots 2 and 3 (exactly their
 // size), which then join the ring.  After the last stage the ring doubles as the per-wave staging
 // tiles of the output stores.
-template <int HD, int R, bool JVP, int SPB = 1, bool DMA = true>
+template <int HD, int R, bool JVP, int SPB = 1, bool DMA = true, int SPLIT = 1>
 struct Fwd16Smem {
     static constexpr int nt = JVP ? 4 : 2;
     static constexpr int slot = nt * Slab<HD>::elems;
-    static constexpr int own = DMA ? (JVP ? 2 : 1) * 4 * Slab<HD>::elems : 0;
-    static_assert(SPB == 1 || (SPB == 2 && R == 4 && own == 2 * slot), "SPB = 2 needs a ring of four slots");
+    static constexpr int own = DMA && SPLIT == 1 ? (JVP ? 2 : 1) * 4 * Slab<HD>::elems : 0;
+    static_assert(SPB == 1 || SPLIT > 1 || (SPB == 2 && R == 4 && own == 2 * slot), "SPB = 2 needs a ring of four slots");
     static constexpr int own_off = SPB == 2 ? 2 * slot : 0;
     static constexpr int ring_off = SPB == 2 ? 0 : own;
-    static constexpr int sink = (SPB == 2 ? R * slot : own + R * slot) * (int)sizeof(elem_t);
+    static constexpr int loop = (SPB == 2 ? R * slot : own + R * slot) * (int)sizeof(elem_t);
+    static constexpr int after = SPLIT > 1 ? Split16Smem<HD, kWaves16, JVP ? 2 : 1>::bytes : 0;
+    static constexpr int sink = loop > after ? loop : after;
     static constexpr int bytes = sink + kSink16;
     static_assert(R * slot >= kWaves16 * StoreStage16<HD>::elems, "ring too small to stage stores");
 };
@@ -39,14 +41,19 @@ struct Fwd16Smem {
 // one stage ahead, and loads its own rows straight into registers.
 // NC: sets of 16 queries per wavefront (NC = 2: four wavefronts, every operand read from LDS feeds both sets; with tangents
 // 202 registers and no gain: 96.6 us against 97.6 at B=8 H=16 L=1024 D=64, 105 against 101 at B=128 H=12 L=256).
-template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1>
+// SPLIT > 1 (launches of few workgroups): the SPLIT waves of a group share 16 queries and take every SPLIT-th stage each, SPLIT
+// stages to a barrier; their partial sums are brought to one maximum and added in LDS, in a fixed order.
+template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1,
+          int SPLIT = 1>
 __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdParams p) {
     constexpr int NT = kThreads16 / NC;  // threads of the workgroup
     static_assert(!ROPE || (HD == 64 && SPB == 1), "the folded rotation covers HD = 64, one stage per barrier");
     constexpr bool DMA = IO == kIoDma;
-    static_assert(DMA || (SPB == 1 && !ROPE), "staged copies run one stage ahead, unrotated");
+    static_assert(DMA || ((SPB == 1 || SPLIT > 1) && !ROPE), "staged copies run one stage ahead, unrotated");
+    static_assert(SPLIT == 1 || (SPB == SPLIT && R == 2 * SPLIT && NC == 1 && !ROPE), "a step is a stage for every part");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    using SM = Fwd16Smem<HD, R, JVP, SPB, DMA>;
+    using SM = Fwd16Smem<HD, R, JVP, SPB, DMA, SPLIT>;
+    constexpr bool OWN_LDS = DMA && SPLIT == 1;  // the own rows come through LDS, else straight into registers
     elem_t* own = reinterpret_cast<elem_t*>(smem_raw) + SM::own_off;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw) + SM::ring_off;
     constexpr int SE = Slab<HD>::elems;
@@ -64,19 +71,29 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     const int bh = bid / p.q_blocks;
     const int qb = bid % p.q_blocks;
     const int b = bh / p.H, h = bh % p.H;
-    const int q0 = qb * kOwned16;
-    const int wrow = q0 + wave * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
+    const int part = SPLIT > 1 ? wave % SPLIT : 0, group = wave / SPLIT;
+    const int q0 = qb * (kOwned16 / SPLIT);
+    const int wrow = q0 + group * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
     const bool wave_active = wrow < p.Lq;
 
     u32x4 qB[NC][KC], tqB[NC][KC];
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, NT>, StagedPlan<T, HD, SM::nt, NT, IO>>;
     constexpr int SPT = StagePlan::N;
-    StagePlan plan;
+    StagePlan plan[DMA ? 1 : SPLIT];
     // slot layout K | V | K_dot | V_dot (primal only: K | V)
     const Src sk{p.k.head(b, h), p.k.sl}, sv{p.v.head(b, h), p.v.sl};
+    if constexpr (!OWN_LDS) {
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const int qrow = wrow + 16 * u + n;
+            load_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
+            if constexpr (JVP)
+                load_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
+        }
+    }
     if constexpr (DMA) {
         // own rows first (issued before the stages, so they land first), then the ring
-        {
+        if constexpr (OWN_LDS) {
             CopyPlan<HD, JVP ? 8 : 4, 4, NT> own_plan;
             if constexpr (JVP)
                 own_plan.init(tid, q0, p.D, smem_raw + SM::sink, Src{p.q.head(b, h), p.q.sl},
@@ -86,44 +103,61 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
             own_plan.issue(own, p.Lq - q0, p.D == HD && q0 + kOwned16 <= p.Lq);
         }
         if constexpr (JVP)
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, sk, sv, Src{p.tk.head(b, h), p.tk.sl},
+            plan[0].init(tid, 0, p.D, smem_raw + SM::sink, sk, sv, Src{p.tk.head(b, h), p.tk.sl},
                       Src{p.tv.head(b, h), p.tv.sl});
         else
-            plan.init(tid, 0, p.D, smem_raw + SM::sink, sk, sv);
+            plan[0].init(tid, 0, p.D, smem_raw + SM::sink, sk, sv);
     } else {
 #pragma unroll
-        for (int u = 0; u < NC; ++u) {
-            const int qrow = wrow + 16 * u + n;
-            staged_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
+        for (int u = 0; u < SPLIT; ++u) {
             if constexpr (JVP)
-                staged_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
-        }
-        if constexpr (JVP) {
-            plan.init(tid, p.D, sk, sv, Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
-        } else {
-            plan.init(tid, p.D, sk, sv);
+                plan[u].init(tid, p.D, sk, sv, Src{p.tk.head(b, h), p.tk.sl}, Src{p.tv.head(b, h), p.tv.sl});
+            else
+                plan[u].init(tid, p.D, sk, sv);
+            plan[u].take(u, SPLIT);
         }
     }
     const int ns = (p.Lk + kStageRows - 1) / kStageRows;
     int issued = 0;
     auto issue_next = [&]() {
         elem_t* slot = ring + (issued % R) * SM::slot;
-        if constexpr (DMA)
-            plan.issue(slot, p.Lk - issued * kStageRows, p.D == HD && (issued + 1) * kStageRows <= p.Lk);
-        else
-            plan.issue(slot, p.Lk - issued * kStageRows);
+        issue_plan(plan[0], slot, p.Lk - issued * kStageRows, p.D == HD && (issued + 1) * kStageRows <= p.Lk);
         ++issued;
     };
-    if constexpr (DMA) {
+    // staged copies: the stages of the next step (`ahead` of it in the ring), each through its own plan
+    auto stage_step = [&](int first) {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int u = 0; u < SPLIT; ++u)
+                if (first + u < ns) plan[u].issue(ring + ((first + u) % R) * SM::slot, p.Lk - (first + u) * kStageRows);
+        }
+    };
+    auto commit_step = [&]() {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int u = 0; u < SPLIT; ++u) plan[u].commit();
+        }
+    };
+    if constexpr (SPLIT > 1 && DMA) {
+        // the stages of the first step only: the loads of the own rows are awaited by a wait for all that is outstanding
+        while (issued < SPLIT && issued < ns) issue_next();
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            asm volatile("" : "+v"(qB[0][c]));
+            if constexpr (JVP) asm volatile("" : "+v"(tqB[0][c]));
+        }
+        while (issued < R && issued < ns) issue_next();
+    } else if constexpr (DMA) {
         while (issued < (SPB == 2 ? 2 : R) && issued < ns) issue_next();
     } else {
-        issue_next();
-        plan.commit();
+        stage_step(0);
+        commit_step();
     }
 
     const float sl2 = p.scale * kLog2e;
     // per set of queries
     float m_i[NC];     // reference maximum (same in the four lanes of a query)
+    float m_sub[NC];   // what the exponentials subtract: m_i, but 0 where no key of this lane's has a score above -inf yet
     float m_true[NC];  // maximum over the keys this lane has seen (for LI)
     float l_i[NC];     // exp-sum over the keys this lane has seen
     float mu_i[NC];    // sum of p * S_dot over the same keys
@@ -133,6 +167,7 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
 #pragma unroll
     for (int u = 0; u < NC; ++u) {
         m_i[u] = m_true[u] = -INFINITY;
+        m_sub[u] = 0.f;
         l_i[u] = mu_i[u] = 0.f;
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
@@ -142,9 +177,10 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     }
 
     // SPB = 1: the own rows and stage 0 were issued before the other stages; SPB = 2: everything
-    if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1);
+    if constexpr (SPLIT > 1) wait_stages<SPT>(DMA && issued > SPLIT ? issued - SPLIT : 0);
+    else if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1);
     workgroup_barrier();
-    if constexpr (DMA) {
+    if constexpr (OWN_LDS) {
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
             const int r0 = wave * 16 * NC + 16 * u;  // of the workgroup's 128 rows, 32 to a slab
@@ -167,7 +203,7 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
         }
     };
     rotate_stage(ring, 0);
-    if constexpr (SPB == 2) {
+    if constexpr (SPB == 2 && OWN_LDS) {
         // the operands must have arrived in registers before the copies below overwrite their slots
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         workgroup_barrier();
@@ -225,8 +261,10 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
 #pragma unroll
             for (int u = 0; u < NC; ++u) {
                 const float m_new = fmaxf(m_i[u], group_max(mloc[u]));
-                const float alpha = fast_exp2(m_i[u] - m_new);  // 0 on the first tile
+                // 0 on the first tile.  A part of a split group may hold nothing but keys that score -inf.
+                const float alpha = SPLIT == 1 || m_i[u] < m_new ? fast_exp2(m_i[u] - m_new) : 1.f;
                 m_i[u] = m_new;
+                m_sub[u] = SPLIT > 1 && m_new == -INFINITY ? 0.f : m_new;
                 l_i[u] *= alpha;
                 if constexpr (JVP) mu_i[u] *= alpha;
 #pragma unroll
@@ -243,7 +281,7 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float pj = fast_exp2(fmaf(s[u][t][j], sl2, -m_i[u]));
+                    const float pj = fast_exp2(fmaf(s[u][t][j], sl2, SPLIT > 1 ? -m_sub[u] : -m_i[u]));
                     s[u][t][j] = pj;
                     l_i[u] += pj;
                     if constexpr (JVP) {
@@ -274,6 +312,7 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     // One trip of the outer loop goes once round the ring, so that every LDS address of the
     // unrolled body is a per-lane constant plus an immediate offset.
     static_assert(R % SPB == 0, "a step must not wrap the ring");
+    const elem_t* part_ring = ring + part * SM::slot;
     for (int i0 = 0; i0 < ns; i0 += R) {
 #pragma unroll
         for (int h = 0; h < R; h += SPB) {
@@ -281,24 +320,87 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
             if (i >= ns) break;
             if (i > 0) {
                 // the stages of this step have landed for every wave; those of the last step are consumed
-                if constexpr (DMA) wait_stages<SPT>(SPB == 2 ? 0 : issued - 1 - i);
+                if constexpr (DMA) wait_stages<SPT>(SPB > 1 ? 0 : issued - 1 - i);
                 workgroup_barrier();
             }
-            if (i > 0 || !DMA) {
+            if constexpr (DMA) {
+                if (i > 0) {
 #pragma unroll
-                for (int u = 0; u < SPB; ++u)
-                    if (issued < ns) issue_next();
+                    for (int u = 0; u < SPB; ++u)
+                        if (issued < ns) issue_next();
+                }
+            } else {
+                stage_step(i + SPB);
             }
             if (i > 0) rotate_stage(ring + h * SM::slot, i * kStageRows);
-            if (wave_active) {
+            if constexpr (SPLIT > 1) {
+                if (wave_active && i + part < ns) compute(part_ring + h * SM::slot, (i + part) * kStageRows);
+            } else if (wave_active) {
 #pragma unroll
                 for (int u = 0; u < SPB; ++u)
                     if (i + u < ns) compute(ring + (h + u) * SM::slot, (i + u) * kStageRows);
             }
-            if constexpr (!DMA) plan.commit();
+            commit_step();
         }
     }
     workgroup_barrier();  // every wave is done reading the ring: it becomes the store staging area
+    if constexpr (SPLIT > 1) {
+        using SP = Split16Smem<HD, kWaves16, JVP ? 2 : 1>;
+        f32x4* red = reinterpret_cast<f32x4*>(smem_raw);
+        float* stat = reinterpret_cast<float*>(smem_raw + SP::red);
+        elem_t* tile = reinterpret_cast<elem_t*>(smem_raw + SP::red + SP::stat) + wave * StoreStage16<HD>::elems;
+        const int64_t so = (int64_t)bh * p.Lr + wrow + n;
+        float l = group_sum(l_i[0]), mu_un = group_sum(mu_i[0]), m_all = -INFINITY, t_all = -INFINITY;
+        if (p.li) m_true[0] = group_max(m_true[0]);
+        float* mine = stat + wave * 64 + n;
+        if (g == 0) {
+            mine[0] = m_i[0];
+            mine[16] = l;
+            mine[32] = mu_un;
+            mine[48] = m_true[0];
+        }
+        workgroup_barrier();
+        const float* all = stat + SPLIT * group * 64 + n;
+#pragma unroll
+        for (int s = 0; s < SPLIT; ++s) {
+            m_all = fmaxf(m_all, all[64 * s]);
+            t_all = fmaxf(t_all, all[64 * s + 48]);
+        }
+        l = mu_un = 0.f;
+#pragma unroll
+        for (int s = 0; s < SPLIT; ++s) {
+            const float f = fast_exp2(all[64 * s] - m_all);  // 0 for a part without keys
+            l += f * all[64 * s + 16];
+            mu_un += f * all[64 * s + 32];
+        }
+        const float inv_l = 1.0f / l, cmu = mu_un * inv_l, f = fast_exp2(m_i[0] - m_all);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            acc[0][d] *= f;
+            if constexpr (JVP) tacc[0][d] = tacc[0][d] * f - cmu * acc[0][d];  // see below
+        }
+        if (g == 0 && part == 0) {
+            // a group without queries gets what a zero query row produces
+            p.lse[so] = wave_active ? (m_all + fast_log2(l)) * kLn2 : fast_log2((float)p.Lk) * kLn2;
+            if constexpr (JVP) p.mu[so] = wave_active ? cmu : 0.f;
+            if (p.li) p.li[so] = wave_active ? l * fast_exp2(m_all - t_all) : (float)p.Lk;
+        }
+        split_put<DT, kWaves16>(red, 0, wave, lane, acc[0]);
+        if constexpr (JVP) split_put<DT, kWaves16>(red, 1, wave, lane, tacc[0]);
+        workgroup_barrier();
+        if (!wave_active) return;
+        if (part == 0) {
+            split_sum<DT, kWaves16, SPLIT>(acc[0], red, 0, group, lane);
+            store_rows16<T, HD, IO>(tile, p.o.head(b, h), p.o.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
+        }
+        if constexpr (JVP) {
+            if (part == 1) {
+                split_sum<DT, kWaves16, SPLIT>(acc[0], red, 1, group, lane);
+                store_rows16<T, HD, IO>(tile, p.to.head(b, h), p.to.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
+            }
+        }
+        return;
+    }
     elem_t* stage_tile = ring + wave * StoreStage16<HD>::elems;
 #pragma unroll
     for (int u = 0; u < NC; ++u) {

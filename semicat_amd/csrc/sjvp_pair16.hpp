@@ -27,7 +27,22 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         // keys on (128 of them 1.02).
         bool wide = false;
         if constexpr (!HAS_G && IO == kIoDma) wide = p.rowfix != 2 && grid >= 1024 && p.Lk >= 256;
-        if (wide) {
+        int split = 1;
+        if constexpr (HD <= 64 && IO != kIoF32) {
+            constexpr int MOST = IO == kIoDma ? 4 : 2;  // (four parts' staged copies do not fit the registers)
+            if (p.rowfix != 2) split = split_rows(grid, (p.Lk + kStageRows - 1) / kStageRows, MOST, true);
+            if (split == 2)
+                rc = launch(bwd_row16_kernel<T, HD, 4, HAS_DO, HAS_G, 2, 0, IO, 1, 2>, grid * 2,
+                            Row16Smem<HD, 4, HAS_G, 2>::bytes, stream, p, kXThreads16);
+            if constexpr (MOST == 4) {
+                if (split == 4)
+                    rc = launch(bwd_row16_kernel<T, HD, 8, HAS_DO, HAS_G, 2, 0, IO, 1, 4>, grid * 4,
+                                Row16Smem<HD, 8, HAS_G, 4>::bytes, stream, p, kXThreads16);
+            }
+        }
+        if (split > 1) {
+            // done above
+        } else if (wide) {
             if constexpr (!HAS_G && IO == kIoDma)
                 rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, HD == 128 ? 2 : 3, 0, IO, 2>, grid / 2, smem, stream, p,
                             kXThreads16);
@@ -59,6 +74,23 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         }
         return launch(bwd_col16p_kernel<T, HD, PR, HAS_DO, HAS_G, IO>, grid, PS::bytes, stream, p, kThreads16);
     } else {
+        if constexpr (HD <= 64 && IO != kIoF32) {
+            constexpr int MOST = IO == kIoDma ? 4 : 2;
+            const int split = rides ? split_rows(grid, (p.Lq + kStageRows - 1) / kStageRows, MOST, IO == kIoDma) : 1;
+            auto go = [&](auto split_tag) {
+                constexpr int SPLIT = decltype(split_tag)::value;
+                constexpr int OWNED = kXOwned16 / SPLIT;
+                BwdParams pr = p;
+                pr.col_workgroups = BH * ((p.Lk + OWNED - 1) / OWNED);
+                constexpr int row = Row16Smem<HD, XR, HAS_G>::bytes, col = Col16Smem<HD, 2 * SPLIT, HAS_DO, HAS_G, SPLIT>::bytes;
+                return launch(bwd_col16_repair_kernel<T, HD, 2 * SPLIT, HAS_DO, HAS_G, 2, IO, 1, SPLIT, XR>,
+                              pr.col_workgroups + BH * (p.Lr / kXOwned16), col > row ? col : row, stream, pr, kXThreads16);
+            };
+            if (split == 2) return go(std::integral_constant<int, 2>{});
+            if constexpr (MOST == 4) {
+                if (split == 4) return go(std::integral_constant<int, 4>{});
+            }
+        }
         // 32 keys per wave where the accumulators leave room for them (as in the row-owned launch): 92 -> 80 us at B=8
         // H=16 L=1024 D=64, cotangent on O only, from two workgroups of 64 keys per compute unit on (512 of them 0.96 to
         // 1.01 of the time, 256 1.16 to 1.23); at D = 32 with both cotangents 129 -> 112 us, from 1024 workgroups and

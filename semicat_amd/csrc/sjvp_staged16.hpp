@@ -123,6 +123,14 @@ struct StagedPlan {
             adv[i] = 32 * s.sl;
         }
     }
+    // Windows first, first + step, ... instead of all of them.
+    __device__ __forceinline__ void take(int first, int step) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            src[i] += first * adv[i];
+            adv[i] *= step;
+        }
+    }
     // Request the next window for `to`; rows_left of its rows exist (zeros beyond).
     __device__ __forceinline__ void issue(elem_t* to, int rows_left) {
         region = to;
@@ -154,6 +162,26 @@ struct StagedPlan {
         }
     }
 };
+
+// B operands (all head-dimension chunks of 32) of one owned row, straight from global memory.
+template <typename T, int HD, int IO>
+__device__ __forceinline__ void load_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
+    if constexpr (IO != kIoDma) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
+#pragma unroll
+    for (int c = 0; c < HD / 32; ++c) {
+        out[c] = u32x4{0u, 0u, 0u, 0u};
+        if (valid && 32 * c + 8 * g < D) out[c] = *reinterpret_cast<const u32x4*>(row + 32 * c + 8 * g);
+    }
+}
+
+// The same from a uniform slice pointer and the lane's byte offset in the slice: whole rows of HD elements
+// that all exist, no predicates, one 32-bit offset for every tensor of equal strides.
+template <int HD>
+__device__ __forceinline__ void load_b_operands16_at(u32x4* out, const elem_t* slice, uint32_t lane_bytes) {
+    const char* base = reinterpret_cast<const char*>(slice);
+#pragma unroll
+    for (int c = 0; c < HD / 32; ++c) out[c] = *reinterpret_cast<const u32x4*>(base + lane_bytes + 64 * c);
+}
 
 // One 16-byte piece (columns 8c ..) of a 16-bit row of any alignment, masked at D.
 __device__ __forceinline__ void store_piece(elem_t* dst, u32x4 v, int d, int D) {

@@ -24,6 +24,19 @@ int fwd16_one(const FwdParams& p, int grid, hipStream_t stream) {
             return launch(fwd16_kernel<T, HD, R, JVP, HD == 128 ? 2 : 4, SPB, ROPE, kIoDma, 2>, grid, smem, stream, p,
                           kThreads16 / 2);
     }
+    if constexpr (HD <= 64 && !ROPE) {
+        // (D = 128: the sums do not fit the LDS.  Up to 128 keys the folded rotation is an alternative to this launch, and
+        // both round alike.)
+        const int split = p.Lk > kOwned16 ? split_rows(grid, (p.Lk + kStageRows - 1) / kStageRows, 4, false) : 1;
+        FwdParams ps = p;
+        ps.q_blocks *= split;
+        if (split == 2)
+            return launch(fwd16_kernel<T, HD, 4, JVP, 4, 2, false, kIoDma, 1, 2>, grid * 2,
+                          Fwd16Smem<HD, 4, JVP, 2, true, 2>::bytes, stream, ps, kThreads16);
+        if (split == 4)
+            return launch(fwd16_kernel<T, HD, 8, JVP, 4, 4, false, kIoDma, 1, 4>, grid * 4,
+                          Fwd16Smem<HD, 8, JVP, 4, true, 4>::bytes, stream, ps, kThreads16);
+    }
     return launch(fwd16_kernel<T, HD, R, JVP, OCC, SPB, ROPE>, grid, smem, stream, p, kThreads16);
 }
 

@@ -316,4 +316,28 @@ __device__ __forceinline__ void store_tile16(elem_t* stage, elem_t* gp, int64_t 
     }
 }
 
+// Sums over the SPLIT waves that share a group of owned rows (waves SPLIT * group + part, NW waves), through LDS in a
+// fixed order.  Tensor k of a wave's accumulators goes to red[k][wave][DT][64]; behind a barrier the wave of part
+// k % SPLIT fetches the sum.
+template <int DT, int NW>
+__device__ __forceinline__ void split_put(f32x4* red, int k, int wave, int lane, const f32x4* acc) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) red[((k * NW + wave) * DT + d) * 64 + lane] = acc[d];
+}
+template <int DT, int NW, int SPLIT>
+__device__ __forceinline__ void split_sum(f32x4* acc, const f32x4* red, int k, int group, int lane) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+        acc[d] = red[((k * NW + SPLIT * group) * DT + d) * 64 + lane];
+#pragma unroll
+        for (int s = 1; s < SPLIT; ++s) acc[d] += red[((k * NW + SPLIT * group + s) * DT + d) * 64 + lane];
+    }
+}
+template <int HD, int NW, int TENSORS>
+struct Split16Smem {  // after the loop: the sums, four statistics of each wave's 16 rows, the waves' staging tiles
+    static constexpr int red = TENSORS * NW * (HD / 16) * 64 * (int)sizeof(f32x4);
+    static constexpr int stat = NW * 4 * 16 * (int)sizeof(float);
+    static constexpr int bytes = red + stat + NW * StoreStage16<HD>::elems * (int)sizeof(elem_t);
+};
+
 }  // namespace sjvp
