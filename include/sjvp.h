@@ -263,6 +263,15 @@ int sjvp_adaln_bwd(const sjvp_adaln* t, int jvp, void* stream);
 int sjvp_gelu(const void* u, const void* tu, const void* dy, const void* dty, void* y, void* ty, int64_t n,
               int reverse, void* stream);
 
+/*
+ * Casts n dense tensors (1 <= n <= SJVP_CAST_MAX, count[i] elements each, any alignment that their type has) from
+ * fp32 to bf16 or fp16, or from bf16 or fp16 to fp32, all in one launch: to nearest even, NaN stays NaN.
+ * No counterpart in the reference, which casts one tensor at a time (semicat/jvp_utils/functional.py:318-331).
+ */
+#define SJVP_CAST_MAX 16
+int sjvp_cast(int n, const void* const* x, void* const* y, const int64_t* count, int in_dtype, int out_dtype,
+              void* stream);
+
 /* Static, NUL-terminated description of a status code. */
 const char* sjvp_strerror(int status);
 

@@ -43,7 +43,7 @@ SJVP_REPAIR_AUTO = 1
 SJVP_REPAIR_ALWAYS = 2
 
 EXPORTS = ("sjvp_fwd", "sjvp_bwd", "sjvp_bwd_parts", "sjvp_bwd_noalloc", "sjvp_fwd_rotary", "sjvp_bwd_rotary", "sjvp_bwd_workspace_bytes", "sjvp_rope",
-           "sjvp_adaln_fwd", "sjvp_adaln_bwd", "sjvp_adaln_workspace_floats", "sjvp_gelu",
+           "sjvp_adaln_fwd", "sjvp_adaln_bwd", "sjvp_adaln_workspace_floats", "sjvp_gelu", "sjvp_cast",
            "sjvp_set_row_sum_repair", "sjvp_strerror", "sjvp_version", "sjvp_build_id")
 
 
@@ -103,6 +103,8 @@ def load() -> ctypes.CDLL:
             vpp = ctypes.POINTER(ctypes.c_void_p)
             lib.sjvp_rope.argtypes = [i, vpp, vpp, i64p, vp, vp, ctypes.c_int64] + [i] * 8 + [vp]
             lib.sjvp_rope.restype = i
+            lib.sjvp_cast.argtypes = [i, vpp, vpp, i64p, i, i, vp]
+            lib.sjvp_cast.restype = i
             ada = ctypes.POINTER(AdaLn)
             lib.sjvp_adaln_fwd.argtypes = lib.sjvp_adaln_bwd.argtypes = [ada, i, vp]
             lib.sjvp_adaln_fwd.restype = lib.sjvp_adaln_bwd.restype = i
@@ -136,7 +138,7 @@ def _load_host(lib: ctypes.CDLL):
         raise RuntimeError(f"{path} was built from other sources than the ones in this tree, or against another torch")
     host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in
                 (lib.sjvp_fwd, lib.sjvp_fwd_rotary, lib.sjvp_bwd_parts, lib.sjvp_bwd_rotary,
-                 lib.sjvp_bwd_workspace_bytes)))
+                 lib.sjvp_bwd_workspace_bytes, lib.sjvp_cast)))
     return host
 
 

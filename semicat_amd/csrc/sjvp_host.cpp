@@ -6,6 +6,7 @@
 // or types, wrappers of functorch or of tensor subclasses, host tensors, empty problems): the caller in kernels.py
 // then goes through its general form, which raises the errors.  They return the status of the C ABI when it is not 0.
 #include <ATen/ATen.h>
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -27,6 +28,7 @@ struct Abi {
     decltype(&sjvp_bwd_parts) bwd_parts = nullptr;
     decltype(&sjvp_bwd_rotary) bwd_rotary = nullptr;
     decltype(&sjvp_bwd_workspace_bytes) workspace_bytes = nullptr;
+    decltype(&sjvp_cast) cast = nullptr;
 };
 Abi abi;  // filled once by bind() when the library is loaded
 
@@ -297,14 +299,82 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(addresses of sjvp_fwd, sjvp_fwd_rotary, sjvp_bwd_parts, sjvp_bwd_rotary, sjvp_bwd_workspace_bytes)
+// cast(list of tensors or None, dtype) -> list; a tensor that has the dtype is handed back itself, the others, dense and
+// between fp32 and one 16-bit type, are copied in as few launches as it takes.  Nothing is recorded for autograd.
+PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 2 || !abi.cast || !PyList_CheckExact(a[0]) || !THPDtype_Check(a[1])) return none();
+    const at::ScalarType to = reinterpret_cast<THPDtype*>(a[1])->scalar_type;
+    constexpr int kMost = 64;
+    const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+    if (count > kMost) return none();
+    auto tag = [](at::ScalarType t) { return t == at::kFloat ? SJVP_FP32 : t == at::kBFloat16 ? SJVP_BF16 : t == at::kHalf ? SJVP_FP16 : -1; };
+    const Tensor* in[kMost] = {};
+    at::ScalarType from = to;
+    const Tensor* some = nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject* obj = PyList_GET_ITEM(a[0], i);
+        if (obj == Py_None) continue;
+        const Tensor* t = plain(obj);
+        if (!t) return none();
+        if (t->scalar_type() == to) continue;
+        if (!some) some = t, from = t->scalar_type();
+        if (t->scalar_type() != from || t->device() != some->device() || !t->is_non_overlapping_and_dense()) return none();
+        in[i] = t;
+    }
+    if (some && (tag(from) < 0 || tag(to) < 0 || (from == at::kFloat) == (to == at::kFloat))) return none();
+    Tensor made[kMost];
+    int rc = SJVP_OK;
+    if (some) {
+        pybind11::gil_scoped_release no_gil;
+        const c10::DeviceGuard guard(some->device());
+        void* stream = c10::hip::getCurrentHIPStream(some->device().index()).stream();
+        const void* x[SJVP_CAST_MAX];
+        void* y[SJVP_CAST_MAX];
+        int64_t numel[SJVP_CAST_MAX];
+        int k = 0;
+        for (Py_ssize_t i = 0; i < count && rc == SJVP_OK; ++i) {
+            if (in[i]) {
+                made[i] = at::empty_like(*in[i], in[i]->options().dtype(to));
+                x[k] = in[i]->const_data_ptr();
+                y[k] = made[i].mutable_data_ptr();
+                numel[k++] = in[i]->numel();
+            }
+            if (k == SJVP_CAST_MAX || (k && i + 1 == count)) {
+                rc = abi.cast(k, x, y, numel, tag(from), tag(to), stream);
+                k = 0;
+            }
+        }
+    }
+    if (rc != SJVP_OK) return PyLong_FromLong(rc);
+    PyObject* res = PyList_New(count);
+    if (!res) return nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject* item;
+        if (in[i]) {
+            item = THPVariable_Wrap(std::move(made[i]));
+        } else {
+            item = PyList_GET_ITEM(a[0], i);
+            Py_INCREF(item);
+        }
+        if (!item) {
+            Py_DECREF(res);
+            return nullptr;
+        }
+        PyList_SET_ITEM(res, i, item);
+    }
+    return res;
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses of sjvp_fwd, sjvp_fwd_rotary, sjvp_bwd_parts, sjvp_bwd_rotary, sjvp_bwd_workspace_bytes, sjvp_cast)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 5) {
-        PyErr_SetString(PyExc_TypeError, "bind() takes five addresses");
+    if (n != 6) {
+        PyErr_SetString(PyExc_TypeError, "bind() takes six addresses");
         return nullptr;
     }
-    void* p[5];
-    for (int i = 0; i < 5; ++i) {
+    void* p[6];
+    for (int i = 0; i < 6; ++i) {
         p[i] = PyLong_AsVoidPtr(a[i]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind(): null address");
@@ -313,7 +383,7 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     abi = {reinterpret_cast<decltype(abi.fwd)>(p[0]), reinterpret_cast<decltype(abi.fwd_rotary)>(p[1]),
            reinterpret_cast<decltype(abi.bwd_parts)>(p[2]), reinterpret_cast<decltype(abi.bwd_rotary)>(p[3]),
-           reinterpret_cast<decltype(abi.workspace_bytes)>(p[4])};
+           reinterpret_cast<decltype(abi.workspace_bytes)>(p[4]), reinterpret_cast<decltype(abi.cast)>(p[5])};
     return none();
 }
 
@@ -325,6 +395,7 @@ const char build_id[] = SJVP_BUILD_ID;
 PyMethodDef methods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
     {"backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(backward)), METH_FASTCALL, nullptr},
+    {"cast", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cast)), METH_FASTCALL, nullptr},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
