@@ -328,11 +328,26 @@ class _CastOf(torch.autograd.Function):
         return g.to(ctx.dtype), None
 
 
+class CastFunction(torch.autograd.Function):
+    """bf16 copies of fp32 parameters, all of them in one launch, and their gradients in fp32 in another."""
+
+    @staticmethod
+    def forward(ctx, *params):
+        ctx.set_materialize_grads(False)
+        return tuple(functional._cast_all(params, (torch.bfloat16,) * len(params)))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        if torch.is_grad_enabled():  # a recorded backward
+            return tuple(None if g is None else g.float() for g in grads)
+        return tuple(functional._cast_all(grads, (torch.float32,) * len(grads)))
+
+
 class LinearFunction(torch.autograd.Function):
     """``x w^T + b`` and ``tx w^T``; in reverse mode one product for both inputs and one, summed over both in fp32, for the
     weight.  Through the general dispatch forward mode adds products with the absent tangents of weight and bias,
     zero fills and sums: 9 products per layer and step instead of 4.
-    bf16 products on a bf16 copy of the fp32 weight, as autocast makes it."""
+    bf16 products on a bf16 copy of the fp32 weight, as autocast makes it (or on one that is handed in)."""
 
     @staticmethod
     def forward(ctx, x, tx, w, b):
@@ -476,23 +491,58 @@ def gelu(u: Tensor) -> Optional[Tensor]:
 
 
 @torch._dynamo.disable
-def linear(layer: nn.Linear, x: Tensor) -> Optional[Tensor]:
-    """The layer on a dual tensor, or None where it is not served (a plain tensor included: that is one product
-    already).  The caller has asked :func:`serves_block`."""
-    w, b = layer.weight, layer.bias
-    if type(layer) is not nn.Linear or not bare(layer) or x.dtype != torch.bfloat16 \
-            or _functorch.get_interpreter_stack() is None:
+def cast(*layers: nn.Linear):
+    """``{layer: (weight, bias)}`` with bf16 copies of the fp32 parameters of linear layers for :func:`linear`, made by one launch
+    where autocast would cast one by one (and once more for each use under forward mode), or None where that is not
+    served.  The caller has asked :func:`serves_block`."""
+    stack = _functorch.get_interpreter_stack()
+    if stack is None:
+        if fwAD._current_level >= 0:
+            return None
+    elif len(stack) != 1 or stack[0].key() != functional.TransformType.Jvp:
+        return None
+    if not all(type(m) is nn.Linear for m in layers) or not bare(*layers):
+        return None
+    params = [p for m in layers for p in (m.weight, m.bias) if p is not None]
+    if any(type(p) not in (Tensor, nn.Parameter) or p.dtype != torch.float32 or p.device != params[0].device or not p.is_cuda
+           or _functorch.is_functorch_wrapped_tensor(p) for p in params):
+        return None
+    if stack is None:
+        copies = iter(CastFunction.apply(*params))
+    else:
+        with functional.retrieve_current_functorch_interpreter().lower():
+            copies = iter(CastFunction.apply(*params))
+    return {m: (next(copies), None if m.bias is None else next(copies)) for m in layers}
+
+
+@torch._dynamo.disable
+def linear(layer: nn.Linear, x: Tensor, copies=None) -> Optional[Tensor]:
+    """The layer on a dual tensor, with the ``copies`` of :func:`cast` where there are any, or None where it is not served (a
+    plain tensor included: that is one product already).  The caller has asked :func:`serves_block`."""
+    if copies is None:
+        if type(layer) is not nn.Linear or not bare(layer):
+            return None
+        w, b, dtype = layer.weight, layer.bias, torch.float32
+    else:
+        (w, b), dtype = copies[layer], torch.bfloat16
+    if x.dtype != torch.bfloat16 or _functorch.get_interpreter_stack() is None:
         return None
     found = _unwrap((x, w, b))
     if found is None:
         return None
     interpreter, (p, w, b), (t, *absent) = found
     if t is None or any(z is not None for z in absent) or t.dtype != p.dtype or t.shape != p.shape or p.numel() == 0 \
-            or any(z.dtype != torch.float32 or z.device != p.device for z in (w, b) if z is not None):
+            or any(z.dtype != dtype or z.device != p.device for z in (w, b) if z is not None):
         return None
     with interpreter.lower():
         y, ty = LinearFunction.apply(p, t, w, b)
     return _dual_above(interpreter, y, ty)
+
+
+@torch._dynamo.disable
+def plain_linear(layer: nn.Linear, x: Tensor, copies) -> Optional[Tensor]:
+    """The layer on a plain tensor with the copies of :func:`cast`; None inside a transform."""
+    return None if _functorch.get_interpreter_stack() is not None else nn.functional.linear(x, *copies[layer])
 
 
 @torch._dynamo.disable

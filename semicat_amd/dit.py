@@ -91,8 +91,10 @@ class TimestepEmbedder(nn.Module):
         return self.mlp(torch.cat((phase.cos(), phase.sin()), dim=-1))
 
 
-def _linear(fused: bool, layer: nn.Linear, x: Tensor) -> Tensor:
-    y = adaln.linear(layer, x) if fused else None
+def _linear(fused: bool, layer: nn.Linear, x: Tensor, copies=None) -> Tensor:
+    y = adaln.linear(layer, x, copies) if fused else None
+    if y is None and copies is not None:
+        y = adaln.plain_linear(layer, x, copies)
     return layer(x) if y is None else y
 
 
@@ -143,11 +145,12 @@ class DDiTBlock(nn.Module):
         B = x.shape[0]
         # one launch for each run of element-wise operations where the library serves them (adaln.py)
         fused = rotary_kernel and attention is safe_sdpa_jvp and self._fuses(x)
-        mod = _linear(fused, self.adaLN_modulation, c)
+        copies = adaln.cast(self.adaLN_modulation, self.attn_qkv, self.attn_out, self.mlp[0], self.mlp[2]) if fused else None
+        mod = _linear(fused, self.adaLN_modulation, c, copies)
         pieces = adaln.chunk(mod, 6) if fused else None
         shift_a, scale_a, gate_a, shift_m, scale_m, gate_m = mod[:, None].chunk(6, dim=2) if pieces is None else pieces
         h = self._norm(fused, x, None, None, self.norm1, scale_a, shift_a)[1]
-        qkv = _linear(fused, self.attn_qkv, h).view(B, self.seq_len, 3, self.n_heads, self.dim // self.n_heads)
+        qkv = _linear(fused, self.attn_qkv, h, copies).view(B, self.seq_len, 3, self.n_heads, self.dim // self.n_heads)
         if rotary_kernel and attention is safe_sdpa_jvp:
             # the attention kernels read q, k, v (and their tangents) as strided views of the fused
             # projection and rotate q, k on chip; gradients come back through the inverse rotation
@@ -156,12 +159,12 @@ class DDiTBlock(nn.Module):
             if a is None:
                 a = safe_sdpa_jvp_rotary(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], cos, sin)
             a = a.reshape(B, self.seq_len, self.dim)
-            x, h = self._norm(fused, x, _linear(fused, self.attn_out, a), gate_a, self.norm2, scale_m, shift_m)
+            x, h = self._norm(fused, x, _linear(fused, self.attn_out, a, copies), gate_a, self.norm2, scale_m, shift_m)
             if not fused:
                 return self.dropout(self.mlp(h) * gate_m) + x
-            h = _linear(fused, self.mlp[0], h)
+            h = _linear(fused, self.mlp[0], h, copies)
             g = adaln.gelu(h)
-            h = _linear(fused, self.mlp[2], self.mlp[1](h) if g is None else g)
+            h = _linear(fused, self.mlp[2], self.mlp[1](h) if g is None else g, copies)
             return self._norm(fused, x, h, gate_m, None, None, None)[0]
         v = qkv[:, :, 2]
         if rotary_kernel:
@@ -205,12 +208,12 @@ class DDiTFinalLayer(nn.Module):
 
     def forward(self, x: Tensor, c: Tensor, fused: bool = False) -> Tensor:
         fused = fused and adaln.serves_block(x) and adaln.bare(self.norm_final)
-        mod = _linear(fused, self.adaLN_modulation, c)
+        copies = adaln.cast(self.adaLN_modulation, self.linear) if fused else None
+        mod = _linear(fused, self.adaLN_modulation, c, copies)
         pieces = adaln.chunk(mod, 2) if fused else None
         shift, scale = mod[:, None].chunk(2, dim=2) if pieces is None else pieces
         both = adaln.gated_norm(x, None, None, self.norm_final, scale, shift) if fused else None
-        return _linear(fused, self.linear,
-                       self.norm_final(x) * (1.0 + scale) + shift if both is None else both[1])
+        return _linear(fused, self.linear, self.norm_final(x) * (1.0 + scale) + shift if both is None else both[1], copies)
 
 
 class DIT(nn.Module):

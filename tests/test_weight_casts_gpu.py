@@ -1,0 +1,84 @@
+"""The linear layers' parameters cast by one launch per block: the bits that autocast's own casts give, in every mode that reaches
+the layers, and none of it where a layer is more than its class."""
+import pytest
+import torch
+
+from semicat_amd import adaln, train_step
+from semicat_amd.dit import DIT
+
+pytestmark = pytest.mark.gpu
+
+
+def _net():
+    torch.manual_seed(0)
+    net = DIT(48, 128, 16, 2, 2, 0.0, 16).cuda()
+    for p in net.parameters():
+        if not p.any():
+            torch.nn.init.normal_(p, std=0.05)
+    return net, torch.randn(4, 16, 48, device="cuda"), torch.randint(0, 48, (4, 16), device="cuda")
+
+
+def _step(net, x0, x1, create_graph=False):
+    t = torch.linspace(0.2, 0.8, 4, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        vf = train_step.vfm_loss(net, x0[2:], x1[2:], t=t[2:])
+        sd = train_step.lag_self_distillation_loss(net, x0[:2], x1[:2], t=t[:2], s=t[:2] / 2)
+    loss = vf if create_graph else vf + sd  # (the op itself cannot be differentiated twice)
+    return [vf, sd, *torch.autograd.grad(loss, list(net.parameters()), create_graph=create_graph)]
+
+
+def test_same_bits_as_autocast(monkeypatch):
+    net, x0, x1 = _net()
+    served = []
+    cast = adaln.cast
+    monkeypatch.setattr(adaln, "cast", lambda *m: served.append(cast(*m)) or served[-1])
+    got = _step(net, x0, x1)
+    assert len(served) == 3 * 3 and all(c is not None for c in served)
+    monkeypatch.setattr(adaln, "cast", lambda *m: None)
+    for a, b in zip(got, _step(net, x0, x1)):
+        assert a.dtype == b.dtype and a.stride() == b.stride() and torch.equal(a, b)
+
+
+def test_frozen_parameters_and_no_grad(monkeypatch):
+    net, x0, x1 = _net()
+    net.blocks[0].attn_qkv.weight.requires_grad_(False)
+    net.blocks[1].mlp[0].bias.requires_grad_(False)
+
+    def run():
+        net.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            loss = train_step.vfm_loss(net, x0, x1, t=torch.full((4,), 0.5, device="cuda"))
+            with torch.no_grad():
+                out = net(x0, *torch.full((2, 4), 0.25, device="cuda"))
+        loss.backward()
+        return [loss, out, *(p.grad for p in net.parameters())]
+
+    got = run()
+    monkeypatch.setattr(adaln, "cast", lambda *m: None)
+    for a, b in zip(got, run()):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+def test_recorded_backward_of_the_casts():
+    w, b = (torch.randn(n, device="cuda", requires_grad=True) for n in (24, 8))
+    w16, b16 = adaln.CastFunction.apply(w, b)
+    assert w16.dtype == b16.dtype == torch.bfloat16
+    gw, = torch.autograd.grad((w16 * w16).sum(), w, create_graph=True)
+    assert gw.dtype == torch.float32 and torch.equal(gw, 2 * w16.float())
+    assert torch.equal(torch.autograd.grad(gw.sum(), w)[0], torch.full_like(w, 2.0))
+
+
+def test_layers_that_are_left_to_pytorch():
+    net, _, _ = _net()
+    block = net.blocks[0]
+    assert adaln.cast(block.attn_qkv, block.attn_out) is not None
+    handle = block.attn_out.register_forward_hook(lambda *a: None)
+    assert adaln.cast(block.attn_qkv, block.attn_out) is None
+    handle.remove()
+    assert adaln.cast(block.attn_qkv, torch.nn.Linear(4, 4)) is None  # another device
+    assert adaln.cast(torch.nn.Linear(4, 4, device="cuda", dtype=torch.bfloat16)) is None
+    assert adaln.cast(torch.nn.utils.parametrizations.weight_norm(torch.nn.Linear(4, 4, device="cuda"))) is None
+    with torch.autograd.forward_ad.dual_level():
+        assert adaln.cast(block.attn_qkv) is None
+    torch.func.vmap(lambda z: (adaln.cast(block.attn_qkv) is None or 1 / 0, z)[1])(torch.zeros(2, device="cuda"))
+    torch.func.grad(lambda z: (adaln.cast(block.attn_qkv) is None or 1 / 0, z)[1])(torch.zeros((), device="cuda"))
