@@ -29,6 +29,10 @@ struct Abi {
     decltype(&sjvp_bwd_rotary) bwd_rotary = nullptr;
     decltype(&sjvp_bwd_workspace_bytes) workspace_bytes = nullptr;
     decltype(&sjvp_cast) cast = nullptr;
+    decltype(&sjvp_adaln_fwd) adaln_fwd = nullptr;
+    decltype(&sjvp_adaln_bwd) adaln_bwd = nullptr;
+    decltype(&sjvp_adaln_workspace_floats) adaln_workspace_floats = nullptr;
+    decltype(&sjvp_gelu) gelu = nullptr;
 };
 Abi abi;  // filled once by bind() when the library is loaded
 
@@ -367,23 +371,111 @@ PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(addresses of sjvp_fwd, sjvp_fwd_rotary, sjvp_bwd_parts, sjvp_bwd_rotary, sjvp_bwd_workspace_bytes, sjvp_cast)
+// The pointer members of sjvp_adaln by the names of the tensors they take.
+struct AdaField {
+    const char* name;
+    void** (*at)(sjvp_adaln&);
+    int mod;  // place in mod_stride, or -1
+};
+#define SJVP_ADA(name, mod) {#name, [](sjvp_adaln& t) { return reinterpret_cast<void**>(const_cast<void*>(static_cast<const void*>(&t.name))); }, mod}
+const AdaField ada_fields[] = {
+    SJVP_ADA(x, -1), SJVP_ADA(tx, -1), SJVP_ADA(a, -1), SJVP_ADA(ta, -1), SJVP_ADA(gate, 0), SJVP_ADA(tgate, 1),
+    SJVP_ADA(scale, 2), SJVP_ADA(tscale, 3), SJVP_ADA(shift, 4), SJVP_ADA(tshift, 5), SJVP_ADA(w, -1), SJVP_ADA(b, -1),
+    SJVP_ADA(y, -1), SJVP_ADA(ty, -1), SJVP_ADA(h, -1), SJVP_ADA(th, -1), SJVP_ADA(dy, -1), SJVP_ADA(dty, -1),
+    SJVP_ADA(dh, -1), SJVP_ADA(dth, -1), SJVP_ADA(dx, -1), SJVP_ADA(dtx, -1), SJVP_ADA(da, -1), SJVP_ADA(dta, -1),
+    SJVP_ADA(dgate, -1), SJVP_ADA(dtgate, -1), SJVP_ADA(dscale, -1), SJVP_ADA(dtscale, -1), SJVP_ADA(dshift, -1),
+    SJVP_ADA(dtshift, -1), SJVP_ADA(dw, -1), SJVP_ADA(db, -1)};
+#undef SJVP_ADA
+constexpr int kAdaFields = sizeof(ada_fields) / sizeof(ada_fields[0]);
+PyObject* ada_names[kAdaFields];  // interned, made by bind()
+
+// adaln(reverse, jvp, B, S, W, eps, {name: tensor or None}) -> status; the caller has laid the tensors out and keeps them
+PyObject* adaln(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 7 || !abi.adaln_fwd || !PyDict_CheckExact(a[6])) return none();
+    sjvp_adaln t{};
+    t.B = static_cast<int>(PyLong_AsLong(a[2]));
+    t.S = static_cast<int>(PyLong_AsLong(a[3]));
+    t.W = static_cast<int>(PyLong_AsLong(a[4]));
+    t.eps = static_cast<float>(PyFloat_AsDouble(a[5]));
+    if (PyErr_Occurred()) return nullptr;
+    const Tensor* x = nullptr;
+    for (int i = 0; i < kAdaFields; ++i) {
+        PyObject* obj = PyDict_GetItem(a[6], ada_names[i]);
+        if (!obj || obj == Py_None) continue;
+        const Tensor* z = plain(obj);
+        if (!z || (x && z->device() != x->device())) return none();
+        if (!x) x = z;
+        *ada_fields[i].at(t) = z->data_ptr();
+        if (ada_fields[i].mod >= 0) t.mod_stride[ada_fields[i].mod] = z->stride(0);
+    }
+    if (!x || !t.x) return none();
+    int rc;
+    {
+        pybind11::gil_scoped_release no_gil;
+        const c10::DeviceGuard guard(x->device());
+        void* stream = c10::hip::getCurrentHIPStream(x->device().index()).stream();
+        if (a[0] == Py_True) {
+            const Tensor workspace = at::empty({static_cast<int64_t>(abi.adaln_workspace_floats(&t))},
+                                               at::TensorOptions().dtype(at::kFloat).device(x->device()));
+            t.workspace = workspace.data_ptr<float>();
+            rc = abi.adaln_bwd(&t, a[1] == Py_True, stream);
+        } else {
+            rc = abi.adaln_fwd(&t, a[1] == Py_True, stream);
+        }
+    }
+    return PyLong_FromLong(rc);
+    END_HANDLE_TH_ERRORS
+}
+
+// gelu(u, tu, dy, dty, y, ty, reverse) -> status; the tensors may be None but for u
+PyObject* gelu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 7 || !abi.gelu) return none();
+    const Tensor* t[6] = {};
+    for (int i = 0; i < 6; ++i)
+        if (a[i] != Py_None && (!(t[i] = plain(a[i])) || !t[0] || t[i]->device() != t[0]->device())) return none();
+    const long reverse = PyLong_AsLong(a[6]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!t[0]) return none();
+    int rc;
+    {
+        pybind11::gil_scoped_release no_gil;
+        const c10::DeviceGuard guard(t[0]->device());
+        rc = abi.gelu(ptr(t[0]), ptr(t[1]), ptr(t[2]), ptr(t[3]), ptr(t[4]), ptr(t[5]), t[0]->numel(), static_cast<int>(reverse),
+                      c10::hip::getCurrentHIPStream(t[0]->device().index()).stream());
+    }
+    return PyLong_FromLong(rc);
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses of the entry points, in the order of Abi)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 6) {
-        PyErr_SetString(PyExc_TypeError, "bind() takes six addresses");
+    constexpr int kEntries = 10;
+    if (n != kEntries) {
+        PyErr_SetString(PyExc_TypeError, "bind() takes ten addresses");
         return nullptr;
     }
-    void* p[6];
-    for (int i = 0; i < 6; ++i) {
+    void* p[kEntries];
+    for (int i = 0; i < kEntries; ++i) {
         p[i] = PyLong_AsVoidPtr(a[i]);
         if (!p[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind(): null address");
             return nullptr;
         }
     }
-    abi = {reinterpret_cast<decltype(abi.fwd)>(p[0]), reinterpret_cast<decltype(abi.fwd_rotary)>(p[1]),
-           reinterpret_cast<decltype(abi.bwd_parts)>(p[2]), reinterpret_cast<decltype(abi.bwd_rotary)>(p[3]),
-           reinterpret_cast<decltype(abi.workspace_bytes)>(p[4]), reinterpret_cast<decltype(abi.cast)>(p[5])};
+    for (int i = 0; i < kAdaFields; ++i)
+        if (!ada_names[i] && !(ada_names[i] = PyUnicode_InternFromString(ada_fields[i].name))) return nullptr;
+    abi = {reinterpret_cast<decltype(abi.fwd)>(p[0]),
+           reinterpret_cast<decltype(abi.fwd_rotary)>(p[1]),
+           reinterpret_cast<decltype(abi.bwd_parts)>(p[2]),
+           reinterpret_cast<decltype(abi.bwd_rotary)>(p[3]),
+           reinterpret_cast<decltype(abi.workspace_bytes)>(p[4]),
+           reinterpret_cast<decltype(abi.cast)>(p[5]),
+           reinterpret_cast<decltype(abi.adaln_fwd)>(p[6]),
+           reinterpret_cast<decltype(abi.adaln_bwd)>(p[7]),
+           reinterpret_cast<decltype(abi.adaln_workspace_floats)>(p[8]),
+           reinterpret_cast<decltype(abi.gelu)>(p[9])};
     return none();
 }
 
@@ -396,6 +488,8 @@ PyMethodDef methods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
     {"backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(backward)), METH_FASTCALL, nullptr},
     {"cast", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cast)), METH_FASTCALL, nullptr},
+    {"adaln", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(adaln)), METH_FASTCALL, nullptr},
+    {"gelu", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gelu)), METH_FASTCALL, nullptr},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
