@@ -15,8 +15,8 @@
 // sample and every lane keeps the column sums of its columns in registers over its rows; six of them are
 // enough for the gradients of gate, scale, shift, their tangents, w and b.  They leave as one partial row per
 // workgroup, which two small launches reduce in a fixed order (no atomics: results repeat bit by bit).
-// Measured at W = 768, S = 128, gated residual + norm: forward with tangents (B = 16, 25 MB) 15.8 us, reverse (38 MB)
-// 37.9; reverse without tangents (B = 48, 57 MB) 36.6 us = 1.5 TB/s.  The reverse is short of waves (one or two
+// Measured at W = 768, S = 128, gated residual + norm: forward with tangents (B = 16, 25 MB) 15.9 us, reverse (38 MB)
+// 27.3; reverse without tangents (B = 48, 57 MB) 25.1 us = 2.3 TB/s.  The reverse is short of waves (one or two
 // workgroups per compute unit) and waits for its chain of row reductions.  gelu_kernel averages 12.8 us forward and
 // 21.2 us in reverse over the step's two shares.  In the place of PyTorch's kernels: LM1B training step 98 -> 67 ms.
 #include <type_traits>
@@ -37,10 +37,20 @@ struct AdaParams {
     float* col_partial;          // [B][2][W]: each sample's share of dw, db
 };
 
+// Sum over the wave, in every lane: DPP moves within rows of 16 lanes, then one read of each row.  Six exchanges through
+// LDS, each waiting for the one before, took longer: W = 768, S = 128, B = 16, reverse of the norm 13.1 -> 8.9 us, of
+// gated residual + norm 15.9 -> 14.2, with tangents 28.8 -> 27.3; forward (B = 48) 16.0 -> 13.7.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
+    auto dpp = [&](auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xF,
+                                                                     0xF, true));
+    };
+    v += dpp(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+    v += dpp(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    v += dpp(std::integral_constant<int, 0x141>{});  // row_half_mirror
+    v += dpp(std::integral_constant<int, 0x140>{});  // row_mirror
+    auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
 }
 
 // One lane's columns of a row: piece i holds columns 4 (lane + 64 i) ...
