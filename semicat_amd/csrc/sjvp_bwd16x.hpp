@@ -66,7 +66,8 @@ struct Row16Smem {
 // second launch can also ride at the end of the column-owned launch, see bwd_col16_repair_kernel)
 // SPLIT > 1 (launches of few workgroups): the SPLIT waves of a group share 16 queries and take every SPLIT-th stage each, SPLIT
 // stages to a barrier (ring of 2 SPLIT); their sums meet in LDS at the end, in a fixed order.
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO, int NC = 1, int SPLIT = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int PASS, int IO, int NC = 1, int SPLIT = 1,
+          int DT = HD / 16>
 __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     constexpr bool SECOND = PASS == 2;   // second launch: sums from the workspace, flagged workgroups only
@@ -76,7 +77,6 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
     constexpr int KC = HD / 32;
-    constexpr int DT = HD / 16;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -445,12 +445,12 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
         if (!wave_active) return;
         if (part == 0) {
             split_sum<DT, kXWaves16, SPLIT>(dq[0], red, 0, group, lane);
-            store_rows16<T, HD, IO>(tile, p.dq.head(b, h), p.dq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
+            store_rows16<T, HD, IO, false, DT>(tile, p.dq.head(b, h), p.dq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
         }
         if constexpr (HAS_G) {
             if (part == 1) {
                 split_sum<DT, kXWaves16, SPLIT>(dq[0], red, 1, group, lane);
-                store_rows16<T, HD, IO>(tile, p.dtq.head(b, h), p.dtq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
+                store_rows16<T, HD, IO, false, DT>(tile, p.dtq.head(b, h), p.dtq.sl, wrow, p.Lq, p.D, dq[0], p.scale, lane);
             }
         }
         return;
@@ -461,16 +461,16 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
 #pragma unroll
     for (int u = 0; u < NC; ++u) {
         const int row0 = wrow + 16 * u;
-        store_rows16<T, HD, IO>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq[u], p.scale, lane);
+        store_rows16<T, HD, IO, false, DT>(stage_tile, p.dq.head(b, h), p.dq.sl, row0, p.Lq, p.D, dq[u], p.scale, lane);
         if constexpr (HAS_G)
-            store_rows16<T, HD, IO>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq[u], p.scale, lane);
+            store_rows16<T, HD, IO, false, DT>(stage_tile, p.dtq.head(b, h), p.dtq.sl, row0, p.Lq, p.D, dtq[u], p.scale, lane);
     }
 }
 
 template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int PASS = 0, int IO = kIoDma, int NC = 1,
-          int SPLIT = 1>
+          int SPLIT = 1, int DT = HD / 16>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_row16_kernel(const BwdParams p) {
-    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO, NC, SPLIT>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_row16_body<T, HD, R, HAS_DO, HAS_G, PASS, IO, NC, SPLIT, DT>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -490,7 +490,8 @@ struct Col16Smem {
 };
 
 // (SPLIT: as in the row-owned kernel)
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int NC = 1, int SPLIT = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int NC = 1, int SPLIT = 1,
+          int DT = HD / 16>
 __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -499,7 +500,6 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     constexpr int SE = Slab<HD>::elems;
     constexpr int oTQ = SE, oG = 2 * SE, oDO = (HAS_G ? 3 : 1) * SE, oST = SM::nt * SE;
     constexpr int KC = HD / 32;
-    constexpr int DT = HD / 16;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -806,7 +806,7 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             if (k % SPLIT != part) continue;  // wave-uniform
             const OutView out = k == 0 ? p.dk : k == 1 ? p.dv : k == 2 ? p.dtk : p.dtv;
             split_sum<DT, kXWaves16, SPLIT>(dk[0], red, k, group, lane);
-            store_rows16<T, HD, IO>(tile, out.head(b, h), out.sl, wrow, p.Lk, p.D, dk[0], k % 2 == 0 ? p.scale : 1.0f, lane);
+            store_rows16<T, HD, IO, false, DT>(tile, out.head(b, h), out.sl, wrow, p.Lk, p.D, dk[0], k % 2 == 0 ? p.scale : 1.0f, lane);
         }
         return;
     }
@@ -823,18 +823,19 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
 #pragma unroll
     for (int u = 0; u < NC; ++u) {
         const int row0 = wrow + 16 * u;
-        store_rows16<T, HD, IO>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk[u], p.scale, lane);
+        store_rows16<T, HD, IO, false, DT>(stage_tile, p.dk.head(b, h), p.dk.sl, row0, p.Lk, p.D, dk[u], p.scale, lane);
         if constexpr (HAS_G)
-            store_rows16<T, HD, IO>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk[u], p.scale, lane);
-        store_rows16<T, HD, IO>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv[u], 1.0f, lane);
+            store_rows16<T, HD, IO, false, DT>(stage_tile, p.dtk.head(b, h), p.dtk.sl, row0, p.Lk, p.D, dtk[u], p.scale, lane);
+        store_rows16<T, HD, IO, false, DT>(stage_tile, p.dv.head(b, h), p.dv.sl, row0, p.Lk, p.D, dv[u], 1.0f, lane);
         if constexpr (HAS_G)
-            store_rows16<T, HD, IO>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv[u], 1.0f, lane);
+            store_rows16<T, HD, IO, false, DT>(stage_tile, p.dtv.head(b, h), p.dtv.sl, row0, p.Lk, p.D, dtv[u], 1.0f, lane);
     }
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1, int SPLIT = 1>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1, int SPLIT = 1,
+          int DT = HD / 16>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdParams p) {
-    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT, DT>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The column-owned launch with the second launch of the row-owned kernel at its end: workgroups
@@ -843,13 +844,13 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_kernel(const BwdPa
 // left).  Nearly all of those workgroups leave at once; dealt out behind the column pass they fill the time in
 // which its last workgroups run alone, where a launch of their own costs a few microseconds.
 template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int OCC, int IO = kIoDma, int NC = 1, int SPLIT = 1,
-          int RROW = R>
+          int RROW = R, int DT = HD / 16>
 __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks)
-        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16_body<T, HD, R, HAS_DO, HAS_G, IO, NC, SPLIT, DT>(p, (int)blockIdx.x, col_blocks);
     else
-        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
+        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO, 1, 1, DT>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
 }
 
 // ---------------------------------------------------------------------------------------------

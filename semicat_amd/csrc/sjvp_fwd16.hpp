@@ -43,8 +43,12 @@ struct Fwd16Smem {
 // 202 registers and no gain: 96.6 us against 97.6 at B=8 H=16 L=1024 D=64, 105 against 101 at B=128 H=12 L=256).
 // SPLIT > 1 (launches of few workgroups): the SPLIT waves of a group share 16 queries and take every SPLIT-th stage each, SPLIT
 // stages to a barrier; their partial sums are brought to one maximum and added in LDS, in a fixed order.
+// DT: 16-wide tiles of the head dimension that hold columns below D.  D <= 48 in the class of 64 needs three of four: a quarter
+// of the output products and of their transposing reads, which the LDS serves at half rate, are left out (here and in the
+// backward pair).  Forward + backward, 4 / 3 tiles: B=4 H=6 333 x 205 D=48 cotangent on TO 35.0 / 32.6 us, B=8 H=8 L=300 D=36
+// 60.2 / 57.7, B=8 H=16 L=1024 D=48 475 / 456, B=64 H=12 L=256 D=48 233 / 229.
 template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1,
-          int SPLIT = 1>
+          int SPLIT = 1, int DT = HD / 16>
 __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdParams p) {
     constexpr int NT = kThreads16 / NC;  // threads of the workgroup
     static_assert(!ROPE || (HD == 64 && SPB == 1), "the folded rotation covers HD = 64, one stage per barrier");
@@ -58,7 +62,6 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw) + SM::ring_off;
     constexpr int SE = Slab<HD>::elems;
     constexpr int KC = HD / 32;  // k-chunks of the score contraction
-    constexpr int DT = HD / 16;  // 16-wide tiles of the head dimension
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -391,12 +394,12 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
         if (!wave_active) return;
         if (part == 0) {
             split_sum<DT, kWaves16, SPLIT>(acc[0], red, 0, group, lane);
-            store_rows16<T, HD, IO>(tile, p.o.head(b, h), p.o.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
+            store_rows16<T, HD, IO, false, DT>(tile, p.o.head(b, h), p.o.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
         }
         if constexpr (JVP) {
             if (part == 1) {
                 split_sum<DT, kWaves16, SPLIT>(acc[0], red, 1, group, lane);
-                store_rows16<T, HD, IO>(tile, p.to.head(b, h), p.to.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
+                store_rows16<T, HD, IO, false, DT>(tile, p.to.head(b, h), p.to.sl, wrow, p.Lq, p.D, acc[0], inv_l, lane);
             }
         }
         return;
@@ -437,9 +440,9 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
 #pragma unroll
             for (int d = 0; d < DT; ++d) tacc[u][d] -= cmu * acc[u][d];
         }
-        store_rows16<T, HD, IO>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc[u], inv_l, lane);
+        store_rows16<T, HD, IO, false, DT>(stage_tile, p.o.head(b, h), p.o.sl, row0, p.Lq, p.D, acc[u], inv_l, lane);
         if constexpr (JVP)
-            store_rows16<T, HD, IO>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc[u], inv_l, lane);
+            store_rows16<T, HD, IO, false, DT>(stage_tile, p.to.head(b, h), p.to.sl, row0, p.Lq, p.D, tacc[u], inv_l, lane);
     }
 }
 

@@ -6,7 +6,7 @@
 
 namespace sjvp {
 
-template <typename T, int HD, int IO>
+template <typename T, int HD, int IO, int DT = HD / 16>
 int fwd16_staged_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
     // the smallest rings whose LDS also holds the store staging tiles
     constexpr int RJ = 2, RP = 4;
@@ -18,7 +18,7 @@ int fwd16_staged_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) 
         auto go = [&](auto jvp_tag, auto split_tag) {
             constexpr bool JVP = decltype(jvp_tag)::value;
             constexpr int SPLIT = decltype(split_tag)::value;
-            return launch(fwd16_kernel<T, HD, 2 * SPLIT, JVP, 2, SPLIT, false, IO, 1, SPLIT>, grid * SPLIT,
+            return launch(fwd16_kernel<T, HD, 2 * SPLIT, JVP, 2, SPLIT, false, IO, 1, SPLIT, DT>, grid * SPLIT,
                           Fwd16Smem<HD, 2 * SPLIT, JVP, SPLIT, false, SPLIT>::bytes, stream, ps, kThreads16);
         };
         constexpr std::integral_constant<int, 2> two{};
@@ -27,15 +27,18 @@ int fwd16_staged_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) 
         if (split == 4) return jvp ? go(std::true_type{}, four) : go(std::false_type{}, four);
     }
     if (jvp)
-        return launch(fwd16_kernel<T, HD, RJ, true, OCC, 1, false, IO>, grid, Fwd16Smem<HD, RJ, true, 1, false>::bytes,
-                      stream, p, kThreads16);
-    return launch(fwd16_kernel<T, HD, RP, false, OCC, 1, false, IO>, grid, Fwd16Smem<HD, RP, false, 1, false>::bytes,
-                  stream, p, kThreads16);
+        return launch(fwd16_kernel<T, HD, RJ, true, OCC, 1, false, IO, 1, 1, DT>, grid,
+                      Fwd16Smem<HD, RJ, true, 1, false>::bytes, stream, p, kThreads16);
+    return launch(fwd16_kernel<T, HD, RP, false, OCC, 1, false, IO, 1, 1, DT>, grid,
+                  Fwd16Smem<HD, RP, false, 1, false>::bytes, stream, p, kThreads16);
 }
 
 template <typename T, int IO>
 int fwd16_staged(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
     if (p.D <= 32) return fwd16_staged_hd<T, 32, IO>(p, grid, jvp, stream);
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 48) return fwd16_staged_hd<T, 64, IO, 3>(p, grid, jvp, stream);
+    }
     if (p.D <= 64) return fwd16_staged_hd<T, 64, IO>(p, grid, jvp, stream);
     return fwd16_staged_hd<T, 128, IO>(p, grid, jvp, stream);
 }

@@ -6,7 +6,7 @@
 
 namespace sjvp {
 
-template <typename T, int HD, bool HAS_DO, bool HAS_G, int IO>
+template <typename T, int HD, bool HAS_DO, bool HAS_G, int IO, int DT>
 int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
     // the row-owned kernel first (besides dQ, dQ_dot it leaves the row sums in the workspace), then
     // the column-owned one; workgroups of four waves own 64 positions
@@ -32,11 +32,11 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
             constexpr int MOST = IO == kIoDma ? 4 : 2;  // (four parts' staged copies do not fit the registers)
             if (p.rowfix != 2) split = split_rows(grid, (p.Lk + kStageRows - 1) / kStageRows, MOST, true);
             if (split == 2)
-                rc = launch(bwd_row16_kernel<T, HD, 4, HAS_DO, HAS_G, 2, 0, IO, 1, 2>, grid * 2,
+                rc = launch(bwd_row16_kernel<T, HD, 4, HAS_DO, HAS_G, 2, 0, IO, 1, 2, DT>, grid * 2,
                             Row16Smem<HD, 4, HAS_G, 2>::bytes, stream, p, kXThreads16);
             if constexpr (MOST == 4) {
                 if (split == 4)
-                    rc = launch(bwd_row16_kernel<T, HD, 8, HAS_DO, HAS_G, 2, 0, IO, 1, 4>, grid * 4,
+                    rc = launch(bwd_row16_kernel<T, HD, 8, HAS_DO, HAS_G, 2, 0, IO, 1, 4, DT>, grid * 4,
                                 Row16Smem<HD, 8, HAS_G, 4>::bytes, stream, p, kXThreads16);
             }
         }
@@ -44,10 +44,10 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
             // done above
         } else if (wide) {
             if constexpr (!HAS_G && IO == kIoDma)
-                rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, HD == 128 ? 2 : 3, 0, IO, 2>, grid / 2, smem, stream, p,
-                            kXThreads16);
-        } else if (p.rowfix == 2) rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 1, IO>, grid, smem, stream, p, kXThreads16);
-        else rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 0, IO>, grid, smem, stream, p, kXThreads16);
+                rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, HD == 128 ? 2 : 3, 0, IO, 2, 1, DT>, grid / 2, smem, stream,
+                            p, kXThreads16);
+        } else if (p.rowfix == 2) rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 1, IO, 1, 1, DT>, grid, smem, stream, p, kXThreads16);
+        else rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 0, IO, 1, 1, DT>, grid, smem, stream, p, kXThreads16);
         // The second launch does not depend on the column-owned pass.  Where nearly all of its workgroups leave
         // at once (repair of flagged workgroups only), they ride at the end of that launch instead of paying for
         // one of their own.
@@ -55,7 +55,7 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         // column-owned kernel, which would lose a resident workgroup per compute unit to it; nor on fp32 rows there)
         rides = p.rowfix == 1 && (parts & SJVP_BWD_COL) && (HD != 128 || (HAS_G && IO != kIoF32));
         if (rc == SJVP_OK && p.rowfix != 0 && !rides)
-            rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 2, IO>, grid, smem, stream, p, kXThreads16);
+            rc = launch(bwd_row16_kernel<T, HD, XR, HAS_DO, HAS_G, OCC, 2, IO, 1, 1, DT>, grid, smem, stream, p, kXThreads16);
     }
     if (rc != SJVP_OK || !(parts & SJVP_BWD_COL)) return rc;
     const int grid = BH * ((p.Lk + kXOwned16 - 1) / kXOwned16);
@@ -83,7 +83,7 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
                 BwdParams pr = p;
                 pr.col_workgroups = BH * ((p.Lk + OWNED - 1) / OWNED);
                 constexpr int row = Row16Smem<HD, XR, HAS_G>::bytes, col = Col16Smem<HD, 2 * SPLIT, HAS_DO, HAS_G, SPLIT>::bytes;
-                return launch(bwd_col16_repair_kernel<T, HD, 2 * SPLIT, HAS_DO, HAS_G, 2, IO, 1, SPLIT, XR>,
+                return launch(bwd_col16_repair_kernel<T, HD, 2 * SPLIT, HAS_DO, HAS_G, 2, IO, 1, SPLIT, XR, DT>,
                               pr.col_workgroups + BH * (p.Lr / kXOwned16), col > row ? col : row, stream, pr, kXThreads16);
             };
             if (split == 2) return go(std::integral_constant<int, 2>{});
@@ -100,7 +100,7 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
                 BwdParams pr = p;
                 pr.col_workgroups = BH * ((p.Lk + 2 * kXOwned16 - 1) / (2 * kXOwned16));
                 constexpr int smem = CS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? CS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
-                return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO, 2>,
+                return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO, 2, 1, XR, DT>,
                               pr.col_workgroups + BH * (p.Lr / kXOwned16), smem, stream, pr, kXThreads16);
             }
         }
@@ -108,23 +108,26 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
             BwdParams pr = p;
             pr.col_workgroups = grid;
             constexpr int smem = CS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? CS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
-            return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO>, grid + BH * (p.Lr / kXOwned16), smem,
-                          stream, pr, kXThreads16);
+            return launch(bwd_col16_repair_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO, 1, 1, XR, DT>,
+                          grid + BH * (p.Lr / kXOwned16), smem, stream, pr, kXThreads16);
         }
-        return launch(bwd_col16_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO>, grid, CS::bytes, stream, p, kXThreads16);
+        return launch(bwd_col16_kernel<T, HD, XR, HAS_DO, HAS_G, 2, IO, 1, 1, DT>, grid, CS::bytes, stream, p, kXThreads16);
     }
 }
 
-template <typename T, int HD, int IO>
+template <typename T, int HD, int IO, int DT = HD / 16>
 int pair_hd(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
-    if (has_do && has_g) return pair_mode<T, HD, true, true, IO>(p, BH, parts, stream);
-    if (has_g) return pair_mode<T, HD, false, true, IO>(p, BH, parts, stream);
-    return pair_mode<T, HD, true, false, IO>(p, BH, parts, stream);
+    if (has_do && has_g) return pair_mode<T, HD, true, true, IO, DT>(p, BH, parts, stream);
+    if (has_g) return pair_mode<T, HD, false, true, IO, DT>(p, BH, parts, stream);
+    return pair_mode<T, HD, true, false, IO, DT>(p, BH, parts, stream);
 }
 
 template <typename T, int IO>
 int bwd_pair16(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
     if (p.D <= 32) return pair_hd<T, 32, IO>(p, BH, has_do, has_g, parts, stream);
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 48) return pair_hd<T, 64, IO, 3>(p, BH, has_do, has_g, parts, stream);
+    }
     if (p.D <= 64) return pair_hd<T, 64, IO>(p, BH, has_do, has_g, parts, stream);
     return pair_hd<T, 128, IO>(p, BH, has_do, has_g, parts, stream);
 }

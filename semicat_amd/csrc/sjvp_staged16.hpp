@@ -225,7 +225,7 @@ __device__ __forceinline__ void issue_plan(StagedPlan<T, HD, NS, NT, IO, P>& pla
 
 // store_tile16 (sjvp_w16.hpp) for rows of any alignment: 16-bit rows leave through the wave's staging tile as there,
 // fp32 rows unrounded straight from the accumulators (four lanes hold 64 consecutive bytes of a row).
-template <typename T, int HD, int IO>
+template <typename T, int HD, int IO, int DT = HD / 16>
 __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, int64_t sl, int row0, int L, int D,
                                                     const f32x4* acc, float mul, int lane) {
     const int n = lane & 15, g = lane >> 4;
@@ -233,12 +233,12 @@ __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, i
         if (row0 + n >= L) return;
         elem_t* row = gp + (int64_t)(row0 + n) * sl;
 #pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt) store_f32x4(row, acc[dt] * mul, 16 * dt + 4 * g, D);
+        for (int dt = 0; dt < DT; ++dt) store_f32x4(row, acc[dt] * mul, 16 * dt + 4 * g, D);
     } else {
         constexpr int P = StoreStage16<HD>::pitch;
         wave_exchange();  // the tile's last readers are done
 #pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt) {
+        for (int dt = 0; dt < DT; ++dt) {
             u32x2 val = {T::pack2(acc[dt][0] * mul, acc[dt][1] * mul), T::pack2(acc[dt][2] * mul, acc[dt][3] * mul)};
             *reinterpret_cast<u32x2*>(stage + n * P + 16 * dt + 4 * g) = val;
         }
@@ -258,11 +258,11 @@ __device__ __forceinline__ void staged_store_tile16(elem_t* stage, elem_t* gp, i
 }
 
 // The wave's 16 rows of an output tensor, whatever its storage.
-template <typename T, int HD, int IO, bool ROPE = false>
+template <typename T, int HD, int IO, bool ROPE = false, int DT = HD / 16>
 __device__ __forceinline__ void store_rows16(elem_t* stage, elem_t* gp, int64_t sl, int row0, int L, int D,
                                              const f32x4* acc, float mul, int lane, const RopeTables* rt = nullptr) {
-    if constexpr (IO == kIoDma) store_tile16<T, HD, ROPE>(stage, gp, sl, row0, L, D, acc, mul, lane, rt);
-    else staged_store_tile16<T, HD, IO>(stage, gp, sl, row0, L, D, acc, mul, lane);
+    if constexpr (IO == kIoDma) store_tile16<T, HD, ROPE, DT>(stage, gp, sl, row0, L, D, acc, mul, lane, rt);
+    else staged_store_tile16<T, HD, IO, DT>(stage, gp, sl, row0, L, D, acc, mul, lane);
 }
 
 }  // namespace sjvp

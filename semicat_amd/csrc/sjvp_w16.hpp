@@ -277,11 +277,11 @@ struct StoreStage16 {
     static constexpr int elems = 16 * pitch;
 };
 
-// Store OUT[row0 + r][0..D) for r < 16 from transposed accumulator tiles acc[HD/16] (lane = row,
+// Store OUT[row0 + r][0..D) for r < 16 from transposed accumulator tiles acc[DT] (lane = row,
 // registers = 4 consecutive columns 16*dt + 4g ..) scaled by mul: 8-byte writes into the wave's
 // staging tile, 16-byte reads back row-major, 16-byte global stores (a 128-byte row per 8 lanes).
-// Issues exactly max(1, HD / 32) global store instructions.
-template <typename T, int HD, bool ROPE = false>
+// Issues exactly max(1, HD / 32) global store instructions.  (DT < HD / 16 where D ends in an earlier tile.)
+template <typename T, int HD, bool ROPE = false, int DT = HD / 16>
 __device__ __forceinline__ void store_tile16(elem_t* stage, elem_t* gp, int64_t sl, int row0, int L, int D,
                                              const f32x4* acc, float mul, int lane,
                                              const RopeTables* rt = nullptr) {
@@ -289,7 +289,7 @@ __device__ __forceinline__ void store_tile16(elem_t* stage, elem_t* gp, int64_t 
     const int n = lane & 15, g = lane >> 4;
     wave_exchange();  // the tile's last readers are done
 #pragma unroll
-    for (int dt = 0; dt < HD / 16; ++dt) {
+    for (int dt = 0; dt < DT; ++dt) {
         u32x2 val = {T::pack2(acc[dt][0] * mul, acc[dt][1] * mul), T::pack2(acc[dt][2] * mul, acc[dt][3] * mul)};
         *reinterpret_cast<u32x2*>(stage + n * P + 16 * dt + 4 * g) = val;
     }
