@@ -76,7 +76,7 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     using SM = Row16Smem<HD, R, HAS_G, SPLIT>;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
-    constexpr int KC = HD / 32;
+    constexpr int KL = HD / 32, KC = (DT + 1) / 2;  // 32-column chunks of a row, and those with columns below D
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -102,8 +102,8 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     }
 
     // The own rows are requested first, as B operands; the set-up of the stage copies runs while they travel.
-    u32x4 qB[NC][KC], tqB[NC][KC], gB[NC][KC], doB[NC][KC];
-    u32x4 oR[NC][KC], toR[NC][KC];
+    u32x4 qB[NC][KL], tqB[NC][KL], gB[NC][KL], doB[NC][KL];
+    u32x4 oR[NC][KL], toR[NC][KL];
     float lse_in[NC], mu_in[NC];
     const int64_t so = (int64_t)bh * p.Lr + wrow + n;  // rows below Lr exist in every statistic
     if (DMA && p.q_side_uniform && p.D == HD && q0 + OWNED <= p.Lq) {
@@ -499,7 +499,7 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw);
     constexpr int SE = Slab<HD>::elems;
     constexpr int oTQ = SE, oG = 2 * SE, oDO = (HAS_G ? 3 : 1) * SE, oST = SM::nt * SE;
-    constexpr int KC = HD / 32;
+    constexpr int KL = HD / 32, KC = (DT + 1) / 2;  // 32-column chunks of a row, and those with columns below D
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -568,7 +568,7 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
         issue_step();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
-    u32x4 kB[NC][KC], vB[NC][KC], tkB[NC][KC], tvB[NC][KC];
+    u32x4 kB[NC][KL], vB[NC][KL], tkB[NC][KL], tvB[NC][KL];
     if (DMA && p.k_side_uniform && p.D == HD && key0 + OWNED <= p.Lk) {
         // the common case: whole rows that all exist, every tensor with k's strides
         const int64_t slice = b * p.k.sb + h * p.k.sh;
@@ -859,7 +859,7 @@ __global__ __launch_bounds__(kXThreads16, OCC) void bwd_col16_repair_kernel(cons
 // registers beside the operands, so the pair splits the work without repeating any of it: member m
 // forms the score-side tiles (S, S_dot, W, XY -> P, P_dot, dS_dot, dS) of the stage's query tile m
 // (16 queries), the two exchange their packed tiles through LDS, and member m accumulates all four
-// gradients for head-dimension columns 64 m .. 64 m + 63 over the stage's 32 queries.  One launch,
+// gradients for head-dimension columns 64 m .. 64 m + 63 (D <= 96: 48 m .. 48 m + 47) over the stage's 32 queries.  One launch,
 // 12 tile contractions (6 + 6), the query side streamed once.
 // LDS: [ring of Q | [Q_dot | G] | [dO] | lse2, mu, s4, s7d stages][exchange: 8 waves x 4 tiles][sink];
 // the ring doubles as store staging after the last stage.
@@ -874,7 +874,7 @@ struct Col16pSmem {
     static_assert(R * slot >= kWaves16 * StoreStage16<64>::elems, "ring too small to stage stores");
 };
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO, int DT = HD / 16>
 __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int block, const int blocks) {
     constexpr bool DMA = IO == kIoDma;
     static_assert(HD == 128, "the paired form exists for the head dimension that needs it");
@@ -884,8 +884,8 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     u32x2* xch = reinterpret_cast<u32x2*>(ring + R * SM::slot);  // [wave][tile 0..3][lane]
     constexpr int SE = Slab<HD>::elems;
     constexpr int oTQ = SE, oG = 2 * SE, oDO = (HAS_G ? 3 : 1) * SE, oST = SM::nt * SE;
-    constexpr int KC = HD / 32;
-    constexpr int DH = HD / 32;  // 16-wide head-dimension tiles per member (half of HD / 16)
+    constexpr int KL = HD / 32, KC = (DT + 1) / 2;
+    constexpr int DH = DT / 2;  // 16-wide head-dimension tiles per member
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -939,7 +939,7 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
         issue_next();
     };
     // the own rows are requested first; the set-up of the stage copies runs while they travel
-    u32x4 kB[KC], vB[KC], tkB[KC], tvB[KC];
+    u32x4 kB[KL], vB[KL], tkB[KL], tvB[KL];
     if (DMA && p.k_side_uniform && p.D == HD && key0 + kXOwned16 <= p.Lk) {
         // the common case: whole rows that all exist, every tensor with k's strides
         const int64_t slice = b * p.k.sb + h * p.k.sh;
@@ -1059,7 +1059,7 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
         }
 #pragma unroll
         for (int d = 0; d < DH; ++d) {
-            const int d0 = 64 * m + 16 * d;
+            const int d0 = 16 * DH * m + 16 * d;
             const u32x4 aq = lds_a_tr16<HD>(sQ, d0, lane);
             dk[d] = T::mfma16(aq, dsB, dk[d]);
             if constexpr (HAS_G) {
@@ -1091,33 +1091,33 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
     if (!pair_active) return;
     elem_t* stage_tile = ring + wave * StoreStage16<64>::elems;
     const int row0 = key0 + pr * 16;
-    const int dcol = 64 * m;
+    const int dcol = 16 * DH * m;
     const int doff = IO == kIoF32 ? 2 * dcol : dcol;  // in the units of the views
-    const int Dm = p.D - dcol;  // columns of this member's half that exist (may be <= 0)
-    store_rows16<T, 64, IO>(stage_tile, p.dk.head(b, h) + doff, p.dk.sl, row0, p.Lk, Dm, dk, p.scale, lane);
+    const int Dm = min(p.D - dcol, 16 * DH);  // columns of this member's half that exist (may be <= 0)
+    store_rows16<T, 64, IO, false, DH>(stage_tile, p.dk.head(b, h) + doff, p.dk.sl, row0, p.Lk, Dm, dk, p.scale, lane);
     if constexpr (HAS_G)
-        store_rows16<T, 64, IO>(stage_tile, p.dtk.head(b, h) + doff, p.dtk.sl, row0, p.Lk, Dm, dtk, p.scale, lane);
-    store_rows16<T, 64, IO>(stage_tile, p.dv.head(b, h) + doff, p.dv.sl, row0, p.Lk, Dm, dv, 1.0f, lane);
+        store_rows16<T, 64, IO, false, DH>(stage_tile, p.dtk.head(b, h) + doff, p.dtk.sl, row0, p.Lk, Dm, dtk, p.scale, lane);
+    store_rows16<T, 64, IO, false, DH>(stage_tile, p.dv.head(b, h) + doff, p.dv.sl, row0, p.Lk, Dm, dv, 1.0f, lane);
     if constexpr (HAS_G)
-        store_rows16<T, 64, IO>(stage_tile, p.dtv.head(b, h) + doff, p.dtv.sl, row0, p.Lk, Dm, dtv, 1.0f, lane);
+        store_rows16<T, 64, IO, false, DH>(stage_tile, p.dtv.head(b, h) + doff, p.dtv.sl, row0, p.Lk, Dm, dtv, 1.0f, lane);
 }
 
-template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO = kIoDma>
+template <typename T, int HD, int R, bool HAS_DO, bool HAS_G, int IO = kIoDma, int DT = HD / 16>
 __global__ __launch_bounds__(kThreads16, 2) void bwd_col16p_kernel(const BwdParams p) {
-    bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, (int)gridDim.x);
+    bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO, DT>(p, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The paired column-owned launch with the second pass of the row-owned kernel at its end (see
 // bwd_col16_repair_kernel).  The row-owned kernel's workgroups have four waves, these eight: in a workgroup that
 // takes a row item the upper four leave at once, and the barriers of the others count the waves that are left.
-template <typename T, int HD, int R, int RROW, bool HAS_DO, bool HAS_G, int IO = kIoDma>
+template <typename T, int HD, int R, int RROW, bool HAS_DO, bool HAS_G, int IO = kIoDma, int DT = HD / 16>
 __global__ __launch_bounds__(kThreads16, 2) void bwd_col16p_repair_kernel(const BwdParams p) {
     const int col_blocks = p.col_workgroups;
     if ((int)blockIdx.x < col_blocks) {
-        bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO>(p, (int)blockIdx.x, col_blocks);
+        bwd_col16p_body<T, HD, R, HAS_DO, HAS_G, IO, DT>(p, (int)blockIdx.x, col_blocks);
     } else {
         if ((int)threadIdx.x >= kXThreads16) return;
-        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
+        bwd_row16_body<T, HD, RROW, HAS_DO, HAS_G, 2, IO, 1, 1, DT>(p, (int)blockIdx.x - col_blocks, (int)gridDim.x - col_blocks);
     }
 }
 

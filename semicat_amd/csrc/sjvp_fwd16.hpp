@@ -47,6 +47,8 @@ struct Fwd16Smem {
 // of the output products and of their transposing reads, which the LDS serves at half rate, are left out (here and in the
 // backward pair).  Forward + backward, 4 / 3 tiles: B=4 H=6 333 x 205 D=48 cotangent on TO 35.0 / 32.6 us, B=8 H=8 L=300 D=36
 // 60.2 / 57.7, B=8 H=16 L=1024 D=48 475 / 456, B=64 H=12 L=256 D=48 233 / 229.
+// D <= 96 in the class of 128 needs six of eight, and three of the score products' four chunks: 8 / 6 tiles at B=8 H=16 L=1024
+// D=80 1012 / 886 us, B=64 H=12 L=128 D=96 181 / 172, L=256 D=80 495 / 448, B=8 H=12 L=512 D=75 (staged) 320 / 292.
 template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1,
           int SPLIT = 1, int DT = HD / 16>
 __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdParams p) {
@@ -61,7 +63,8 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     elem_t* own = reinterpret_cast<elem_t*>(smem_raw) + SM::own_off;
     elem_t* ring = reinterpret_cast<elem_t*>(smem_raw) + SM::ring_off;
     constexpr int SE = Slab<HD>::elems;
-    constexpr int KC = HD / 32;  // k-chunks of the score contraction
+    constexpr int KL = HD / 32;        // 32-column chunks of a row
+    constexpr int KC = (DT + 1) / 2;  // those with columns below D: k-chunks of the score contraction
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -79,7 +82,7 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     const int wrow = q0 + group * 16 * NC;  // the wave's first query; the lane's are wrow + 16 u + n
     const bool wave_active = wrow < p.Lq;
 
-    u32x4 qB[NC][KC], tqB[NC][KC];
+    u32x4 qB[NC][KL], tqB[NC][KL];
     using StagePlan = std::conditional_t<DMA, CopyPlan<HD, SM::nt, 1, NT>, StagedPlan<T, HD, SM::nt, NT, IO>>;
     constexpr int SPT = StagePlan::N;
     StagePlan plan[DMA ? 1 : SPLIT];

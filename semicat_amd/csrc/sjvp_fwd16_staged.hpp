@@ -40,6 +40,9 @@ int fwd16_staged(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
         if (p.D <= 48) return fwd16_staged_hd<T, 64, IO, 3>(p, grid, jvp, stream);
     }
     if (p.D <= 64) return fwd16_staged_hd<T, 64, IO>(p, grid, jvp, stream);
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 96) return fwd16_staged_hd<T, 128, IO, 6>(p, grid, jvp, stream);
+    }
     return fwd16_staged_hd<T, 128, IO>(p, grid, jvp, stream);
 }
 

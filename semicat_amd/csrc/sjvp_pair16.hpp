@@ -69,10 +69,10 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
             BwdParams pr = p;
             pr.col_workgroups = grid;
             constexpr int smem = PS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? PS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;
-            return launch(bwd_col16p_repair_kernel<T, HD, PR, XR, HAS_DO, HAS_G, IO>, grid + BH * (p.Lr / kXOwned16), smem,
+            return launch(bwd_col16p_repair_kernel<T, HD, PR, XR, HAS_DO, HAS_G, IO, DT>, grid + BH * (p.Lr / kXOwned16), smem,
                           stream, pr, kThreads16);
         }
-        return launch(bwd_col16p_kernel<T, HD, PR, HAS_DO, HAS_G, IO>, grid, PS::bytes, stream, p, kThreads16);
+        return launch(bwd_col16p_kernel<T, HD, PR, HAS_DO, HAS_G, IO, DT>, grid, PS::bytes, stream, p, kThreads16);
     } else {
         if constexpr (HD <= 64 && IO != kIoF32) {
             constexpr int MOST = IO == kIoDma ? 4 : 2;
@@ -129,6 +129,9 @@ int bwd_pair16(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, h
         if (p.D <= 48) return pair_hd<T, 64, IO, 3>(p, BH, has_do, has_g, parts, stream);
     }
     if (p.D <= 64) return pair_hd<T, 64, IO>(p, BH, has_do, has_g, parts, stream);
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 96) return pair_hd<T, 128, IO, 6>(p, BH, has_do, has_g, parts, stream);
+    }
     return pair_hd<T, 128, IO>(p, BH, has_do, has_g, parts, stream);
 }
 

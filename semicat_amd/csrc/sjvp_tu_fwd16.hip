@@ -64,6 +64,7 @@ int fwd_vec<SJVP_T>(const FwdParams& p, int grid, bool jvp, hipStream_t stream) 
     if (p.D <= 32) return fwd16_hd<SJVP_T, 32>(p, grid, jvp, stream);
     if (p.D <= 48) return fwd16_hd<SJVP_T, 64, 3>(p, grid, jvp, stream);
     if (p.D <= 64) return fwd16_hd<SJVP_T, 64>(p, grid, jvp, stream);
+    if (p.D <= 96) return fwd16_hd<SJVP_T, 128, 6>(p, grid, jvp, stream);
     return fwd16_hd<SJVP_T, 128>(p, grid, jvp, stream);
 }
 
