@@ -35,6 +35,9 @@ int fwd16_staged_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) 
 
 template <typename T, int IO>
 int fwd16_staged(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 16) return fwd16_staged_hd<T, 32, IO, 1>(p, grid, jvp, stream);
+    }
     if (p.D <= 32) return fwd16_staged_hd<T, 32, IO>(p, grid, jvp, stream);
     if constexpr (IO != kIoF32) {
         if (p.D <= 48) return fwd16_staged_hd<T, 64, IO, 3>(p, grid, jvp, stream);

@@ -124,6 +124,9 @@ int pair_hd(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipS
 
 template <typename T, int IO>
 int bwd_pair16(const BwdParams& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream) {
+    if constexpr (IO != kIoF32) {
+        if (p.D <= 16) return pair_hd<T, 32, IO, 1>(p, BH, has_do, has_g, parts, stream);
+    }
     if (p.D <= 32) return pair_hd<T, 32, IO>(p, BH, has_do, has_g, parts, stream);
     if constexpr (IO != kIoF32) {
         if (p.D <= 48) return pair_hd<T, 64, IO, 3>(p, BH, has_do, has_g, parts, stream);

@@ -61,6 +61,7 @@ int fwd16_hd(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
 
 template <>
 int fwd_vec<SJVP_T>(const FwdParams& p, int grid, bool jvp, hipStream_t stream) {
+    if (p.D <= 16) return fwd16_hd<SJVP_T, 32, 1>(p, grid, jvp, stream);
     if (p.D <= 32) return fwd16_hd<SJVP_T, 32>(p, grid, jvp, stream);
     if (p.D <= 48) return fwd16_hd<SJVP_T, 64, 3>(p, grid, jvp, stream);
     if (p.D <= 64) return fwd16_hd<SJVP_T, 64>(p, grid, jvp, stream);

@@ -11,11 +11,11 @@ GRADS = ("dq", "dk", "dv", "dtq", "dtk", "dtv")
 
 
 @pytest.mark.parametrize("B,H,Lq,Lk", [(1, 2, 90, 70), (1, 3, 300, 170), (8, 12, 77, 333), (1, 150, 200, 260), (2, 300, 130, 257)])
-@pytest.mark.parametrize("D", [33, 40, 47, 48, 49, 56, 65, 72, 80, 95, 96, 97, 104])
+@pytest.mark.parametrize("D", [16, 17, 24, 33, 40, 47, 48, 49, 56, 65, 72, 80, 95, 96, 97, 104])
 @pytest.mark.parametrize("mode", ["both", "dO", "dTO", "primal"])
 def test_head_dimensions_at_the_edges_of_tiles(B, H, Lq, Lk, D, mode):
     from semicat_amd import kernels as K
-    if B * H >= 150 and (D % 8 or D in (56, 72, 104)):
+    if B * H >= 150 and (D % 8 or D in (24, 56, 72, 104)):
         pytest.skip("wide waves take 16-byte aligned rows, and two sizes on a side are enough")
     print(f"[tiles] {B} {H} {Lq} {Lk} {D} {mode}", flush=True)
     dtype = torch.float16 if (D + Lq) % 2 else torch.bfloat16
