@@ -49,7 +49,7 @@ struct Fwd16Smem {
 // 60.2 / 57.7, B=8 H=16 L=1024 D=48 475 / 456, B=64 H=12 L=256 D=48 233 / 229.
 // D <= 96 in the class of 128 needs six of eight, and three of the score products' four chunks: 8 / 6 tiles at B=8 H=16 L=1024
 // D=80 1012 / 886 us, B=64 H=12 L=128 D=96 181 / 172, L=256 D=80 495 / 448, B=8 H=12 L=512 D=75 (staged) 320 / 292.
-// D = 16 in the class of 32 needs one of two: B=8 H=16 L=1024 250 / 233 us, B=64 H=12 L=256 134 / 120.
+// D = 16 in the class of 32 needs one of two: B=64 H=12 L=256 134 / 120 us, B=8 H=16 L=1024 233 where D = 32 takes 251.
 template <typename T, int HD, int R, bool JVP, int OCC, int SPB = 1, bool ROPE = false, int IO = kIoDma, int NC = 1,
           int SPLIT = 1, int DT = HD / 16>
 __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdParams p) {
