@@ -164,13 +164,18 @@ struct StagedPlan {
 };
 
 // B operands (all head-dimension chunks of 32) of one owned row, straight from global memory.
-template <typename T, int HD, int IO>
+// (GROUPED: the zeros come as one register group.  Joined with the loaded piece element by element, as the compiler may do, the
+// piece is awaited as soon as it is requested.  Row-owned kernel at D = 80, 1476 queries on 10 keys: 278 -> 245 us; the forward
+// of few workgroups, whose pieces were not affected, loses by it: 333 x 205, D = 48 8.9 -> 9.8 us.)
+template <typename T, int HD, int IO, bool GROUPED = false>
 __device__ __forceinline__ void load_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
     if constexpr (IO != kIoDma) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
 #pragma unroll
     for (int c = 0; c < HD / 32; ++c) {
-        out[c] = u32x4{0u, 0u, 0u, 0u};
-        if (valid && 32 * c + 8 * g < D) out[c] = *reinterpret_cast<const u32x4*>(row + 32 * c + 8 * g);
+        u32x4 piece = {0u, 0u, 0u, 0u};
+        if constexpr (GROUPED) asm volatile("" : "+v"(piece));
+        if (valid && 32 * c + 8 * g < D) piece = *reinterpret_cast<const u32x4*>(row + 32 * c + 8 * g);
+        out[c] = piece;
     }
 }
 
