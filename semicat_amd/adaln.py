@@ -18,6 +18,7 @@ is what PyTorch's layer_norm does there, and a network's gradients are the same 
 not the full derivative of the tangent."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 from typing import Optional
@@ -332,31 +333,17 @@ class _CastOf(torch.autograd.Function):
         return g.to(ctx.dtype), None
 
 
-class CastFunction(torch.autograd.Function):
-    """bf16 copies of fp32 parameters, all of them in one launch, and their gradients in fp32 in another."""
-
-    @staticmethod
-    def forward(ctx, *params):
-        ctx.set_materialize_grads(False)
-        return tuple(functional._cast_all(params, (torch.bfloat16,) * len(params)))
-
-    @staticmethod
-    def backward(ctx, *grads):
-        if torch.is_grad_enabled():  # a recorded backward
-            return tuple(None if g is None else g.float() for g in grads)
-        return tuple(functional._cast_all(grads, (torch.float32,) * len(grads)))
-
-
 class LinearFunction(torch.autograd.Function):
     """``x w^T + b`` and ``tx w^T``; in reverse mode one product for both inputs and one, summed over both in fp32, for the
     weight.  Through the general dispatch forward mode adds products with the absent tangents of weight and bias,
     zero fills and sums: 9 products per layer and step instead of 4.
-    bf16 products on a bf16 copy of the fp32 weight, as autocast makes it (or on one that is handed in)."""
+    bf16 products on bf16 copies of the fp32 parameters, as autocast makes them; ``w16`` and ``b16`` are copies that are
+    there already, values without a graph of their own."""
 
     @staticmethod
-    def forward(ctx, x, tx, w, b):
+    def forward(ctx, x, tx, w, b, w16=None, b16=None):
         ctx.set_materialize_grads(False)
-        w16 = w.to(x.dtype)
+        w16 = w.to(x.dtype) if w16 is None else w16
         # two products, so that each output has its own storage (see _outputs); the bias enters the product's
         # accumulator: added behind it, y would be rounded twice
         y, ty = _outputs(x, shape=(*x.shape[:-1], w.shape[0]))
@@ -364,7 +351,7 @@ class LinearFunction(torch.autograd.Function):
         if b is None:
             torch.mm(rows, w16.t(), out=y.view(-1, w.shape[0]))
         else:
-            torch.addmm(b.to(x.dtype), rows, w16.t(), out=y.view(-1, w.shape[0]))
+            torch.addmm(b.to(x.dtype) if b16 is None else b16, rows, w16.t(), out=y.view(-1, w.shape[0]))
         torch.mm(t_rows, w16.t(), out=ty.view(-1, w.shape[0]))
         ctx.save_for_backward(x, tx, w16)
         ctx.w_dtype = w.dtype
@@ -375,11 +362,12 @@ class LinearFunction(torch.autograd.Function):
     def backward(ctx, dy, dty):
         x, tx, w16 = ctx.saved_tensors
         if dy is None and dty is None:
-            return (None,) * 4
-        if torch.is_grad_enabled():
+            return (None,) * 6
+        recorded = torch.is_grad_enabled()
+        if recorded:
             w16 = _CastOf.apply(ctx.weight, w16)
         dx = dtx = dw = db = None
-        need_x, need_tx, need_w, need_b = ctx.needs_input_grad
+        need_x, need_tx, need_w, need_b = ctx.needs_input_grad[:4]
         if dy is not None and dty is not None:
             g, rows = _stacked(dy, dty), lambda: _stacked(x, tx)
         else:
@@ -390,10 +378,14 @@ class LinearFunction(torch.autograd.Function):
             dx = None if dy is None else next(pieces)
             dtx = None if dty is None else next(pieces)
         if need_w:
-            dw = torch.mm(g.t(), rows()).to(ctx.w_dtype)
+            dw = torch.mm(g.t(), rows())
         if need_b and dy is not None:
-            db = dy.reshape(-1, w16.shape[0]).sum(0).to(ctx.w_dtype)
-        return dx, dtx, dw, db
+            db = dy.reshape(-1, w16.shape[0]).sum(0)
+        if recorded:
+            dw, db = (None if d is None else d.to(ctx.w_dtype) for d in (dw, db))
+        else:
+            dw, db = functional._cast_all((dw, db), (ctx.w_dtype,) * 2)
+        return dx, dtx, dw, db, None, None
 
 
 def _heads(qkv: Tensor):
@@ -500,9 +492,11 @@ def gelu(u: Tensor) -> Optional[Tensor]:
 
 @torch._dynamo.disable
 def cast(*layers: nn.Linear):
-    """``{layer: (weight, bias)}`` with bf16 copies of the fp32 parameters of linear layers for :func:`linear`, made by one launch
-    where autocast would cast one by one (and once more for each use under forward mode), or None where that is not
-    served.  The caller has asked :func:`serves_block`."""
+    """``{layer: (weight, bias)}`` for :func:`linear` and :func:`plain_linear`: bf16 copies of the fp32 parameters, made by one
+    launch where autocast would cast one by one (and once more for each use under forward mode).  The copies are values
+    without a graph.  A plain call that records gradients gets the parameters themselves, which autocast casts each with a
+    node of its own: one node for all would compute the gradients of frozen parameters too, and hand over none
+    before the last is there.  None where that is not served.  The caller has asked :func:`serves_block`."""
     stack = _functorch.get_interpreter_stack()
     if stack is None:
         if fwAD._current_level >= 0:
@@ -515,11 +509,11 @@ def cast(*layers: nn.Linear):
     if any(type(p) not in (Tensor, nn.Parameter) or p.dtype != torch.float32 or p.device != params[0].device or not p.is_cuda
            or _functorch.is_functorch_wrapped_tensor(p) for p in params):
         return None
-    if stack is None:
-        copies = iter(CastFunction.apply(*params))
-    else:
-        with functional.retrieve_current_functorch_interpreter().lower():
-            copies = iter(CastFunction.apply(*params))
+    if stack is None and torch.is_grad_enabled() and any(p.requires_grad for p in params):
+        return {m: (m.weight, m.bias) for m in layers}
+    below = contextlib.nullcontext() if stack is None else functional.retrieve_current_functorch_interpreter().lower()
+    with below, torch.no_grad():
+        copies = iter(functional._cast_all(params, (torch.bfloat16,) * len(params)))
     return {m: (next(copies), None if m.bias is None else next(copies)) for m in layers}
 
 
@@ -527,12 +521,9 @@ def cast(*layers: nn.Linear):
 def linear(layer: nn.Linear, x: Tensor, copies=None) -> Optional[Tensor]:
     """The layer on a dual tensor, with the ``copies`` of :func:`cast` where there are any, or None where it is not served (a
     plain tensor included: that is one product already).  The caller has asked :func:`serves_block`."""
-    if copies is None:
-        if type(layer) is not nn.Linear or not bare(layer):
-            return None
-        w, b, dtype = layer.weight, layer.bias, torch.float32
-    else:
-        (w, b), dtype = copies[layer], torch.bfloat16
+    w, b = layer.weight, layer.bias
+    if copies is None and (type(layer) is not nn.Linear or not bare(layer)):
+        return None
     if x.dtype != torch.bfloat16 or _functorch.get_interpreter_stack() is None:
         return None
     found = _unwrap((x, w, b))
@@ -540,16 +531,16 @@ def linear(layer: nn.Linear, x: Tensor, copies=None) -> Optional[Tensor]:
         return None
     interpreter, (p, w, b), (t, *absent) = found
     if t is None or any(z is not None for z in absent) or t.dtype != p.dtype or t.shape != p.shape or p.numel() == 0 \
-            or any(z.dtype != dtype or z.device != p.device for z in (w, b) if z is not None):
+            or any(z.dtype != torch.float32 or z.device != p.device for z in (w, b) if z is not None):
         return None
     with interpreter.lower():
-        y, ty = LinearFunction.apply(p, t, w, b)
+        y, ty = LinearFunction.apply(p, t, w, b, *(() if copies is None else copies[layer]))
     return _dual_above(interpreter, y, ty)
 
 
 @torch._dynamo.disable
 def plain_linear(layer: nn.Linear, x: Tensor, copies) -> Optional[Tensor]:
-    """The layer on a plain tensor with the copies of :func:`cast`; None inside a transform."""
+    """The layer on a plain tensor with what :func:`cast` gave; None inside a transform."""
     return None if _functorch.get_interpreter_stack() is not None else nn.functional.linear(x, *copies[layer])
 
 

@@ -59,13 +59,26 @@ def test_frozen_parameters_and_no_grad(monkeypatch):
         assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
 
 
-def test_recorded_backward_of_the_casts():
-    w, b = (torch.randn(n, device="cuda", requires_grad=True) for n in (24, 8))
-    w16, b16 = adaln.CastFunction.apply(w, b)
-    assert w16.dtype == b16.dtype == torch.bfloat16
-    gw, = torch.autograd.grad((w16 * w16).sum(), w, create_graph=True)
-    assert gw.dtype == torch.float32 and torch.equal(gw, 2 * w16.float())
-    assert torch.equal(torch.autograd.grad(gw.sum(), w)[0], torch.full_like(w, 2.0))
+def test_recorded_backward(monkeypatch):
+    """Gradients that are recorded, of the network's plain call and of a dual layer, and the gradients of those."""
+    net, x0, x1 = _net()
+    got = _step(net, x0, x1, create_graph=True)
+    cast = adaln.cast
+    monkeypatch.setattr(adaln, "cast", lambda *m: None)
+    for a, b in zip(got, _step(net, x0, x1, create_graph=True)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+    monkeypatch.setattr(adaln, "cast", cast)
+    layer = torch.nn.Linear(24, 40, device="cuda")
+
+    def twice(copies):
+        torch.manual_seed(1)
+        x, t = (torch.randn(6, 24, device="cuda").bfloat16().requires_grad_() for _ in range(2))
+        out = torch.func.jvp(lambda z: adaln.linear(layer, z, adaln.cast(layer) if copies else None), (x,), (t,))
+        first = torch.autograd.grad(out, [x, t, layer.weight, layer.bias], [torch.ones_like(z) for z in out], create_graph=True)
+        return [*out, *first, *torch.autograd.grad(sum(g.float().pow(2).sum() for g in first), [x, t, layer.weight])]
+
+    for a, b in zip(twice(True), twice(False)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
 
 
 def test_layers_that_are_left_to_pytorch():
