@@ -8,6 +8,7 @@
 #include <ATen/ATen.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <c10/core/DeviceGuard.h>
@@ -303,11 +304,26 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// cast(list of tensors or None, dtype) -> list; a tensor that has the dtype is handed back itself, the others, dense and
-// between fp32 and one 16-bit type, are copied in as few launches as it takes.  Nothing is recorded for autograd.
+// A copy as part of the graph of the tensor it was cast from: one node for each, so that a tensor that needs no gradient
+// has none and one that does gets it as soon as it is there.
+struct CastNode : torch::autograd::Function<CastNode> {
+    static constexpr bool is_traceable = true;
+    static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& from, Tensor* copy) {
+        ctx->saved_data["type"] = static_cast<int64_t>(from.scalar_type());
+        return std::move(*copy);
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+        const auto type = static_cast<at::ScalarType>(ctx->saved_data["type"].toInt());
+        return {grads[0].defined() ? grads[0].to(type) : Tensor(), Tensor()};
+    }
+};
+
+// cast(list of tensors or None, dtype, recorded) -> list; a tensor that has the dtype is handed back itself, the others, dense
+// and between fp32 and one 16-bit type, are copied in as few launches as it takes.  Autograd sees it only where `recorded`.
 PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 2 || !abi.cast || !PyList_CheckExact(a[0]) || !THPDtype_Check(a[1])) return none();
+    if (n < 2 || n > 3 || !abi.cast || !PyList_CheckExact(a[0]) || !THPDtype_Check(a[1])) return none();
+    const bool recorded = n == 3 && a[2] == Py_True && at::GradMode::is_enabled();
     const at::ScalarType to = reinterpret_cast<THPDtype*>(a[1])->scalar_type;
     constexpr int kMost = 64;
     const Py_ssize_t count = PyList_GET_SIZE(a[0]);
@@ -351,6 +367,8 @@ PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
     }
     if (rc != SJVP_OK) return PyLong_FromLong(rc);
+    for (Py_ssize_t i = 0; i < count; ++i)
+        if (recorded && in[i] && in[i]->requires_grad()) made[i] = CastNode::apply(*in[i], &made[i]);
     PyObject* res = PyList_New(count);
     if (!res) return nullptr;
     for (Py_ssize_t i = 0; i < count; ++i) {

@@ -1,6 +1,5 @@
 """The copies that a block's linear layers share are values: a layer's parameters keep their own places in the graph.  (CPU; the
 cast itself is PyTorch's here.)"""
-import pytest
 import torch
 from torch import nn
 
@@ -86,22 +85,3 @@ def test_copies_give_what_each_layers_own_cast_gives(monkeypatch):
         res.append([*out, *torch.autograd.grad(out, [p for m in layers for p in m.parameters()], [torch.ones_like(z) for z in out])])
     for a, b in zip(*res):
         assert a.dtype == b.dtype and torch.equal(a, b)
-
-
-@pytest.mark.parametrize("frozen", [False, True])
-def test_plain_calls(monkeypatch, frozen):
-    """Where gradients are recorded autocast casts each parameter with a node of its own."""
-    layers = _layers(monkeypatch)
-    if frozen:
-        layers[0].weight.requires_grad_(False)
-    with torch.autocast("cpu", dtype=torch.bfloat16):
-        copies = adaln.cast(*layers)
-        assert all((p is None) == (c is None) and (p is None or c.requires_grad == p.requires_grad)
-                   for m in layers for p, c in zip((m.weight, m.bias), copies[m]))
-        y = adaln.plain_linear(layers[0], torch.randn(3, 24).bfloat16(), copies)
-    y.sum().backward()
-    assert y.dtype == torch.bfloat16 and (layers[0].weight.grad is None) == frozen and layers[0].bias.grad is not None
-    for m in layers:
-        m.requires_grad_(False)
-    copies = adaln.cast(*layers)
-    assert all(c.dtype == torch.bfloat16 and not c.requires_grad for m in layers for c in copies[m] if c is not None)

@@ -59,6 +59,43 @@ def test_frozen_parameters_and_no_grad(monkeypatch):
         assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
 
 
+def test_copies_of_plain_calls():
+    """A node for each parameter that needs one; gradients reach the layers one after the other."""
+    layers = [torch.nn.Linear(24, 40, device="cuda"), torch.nn.Linear(40, 16, device="cuda")]
+    layers[0].weight.requires_grad_(False)
+    order = []
+    for i, m in enumerate(layers):
+        m.bias.register_post_accumulate_grad_hook(lambda p, i=i: order.append(i))
+    copies = adaln.cast(*layers)
+    for m in layers:
+        for p, c in zip((m.weight, m.bias), copies[m]):
+            assert c.dtype == torch.bfloat16 and c.requires_grad == p.requires_grad and torch.equal(c, p.bfloat16())
+    z = adaln.plain_linear(layers[0], torch.randn(3, 24, device="cuda").bfloat16(), copies)
+    z.register_hook(lambda g: order.append("between"))
+    y = adaln.plain_linear(layers[1], z, copies)
+    only, = torch.autograd.grad(y.sum(), layers[1].bias, retain_graph=True)
+    assert order == [] and only.dtype == torch.float32
+    y.sum().backward()
+    assert order.index(1) < order.index(0) and layers[0].weight.grad is None and torch.equal(layers[1].bias.grad, only)
+    with torch.no_grad():
+        assert not any(c.requires_grad for c in adaln.cast(*layers)[layers[1]])
+
+
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode])
+def test_calls_in_one_autocast_region(mode):
+    """A call without gradients leaves the ones behind it theirs; two that record add theirs up in float32."""
+    layer = torch.nn.Linear(24, 40, device="cuda")
+    x = torch.randn(3, 24, device="cuda").bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        with mode():
+            y = adaln.plain_linear(layer, x, adaln.cast(layer))
+        ys = [adaln.plain_linear(layer, x * scale, adaln.cast(layer)) for scale in (1.0, 2 ** -9)]
+    assert not y.requires_grad and torch.equal(y, ys[0])
+    grads = [torch.autograd.grad(z.sum(), layer.weight, retain_graph=True)[0] for z in ys]
+    (ys[0].sum() + ys[1].sum()).backward()
+    assert torch.equal(layer.weight.grad, grads[0] + grads[1])
+
+
 def test_recorded_backward(monkeypatch):
     """Gradients that are recorded, of the network's plain call and of a dual layer, and the gradients of those."""
     net, x0, x1 = _net()
