@@ -75,23 +75,8 @@ int check_rotary(const float* cos, const float* sin, int64_t cs_stride, int tabl
 
 inline float resolve_scale(float scale, int D) { return scale > 0.f ? scale : 1.0f / sqrtf((float)D); }
 
-constexpr int kMaxDevices = 64;
-
 // Process-wide setting of sjvp_set_row_sum_repair().
 std::atomic<int> g_row_sum_repair{SJVP_REPAIR_AUTO};
-
-// Compute units of the current device (looked up once per device).
-int compute_units() {
-    static std::atomic<int> cached[kMaxDevices] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
-    int n = cached[dev].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-        cached[dev].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
 
 // Whether the backward takes the single launch, else the row + column pair.
 bool bwd_single(const BwdParams& p, int BH, int parts) {

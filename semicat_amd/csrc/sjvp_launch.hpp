@@ -62,19 +62,36 @@ int launch(K kernel, int grid, int smem_bytes, hipStream_t stream, const P& para
     return rc == hipSuccess ? SJVP_OK : SJVP_ERR_LAUNCH;
 }
 
+constexpr int kMaxDevices = 64;
+
+// Compute units of the current device (looked up once per device; 256 for a whole MI355X, fewer for a partition of one).
+inline int compute_units() {
+    static std::atomic<int> cached[kMaxDevices] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        cached[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
 // Waves that share a group of 16 owned rows (SPLIT of the 16-wide kernels) in a launch of `grid` workgroups that would walk
-// `stages` stages each.  A workgroup of a launch that does not fill the chip is a serial chain of stages; split, it is as
-// many times shorter, plus the exchange of the sums (two or three stages' time).  So: while every split workgroup still has
+// `stages` stages each, on `units` compute units.  A workgroup of a launch that does not fill the chip is a serial chain of
+// stages; split, it is as many times shorter, plus the exchange of the sums.  So: while every split workgroup still has
 // a compute unit of its own, or two share one (`pairs`) and the chain is long.  Times of the split launch over the whole
 // one at D = 64: all have a unit 0.49 to 0.89; two to a unit, 16 or 32 stages 0.81 to 0.95, 7 stages 1.05; more 1.1 to 3.5
-// (the forward, whose workgroups have eight waves, 1.1 to 1.3 already with two).
+// (the forward, whose workgroups have eight waves, 1.1 to 1.3 already with two).  The shortest chains that are split, us whole /
+// split: row kernel 4 stages in two 8.6 / 7.0, 5 in four 9.8 / 7.6; column kernel 4 in two 8.2 / 6.9, 5 in four 8.8 / 6.6;
+// forward 5 in four 8.5 / 7.2, 5 in two 8.9 / 8.4, 6 in two 9.7 / 8.2; rows of odd lengths, row kernel 4 in two
+// 11.6 / 9.8, column kernel 10.6 / 9.3.
 // Forward + backward, whole / split: B=1 H=8 L=256 33.7 / 21.6 us, B=1 H=4 L=2048 173 / 96, B=1 H=12 L=512 without tangents
 // 34.5 / 24.4, B=4 H=6 333 x 205 D=48 cotangent on TO 40.2 / 35.1, B=2 H=12 L=300 D=36 50.8 / 44.1.
-constexpr int kComputeUnits = 256;
-inline int split_rows(int64_t grid, int stages, int most, bool pairs) {
-    if (most >= 4 && 4 * grid <= kComputeUnits && stages > 4) return 4;
-    if (2 * grid <= kComputeUnits && stages > 3) return 2;
-    return pairs && 2 * grid <= 2 * kComputeUnits && stages >= 12 ? 2 : 1;
+inline int split_rows(int64_t grid, int stages, int most, bool pairs, int units = compute_units()) {
+    if (most >= 4 && 4 * grid <= units && stages > 4) return 4;
+    if (2 * grid <= units && stages > 3) return 2;
+    return pairs && grid <= units && stages >= 12 ? 2 : 1;
 }
 
 // Forward: stages by LDS-DMA (16-byte aligned rows), or through registers (any alignment).

@@ -26,7 +26,7 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         // of 64 queries per compute unit on (1024 of them 0.76 to 1.01 of the time, 512 1.03 to 1.13), and from 256
         // keys on (128 of them 1.02).
         bool wide = false;
-        if constexpr (!HAS_G && IO == kIoDma) wide = p.rowfix != 2 && grid >= 1024 && p.Lk >= 256;
+        if constexpr (!HAS_G && IO == kIoDma) wide = p.rowfix != 2 && grid >= 4 * compute_units() && p.Lk >= 256;
         int split = 1;
         if constexpr (HD <= 64 && IO != kIoF32) {
             constexpr int MOST = IO == kIoDma ? 4 : 2;  // (four parts' staged copies do not fit the registers)
@@ -96,7 +96,8 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
         // 1.01 of the time, 256 1.16 to 1.23); at D = 32 with both cotangents 129 -> 112 us, from 1024 workgroups and
         // 512 queries on (1024 and 256: 0.97 to 1.04).
         if constexpr (IO == kIoDma && (!HAS_G || HD == 32)) {
-            if (rides && (HAS_G ? grid >= 1024 && p.Lq >= 512 : grid >= 512 && p.Lq >= 256)) {
+            const int rounds = grid / compute_units();
+            if (rides && (HAS_G ? rounds >= 4 && p.Lq >= 512 : rounds >= 2 && p.Lq >= 256)) {
                 BwdParams pr = p;
                 pr.col_workgroups = BH * ((p.Lk + 2 * kXOwned16 - 1) / (2 * kXOwned16));
                 constexpr int smem = CS::bytes > Row16Smem<HD, XR, HAS_G>::bytes ? CS::bytes : Row16Smem<HD, XR, HAS_G>::bytes;

@@ -20,7 +20,8 @@ int fwd16_one(const FwdParams& p, int grid, hipStream_t stream) {
     // chip holds (D <= 64: 1024 of them 0.90 to 1.01 of the time, 512 0.97 to 1.08; D = 128: 512 of them from 1024 keys
     // on 0.95 to 0.98, with 256 to 512 keys 1.01 to 1.07).
     if constexpr (!JVP && SPB == 2) {
-        if (HD == 128 ? grid >= 512 && p.Lk >= 1024 : grid >= 1024)
+        const int rounds = grid / compute_units();
+        if (HD == 128 ? rounds >= 2 && p.Lk >= 1024 : rounds >= 4)
             return launch(fwd16_kernel<T, HD, R, JVP, HD == 128 ? 2 : 4, SPB, ROPE, kIoDma, 2, 1, DT>, grid, smem, stream, p,
                           kThreads16 / 2);
     }
