@@ -76,13 +76,18 @@ int pair_mode(const BwdParams& p, int BH, int parts, hipStream_t stream) {
     } else {
         if constexpr (HD <= 64 && IO != kIoF32) {
             constexpr int MOST = IO == kIoDma ? 4 : 2;
-            const int split = rides ? split_rows(grid, (p.Lq + kStageRows - 1) / kStageRows, MOST, IO == kIoDma) : 1;
+            // (whether or not the second row launch rides along: dK, dV are the same bits with the repair off, or in a call
+            // for this part alone; as in the row launch, "always" keeps to whole workgroups)
+            const int split = p.rowfix != 2 ? split_rows(grid, (p.Lq + kStageRows - 1) / kStageRows, MOST, IO == kIoDma) : 1;
             auto go = [&](auto split_tag) {
                 constexpr int SPLIT = decltype(split_tag)::value;
                 constexpr int OWNED = kXOwned16 / SPLIT;
                 BwdParams pr = p;
                 pr.col_workgroups = BH * ((p.Lk + OWNED - 1) / OWNED);
                 constexpr int row = Row16Smem<HD, XR, HAS_G>::bytes, col = Col16Smem<HD, 2 * SPLIT, HAS_DO, HAS_G, SPLIT>::bytes;
+                if (!rides)
+                    return launch(bwd_col16_kernel<T, HD, 2 * SPLIT, HAS_DO, HAS_G, 2, IO, 1, SPLIT, DT>, pr.col_workgroups, col,
+                                  stream, pr, kXThreads16);
                 return launch(bwd_col16_repair_kernel<T, HD, 2 * SPLIT, HAS_DO, HAS_G, 2, IO, 1, SPLIT, XR, DT>,
                               pr.col_workgroups + BH * (p.Lr / kXOwned16), col > row ? col : row, stream, pr, kXThreads16);
             };
