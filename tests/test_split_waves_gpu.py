@@ -1,5 +1,5 @@
 """The 16-bit kernels in which several wavefronts share a group of rows, which launches of few workgroups take: every part's
-remainder, groups and waves without rows, keys without a probability in a part, and flagged rows."""
+remainder, groups and waves without rows, and keys without a probability in a part."""
 import pytest
 import torch
 
@@ -8,6 +8,8 @@ from oracle import attn_jvp_oracle as orc
 pytestmark = pytest.mark.gpu
 ORDER = ("q", "k", "v", "tq", "tk", "tv")
 GRADS = ("dq", "dk", "dv", "dtq", "dtk", "dtv")
+# the bound of the other parity tests, by the unit roundoff of the type (2^-8 and 2^-11)
+BOUND = {torch.bfloat16: 1e-2, torch.float16: 1e-2 / 8}
 
 
 def _run(x, mode):
@@ -44,7 +46,7 @@ def test_parts_of_a_group(H, Lq, Lk, D, dtype, step, mode):
     for n, t in res.items():
         if n in ref and n not in ("lse", "mu", "li"):
             err = orc.rel_frobenius(t, ref[n])
-            assert err <= 1e-2, (n, err)  # the bound of the other parity tests (also false for NaN)
+            assert err <= BOUND[dtype], (n, err)  # (also false for NaN)
     cf = orc.attention_jvp_closed_form(*[x[n] for n in ORDER])
     assert torch.allclose(res["lse"][..., :Lq].double(), torch.as_tensor(cf["lse"]).double(), rtol=2e-5, atol=2e-5)
     assert torch.allclose(res["lse"][..., Lq:], torch.full_like(res["lse"][..., Lq:], Lk).log(), rtol=1e-6)
