@@ -26,7 +26,8 @@ int fwd16_one(const FwdParams& p, int grid, hipStream_t stream) {
                           kThreads16 / 2);
     }
     if constexpr (HD <= 64 && !ROPE) {
-        // (D = 128: the sums do not fit the LDS.  Up to 128 keys the folded rotation is an alternative to this launch, and
+        // (D > 64 is left whole: with tangents at D = 128 the sums of eight waves do not fit the LDS (168 KB); the other forms
+        // would fit and have not been measured.  Up to 128 keys the folded rotation is an alternative to this launch, and
         // both round alike.)
         const int split = p.Lk > kOwned16 ? split_rows(grid, (p.Lk + kStageRows - 1) / kStageRows, 4, false) : 1;
         FwdParams ps = p;
