@@ -85,3 +85,25 @@ def test_copies_give_what_each_layers_own_cast_gives(monkeypatch):
         res.append([*out, *torch.autograd.grad(out, [p for m in layers for p in m.parameters()], [torch.ones_like(z) for z in out])])
     for a, b in zip(*res):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_calls_without_gradients_share_the_regions_casts(monkeypatch):
+    """What autocast keeps for a region is not cast once more for each call in it; what it does not keep still is."""
+    layers = _layers(monkeypatch)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *device: True)
+    with torch.no_grad():
+        assert torch.is_autocast_cache_enabled() and adaln.cast(*layers) is None
+        assert adaln.cast(layers[0], nn.Sequential(layers[1])) is None  # no weight of its own
+        layers[1].weight.requires_grad_(False)
+        copies = adaln.cast(*layers)
+        own = [c is not p for m in layers for p, c in zip((m.weight, m.bias), copies[m]) if p is not None]
+        assert own == [False, False, True, False, False] and torch.equal(copies[layers[1]][0], layers[1].weight.bfloat16())
+        torch.set_autocast_cache_enabled(False)
+        try:
+            copies = adaln.cast(*layers)
+        finally:
+            torch.set_autocast_cache_enabled(True)
+    assert all(c is None or c.dtype == torch.bfloat16 for pair in copies.values() for c in pair)
+    for m in layers:
+        m.requires_grad_(False)
+    assert all(c is None or c.dtype == torch.bfloat16 for pair in adaln.cast(*layers).values() for c in pair)

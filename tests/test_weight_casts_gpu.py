@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from semicat_amd import adaln, train_step
-from semicat_amd.dit import DIT
+from semicat_amd.dit import DIT, _linear
 
 pytestmark = pytest.mark.gpu
 
@@ -88,12 +88,34 @@ def test_calls_in_one_autocast_region(mode):
     x = torch.randn(3, 24, device="cuda").bfloat16()
     with torch.autocast("cuda", dtype=torch.bfloat16):
         with mode():
-            y = adaln.plain_linear(layer, x, adaln.cast(layer))
+            y = _linear(True, layer, x, adaln.cast(layer))
         ys = [adaln.plain_linear(layer, x * scale, adaln.cast(layer)) for scale in (1.0, 2 ** -9)]
     assert not y.requires_grad and torch.equal(y, ys[0])
     grads = [torch.autograd.grad(z.sum(), layer.weight, retain_graph=True)[0] for z in ys]
     (ys[0].sum() + ys[1].sum()).backward()
     assert torch.equal(layer.weight.grad, grads[0] + grads[1])
+
+
+def test_region_without_gradients(monkeypatch):
+    """Calls of the network in one region cast its parameters once, frozen ones excepted; the bits are autocast's own."""
+    net, x0, _ = _net()
+    net.blocks[0].attn_qkv.weight.requires_grad_(False)
+    t = torch.full((4,), 0.25, device="cuda")
+    made = []
+    cast_all = adaln.functional._cast_all
+    monkeypatch.setattr(adaln.functional, "_cast_all", lambda ts, ds: made.append(sum(z is not None for z in ts)) or cast_all(ts, ds))
+
+    def run(**region):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, **region):
+            return [net(x0, t, t), net(x0, t, t)]
+
+    got = run()
+    assert made == [1, 1]
+    got += run(cache_enabled=False)
+    assert made[2:] == [8, 8, 4] * 2
+    monkeypatch.setattr(adaln, "cast", lambda *m: None)
+    want = run()[0]
+    assert all(torch.equal(y, want) for y in got)
 
 
 def test_recorded_backward(monkeypatch):
