@@ -15,6 +15,9 @@
 //     y: sub-tile e of the output holds columns d = 4 c + e, and a lane ends up with 16 consecutive columns of
 //     output row x.  No shuffle, no LDS, no transposition.
 //
+// Problems that fill the chip go to the kernels of sjvp_f32x3.hpp (the rule is in sjvp_f32.hip); these serve the smaller ones, short
+// axes, and waves that hold numbers which those cannot take.
+//
 // What bounds it: the matrix pipe (157 TFLOP/s in fp32), once a wave's operand loads are out of its way.  A
 // 16-byte load serves 4 to 8 matrix instructions of 32 cycles each, so the operands come straight from global
 // memory (L1 / L2: at most 21 bytes per clock and CU at D = 64, where the L1 delivers 64) and the loops have no
@@ -283,13 +286,11 @@ constexpr int f32_red_floats() { return SPLIT > 1 ? SPLIT * HD / 16 * 4 * 64 : 1
 
 // ---------------------------------------------------------------------------------------------
 // Forward (ryu_triton.py:188-291 in fp32): O, TO, lse, mu, li.
+// (`red`, `stat`: LDS for the sums of a split group.)
 template <int HD, bool JVP, int SPLIT, F32Columns COLS>
-__global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel(const FwdParamsF32 p) {
-    __shared__ float red[f32_red_floats<HD, SPLIT>()];
-    __shared__ float stat[SPLIT > 1 ? SPLIT * 3 * kF32Rows : 1];
+__device__ __forceinline__ void fwd_f32_wave(const FwdParamsF32& p, const F32Place& w, float* red, float* stat) {
     constexpr int M = HD / 16, T = HD / 16;
     constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
-    const F32Place w = f32_place<SPLIT>(p.blocks, p.H);
     const int qrow = w.row0 + w.n;
     const bool qvalid = qrow < p.Lq;
     const int64_t so = (int64_t)w.bh * p.Lr + qrow;  // rows below Lr exist
@@ -444,15 +445,19 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel
         f32_store<HD, VEC, SPLIT>(red, p.to.head(w.b, w.h) + (int64_t)qrow * p.to.sl, tacc, inv_l, w, p.D, qvalid);
     }
 }
+template <int HD, bool JVP, int SPLIT, F32Columns COLS>
+__global__ __launch_bounds__(kF32Threads, HD == 128 ? 1 : 2) void fwd_f32_kernel(const FwdParamsF32 p) {
+    __shared__ float red[f32_red_floats<HD, SPLIT>()];
+    __shared__ float stat[SPLIT > 1 ? SPLIT * 3 * kF32Rows : 1];
+    fwd_f32_wave<HD, JVP, SPLIT, COLS>(p, f32_place<SPLIT>(p.blocks, p.H), red, stat);
+}
 
 // ---------------------------------------------------------------------------------------------
 // Row-owned backward: dQ (, dQ_dot) and the row sums for the column-owned kernel.
 template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
-__global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_row_f32_kernel(const BwdParamsF32 p) {
-    __shared__ float red[f32_red_floats<HD, SPLIT>()];
+__device__ __forceinline__ void bwd_row_f32_wave(const BwdParamsF32& p, const F32Place& w, float* red) {
     constexpr int M = HD / 16, T = HD / 16;
     constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
-    const F32Place w = f32_place<SPLIT>(p.q_blocks, p.H);
     if (w.row0 >= p.Lq) return;
     const int qrow = w.row0 + w.n;
     const bool qvalid = qrow < p.Lq;
@@ -591,15 +596,18 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
     if constexpr (HAS_G)
         f32_store<HD, VEC, SPLIT>(red, p.dtq.head(w.b, w.h) + (int64_t)qrow * p.dtq.sl, dtq, p.scale, w, p.D, qvalid);
 }
+template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
+__global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_row_f32_kernel(const BwdParamsF32 p) {
+    __shared__ float red[f32_red_floats<HD, SPLIT>()];
+    bwd_row_f32_wave<HD, HAS_DO, HAS_G, SPLIT, COLS>(p, f32_place<SPLIT>(p.q_blocks, p.H), red);
+}
 
 // ---------------------------------------------------------------------------------------------
 // Column-owned backward: dK, dV (, dK_dot, dV_dot).
 template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
-__global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_col_f32_kernel(const BwdParamsF32 p) {
-    __shared__ float red[f32_red_floats<HD, SPLIT>()];
+__device__ __forceinline__ void bwd_col_f32_wave(const BwdParamsF32& p, const F32Place& w, float* red) {
     constexpr int M = HD / 16, T = HD / 16;
     constexpr bool VEC = COLS != kColumnsCut, MASK = COLS != kColumnsAll;
-    const F32Place w = f32_place<SPLIT>(p.k_blocks, p.H);
     if (w.row0 >= p.Lk) return;
     const int krow = w.row0 + w.n;
     const bool kvalid = krow < p.Lk;
@@ -750,6 +758,11 @@ __global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 :
         f32_store<HD, VEC, SPLIT>(red, p.dtk.head(w.b, w.h) + (int64_t)krow * p.dtk.sl, dtk, p.scale, w, p.D, kvalid);
         f32_store<HD, VEC, SPLIT>(red, p.dtv.head(w.b, w.h) + (int64_t)krow * p.dtv.sl, dtv, 1.0f, w, p.D, kvalid);
     }
+}
+template <int HD, bool HAS_DO, bool HAS_G, int SPLIT, F32Columns COLS>
+__global__ __launch_bounds__(kF32Threads, HD == 128 || (HD == 64 && HAS_G) ? 1 : 2) void bwd_col_f32_kernel(const BwdParamsF32 p) {
+    __shared__ float red[f32_red_floats<HD, SPLIT>()];
+    bwd_col_f32_wave<HD, HAS_DO, HAS_G, SPLIT, COLS>(p, f32_place<SPLIT>(p.k_blocks, p.H), red);
 }
 
 }  // namespace sjvp

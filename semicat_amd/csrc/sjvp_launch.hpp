@@ -113,5 +113,9 @@ int bwd_pair_f32io(const BwdParams& p, int BH, bool has_do, bool has_g, int part
 // fp32 correctness mode: forward, and the row-owned + column-owned backward pair.
 int fwd_f32(const FwdParamsF32& p, int BH, bool jvp, hipStream_t stream);
 int bwd_f32(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int parts, hipStream_t stream);
+// The same on the bf16 matrix pipe, operands in three parts (sjvp_f32x3.hpp), with four or eight waves in a workgroup; the
+// two above choose.  `part`: SJVP_BWD_ROW or SJVP_BWD_COL.
+int fwd_f32x3(const FwdParamsF32& p, int BH, bool jvp, int waves, hipStream_t stream);
+int bwd_f32x3(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int part, int waves, hipStream_t stream);
 
 }  // namespace sjvp

@@ -1,0 +1,113 @@
+"""The fp32 kernels that take their operands in three bf16 parts, at the edges of their tiles, workgroups and head-dimension
+classes, against the fp64 oracle; and heads that hold numbers for the fp32 unit, against the same heads in a call that the fp32
+unit's kernels serve as a whole."""
+import pytest
+import torch
+from torch.profiler import ProfilerActivity, profile
+
+from oracle import attn_jvp_oracle as orc
+
+pytestmark = pytest.mark.gpu
+NAMES = ("o", "to", "lse", "mu", "dq", "dk", "dv", "dtq", "dtk", "dtv")
+TOL = 1e-5  # the bound that the fp32 mode is held to elsewhere
+
+
+def _step(x, mode="both"):
+    from semicat_amd import kernels as K
+    ins = [x[n] for n in ("q", "k", "v", "tq", "tk", "tv")]
+    o, to, lse, mu, _ = K.attention_jvp_forward(*ins, with_li=False)
+    if mode == "dO":
+        ins[3:] = [None] * 3
+    g = K.attention_jvp_backward(*ins, o, None if mode == "dO" else to, lse, None if mode == "dO" else mu,
+                                 dO=None if mode == "dTO" else x["dO"], dTO=None if mode == "dO" else x["dTO"])
+    return dict(zip(NAMES, (o, to, lse, mu, *g)))
+
+
+def _kernels(run):
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        res = run()
+        torch.cuda.synchronize()
+    return res, [e.key for e in prof.key_averages() if "f32" in e.key]
+
+
+@pytest.mark.parametrize("mode", ["both", "dO", "dTO"])
+@pytest.mark.parametrize("B,H,Lq,Lk,D,offset", [
+    (40, 12, 75, 90, 64, 0),   # eight waves, ragged rows and last stage; waves and a workgroup's half without rows
+    (25, 4, 100, 97, 64, 1),   # four waves, a last stage of one row, no 16-byte alignment
+    (30, 12, 129, 100, 48, 0),  # a second workgroup with one row
+    (40, 12, 96, 127, 33, 3),  # odd columns
+    (30, 12, 100, 120, 32, 0), (30, 12, 100, 120, 21, 1), (30, 12, 80, 96, 16, 0),
+    (20, 12, 90, 90, 80, 0), (20, 12, 90, 95, 67, 2), (16, 12, 100, 100, 128, 0), (20, 12, 120, 110, 101, 1)])
+def test_parts_at_the_edges(mode, B, H, Lq, Lk, D, offset):
+    x = orc.make_inputs(B, H, Lq, Lk, D, seed=7, tangent_scale=0.5, dtype=torch.float32)
+    cot = {n: x[n] for n in ("dO", "dTO") if mode in ("both", n)}
+    ref = orc.attention_jvp_autograd(*[x[n] for n in orc.TENSOR_ORDER[:6]], **cot)
+    d = {}
+    for n, t in x.items():  # views that start `offset` elements into their storage, in [B,L,H,D] memory
+        buf = torch.empty(t.numel() + offset, device="cuda")
+        d[n] = buf[offset:].view(B, t.shape[2], H, D).transpose(1, 2)
+        d[n].copy_(t)
+    print(f"[f32 parts] {(B, H, Lq, Lk, D, offset)} {mode}", flush=True)
+    res, names = _kernels(lambda: _step(d, mode))
+    assert any("fwd_f32x3" in n for n in names) and any("row_f32x3" in n for n in names), names
+    assert any("col_f32x3" in n for n in names) == (D <= 96 or mode == "dO"), names
+    for n, t in res.items():
+        if t is not None and n not in ("lse", "mu"):
+            err = orc.rel_frobenius(t.cpu(), ref[n.upper() if n in ("o", "to") else n])
+            assert err <= TOL, (n, err)
+    assert (res["lse"][..., Lq:] - torch.tensor(float(Lk)).log().item()).abs().max() <= 1e-5
+    assert not res["mu"][..., Lq:].any()
+    from semicat_amd import kernels as K
+    o, lse = K.attention_forward(d["q"], d["k"], d["v"])
+    assert orc.rel_frobenius(o.cpu(), ref["O"]) <= TOL and torch.allclose(lse, res["lse"], rtol=1e-6, atol=1e-6)
+
+
+def _at(name, row, value, column=0):
+    def put(x, b):
+        x[name][b, 0, row, column] = value
+    return put
+
+
+def _overflowing(x, b):  # one score beyond the range
+    for n in ("q", "k", "tq", "tk"):
+        x[n][b, 0, :, 0] = 0.0
+    x["q"][b, 0, 5, 0], x["k"][b, 0, 9, 0] = 1e25, -1e25
+
+
+def _lowest(x, b):
+    x["q"][b, 0, :, 0] = 8.0
+    x["k"][b, 0, 40:, 0] = torch.finfo(torch.float32).min
+    x["tq"][b, 0, :, 0] = x["tk"][b, 0, :, 0] = 0.0
+
+
+SPECIAL = [_at("k", 3, float("inf")), _at("k", 33, float("-inf"), 7), _at("q", 17, float("nan")), _at("v", 40, float("inf"), 20),
+           _at("tv", 0, float("-inf")), _at("tk", 8, 1e30), _at("dTO", 11, float("inf"), 3), _at("dO", 70, float("nan"), 31),
+           _overflowing, _lowest, _at("v", 2, torch.finfo(torch.float32).max), _at("tq", 1, 1e25)]
+
+
+@pytest.mark.parametrize("D", [32, 64, 80])
+def test_numbers_for_the_fp32_unit(D):
+    """They reach the same outputs, as the same infinities and NaN, and no other head."""
+    B, L = 480, 110 if D == 80 else 75
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    x = {n: torch.randn((B, 1, L, D), device="cuda", generator=gen) * (0.5 if n[0] == "t" else 1.0)
+         for n in ("q", "k", "v", "tq", "tk", "tv", "dO", "dTO")}
+    clean, names = _kernels(lambda: _step(x))
+    assert all("f32x3" in n for n in names), names
+    heads = [37 * i + 5 for i in range(len(SPECIAL))]
+    for b, put in zip(heads, SPECIAL):
+        put(x, b)
+    print(f"[f32 unit's numbers] D={D}", flush=True)
+    got = _step(x)
+    unit, names = _kernels(lambda: _step({n: t[heads].contiguous() for n, t in x.items()}))
+    assert not any("f32x3" in n for n in names), names
+    others = [b for b in range(B) if b not in heads]
+    for n in NAMES:
+        assert torch.equal(got[n][others], clean[n][others]), n
+        a, r = got[n][heads], unit[n]
+        for i in range(len(heads)):
+            finite = r[i].isfinite()
+            assert torch.equal(a[i].isfinite(), finite) and torch.equal(a[i].isnan(), r[i].isnan()), (n, i)
+            assert torch.equal(a[i][r[i].isinf()], r[i][r[i].isinf()]), (n, i)
+            if finite.any():  # sums of the same products in another order
+                assert (a[i][finite] - r[i][finite]).abs().max() <= TOL * r[i][finite].abs().max(), (n, i)
