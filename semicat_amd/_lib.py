@@ -139,7 +139,7 @@ def _load_host(lib: ctypes.CDLL):
     host.bind(*(ctypes.cast(fn, ctypes.c_void_p).value for fn in
                 (lib.sjvp_fwd, lib.sjvp_fwd_rotary, lib.sjvp_bwd_parts, lib.sjvp_bwd_rotary,
                  lib.sjvp_bwd_workspace_bytes, lib.sjvp_cast, lib.sjvp_adaln_fwd, lib.sjvp_adaln_bwd,
-                 lib.sjvp_adaln_workspace_floats, lib.sjvp_gelu)))
+                 lib.sjvp_adaln_workspace_floats, lib.sjvp_gelu, lib.sjvp_rope)))
     return host
 
 

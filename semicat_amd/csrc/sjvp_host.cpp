@@ -34,6 +34,7 @@ struct Abi {
     decltype(&sjvp_adaln_bwd) adaln_bwd = nullptr;
     decltype(&sjvp_adaln_workspace_floats) adaln_workspace_floats = nullptr;
     decltype(&sjvp_gelu) gelu = nullptr;
+    decltype(&sjvp_rope) rope = nullptr;
 };
 Abi abi;  // filled once by bind() when the library is loaded
 
@@ -389,6 +390,76 @@ PyObject* cast(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// rope(sequence of one to four [B,S,H,D] tensors, cos, sin, dtype of the results or None, inverse) -> tuple of contiguous
+// [B,S,H,D] tensors; cos and sin None: no rotation
+PyObject* rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 5 || !abi.rope || !PyTuple_CheckExact(a[0]) || (a[3] != Py_None && !THPDtype_Check(a[3]))) return none();
+    if (a[4] != Py_True && a[4] != Py_False) return none();
+    constexpr int kMost = 4;
+    const Py_ssize_t count = PyTuple_GET_SIZE(a[0]);
+    if (count < 1 || count > kMost) return none();
+    const Tensor* x[kMost];
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        x[i] = plain(PyTuple_GET_ITEM(a[0], i));
+        if (!x[i] || x[i]->dim() != 4 || x[i]->sizes() != x[0]->sizes() || x[i]->scalar_type() != x[0]->scalar_type() ||
+            x[i]->device() != x[0]->device() || x[i]->stride(3) != 1)
+            return none();
+    }
+    auto tag = [](at::ScalarType t) { return t == at::kFloat ? SJVP_FP32 : t == at::kBFloat16 ? SJVP_BF16 : t == at::kHalf ? SJVP_FP16 : -1; };
+    const at::ScalarType from = x[0]->scalar_type(), to = a[3] == Py_None ? from : reinterpret_cast<THPDtype*>(a[3])->scalar_type;
+    const int64_t B = x[0]->size(0), S = x[0]->size(1), H = x[0]->size(2), D = x[0]->size(3);
+    if (tag(from) < 0 || tag(to) < 0 || B < 1 || S < 1 || H < 1 || D < 1 || B > INT_MAX || S > INT_MAX || H > INT_MAX || D > INT_MAX)
+        return none();
+    const Tensor *cos = nullptr, *sin = nullptr;
+    if (a[1] != Py_None || a[2] != Py_None) {
+        cos = plain(a[1]);
+        sin = plain(a[2]);
+        if (!cos || !sin || cos->dim() != 2 || cos->sizes() != sin->sizes() || cos->size(0) < S || 2 * cos->size(1) > D ||
+            cos->stride(0) != sin->stride(0))
+            return none();
+        for (const Tensor* t : {cos, sin})
+            if (t->scalar_type() != at::kFloat || t->device() != x[0]->device() || t->stride(1) != 1) return none();
+    }
+    Tensor made[kMost];
+    int rc;
+    {
+        pybind11::gil_scoped_release no_gil;
+        const void* in[kMost];
+        void* out[kMost];
+        int64_t strides[6 * kMost];  // of [B,H,S,D], inputs and results in turn
+        for (Py_ssize_t i = 0; i < count; ++i) {
+            made[i] = at::empty({B, S, H, D}, x[0]->options().dtype(to));
+            in[i] = x[i]->const_data_ptr();
+            out[i] = made[i].mutable_data_ptr();
+            int64_t* at = strides + 6 * i;
+            for (const Tensor* t : {x[i], static_cast<const Tensor*>(&made[i])}) {
+                *at++ = t->stride(0);
+                *at++ = t->stride(2);
+                *at++ = t->stride(1);
+            }
+        }
+        const c10::DeviceGuard guard(x[0]->device());
+        rc = abi.rope(static_cast<int>(count), in, out, strides, cos ? cos->const_data_ptr<float>() : nullptr,
+                      sin ? sin->const_data_ptr<float>() : nullptr, cos ? cos->stride(0) : 0, static_cast<int>(B),
+                      static_cast<int>(H), static_cast<int>(S), static_cast<int>(D), cos ? static_cast<int>(2 * cos->size(1)) : 0,
+                      tag(from), tag(to), a[4] == Py_True, c10::hip::getCurrentHIPStream(x[0]->device().index()).stream());
+    }
+    if (rc != SJVP_OK) return PyLong_FromLong(rc);
+    PyObject* res = PyTuple_New(count);
+    if (!res) return nullptr;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+        PyObject* item = THPVariable_Wrap(std::move(made[i]));
+        if (!item) {
+            Py_DECREF(res);
+            return nullptr;
+        }
+        PyTuple_SET_ITEM(res, i, item);
+    }
+    return res;
+    END_HANDLE_TH_ERRORS
+}
+
 // The pointer members of sjvp_adaln by the names of the tensors they take.
 struct AdaField {
     const char* name;
@@ -469,9 +540,9 @@ PyObject* gelu(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // bind(addresses of the entry points, in the order of Abi)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    constexpr int kEntries = 10;
+    constexpr int kEntries = 11;
     if (n != kEntries) {
-        PyErr_SetString(PyExc_TypeError, "bind() takes ten addresses");
+        PyErr_SetString(PyExc_TypeError, "bind() takes eleven addresses");
         return nullptr;
     }
     void* p[kEntries];
@@ -493,7 +564,8 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
            reinterpret_cast<decltype(abi.adaln_fwd)>(p[6]),
            reinterpret_cast<decltype(abi.adaln_bwd)>(p[7]),
            reinterpret_cast<decltype(abi.adaln_workspace_floats)>(p[8]),
-           reinterpret_cast<decltype(abi.gelu)>(p[9])};
+           reinterpret_cast<decltype(abi.gelu)>(p[9]),
+           reinterpret_cast<decltype(abi.rope)>(p[10])};
     return none();
 }
 
@@ -508,6 +580,7 @@ PyMethodDef methods[] = {
     {"cast", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(cast)), METH_FASTCALL, nullptr},
     {"adaln", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(adaln)), METH_FASTCALL, nullptr},
     {"gelu", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gelu)), METH_FASTCALL, nullptr},
+    {"rope", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(rope)), METH_FASTCALL, nullptr},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -250,22 +250,26 @@ class SDPASeqMajorFunction(torch.autograd.Function):
     """:class:`SDPAFusedFunction` on ``[B,S,H,D]`` tensors, for tensors below the forward-mode level (see
     :func:`_below_jvp`): the change of axes, and the casts to the dtype ``compute`` and back, happen in here, where they
     leave no autograd nodes.  With ``compute`` only its copies are kept for the backward: the caller may write to its
-    own tensors and to the result."""
+    own tensors and to the result.  With ``apart`` the rotation by ``cos``, ``sin`` is a launch of its own in front of the
+    attention kernels (and behind them in reverse mode) instead of folded into them; the rotated tensors are what is kept."""
 
     @staticmethod
-    def forward(ctx, q, k, v, t_q, t_k, t_v, arith, cos, sin, compute):
-        ctx.rope = None if cos is None else (cos, sin)
-        ctx.arith, ctx.compute = arith, compute
+    def forward(ctx, q, k, v, t_q, t_k, t_v, arith, cos, sin, compute, apart=False):
+        ctx.rope = None if cos is None or apart else (cos, sin)
+        ctx.arith, ctx.compute, ctx.apart = arith, compute, apart
         given = (q, k, v, t_q, t_k, t_v)
         ctx.dtypes = [t.dtype for t in given]
         if compute is not None:
             given = _cast_all(given, (compute,) * 6)
+        if apart:
+            q, k, t_q, t_k = kernels.rotary_embedding((q, k, t_q, t_k), cos, sin)
+            given = (q, k, v, t_q, t_k, t_v)
         B, S, H, _ = q.shape
         y, t_y = (torch.empty((B, S, H, v.shape[-1]), device=q.device, dtype=given[0].dtype) for _ in range(2))
         *inputs, o, to = (t.transpose(1, 2) for t in (*given, y, t_y))
         _, _, M, MU, _ = kernels.attention_jvp_forward(*inputs, o=o, to=to, with_li=False, arithmetic=arith,
                                                        rope=ctx.rope)
-        ctx.save_for_backward(*given, y, t_y, M, MU, *(ctx.rope or ()))
+        ctx.save_for_backward(*given, y, t_y, M, MU, *(() if cos is None else (cos, sin)))
         ctx.rope = ctx.rope is not None
         ctx.set_materialize_grads(False)
         return (y, t_y) if compute is None else tuple(_cast_all((y, t_y), (q.dtype,) * 2))
@@ -273,9 +277,10 @@ class SDPASeqMajorFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d_y, d_t_y):
         if d_y is None and d_t_y is None:
-            return (None,) * 10
+            return (None,) * 11
         *tensors, M, MU = ctx.saved_tensors[:10]
-        rope = ctx.saved_tensors[10:] if ctx.rope else None
+        tables = ctx.saved_tensors[10:]
+        rope = tables if ctx.rope else None
         with torch.no_grad():
             q, k, v, t_q, t_k, t_v, y, t_y = (t.transpose(1, 2) for t in tensors)
             if ctx.compute is not None:
@@ -283,8 +288,12 @@ class SDPASeqMajorFunction(torch.autograd.Function):
             d_y, d_t_y = (None if d is None else d.transpose(1, 2) for d in (d_y, d_t_y))
             grads = kernels.attention_jvp_backward(q, k, v, t_q, t_k, t_v, y, t_y, M, MU, dO=d_y, dTO=d_t_y,
                                                    arithmetic=ctx.arith, rope=rope)
-            grads = _cast_all([None if g is None else g.transpose(1, 2) for g in grads], ctx.dtypes)
-            return *grads, None, None, None, None
+            grads = [None if g is None else g.transpose(1, 2) for g in grads]
+            if ctx.apart:
+                turned = [i for i in (0, 1, 3, 4) if grads[i] is not None]
+                for i, g in zip(turned, kernels.rotary_embedding([grads[i] for i in turned], *tables, inverse=True)):
+                    grads[i] = g
+            return *_cast_all(grads, ctx.dtypes), None, None, None, None, None
 
 
 def _below_jvp(tensors):
@@ -336,12 +345,12 @@ def _sdpa_seq_major(q: Tensor, k: Tensor, v: Tensor, arith: Optional[str] = None
     return _seq_major_below(below, arith, cos, sin)
 
 
-def _seq_major_below(below, arith=None, cos=None, sin=None, compute=None) -> Tensor:
+def _seq_major_below(below, arith=None, cos=None, sin=None, compute=None, apart=False) -> Tensor:
     interpreter, duals = below
     with interpreter.lower():
         primals = [p for p, _ in duals]
         tangents = [torch.zeros_like(p) if t is None else t for p, t in duals]
-        y, t_y = SDPASeqMajorFunction.apply(*primals, *tangents, arith, cos, sin, compute)
+        y, t_y = SDPASeqMajorFunction.apply(*primals, *tangents, arith, cos, sin, compute, apart)
     return _dual_above(interpreter, y, t_y)
 
 
@@ -428,11 +437,15 @@ def safe_sdpa_jvp_rotary(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tens
         interpreter, duals = below
         with interpreter.lower():
             (qh, tq), (kh, tk), (vh, tv) = [[None if t is None else t.transpose(1, 2) for t in d] for d in duals]
-            fusable = not _functorch.is_functorch_wrapped_tensor(cos) \
-                and not _functorch.is_functorch_wrapped_tensor(sin) \
-                and kernels.rotary_fusable(qh, kh, cos, (vh, tq, tk, tv), sin=sin)
+            plain = not _functorch.is_functorch_wrapped_tensor(cos) and not _functorch.is_functorch_wrapped_tensor(sin)
+            fusable = plain and kernels.rotary_fusable(qh, kh, cos, (vh, tq, tk, tv), sin=sin)
         if fusable:
             return _seq_major_below(below, None, cos, sin)
+        if plain and q.dtype in (torch.bfloat16, torch.float16) and all(
+                z.dtype == q.dtype and z.ndim == 4 for pair in duals for z in pair if z is not None):
+            # The rotary launch below the level too: as a function of its own under the transform it goes through functorch's
+            # general dispatch three times (forward + backward at B=4 H=12 S=256 D=64 1160 us, here 427).
+            return _seq_major_below(below, None, cos, sin, apart=True)
     qh, kh, vh = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
     tangents = [fwAD.unpack_dual(t).tangent for t in (qh, kh, vh)]
     if AUTOGRAD_WIRING != "reference" and kernels.rotary_fusable(

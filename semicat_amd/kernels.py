@@ -468,6 +468,10 @@ def rotary_embedding(xs: Sequence[torch.Tensor], cos: Optional[torch.Tensor], si
     if not 1 <= len(xs) <= 4:
         raise ValueError("rotary_embedding takes one to four tensors")
     x0 = xs[0]
+    if _on_gpu(x0) and (out_dtype is None or isinstance(out_dtype, torch.dtype)):
+        res = _lib.host().rope(xs, cos, sin, out_dtype, bool(inverse))
+        if res is not None:
+            return _host_result(res)
     if not x0.is_cuda:
         raise RuntimeError("semicat_amd kernels run on an AMD GPU only; got a tensor on "
                            f"{x0.device} (there is no CPU fallback)")

@@ -116,8 +116,14 @@ def attention_jvp_backward(q, k, v, tq, tk, tv, o, to, lse, mu, dO=None, dTO=Non
     return grads
 
 
+def rotary_embedding(xs, cos, sin, out_dtype=None, inverse=False):
+    out = (_rot(x.detach().float().transpose(1, 2), (cos, sin), inverse).transpose(1, 2) for x in xs)
+    return tuple(y.to(out_dtype or x.dtype).contiguous() for x, y in zip(xs, out))
+
+
 def install(monkeypatch):
     import semicat_amd.kernels as K
     monkeypatch.setattr(K, "attention_jvp_forward", attention_jvp_forward)
     monkeypatch.setattr(K, "attention_forward", attention_forward)
     monkeypatch.setattr(K, "attention_jvp_backward", attention_jvp_backward)
+    monkeypatch.setattr(K, "rotary_embedding", rotary_embedding)

@@ -6,13 +6,13 @@ from semicat_amd import functional
 from tests import eager_backend
 
 
-def _run(x, g, wrapped, cot, grad_mode=True, hooks=None):
+def _run(x, g, wrapped, cot, grad_mode=True, hooks=None, op=None):
     """Outputs and gradients; ``wrapped`` says which of q, k, v carry a tangent (the others are constants)."""
     x = [t.detach().clone().requires_grad_() for t in x]
 
     def f(*dual):
         dual = iter(dual)
-        return functional.safe_sdpa_jvp(*[next(dual) if w else t for w, t in zip(wrapped, x[:3])])
+        return (op or functional.safe_sdpa_jvp)(*[next(dual) if w else t for w, t in zip(wrapped, x[:3])])
 
     primals = tuple(t for w, t in zip(wrapped, x[:3]) if w)
     tangents = tuple(t for w, t in zip(wrapped, x[3:]) if w)
@@ -96,3 +96,14 @@ def test_saved_tensor_hooks_and_no_grad(monkeypatch):
     assert packed
     y, ty = _both(monkeypatch, lambda: _run(x, g, (1, 1, 1), "both", grad_mode=False))
     assert not y.requires_grad and not ty.requires_grad
+
+
+@pytest.mark.parametrize("wrapped", [(1, 1, 1), (1, 0, 1), (0, 1, 0), (0, 0, 1)])
+@pytest.mark.parametrize("cot", ["both", "y", "ty"])
+@pytest.mark.parametrize("dtype,rot", [(torch.bfloat16, 16), (torch.float16, 8), (torch.float32, 16)])
+def test_rotation_in_front_of_the_kernels(monkeypatch, wrapped, cot, dtype, rot):
+    """Shapes that the folded rotation does not serve, a part of the head dimension rotated among them."""
+    eager_backend.install(monkeypatch)
+    x, g = _inputs(dtype)
+    cos, sin = torch.randn(2, 11, rot // 2, generator=torch.Generator().manual_seed(1))
+    _both(monkeypatch, lambda: _run(x, g, wrapped, cot, op=lambda q, k, v: functional.safe_sdpa_jvp_rotary(q, k, v, cos, sin)))

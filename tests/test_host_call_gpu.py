@@ -97,3 +97,16 @@ def test_refused_scales_and_expanded_inputs(monkeypatch):
     monkeypatch.setattr(kernels, "_on_gpu", lambda q: False)
     for a, b in zip(res, _step(x, True, True)):
         assert (a is None and b is None) or (torch.equal(a, b) and a.stride() == b.stride())
+
+
+@pytest.mark.parametrize("n,D,half,dtype,out_dtype,inverse", [
+    (4, 64, 32, torch.bfloat16, None, False), (2, 128, 32, torch.bfloat16, torch.float32, True),
+    (1, 20, 10, torch.float16, None, True), (3, 48, 0, torch.float32, torch.bfloat16, False)])
+def test_rotation_through_the_host_extension(monkeypatch, n, D, half, dtype, out_dtype, inverse):
+    fused = torch.randn(2, 33, n, 3, D, device="cuda").to(dtype)
+    xs = fused.unbind(2)
+    tables = (None, None) if half == 0 else tuple(torch.randn(40, 3 * half, device="cuda")[:, :half] for _ in range(2))
+    res = kernels.rotary_embedding(xs, *tables, out_dtype=out_dtype, inverse=inverse)
+    monkeypatch.setattr(kernels, "_on_gpu", lambda q: False)
+    for a, b in zip(res, kernels.rotary_embedding(xs, *tables, out_dtype=out_dtype, inverse=inverse), strict=True):
+        assert torch.equal(a, b) and a.stride() == b.stride() and a.dtype == b.dtype
