@@ -124,8 +124,8 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     } else {
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
-            const int64_t qrow = wrow + 16 * u + n;
-            const bool qvalid = qrow < p.Lq;
+            const bool qvalid = wrow + 16 * u + n < p.Lq;
+            const int64_t qrow = IO == kIoAny ? own_row(wrow + 16 * u + n, p.Lq) : wrow + 16 * u + n;
             load_b_operands16<T, HD, IO, true>(qB[u], p.q.head(b, h) + qrow * p.q.sl, g, p.D, qvalid);
             if constexpr (!SECOND) load_b_operands16<T, HD, IO, true>(oR[u], p.o.head(b, h) + qrow * p.o.sl, g, p.D, qvalid);
             if constexpr (HAS_G) {
@@ -177,6 +177,20 @@ __device__ __forceinline__ void bwd_row16_body(const BwdParams p, const int bloc
     // outstanding (the compiler cannot tell them from the stage copies), so the later stages are issued once
     // the own rows are in registers and land under the first stage's arithmetic.
     issue_step();
+    if constexpr (IO == kIoAny) {
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const bool qvalid = wrow + 16 * u + n < p.Lq;
+            finish_b_operands16<HD, IO>(qB[u], g, p.D, qvalid);
+            if constexpr (!SECOND) finish_b_operands16<HD, IO>(oR[u], g, p.D, qvalid);
+            if constexpr (HAS_G) {
+                finish_b_operands16<HD, IO>(tqB[u], g, p.D, qvalid);
+                finish_b_operands16<HD, IO>(gB[u], g, p.D, qvalid);
+                if constexpr (!SECOND) finish_b_operands16<HD, IO>(toR[u], g, p.D, qvalid);
+            }
+            if constexpr (HAS_DO) finish_b_operands16<HD, IO>(doB[u], g, p.D, qvalid);
+        }
+    }
     // The own rows as whole pieces, behind the copies: used by their elements alone (the row sums below), a piece is joined
     // element by element where the two paths above meet, and an element that changes its register there is awaited in front
     // of the copies (D = 128, 1476 queries on 10 keys, cotangent on TO: 372 us against 331).
@@ -605,8 +619,8 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
     } else {
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
-            const int64_t krow = wrow + 16 * u + n;
-            const bool kvalid = krow < p.Lk;
+            const bool kvalid = wrow + 16 * u + n < p.Lk;
+            const int64_t krow = IO == kIoAny ? own_row(wrow + 16 * u + n, p.Lk) : wrow + 16 * u + n;
             load_b_operands16<T, HD, IO>(kB[u], p.k.head(b, h) + krow * p.k.sl, g, p.D, kvalid);
             load_b_operands16<T, HD, IO>(vB[u], p.v.head(b, h) + krow * p.v.sl, g, p.D, kvalid);
             if constexpr (HAS_G) {
@@ -615,6 +629,16 @@ __device__ __forceinline__ void bwd_col16_body(const BwdParams p, const int bloc
             }
         }
         begin_copies();
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const bool kvalid = wrow + 16 * u + n < p.Lk;
+            finish_b_operands16<HD, IO>(kB[u], g, p.D, kvalid);
+            finish_b_operands16<HD, IO>(vB[u], g, p.D, kvalid);
+            if constexpr (HAS_G) {
+                finish_b_operands16<HD, IO>(tkB[u], g, p.D, kvalid);
+                finish_b_operands16<HD, IO>(tvB[u], g, p.D, kvalid);
+            }
+        }
     }
 #pragma unroll
     for (int u = 0; u < NC; ++u)
@@ -971,13 +995,20 @@ __device__ __forceinline__ void bwd_col16p_body(const BwdParams p, const int blo
         }
         begin_copies();
     } else {
-        load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + (int64_t)krow * p.k.sl, g, p.D, kvalid);
-        load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + (int64_t)krow * p.v.sl, g, p.D, kvalid);
+        const int64_t row = IO == kIoAny ? own_row(krow, p.Lk) : krow;
+        load_b_operands16<T, HD, IO>(kB, p.k.head(b, h) + row * p.k.sl, g, p.D, kvalid);
+        load_b_operands16<T, HD, IO>(vB, p.v.head(b, h) + row * p.v.sl, g, p.D, kvalid);
         if constexpr (HAS_G) {
-            load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + (int64_t)krow * p.tk.sl, g, p.D, kvalid);
-            load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + (int64_t)krow * p.tv.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tkB, p.tk.head(b, h) + row * p.tk.sl, g, p.D, kvalid);
+            load_b_operands16<T, HD, IO>(tvB, p.tv.head(b, h) + row * p.tv.sl, g, p.D, kvalid);
         }
         begin_copies();
+        finish_b_operands16<HD, IO>(kB, g, p.D, kvalid);
+        finish_b_operands16<HD, IO>(vB, g, p.D, kvalid);
+        if constexpr (HAS_G) {
+            finish_b_operands16<HD, IO>(tkB, g, p.D, kvalid);
+            finish_b_operands16<HD, IO>(tvB, g, p.D, kvalid);
+        }
     }
 #pragma unroll
     for (int c = 0; c < KC; ++c) {  // the own rows are awaited here

@@ -92,10 +92,10 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
     if constexpr (!OWN_LDS) {
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
-            const int qrow = wrow + 16 * u + n;
-            load_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + (int64_t)qrow * p.q.sl, g, p.D, qrow < p.Lq);
-            if constexpr (JVP)
-                load_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + (int64_t)qrow * p.tq.sl, g, p.D, qrow < p.Lq);
+            const bool qvalid = wrow + 16 * u + n < p.Lq;
+            const int64_t qrow = IO == kIoAny ? own_row(wrow + 16 * u + n, p.Lq) : wrow + 16 * u + n;
+            load_b_operands16<T, HD, IO>(qB[u], p.q.head(b, h) + qrow * p.q.sl, g, p.D, qvalid);
+            if constexpr (JVP) load_b_operands16<T, HD, IO>(tqB[u], p.tq.head(b, h) + qrow * p.tq.sl, g, p.D, qvalid);
         }
     }
     if constexpr (DMA) {
@@ -158,6 +158,12 @@ __global__ __launch_bounds__(kThreads16 / NC, OCC) void fwd16_kernel(const FwdPa
         while (issued < (SPB == 2 ? 2 : R) && issued < ns) issue_next();
     } else {
         stage_step(0);
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            const bool qvalid = wrow + 16 * u + n < p.Lq;
+            finish_b_operands16<HD, IO>(qB[u], g, p.D, qvalid);
+            if constexpr (JVP) finish_b_operands16<HD, IO>(tqB[u], g, p.D, qvalid);
+        }
         commit_step();
         // The own rows are awaited here, once: left to their first use, the wait stands inside the loop and takes the next
         // stage's copies with it (B=50 H=10 L=292, D = 21 44 -> 48 us, D = 36 70 -> 73.5).

@@ -59,7 +59,7 @@ __device__ __forceinline__ u32x4 shift_down(u32x4 v, int s) {
     return v;
 }
 
-// B operands (all head-dimension chunks of 32) of one owned row.
+// B operands (all head-dimension chunks of 32) of one owned row of fp32 elements.
 template <typename T, int HD, int IO>
 __device__ __forceinline__ void staged_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
     Raw8<IO> raw[HD / 32];
@@ -72,6 +72,21 @@ __device__ __forceinline__ void staged_b_operands16(u32x4* out, const elem_t* ro
     for (int c = 0; c < HD / 32; ++c) {
         out[c] = raw[c].template get<T>();
         if (D != HD) out[c] = shift_down(out[c], piece_shift(32 * c + 8 * g, D));
+    }
+}
+// 16-bit rows of any alignment: the pieces are requested here, as they lie in a row that exists (own_row), and made operands by
+// finish_b_operands16 once all of a wave's rows have been requested.  Made operands one row after the other, each row is
+// awaited before the next is requested: forward + backward, in turn / together, B=8 H=8 L=300 D=36 56.7 / 54.0 us, B=64 H=12 L=128
+// D=20 61.9 / 56.5, B=100 H=9 30 x 20 D=36 72.0 / 62.3, B=8 H=16 L=512 D=100 354 / 337.
+__device__ __forceinline__ int64_t own_row(int64_t row, int L) { return row < L ? row : L - 1; }
+template <int HD, int IO>
+__device__ __forceinline__ void finish_b_operands16(u32x4* out, int g, int D, bool valid) {
+    if constexpr (IO == kIoAny) {
+#pragma unroll
+        for (int c = 0; c < HD / 32; ++c) {
+            if (D != HD) out[c] = shift_down(out[c], piece_shift(32 * c + 8 * g, D));
+            if (!valid) out[c] = u32x4{0u, 0u, 0u, 0u};
+        }
     }
 }
 
@@ -163,13 +178,18 @@ struct StagedPlan {
     }
 };
 
-// B operands (all head-dimension chunks of 32) of one owned row, straight from global memory.
+// B operands (all head-dimension chunks of 32) of one owned row, straight from global memory (kIoAny: own_row of it, to be finished).
 // (GROUPED: the zeros come as one register group.  Joined with the loaded piece element by element, as the compiler may do, the
 // piece is awaited as soon as it is requested.  Row-owned kernel at D = 80, 1476 queries on 10 keys: 278 -> 245 us; the forward
 // of few workgroups, whose pieces were not affected, loses by it: 333 x 205, D = 48 8.9 -> 9.8 us.)
 template <typename T, int HD, int IO, bool GROUPED = false>
 __device__ __forceinline__ void load_b_operands16(u32x4* out, const elem_t* row, int g, int D, bool valid) {
-    if constexpr (IO != kIoDma) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
+    if constexpr (IO == kIoF32) return staged_b_operands16<T, HD, IO>(out, row, g, D, valid);
+    if constexpr (IO == kIoAny) {
+#pragma unroll
+        for (int c = 0; c < HD / 32; ++c) __builtin_memcpy(&out[c], row + piece_col(32 * c + 8 * g, D), sizeof(out[c]));
+        return;
+    }
 #pragma unroll
     for (int c = 0; c < HD / 32; ++c) {
         u32x4 piece = {0u, 0u, 0u, 0u};
