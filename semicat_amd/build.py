@@ -53,7 +53,7 @@ def hipcc_path() -> str:
 
 # Flags of the host extension (g++; the include and library folders of torch, ROCm and Python come on top).
 HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
-HOST_LIBS = ["-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+HOST_LIBS = ["-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10"]
 
 
 def _hash(what: str, paths) -> str:
