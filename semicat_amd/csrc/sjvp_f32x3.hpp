@@ -15,9 +15,9 @@
 // for the score-like tiles, transposing reads for the output ones); the owned side is split once, and each tile
 // once, before the output contractions that it enters.
 //
-// Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4464 / 2178 us (the matrix pipe busy
-// 52, 60 and 55 % of the forward's, row and column kernel's cycles), without tangents at B=8 H=8 L=512 337 / 165, B=64 H=12 L=128
-// D=64 519 / 316, B=8 H=12 L=500 D=32 568 / 268, B=8 H=16 L=512 D=128 2141 / 1868 (one wave per SIMD there, the column kernel left
+// Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4497 / 2198 us (the matrix pipe busy
+// 52, 60 and 55 % of the forward's, row and column kernel's cycles), without tangents at B=8 H=8 L=512 336 / 167, B=64 H=12 L=128
+// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2148 / 1873 (one wave per SIMD there, the column kernel left
 // on the fp32 unit).  What is left between the contractions is the split of the stage and of the tiles, softmax and barriers.
 // Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 5.4e-7.
 //
@@ -391,6 +391,10 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void fwd_f32x3_kern
         f32x4 s[2], ts[2];
         zero_tiles<2>(s);
         zero_tiles<2>(ts);
+        // the score contractions go first: a wave that is through with them has vector work that runs beside another's (row and
+        // column kernel, without / with: B=8 H=12 L=500 D=32 85 and 117 / 78 and 113 us, B=8 H=8 L=256 D=64 36.2 and 45.9 / 35.2 and
+        // 45.0, L=1024 688 and 957 / 685 and 944; the forward 68.0 / 67.6, 504 / 502)
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             const Op3 a0 = rows3<HD>(buf, 0, c, w.n, w.g), a1 = rows3<HD>(buf, 1, c, w.n, w.g);
@@ -400,6 +404,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void fwd_f32x3_kern
                 mfma6(rows3<HD>(buf + 6 * SE, 0, c, w.n, w.g), q[c], ts[0], rows3<HD>(buf + 6 * SE, 1, c, w.n, w.g), q[c], ts[1]);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         s[0] *= sl2;
         s[1] *= sl2;
         if (k0 + kStageRows > p.Lk) {  // wave-uniform
@@ -540,6 +545,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
         zero_tiles<2>(ts);
         zero_tiles<2>(wt);
         zero_tiles<2>(xy);
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             auto rows = [&](int tensor, int t) { return rows3<HD>(buf + 3 * tensor * SE, t, c, w.n, w.g); };
@@ -556,6 +562,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
                 mfma6(rows(3, 0), g[c], xy[0], rows(3, 1), g[c], xy[1]);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         f32x4 ds[2], dts[2];
         zero_tiles<2>(dts);
 #pragma unroll
@@ -661,6 +668,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
         zero_tiles<2>(ts);
         zero_tiles<2>(wt);
         zero_tiles<2>(xy);
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
             auto rows = [&](int slab, int t) { return rows3<HD>(buf + slab * SE, t, c, w.n, w.g); };
@@ -677,6 +685,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             }
             if constexpr (HAS_DO && DK) mfma6(rows(kDo, 0), v[c], xy[0], rows(kDo, 1), v[c], xy[1]);
         }
+        __builtin_amdgcn_s_setprio(0);
         f32x4 pr[2], pn[2], ds[2], dts[2];
         zero_tiles<2>(pn);
         zero_tiles<2>(dts);
