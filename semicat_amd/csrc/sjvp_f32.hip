@@ -31,9 +31,8 @@ inline int split(int BH, int rows, int streamed) {
 // A launch costs rounds of workgroups times streamed tiles; per tile, in fortieths of what a round of the fp32 unit's whole
 // groups takes: 28 (four waves; D > 64: 32) or 37 (eight), the forward without tangents 40 and 50; the fp32 unit's 40, 13 for each
 // round of split groups.  Both sides in us, fp32 unit / here, L = 256: D = 64 512 groups 26 / 27 forward, 37 / 34 row, 40 / 44 column;
-// 640 31 / 26, 54 / 33, 59 / 41; 4096 142 / 78, 201 / 105, 250 / 139; D = 80 640 62 / 48, 90 / 58, 113 / 100; D = 32 without
-// tangents, forward, 640 9.0 / 11.2, 2048 17 / 13.  The column launch with tangents has no registers for it beyond D = 96 (its
-// two passes: 1024 groups 118 / 127, 4096 485 / 530).
+// 640 31 / 26, 54 / 33, 59 / 41; 4096 142 / 78, 201 / 105, 250 / 139; D = 80 640 62 / 50, 90 / 60, 113 / 57; D = 128
+// 448 44 / 51, 70 / 70, 73 / 71, 576 64 / 53, 104 / 70, 108 / 72; D = 32 without tangents, forward, 640 9.0 / 11.2, 2048 17 / 13.
 inline int x3_waves(int BH, int groups_of, int rows, int streamed, int D, bool forward, bool tangents, int split) {
     const int units = compute_units();
     const int64_t four = (int64_t)BH * ((rows + 63) / 64), eight = (int64_t)BH * ((rows + 127) / 128);
@@ -76,7 +75,7 @@ int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
 template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int col_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lk, p.Lq);
-    if (const int waves = HAS_G && p.D > 96 ? 0 : x3_waves(BH, p.Lk, p.Lk, p.Lq, p.D, false, HAS_G, sp))
+    if (const int waves = x3_waves(BH, p.Lk, p.Lk, p.Lq, p.D, false, HAS_G, sp))
         return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_COL, waves, stream);
     p.k_blocks = blocks(p.Lk, sp);
     const int grid = BH * p.k_blocks;

@@ -22,14 +22,12 @@ int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
 
 template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW>
 int col_one(BwdParamsF32 p, int BH, hipStream_t stream) {
-    p.k_blocks = (p.Lk + 16 * NW - 1) / (16 * NW);
-    const int grid = BH * p.k_blocks;
-    constexpr int smem = TriSmem<HD, HAS_G ? (HAS_DO ? 4 : 3) : 2>::bytes;
     if constexpr (HD == 128 && HAS_G) {
-        const int rc = launch(bwd_col_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW, 1>, grid, smem, stream, p, 64 * NW);
-        return rc != SJVP_OK ? rc : launch(bwd_col_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW, 2>, grid, smem, stream, p, 64 * NW);
+        p.k_blocks = (p.Lk + 16 * kPairs - 1) / (16 * kPairs);
+        return launch(bwd_col_f32x3_pair_kernel<HD, DT, HAS_DO>, BH * p.k_blocks, pair_smem<HD, HAS_DO ? 4 : 3>(), stream, p, 128 * kPairs);
     } else {
-        return launch(bwd_col_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW, 3>, grid, smem, stream, p, 64 * NW);
+        p.k_blocks = (p.Lk + 16 * NW - 1) / (16 * NW);
+        return launch(bwd_col_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW>, BH * p.k_blocks, TriSmem<HD, HAS_G ? (HAS_DO ? 4 : 3) : 2>::bytes, stream, p, 64 * NW);
     }
 }
 
@@ -73,8 +71,7 @@ int bwd_f32x3(const BwdParamsF32& p, int BH, bool has_do, bool has_g, int part, 
             return by_waves<HD == 64 && G>(waves, [&](auto nw) {
                 constexpr int NW = decltype(nw)::value;
                 if (part == SJVP_BWD_ROW) return row_one<HD, DT, DO, G, NW>(p, BH, stream);
-                if constexpr (DT == 8 && G) return (int)SJVP_ERR_HEAD_DIM;  // not asked for (x3_waves)
-                else return col_one<HD, DT, DO, G, NW>(p, BH, stream);
+                return col_one<HD, DT, DO, G, NW>(p, BH, stream);
             });
         };
         if (has_do && has_g) return go(std::true_type{}, std::true_type{});

@@ -17,8 +17,8 @@
 //
 // Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4497 / 2198 us (the matrix pipe busy
 // 52, 60 and 55 % of the forward's, row and column kernel's cycles), without tangents at B=8 H=8 L=512 336 / 167, B=64 H=12 L=128
-// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2148 / 1873 (one wave per SIMD there, the column kernel left
-// on the fp32 unit).  What is left between the contractions is the split of the stage and of the tiles, softmax and barriers.
+// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2150 / 1546, B=4 H=16 300 queries
+// on 700 keys D=80 1057 / 759.  What is left between the contractions is the split of the stage and of the tiles, softmax and barriers.
 // Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 5.4e-7.
 //
 // Numbers that the split does not hold (infinities, NaN) or whose products could overflow one by one where their sum does
@@ -608,13 +608,9 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
 
 // ---------------------------------------------------------------------------------------------
 // Column-owned backward: dK, dV (, dK_dot, dV_dot).
-// PARTS: bit 0 the gradients of K, bit 1 those of V.  With four owned tensors in three parts and four accumulators a wave at
-// D > 64 has no registers left, so there each pair of gradients has a launch of its own, with 9 and 6 contractions where
-// one would have 12.
-template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW, int PARTS>
+template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW>
 __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_kernel(const BwdParamsF32 p) {
     constexpr int NS = HAS_G ? (HAS_DO ? 4 : 3) : 2, NT = 64 * NW, KC = (DT + 1) / 2, SE = Slab<HD>::elems;
-    constexpr bool DK = PARTS & 1, DV = PARTS & 2;
     // (the eight registers of the sums beside the accumulators are spilled where the wave has 256: 63 -> 73 us at B=64 L=256)
     constexpr bool ONTO = !(HD == 64 && HAS_G && NW == 8);
     // slabs: Q, then Q_dot, G (HAS_G), then dO (HAS_DO)
@@ -645,10 +641,10 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             own_split<KC>(to, x, sq);
         };
         fetch(k, k_own);
-        if constexpr (DK) fetch(v, v_own);
+        fetch(v, v_own);
         if constexpr (HAS_G) {
             fetch(tk, tk_own);
-            if constexpr (DK) fetch(tv, tv_own);
+            fetch(tv, tv_own);
         }
         met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
     }
@@ -677,13 +673,11 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             if constexpr (HAS_G) {
                 mfma6(a0, tk[c], ts[0], a1, tk[c], ts[1]);
                 mfma6(rows(kTq, 0), k[c], ts[0], rows(kTq, 1), k[c], ts[1]);
-                if constexpr (DK) {
-                    const Op3 g0 = rows(kG, 0), g1 = rows(kG, 1);
-                    mfma6(g0, v[c], wt[0], g1, v[c], wt[1]);
-                    mfma6(g0, tv[c], xy[0], g1, tv[c], xy[1]);
-                }
+                const Op3 g0 = rows(kG, 0), g1 = rows(kG, 1);
+                mfma6(g0, v[c], wt[0], g1, v[c], wt[1]);
+                mfma6(g0, tv[c], xy[0], g1, tv[c], xy[1]);
             }
-            if constexpr (HAS_DO && DK) mfma6(rows(kDo, 0), v[c], xy[0], rows(kDo, 1), v[c], xy[1]);
+            if constexpr (HAS_DO) mfma6(rows(kDo, 0), v[c], xy[0], rows(kDo, 1), v[c], xy[1]);
         }
         __builtin_amdgcn_s_setprio(0);
         f32x4 pr[2], pn[2], ds[2], dts[2];
@@ -725,7 +719,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             }
         }
         float sq = 0.f;
-        if constexpr (DK) {
+        {
             const Op3 dsb = split_tiles(ds[0], ds[1], sq);
             Op3 dtsb;
             if constexpr (HAS_G) dtsb = split_tiles(dts[0], dts[1], sq);
@@ -736,7 +730,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
                 tri_out<HD, DT>(buf, w.lane, dsb, dk);
             }
         }
-        if constexpr (DV) {
+        {
             const Op3 prb = split_tiles(pr[0], pr[1], sq);
             Op3 pnb;
             if constexpr (HAS_G) pnb = split_tiles(pn[0], pn[1], sq);
@@ -747,10 +741,215 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
     });
     if (!active) return;
     if (__builtin_expect(met, 0)) return bwd_col_f32_wave<HD, HAS_DO, HAS_G, 1, kColumnsCut>(p, w, nullptr);
-    if constexpr (DK) tri_store<DT>(p.dk.head(w.b, w.h) + (int64_t)krow * p.dk.sl, dk, p.scale, p.D, w.g, kvalid);
-    if constexpr (DV) tri_store<DT>(p.dv.head(w.b, w.h) + (int64_t)krow * p.dv.sl, dv, 1.0f, p.D, w.g, kvalid);
-    if constexpr (HAS_G && DK) tri_store<DT>(p.dtk.head(w.b, w.h) + (int64_t)krow * p.dtk.sl, dtk, p.scale, p.D, w.g, kvalid);
-    if constexpr (HAS_G && DV) tri_store<DT>(p.dtv.head(w.b, w.h) + (int64_t)krow * p.dtv.sl, dtv, 1.0f, p.D, w.g, kvalid);
+    tri_store<DT>(p.dk.head(w.b, w.h) + (int64_t)krow * p.dk.sl, dk, p.scale, p.D, w.g, kvalid);
+    tri_store<DT>(p.dv.head(w.b, w.h) + (int64_t)krow * p.dv.sl, dv, 1.0f, p.D, w.g, kvalid);
+    if constexpr (HAS_G) {
+        tri_store<DT>(p.dtk.head(w.b, w.h) + (int64_t)krow * p.dtk.sl, dtk, p.scale, p.D, w.g, kvalid);
+        tri_store<DT>(p.dtv.head(w.b, w.h) + (int64_t)krow * p.dtv.sl, dtv, 1.0f, p.D, w.g, kvalid);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same with tangents at D > 64, by pairs of waves: four owned tensors in three parts and four accumulators are more registers
+// than a wave has.  One wave owns k, k_dot and the gradients of them, the other v, v_dot and theirs, of the same 16 rows; each
+// forms the scores of its own tensors, they exchange what the other one's element-wise part needs through LDS, and each enters
+// its own output contractions: three and three of both, nothing twice, in half the registers, so that a SIMD has two waves.
+// Against the fp32 unit (D > 96) and two launches of 9 and 6 contractions, one for each half: B=8 H=16 L=512 D=128 887 -> 564 us,
+// B=8 H=12 L=500 D=96 594 -> 319, B=4 H=16 L=512 D=80 397 -> 212.
+// With o, o_dot the owned pair, y1, y2 the streamed one (q, q_dot or dO_dot, dO) and t1, t2 the tiles (dS_dot, dS or P, P_dot), both waves do
+//     x1 = y1 o, x2 = y1 o_dot + y2 o;   d(o_dot) = t1^T y1, d(o) = t2^T y1 + t1^T y2.
+constexpr int kPairs = 4;  // of a workgroup: 64 owned rows
+template <int HD, int NS>
+constexpr int pair_smem() { return TriSmem<HD, NS>::bytes + kPairs * 2 * 4 * 64 * (int)sizeof(f32x4); }
+
+// The two gradients of a wave on the fp32 unit, its operands read where they are used: for the wave's few registers, and for the
+// rows whose numbers the split does not hold.
+template <int HD, bool HAS_DO>
+__device__ __forceinline__ void bwd_col_f32_half(const BwdParamsF32& p, const F32Place& w, int role) {
+    constexpr int M = HD / 16, T = F32Cols<HD>::tiles;
+    const int krow = w.row0 + w.n;
+    const bool kvalid = krow < p.Lk;
+    f32x4 acc[T], tacc[T];
+    zero_tiles<T>(acc);
+    zero_tiles<T>(tacc);
+    const int64_t so = (int64_t)w.bh * p.Lr + 4 * w.g;
+#pragma unroll 1
+    for (int q0 = 0; q0 < p.Lq; q0 += kF32Rows) {
+        int own_row = krow;  // read anew for every tile: kept through the loop, the owned rows are more registers than there are
+        asm volatile("" : "+v"(own_row));
+        auto dot = [&](const F32In& rows, const F32In& own) {
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 a[M], b[M], c = {0.f, 0.f, 0.f, 0.f};
+            f32_load_own<HD, false, true>(a, rows.head(w.b, w.h), rows.sl, q0 + w.n, p.Lq, p.D, w.g);
+            f32_load_own<HD, false, true>(b, own.head(w.b, w.h), own.sl, own_row, p.Lk, p.D, w.g);
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c = mfma_f32(a[m][e], b[m][e], c);
+            return c;
+        };
+        const f32x4 s = dot(p.q, p.k), ts = dot(p.tq, p.k) + dot(p.q, p.tk);
+        f32x4 wt = {0.f, 0.f, 0.f, 0.f}, xy = wt, t1, t2;
+        if (role == 0) {
+            wt = dot(p.dTO, p.v);
+            xy = dot(p.dTO, p.tv);
+            if constexpr (HAS_DO) xy = dot(p.dO, p.v) + xy;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t at = so + q0 + j;
+            const float pj = kvalid ? fast_exp2(fmaf(s[j], p.scale * kLog2e, -p.lse2[at])) : 0.f;
+            const float nn = fmaf(ts[j], p.scale, -p.mu[at]), dts = pj * (wt[j] - p.s4[at]);
+            t1[j] = role ? pj : dts;
+            t2[j] = role ? pj * nn : fmaf(dts, nn, pj * (xy[j] - p.s7d[at]));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = q0 + 4 * w.g + j;
+            const bool qvalid = row < p.Lq;
+            t1[j] = qvalid ? t1[j] : 0.f;
+            t2[j] = qvalid ? t2[j] : 0.f;
+            float y[T];
+            auto cols = [&](const F32In& x) {
+                __builtin_amdgcn_sched_barrier(0);
+                f32_load_cols<HD, false, true>(y, x.head(w.b, w.h), x.sl, row, p.Lq, p.D, w.n);
+                f32_cut_cols<HD, false, true>(y, p.D, w.n);
+                f32_zero_unless<T>(y, qvalid);
+            };
+            if (role) cols(p.dTO);
+            else cols(p.q);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                acc[t] = mfma_f32(y[t], t2[j], acc[t]);
+                tacc[t] = mfma_f32(y[t], t1[j], tacc[t]);
+            }
+            if (HAS_DO || role == 0) {
+                if (role) cols(p.dO);
+                else cols(p.tq);
+#pragma unroll
+                for (int t = 0; t < T; ++t) acc[t] = mfma_f32(y[t], t1[j], acc[t]);
+            }
+        }
+    }
+    const F32Out &d = role ? p.dv : p.dk, &td = role ? p.dtv : p.dtk;
+    const float mul = role ? 1.0f : p.scale;
+    f32_store<HD, false, 1>(nullptr, d.head(w.b, w.h) + (int64_t)krow * d.sl, acc, mul, w, p.D, kvalid);
+    f32_store<HD, false, 1>(nullptr, td.head(w.b, w.h) + (int64_t)krow * td.sl, tacc, mul, w, p.D, kvalid);
+}
+
+template <int HD, int DT, bool HAS_DO>
+__global__ __launch_bounds__(128 * kPairs, 2) void bwd_col_f32x3_pair_kernel(const BwdParamsF32 p) {
+    constexpr int NS = HAS_DO ? 4 : 3, NT = 128 * kPairs, KC = (DT + 1) / 2, SE = Slab<HD>::elems;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    F32Place w = tri_place<kPairs>(p.k_blocks, p.H);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), role = wave / kPairs;  // 0: k, 1: v
+    w.row0 -= role * 16 * kPairs;
+    f32x4* exchange = reinterpret_cast<f32x4*>(smem_raw + TriSmem<HD, NS>::bytes) + (wave % kPairs) * 512 + w.lane;
+    f32x4 *mine = exchange + 256 * role, *other = exchange + 256 * (1 - role);
+    const int krow = w.row0 + w.n;
+    const bool kvalid = krow < p.Lk, active = w.row0 < p.Lk;
+    TriPlan<HD, NS, NT> plan;
+    {
+        auto src = [&](const F32In& t) { return Src32{t.head(w.b, w.h), t.sl}; };
+        if constexpr (HAS_DO) plan.init(threadIdx.x, p.D, src(p.q), src(p.tq), src(p.dTO), src(p.dO));
+        else plan.init(threadIdx.x, p.D, src(p.q), src(p.tq), src(p.dTO));
+    }
+    Op3 own[KC], town[KC];
+    bool met;  // an element for the fp32 unit (wave-uniform)
+    {
+        F32x8 x[KC];
+        float sq = 0.f;
+        auto fetch = [&](Op3* to, const F32In& t) {
+            own_load<KC>(x, t.head(w.b, w.h) + (int64_t)krow * t.sl, w.g, p.D, kvalid);
+            own_cut<KC>(x, w.g, p.D);
+            own_split<KC>(to, x, sq);
+        };
+        fetch(own, role ? p.v : p.k);
+        fetch(town, role ? p.tv : p.tk);
+        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+    }
+    f32x4 acc[DT], tacc[DT];
+    zero_tiles<DT>(acc);
+    zero_tiles<DT>(tacc);
+    const int64_t so = (int64_t)w.bh * p.Lr + 4 * w.g;  // rows below Lr exist in every statistic
+    const float sl2 = p.scale * kLog2e;
+
+    tri_walk<HD, NS, NT>(smem_raw, plan, p.Lq, [&](const elem_t* buf, int q0, bool stage_special) {
+        met = met || stage_special;
+        const elem_t *y1 = buf + role * 6 * SE, *y2 = y1 + 3 * SE;
+        const bool has_y2 = HAS_DO || role == 0;
+        f32x4 x1[2], x2[2];
+        zero_tiles<2>(x1);
+        zero_tiles<2>(x2);
+        if (active) {
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int c = 0; c < KC; ++c) {
+                const Op3 a0 = rows3<HD>(y1, 0, c, w.n, w.g), a1 = rows3<HD>(y1, 1, c, w.n, w.g);
+                mfma6(a0, own[c], x1[0], a1, own[c], x1[1]);
+                mfma6(a0, town[c], x2[0], a1, town[c], x2[1]);
+                if (has_y2) mfma6(rows3<HD>(y2, 0, c, w.n, w.g), own[c], x2[0], rows3<HD>(y2, 1, c, w.n, w.g), own[c], x2[1]);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            // x1, x2 become P and N, or W - s4 and XY - s7d; what the other wave needs of them goes to it
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int64_t at = so + q0 + 16 * t;
+                const f32x4 c1 = *reinterpret_cast<const f32x4*>((role ? p.s4 : p.lse2) + at);
+                const f32x4 c2 = *reinterpret_cast<const f32x4*>((role ? p.s7d : p.mu) + at);
+                f32x4 second;
+                if (role == 0) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        // a key or a query that does not exist contributes nothing
+                        const bool valid = kvalid && q0 + 16 * t + 4 * w.g + j < p.Lq;
+                        const float pj = valid ? fast_exp2(fmaf(x1[t][j], sl2, -c1[j])) : 0.f;
+                        const float nn = fmaf(x2[t][j], p.scale, -c2[j]);
+                        x1[t][j] = pj;
+                        x2[t][j] = nn;
+                        second[j] = valid ? pj * nn : 0.f;
+                    }
+                } else {
+                    x1[t] -= c1;
+                    x2[t] -= c2;
+                    second = x2[t];
+                }
+                mine[64 * t] = x1[t];
+                mine[64 * (2 + t)] = second;
+            }
+        }
+        workgroup_barrier();
+        if (!active) return;
+        f32x4 t1[2], t2[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            t1[t] = other[64 * t];
+            t2[t] = other[64 * (2 + t)];
+            if (role == 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool valid = kvalid && q0 + 16 * t + 4 * w.g + j < p.Lq;
+                    const float dts = x1[t][j] * t1[t][j], ds = fmaf(dts, x2[t][j], x1[t][j] * t2[t][j]);
+                    t1[t][j] = valid ? dts : 0.f;
+                    t2[t][j] = valid ? ds : 0.f;
+                }
+        }
+        float sq = 0.f;
+        const Op3 b1 = split_tiles(t1[0], t1[1], sq), b2 = split_tiles(t2[0], t2[1], sq);
+        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        tri_out<HD, DT>(y1, w.lane, b2, acc, b1, tacc);
+        if (has_y2) tri_out<HD, DT>(y2, w.lane, b1, acc);
+    });
+    volatile int* flag = reinterpret_cast<volatile int*>(smem_raw + TriSmem<HD, NS>::bytes);
+    workgroup_barrier();  // the last stage's tiles are read
+    if (w.lane == 0) flag[wave] = met;
+    workgroup_barrier();
+    if (!active) return;
+    if (__builtin_expect(met || __builtin_amdgcn_readfirstlane(flag[wave ^ kPairs]) != 0, 0)) return bwd_col_f32_half<HD, HAS_DO>(p, w, role);
+    const F32Out &d = role ? p.dv : p.dk, &td = role ? p.dtv : p.dtk;
+    const float mul = role ? 1.0f : p.scale;
+    tri_store<DT>(d.head(w.b, w.h) + (int64_t)krow * d.sl, acc, mul, p.D, w.g, kvalid);
+    tri_store<DT>(td.head(w.b, w.h) + (int64_t)krow * td.sl, tacc, mul, p.D, w.g, kvalid);
 }
 
 }  // namespace sjvp
