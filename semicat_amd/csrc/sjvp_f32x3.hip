@@ -16,8 +16,13 @@ int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
 
 template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW>
 int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
-    p.q_blocks = (p.Lq + 16 * NW - 1) / (16 * NW);
-    return launch(bwd_row_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW>, BH * p.q_blocks, TriSmem<HD, HAS_G ? 4 : 2>::bytes, stream, p, 64 * NW);
+    if constexpr (HD == 128 && HAS_G) {
+        p.q_blocks = (p.Lq + 16 * kPairs - 1) / (16 * kPairs);
+        return launch(bwd_row_f32x3_pair_kernel<HD, DT, HAS_DO>, BH * p.q_blocks, pair_smem<HD, 4>(), stream, p, 128 * kPairs);
+    } else {
+        p.q_blocks = (p.Lq + 16 * NW - 1) / (16 * NW);
+        return launch(bwd_row_f32x3_kernel<HD, DT, HAS_DO, HAS_G, NW>, BH * p.q_blocks, TriSmem<HD, HAS_G ? 4 : 2>::bytes, stream, p, 64 * NW);
+    }
 }
 
 template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW>

@@ -17,8 +17,9 @@
 //
 // Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4497 / 2198 us (the matrix pipe busy
 // 52, 60 and 55 % of the forward's, row and column kernel's cycles), without tangents at B=8 H=8 L=512 336 / 167, B=64 H=12 L=128
-// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2150 / 1546, B=4 H=16 300 queries
-// on 700 keys D=80 1057 / 759.  What is left between the contractions is the split of the stage and of the tiles, softmax and barriers.
+// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2154 / 1475, B=8 H=12 L=500
+// D=96 1936 / 913, B=4 H=16 300 queries on 700 keys D=80 1059 / 724.  What is left between the contractions is the split of the
+// stage and of the tiles, softmax and barriers.
 // Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 5.4e-7.
 //
 // Numbers that the split does not hold (infinities, NaN) or whose products could overflow one by one where their sum does
@@ -229,23 +230,23 @@ __device__ __forceinline__ Op3 cols3(const elem_t* slabs, int d0, int lane) {
     return Op3{lds_a_tr16<HD>(slabs, d0, lane), lds_a_tr16<HD>(slabs + SE, d0, lane), lds_a_tr16<HD>(slabs + 2 * SE, d0, lane)};
 }
 
-// x[d] += Y'[d] tile, and z[d] += Y'[d] more.
+// x[d] += Y'[d] tile, and z[d] += Y'[d] more; tile d of the columns from `col` on.
 template <int HD, int DT, bool ONTO = true>
-__device__ __forceinline__ void tri_out(const elem_t* slabs, int lane, const Op3& tile, f32x4* x, const Op3& more, f32x4* z) {
+__device__ __forceinline__ void tri_out(const elem_t* slabs, int lane, const Op3& tile, f32x4* x, const Op3& more, f32x4* z, int col = 0) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-        const Op3 a = cols3<HD>(slabs, 16 * d, lane);
+        const Op3 a = cols3<HD>(slabs, col + 16 * d, lane);
         if constexpr (ONTO) mfma6_onto(a, tile, x[d], a, more, z[d]);
         else mfma6(a, tile, x[d], a, more, z[d]);
     }
 }
 template <int HD, int DT>
-__device__ __forceinline__ void tri_out(const elem_t* slabs, int lane, const Op3& tile, f32x4* x) {
+__device__ __forceinline__ void tri_out(const elem_t* slabs, int lane, const Op3& tile, f32x4* x, int col = 0) {
 #pragma unroll
     for (int d = 0; d + 1 < DT; d += 2)
-        mfma6_onto(cols3<HD>(slabs, 16 * d, lane), tile, x[d], cols3<HD>(slabs, 16 * d + 16, lane), tile, x[d + 1]);
+        mfma6_onto(cols3<HD>(slabs, col + 16 * d, lane), tile, x[d], cols3<HD>(slabs, col + 16 * d + 16, lane), tile, x[d + 1]);
     if constexpr (DT % 2 != 0) {
-        const Op3 a = cols3<HD>(slabs, 16 * DT - 16, lane);
+        const Op3 a = cols3<HD>(slabs, col + 16 * DT - 16, lane);
         f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = t0;
         t0 = Bf16::mfma16(a.p[2], tile.p[0], t0);
         t1 = Bf16::mfma16(a.p[1], tile.p[1], t1);
@@ -607,6 +608,228 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
 }
 
 // ---------------------------------------------------------------------------------------------
+// The same with tangents at D > 64, by pairs of waves: four owned tensors in three parts and the accumulators are more registers than
+// leave a second wave room on its SIMD.  The pair shares 16 owned rows; one wave owns two tensors o, o_dot and streams y1, y2 against them,
+//     x1 = y1 o, x2 = y1 o_dot + y2 o,
+// here q, q_dot against k, k_dot and G, dO against v, v_dot: three contractions of both.  They exchange what the other one's element-wise
+// part needs through LDS.  dQ, dQ_dot need all of it: each wave takes half of their columns.  One wave per SIMD with everything / pairs:
+// B=8 H=16 L=512 D=128 552 / 480 us, B=8 H=12 L=500 D=96 325 / 289, B=32 H=8 L=128 D=80 74 / 66.
+constexpr int kPairs = 4;  // of a workgroup: 64 owned rows
+template <int HD, int NS>
+constexpr int pair_smem() { return TriSmem<HD, NS>::bytes + kPairs * 2 * 4 * 64 * (int)sizeof(f32x4); }
+
+// Whether a wave of the pair met an element for the fp32 unit.
+template <int HD, int NS>
+__device__ __forceinline__ bool pair_met(unsigned char* smem, bool met, int wave, int lane) {
+    volatile int* flag = reinterpret_cast<volatile int*>(smem + TriSmem<HD, NS>::bytes);
+    workgroup_barrier();  // the last stage's tiles are read
+    if (lane == 0) flag[wave] = met;
+    workgroup_barrier();
+    return __builtin_expect(met || __builtin_amdgcn_readfirstlane(flag[wave ^ kPairs]) != 0, 0);
+}
+
+// The forms of the pairs on the fp32 unit, for rows whose numbers the split does not hold: operands are read where they are used.
+// Score-like tile: streamed rows (the lane's `row` of L) times the owned one.
+template <int HD>
+__device__ __forceinline__ f32x4 unit_dot(const BwdParamsF32& p, const F32Place& w, const F32In& rows, int row, int L, const F32In& own, int own_row,
+                                          int own_L) {
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 a[HD / 16], b[HD / 16], c = {0.f, 0.f, 0.f, 0.f};
+    f32_load_own<HD, false, true>(a, rows.head(w.b, w.h), rows.sl, row, L, p.D, w.g);
+    f32_load_own<HD, false, true>(b, own.head(w.b, w.h), own.sl, own_row, own_L, p.D, w.g);
+#pragma unroll
+    for (int m = 0; m < HD / 16; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c = mfma_f32(a[m][e], b[m][e], c);
+    return c;
+}
+// Output-side operand of a streamed row.
+template <int HD>
+__device__ __forceinline__ void unit_cols(float* y, const BwdParamsF32& p, const F32Place& w, const F32In& x, int row, int L) {
+    __builtin_amdgcn_sched_barrier(0);
+    f32_load_cols<HD, false, true>(y, x.head(w.b, w.h), x.sl, row, L, p.D, w.n);
+    f32_cut_cols<HD, false, true>(y, p.D, w.n);
+    f32_zero_unless<F32Cols<HD>::tiles>(y, row < L);
+}
+
+// dQ, dQ_dot of 16 rows.
+template <int HD, bool HAS_DO>
+__device__ __forceinline__ void bwd_row_f32_unit(const BwdParamsF32& p, const F32Place& w, float s4, float s7d) {
+    constexpr int T = F32Cols<HD>::tiles;
+    const int qrow = w.row0 + w.n;
+    const bool qvalid = qrow < p.Lq;
+    const int64_t so = (int64_t)w.bh * p.Lr + qrow;
+    const float lse2 = p.lse[so] * kLog2e, mu = p.mu[so];
+    f32x4 acc[T], tacc[T];
+    zero_tiles<T>(acc);
+    zero_tiles<T>(tacc);
+#pragma unroll 1
+    for (int k0 = 0; k0 < p.Lk; k0 += kF32Rows) {
+        int own_row = qrow;  // read anew for every tile: kept through the loop, the owned rows are more registers than there are
+        asm volatile("" : "+v"(own_row));
+        auto dot = [&](const F32In& rows, const F32In& own) { return unit_dot<HD>(p, w, rows, k0 + w.n, p.Lk, own, own_row, p.Lq); };
+        const f32x4 s = dot(p.k, p.q), ts = dot(p.k, p.tq) + dot(p.tk, p.q), wt = dot(p.v, p.dTO);
+        f32x4 xy = dot(p.tv, p.dTO);
+        if constexpr (HAS_DO) xy = dot(p.v, p.dO) + xy;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = k0 + 4 * w.g + j;
+            const float pj = fast_exp2(fmaf(s[j], p.scale * kLog2e, -lse2));
+            float dts = pj * (wt[j] - s4), ds = fmaf(dts, fmaf(ts[j], p.scale, -mu), pj * (xy[j] - s7d));
+            dts = row < p.Lk ? dts : 0.f;
+            ds = row < p.Lk ? ds : 0.f;
+            float y[T];
+            unit_cols<HD>(y, p, w, p.k, row, p.Lk);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                acc[t] = mfma_f32(y[t], ds, acc[t]);
+                tacc[t] = mfma_f32(y[t], dts, tacc[t]);
+            }
+            unit_cols<HD>(y, p, w, p.tk, row, p.Lk);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = mfma_f32(y[t], dts, acc[t]);
+        }
+    }
+    f32_store<HD, false, 1>(nullptr, p.dq.head(w.b, w.h) + (int64_t)qrow * p.dq.sl, acc, p.scale, w, p.D, qvalid);
+    f32_store<HD, false, 1>(nullptr, p.dtq.head(w.b, w.h) + (int64_t)qrow * p.dtq.sl, tacc, p.scale, w, p.D, qvalid);
+}
+
+template <int HD, int DT, bool HAS_DO>
+__global__ __launch_bounds__(128 * kPairs, 2) void bwd_row_f32x3_pair_kernel(const BwdParamsF32 p) {
+    constexpr int NS = 4, NT = 128 * kPairs, KC = (DT + 1) / 2, SE = Slab<HD>::elems, HT = DT / 2;
+    static_assert(DT % 2 == 0, "half of the columns each");
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    F32Place w = tri_place<kPairs>(p.q_blocks, p.H);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), role = wave / kPairs;  // 0: k, 1: v
+    w.row0 -= role * 16 * kPairs;
+    f32x4* exchange = reinterpret_cast<f32x4*>(smem_raw + TriSmem<HD, NS>::bytes) + (wave % kPairs) * 512 + w.lane;
+    f32x4 *mine = exchange + 256 * role, *other = exchange + 256 * (1 - role);
+    const int qrow = w.row0 + w.n;
+    const bool qvalid = qrow < p.Lq, active = w.row0 < p.Lq;
+    TriPlan<HD, NS, NT> plan;
+    {
+        auto src = [&](const F32In& t) { return Src32{t.head(w.b, w.h), t.sl}; };
+        plan.init(threadIdx.x, p.D, src(p.k), src(p.v), src(p.tk), src(p.tv));
+    }
+    const int64_t so = (int64_t)w.bh * p.Lr + qrow;  // rows below Lr exist
+    Op3 own[KC], town[KC];
+    float c1 = 0.f, c2 = 0.f;  // of the row: log-sum-exp (log2 units) and mu, or s4 and s7d
+    bool met;                  // an element for the fp32 unit (wave-uniform)
+    {
+        F32x8 x[KC], o[KC];
+        float sq = 0.f;
+        auto fetch = [&](F32x8* to, const F32In& t) {
+            own_load<KC>(to, t.head(w.b, w.h) + (int64_t)qrow * t.sl, w.g, p.D, qvalid);
+            own_cut<KC>(to, w.g, p.D);
+        };
+        if (role == 0) {
+            fetch(x, p.q);
+            own_split<KC>(own, x, sq);
+            fetch(x, p.tq);
+            own_split<KC>(town, x, sq);
+            if (active) {
+                c1 = p.lse[so] * kLog2e;
+                c2 = p.mu[so];
+                if (w.g == 0) p.lse2[so] = c1;
+            }
+        } else {
+            fetch(o, p.o);
+            if constexpr (HAS_DO) {
+                fetch(x, p.dO);
+                c2 = own_dot<KC>(x, o, c2);
+                own_split<KC>(town, x, sq);
+            }
+            fetch(x, p.dTO);
+            c1 = own_dot<KC>(x, o, c1);
+            fetch(o, p.to);
+            c2 = own_dot<KC>(x, o, c2);
+            own_split<KC>(own, x, sq);
+            c1 = group_sum(c1);
+            c2 = group_sum(c2);
+            if (active && w.g == 0) {
+                p.s4[so] = c1;
+                p.s7d[so] = c2;
+            }
+        }
+        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+    }
+    f32x4 dq[HT], dtq[HT];
+    zero_tiles<HT>(dq);
+    zero_tiles<HT>(dtq);
+    const int col = 16 * HT * role;
+    const float sl2 = p.scale * kLog2e;
+
+    tri_walk<HD, NS, NT>(smem_raw, plan, p.Lk, [&](const elem_t* buf, int k0, bool stage_special) {
+        met = met || stage_special;
+        const elem_t *y1 = buf + role * 3 * SE, *y2 = y1 + 6 * SE;
+        f32x4 x1[2], x2[2];
+        zero_tiles<2>(x1);
+        zero_tiles<2>(x2);
+        if (active) {
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int c = 0; c < KC; ++c) {
+                const Op3 a0 = rows3<HD>(y1, 0, c, w.n, w.g), a1 = rows3<HD>(y1, 1, c, w.n, w.g);
+                mfma6(a0, own[c], x1[0], a1, own[c], x1[1]);
+                if (HAS_DO || role == 0) mfma6(a0, town[c], x2[0], a1, town[c], x2[1]);
+                mfma6(rows3<HD>(y2, 0, c, w.n, w.g), own[c], x2[0], rows3<HD>(y2, 1, c, w.n, w.g), own[c], x2[1]);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            // P and N, or W - s4 and XY - s7d
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (role == 0) {
+                        x1[t][j] = fast_exp2(fmaf(x1[t][j], sl2, -c1));
+                        x2[t][j] = fmaf(x2[t][j], p.scale, -c2);
+                    } else {
+                        x1[t][j] -= c1;
+                        x2[t][j] -= c2;
+                    }
+                mine[64 * t] = x1[t];
+                mine[64 * (2 + t)] = x2[t];
+            }
+        }
+        workgroup_barrier();
+        if (!active) return;
+        f32x4 ds[2], dts[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const f32x4 z1 = other[64 * t], z2 = other[64 * (2 + t)];
+            const f32x4 pr = role ? z1 : x1[t], nn = role ? z2 : x2[t], wt = role ? x1[t] : z1, xy = role ? x2[t] : z2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                dts[t][j] = pr[j] * wt[j];
+                ds[t][j] = fmaf(dts[t][j], nn[j], pr[j] * xy[j]);
+            }
+        }
+        if (k0 + kStageRows > p.Lk) {  // keys that do not exist contribute nothing
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool kvalid = k0 + 16 * t + 4 * w.g + j < p.Lk;
+                    ds[t][j] = kvalid ? ds[t][j] : 0.f;
+                    dts[t][j] = kvalid ? dts[t][j] : 0.f;
+                }
+        }
+        float sq = 0.f;
+        const Op3 dsb = split_tiles(ds[0], ds[1], sq), dtsb = split_tiles(dts[0], dts[1], sq);
+        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        tri_out<HD, HT>(buf, w.lane, dsb, dq, dtsb, dtq, col);
+        tri_out<HD, HT>(buf + 6 * SE, w.lane, dtsb, dq, col);
+    });
+    if (pair_met<HD, NS>(smem_raw, met, wave, w.lane)) {
+        if (active && role == 1) bwd_row_f32_unit<HD, HAS_DO>(p, w, c1, c2);
+        return;
+    }
+    if (!active) return;
+    tri_store<HT>(p.dq.head(w.b, w.h) + (int64_t)qrow * p.dq.sl + col, dq, p.scale, p.D - col, w.g, qvalid);
+    tri_store<HT>(p.dtq.head(w.b, w.h) + (int64_t)qrow * p.dtq.sl + col, dtq, p.scale, p.D - col, w.g, qvalid);
+}
+
+// ---------------------------------------------------------------------------------------------
 // Column-owned backward: dK, dV (, dK_dot, dV_dot).
 template <int HD, int DT, bool HAS_DO, bool HAS_G, int NW>
 __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_kernel(const BwdParamsF32 p) {
@@ -750,23 +973,13 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
 }
 
 // ---------------------------------------------------------------------------------------------
-// The same with tangents at D > 64, by pairs of waves: four owned tensors in three parts and four accumulators are more registers
-// than a wave has.  One wave owns k, k_dot and the gradients of them, the other v, v_dot and theirs, of the same 16 rows; each
-// forms the scores of its own tensors, they exchange what the other one's element-wise part needs through LDS, and each enters
-// its own output contractions: three and three of both, nothing twice, in half the registers, so that a SIMD has two waves.
-// Against the fp32 unit (D > 96) and two launches of 9 and 6 contractions, one for each half: B=8 H=16 L=512 D=128 887 -> 564 us,
-// B=8 H=12 L=500 D=96 594 -> 319, B=4 H=16 L=512 D=80 397 -> 212.
-// With o, o_dot the owned pair, y1, y2 the streamed one (q, q_dot or dO_dot, dO) and t1, t2 the tiles (dS_dot, dS or P, P_dot), both waves do
-//     x1 = y1 o, x2 = y1 o_dot + y2 o;   d(o_dot) = t1^T y1, d(o) = t2^T y1 + t1^T y2.
-constexpr int kPairs = 4;  // of a workgroup: 64 owned rows
-template <int HD, int NS>
-constexpr int pair_smem() { return TriSmem<HD, NS>::bytes + kPairs * 2 * 4 * 64 * (int)sizeof(f32x4); }
-
-// The two gradients of a wave on the fp32 unit, its operands read where they are used: for the wave's few registers, and for the
-// rows whose numbers the split does not hold.
+// By pairs of waves, as the row kernel's: one wave owns k, k_dot and the gradients of them, the other v, v_dot and theirs.  With
+// t1, t2 the tiles (dS_dot, dS or P, P_dot) the output contractions are three of both waves too, and nothing is done twice:
+//     d(o_dot) = t1^T y1, d(o) = t2^T y1 + t1^T y2.
+// The two gradients of a wave.
 template <int HD, bool HAS_DO>
 __device__ __forceinline__ void bwd_col_f32_half(const BwdParamsF32& p, const F32Place& w, int role) {
-    constexpr int M = HD / 16, T = F32Cols<HD>::tiles;
+    constexpr int T = F32Cols<HD>::tiles;
     const int krow = w.row0 + w.n;
     const bool kvalid = krow < p.Lk;
     f32x4 acc[T], tacc[T];
@@ -777,17 +990,7 @@ __device__ __forceinline__ void bwd_col_f32_half(const BwdParamsF32& p, const F3
     for (int q0 = 0; q0 < p.Lq; q0 += kF32Rows) {
         int own_row = krow;  // read anew for every tile: kept through the loop, the owned rows are more registers than there are
         asm volatile("" : "+v"(own_row));
-        auto dot = [&](const F32In& rows, const F32In& own) {
-            __builtin_amdgcn_sched_barrier(0);
-            f32x4 a[M], b[M], c = {0.f, 0.f, 0.f, 0.f};
-            f32_load_own<HD, false, true>(a, rows.head(w.b, w.h), rows.sl, q0 + w.n, p.Lq, p.D, w.g);
-            f32_load_own<HD, false, true>(b, own.head(w.b, w.h), own.sl, own_row, p.Lk, p.D, w.g);
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) c = mfma_f32(a[m][e], b[m][e], c);
-            return c;
-        };
+        auto dot = [&](const F32In& rows, const F32In& own) { return unit_dot<HD>(p, w, rows, q0 + w.n, p.Lq, own, own_row, p.Lk); };
         const f32x4 s = dot(p.q, p.k), ts = dot(p.tq, p.k) + dot(p.q, p.tk);
         f32x4 wt = {0.f, 0.f, 0.f, 0.f}, xy = wt, t1, t2;
         if (role == 0) {
@@ -810,12 +1013,7 @@ __device__ __forceinline__ void bwd_col_f32_half(const BwdParamsF32& p, const F3
             t1[j] = qvalid ? t1[j] : 0.f;
             t2[j] = qvalid ? t2[j] : 0.f;
             float y[T];
-            auto cols = [&](const F32In& x) {
-                __builtin_amdgcn_sched_barrier(0);
-                f32_load_cols<HD, false, true>(y, x.head(w.b, w.h), x.sl, row, p.Lq, p.D, w.n);
-                f32_cut_cols<HD, false, true>(y, p.D, w.n);
-                f32_zero_unless<T>(y, qvalid);
-            };
+            auto cols = [&](const F32In& x) { unit_cols<HD>(y, p, w, x, row, p.Lq); };
             if (role) cols(p.dTO);
             else cols(p.q);
 #pragma unroll
@@ -940,12 +1138,9 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_col_f32x3_pair_kernel(con
         tri_out<HD, DT>(y1, w.lane, b2, acc, b1, tacc);
         if (has_y2) tri_out<HD, DT>(y2, w.lane, b1, acc);
     });
-    volatile int* flag = reinterpret_cast<volatile int*>(smem_raw + TriSmem<HD, NS>::bytes);
-    workgroup_barrier();  // the last stage's tiles are read
-    if (w.lane == 0) flag[wave] = met;
-    workgroup_barrier();
+    const bool unit = pair_met<HD, NS>(smem_raw, met, wave, w.lane);
     if (!active) return;
-    if (__builtin_expect(met || __builtin_amdgcn_readfirstlane(flag[wave ^ kPairs]) != 0, 0)) return bwd_col_f32_half<HD, HAS_DO>(p, w, role);
+    if (unit) return bwd_col_f32_half<HD, HAS_DO>(p, w, role);
     const F32Out &d = role ? p.dv : p.dk, &td = role ? p.dtv : p.dtk;
     const float mul = role ? 1.0f : p.scale;
     tri_store<DT>(d.head(w.b, w.h) + (int64_t)krow * d.sl, acc, mul, p.D, w.g, kvalid);
