@@ -20,8 +20,9 @@ inline int split(int BH, int rows, int streamed) {
     return streamed > kF32Rows && 13 * quarter < 10 * whole ? 4 : 1;
 }
 
-// Waves of a workgroup for which the kernels on the bf16 matrix pipe (sjvp_f32x3.hpp) take the launch, 0 where the ones on the
-// fp32 unit keep it.  `rows`: owned rows of a (batch, head) pair (padded in the forward), `streamed`: the other axis.
+// The kernels on the bf16 matrix pipe (sjvp_f32x3.hpp) take all three launches of a problem or none: the backward forms the
+// scores again, and against the log-sum-exp of the other set's scores its error grows (dV of 200 queries on 32 keys, D = 100: 1.16 times
+// the fp32 unit's, by one set 0.8).  `rows`: owned rows of a (batch, head) pair (padded in the forward), `streamed`: the other axis.
 //
 // Four waves while every workgroup of 64 rows has a compute unit, else eight, whose workgroups split the streamed side once
 // for 128 rows (D = 64, L = 256, 1024 / 2048 groups of 16 rows, four / eight: forward 28 / 36 and 54 / 40 us, row kernel 37 / 47 and
@@ -29,22 +30,32 @@ inline int split(int BH, int rows, int streamed) {
 // groups, 33 / 32 and 48 / 57) and without tangents (D = 64: 27 / 25 and 34 / 44) keeps to four, so does all of D > 64.
 //
 // A launch costs rounds of workgroups times streamed tiles; per tile, in fortieths of what a round of the fp32 unit's whole
-// groups takes: 28 (four waves; D > 64: 32) or 37 (eight), the forward without tangents 40 and 50; the fp32 unit's 40, 13 for each
-// round of split groups.  Both sides in us, fp32 unit / here, L = 256: D = 64 512 groups 26 / 27 forward, 37 / 34 row, 40 / 44 column;
-// 640 31 / 26, 54 / 33, 59 / 41; 4096 142 / 78, 201 / 105, 250 / 139; D = 80 640 62 / 50, 90 / 60, 113 / 57; D = 128
-// 448 44 / 51, 70 / 70, 73 / 71, 576 64 / 53, 104 / 70, 108 / 72; D = 32 without tangents, forward, 640 9.0 / 11.2, 2048 17 / 13.
-inline int x3_waves(int BH, int groups_of, int rows, int streamed, int D, bool forward, bool tangents, int split) {
-    const int units = compute_units();
-    const int64_t four = (int64_t)BH * ((rows + 63) / 64), eight = (int64_t)BH * ((rows + 127) / 128);
-    const int waves = D > 64 || four <= units || (!forward && (D <= 32 || !tangents)) ? 4 : 8;
+// groups takes: 28 (four waves; D > 64: 32) or 37 (eight), the forward without tangents 40 and 50, the backward by pairs of waves 25
+// (D > 96 on more than 256 rows: 27); the fp32 unit's 40, 13 for each round of split groups.
+// Both sides in us, fp32 unit / here, L = 256: D = 64 512 groups 26 / 27 forward, 37 / 34 row, 40 / 44 column; 640 31 / 26, 54 / 33, 59 / 41; 4096 142 / 78, 201 / 105, 250 / 139; D = 80 384 42 / 50, 61 / 53, 74 / 56,
+// 640 62 / 50, 90 / 53, 113 / 57; D = 128 384 43 / 51, 70 / 61, 73 / 70 (L = 1024: 125 / 187, 202 / 206, 218 / 239), 576 64 / 53, 104 / 62,
+// 108 / 72; D = 32 without tangents, forward, 640 9.0 / 11.2, 2048 17 / 13.
+inline int x3_width(int BH, int rows, int D, bool forward, bool tangents) {
+    const int64_t four = (int64_t)BH * ((rows + 63) / 64);
+    return D > 64 || four <= compute_units() || (!forward && (D <= 32 || !tangents)) ? 4 : 8;
+}
+// What a launch saves there, in tenths of fortieths.
+inline int64_t x3_saves(int BH, int groups_of, int rows, int streamed, int D, bool forward, bool tangents) {
+    const int units = compute_units(), waves = x3_width(BH, rows, D, forward, tangents);
     // tenths; workgroups of four that share a compute unit (48 KB of LDS, or less) add 0.7 of a round each
-    int64_t rounds = ((waves == 4 ? four : eight) + units - 1) / units;
+    int64_t rounds = ((int64_t)BH * ((rows + 16 * waves - 1) / (16 * waves)) + units - 1) / units;
     rounds = waves == 4 && (D <= 32 || (D <= 64 && !tangents)) ? 7 * rounds + 3 : 10 * rounds;
-    const int per_tile = forward && !tangents ? (waves == 4 ? 40 : 50) : D > 64 ? 32 : waves == 4 ? 28 : 37;
+    const int pairs = D > 96 && streamed > 256 ? 27 : 25;
+    const int per_tile = forward && !tangents ? (waves == 4 ? 40 : 50) : D > 64 ? (!forward && tangents ? pairs : 32) : waves == 4 ? 28 : 37;
     const int64_t groups = (int64_t)BH * ((groups_of + kF32Rows - 1) / kF32Rows);
-    const int64_t unit = split == 4 ? 13 * ((4 * groups + kSimds - 1) / kSimds) : 40 * ((groups + kSimds - 1) / kSimds);
+    const int64_t unit = split(BH, groups_of, streamed) == 4 ? 13 * ((4 * groups + kSimds - 1) / kSimds) : 40 * ((groups + kSimds - 1) / kSimds);
     const int64_t tiles = (streamed + kF32Rows - 1) / kF32Rows, stages = (streamed + kStageRows - 1) / kStageRows;
-    return 2 * stages * rounds * per_tile < 10 * tiles * unit ? waves : 0;
+    return 10 * tiles * unit - 2 * stages * rounds * per_tile;
+}
+inline bool x3_takes(int BH, int Lq, int Lr, int Lk, int D, bool tangents) {
+    // by the contractions of forward, row and column launch: 6, 9 and 12, without tangents 2, 3 and 4
+    return 2 * x3_saves(BH, Lq, Lr, Lk, D, true, tangents) + 3 * x3_saves(BH, Lq, Lq, Lk, D, false, tangents) +
+               4 * x3_saves(BH, Lk, Lk, Lq, D, false, tangents) > 0;
 }
 inline int blocks(int rows, int split) {
     const int per = split > 1 ? kF32Rows : kF32Rows * kF32Waves;
@@ -54,7 +65,7 @@ inline int blocks(int rows, int split) {
 template <int HD, bool JVP, F32Columns COLS>
 int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
-    if (const int waves = x3_waves(BH, p.Lq, p.Lr, p.Lk, p.D, true, JVP, sp)) return fwd_f32x3(p, BH, JVP, waves, stream);
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, JVP)) return fwd_f32x3(p, BH, JVP, x3_width(BH, p.Lr, p.D, true, JVP), stream);
     p.blocks = blocks(p.Lr, sp);  // the statistics cover rows below Lr
     const int grid = BH * p.blocks;
     if (sp == 4) return launch(fwd_f32_kernel<HD, JVP, 4, COLS>, grid, 0, stream, p, kF32Threads);
@@ -64,8 +75,8 @@ int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
 template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
-    if (const int waves = x3_waves(BH, p.Lq, p.Lq, p.Lk, p.D, false, HAS_G, sp))
-        return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_ROW, waves, stream);
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, HAS_G))
+        return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_ROW, x3_width(BH, p.Lq, p.D, false, HAS_G), stream);
     p.q_blocks = blocks(p.Lq, sp);
     const int grid = BH * p.q_blocks;
     if (sp == 4) return launch(bwd_row_f32_kernel<HD, HAS_DO, HAS_G, 4, COLS>, grid, 0, stream, p, kF32Threads);
@@ -75,8 +86,8 @@ int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
 template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int col_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lk, p.Lq);
-    if (const int waves = x3_waves(BH, p.Lk, p.Lk, p.Lq, p.D, false, HAS_G, sp))
-        return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_COL, waves, stream);
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, HAS_G))
+        return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_COL, x3_width(BH, p.Lk, p.D, false, HAS_G), stream);
     p.k_blocks = blocks(p.Lk, sp);
     const int grid = BH * p.k_blocks;
     if (sp == 4) return launch(bwd_col_f32_kernel<HD, HAS_DO, HAS_G, 4, COLS>, grid, 0, stream, p, kF32Threads);
