@@ -154,7 +154,7 @@ def _on_gpu(q) -> bool:
     """Whether the host extension (csrc/sjvp_host.cpp) is asked first.  It serves the calls that pass every check of
     the general forms below, with the same results, and answers None to all others, which the general form then
     refuses or takes.  Forward + backward of a 2x2x16x16x32 problem: 55 us through Python and ctypes alone,
-    15 us with it (toy problem in a loop, kernels included)."""
+    14 us with it (toy problem in a loop, kernels included)."""
     return isinstance(q, torch.Tensor) and q.is_cuda and bool(_lib.host())
 
 
