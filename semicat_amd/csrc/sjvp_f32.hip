@@ -20,9 +20,10 @@ inline int split(int BH, int rows, int streamed) {
     return streamed > kF32Rows && 13 * quarter < 10 * whole ? 4 : 1;
 }
 
-// The kernels on the bf16 matrix pipe (sjvp_f32x3.hpp) take all three launches of a problem or none: the backward forms the
-// scores again, and against the log-sum-exp of the other set's scores its error grows (dV of 200 queries on 32 keys, D = 100: 1.16 times
-// the fp32 unit's, by one set 0.8).  `rows`: owned rows of a (batch, head) pair (padded in the forward), `streamed`: the other axis.
+// The kernels on the bf16 matrix pipe (sjvp_f32x3.hpp) take all launches on a shape or none: the backward forms the
+// scores again, and against the log-sum-exp of the other set's scores its error grows (dQ of 200 queries on 32 keys, D = 100: 1.18 times
+// the fp32 unit's, by one set 0.99).  A backward does not know whether its forward had tangents (for a cotangent on O alone it is
+// given none), so the rule asks the shape alone.  `rows`: owned rows of a (batch, head) pair (padded in the forward), `streamed`: the other axis.
 //
 // Four waves while every workgroup of 64 rows has a compute unit, else eight, whose workgroups split the streamed side once
 // for 128 rows (D = 64, L = 256, 1024 / 2048 groups of 16 rows, four / eight: forward 28 / 36 and 54 / 40 us, row kernel 37 / 47 and
@@ -52,10 +53,21 @@ inline int64_t x3_saves(int BH, int groups_of, int rows, int streamed, int D, bo
     const int64_t tiles = (streamed + kF32Rows - 1) / kF32Rows, stages = (streamed + kStageRows - 1) / kStageRows;
     return 10 * tiles * unit - 2 * stages * rounds * per_tile;
 }
-inline bool x3_takes(int BH, int Lq, int Lr, int Lk, int D, bool tangents) {
-    // by the contractions of forward, row and column launch: 6, 9 and 12, without tangents 2, 3 and 4
-    return 2 * x3_saves(BH, Lq, Lr, Lk, D, true, tangents) + 3 * x3_saves(BH, Lq, Lq, Lk, D, false, tangents) +
-               4 * x3_saves(BH, Lk, Lk, Lq, D, false, tangents) > 0;
+// By the launches of a call with tangents.  Plain calls (the forward without, or a cotangent on O alone) go with them, and what their
+// costs, which are on the high side, say against it counts only where a launch leaves more than half of the compute units without a
+// workgroup.  Forward + backward with and without tangents, fp32 unit / here, us, at shapes where the two kinds' costs disagree:
+//   stays on the unit: 78 heads, 52 queries on 3516 keys, D = 20 505 / 564 and 204 / 313; 24 heads, 250 on 2586, D = 16 349 / 350 and 142 / 193;
+//   goes here: 60 heads, 259 x 259, D = 48 321 / 153 and 125 / 82; 120 heads, 803 x 803, D = 128 5470 / 3742 and 2428 / 1596; the worst
+//   of 80 such shapes 186 heads, 44 on 1663, D = 100 1539 / 1694 and 618 / 739; with half of the units idle at D > 64, 104 heads, 59 on 424,
+//   D = 100 295 / 293 and 122 / 136, 35 heads, 280 on 154, D = 80 220 / 140 and 89 / 74.
+// (Where the plain launches alone would gain: 144 heads, 144 x 144, D = 64 plain 80 / 60; with tangents 221 on the unit.)
+inline bool x3_takes(int BH, int Lq, int Lr, int Lk, int D) {
+    auto gains = [&](bool tangents) {  // by the contractions of forward, row and column launch: 6, 9 and 12, without tangents 2, 3 and 4
+        return 2 * x3_saves(BH, Lq, Lr, Lk, D, true, tangents) + 3 * x3_saves(BH, Lq, Lq, Lk, D, false, tangents) +
+                   4 * x3_saves(BH, Lk, Lk, Lq, D, false, tangents) > 0;
+    };
+    const int64_t fewest = (int64_t)BH * (((Lq < Lk ? Lq : Lk) + 63) / 64);
+    return gains(true) && (D > 64 || 2 * fewest >= compute_units() || gains(false));
 }
 inline int blocks(int rows, int split) {
     const int per = split > 1 ? kF32Rows : kF32Rows * kF32Waves;
@@ -65,7 +77,7 @@ inline int blocks(int rows, int split) {
 template <int HD, bool JVP, F32Columns COLS>
 int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
-    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, JVP)) return fwd_f32x3(p, BH, JVP, x3_width(BH, p.Lr, p.D, true, JVP), stream);
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D)) return fwd_f32x3(p, BH, JVP, x3_width(BH, p.Lr, p.D, true, JVP), stream);
     p.blocks = blocks(p.Lr, sp);  // the statistics cover rows below Lr
     const int grid = BH * p.blocks;
     if (sp == 4) return launch(fwd_f32_kernel<HD, JVP, 4, COLS>, grid, 0, stream, p, kF32Threads);
@@ -75,7 +87,7 @@ int fwd_one(FwdParamsF32 p, int BH, hipStream_t stream) {
 template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lq, p.Lk);
-    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, HAS_G))
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D))
         return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_ROW, x3_width(BH, p.Lq, p.D, false, HAS_G), stream);
     p.q_blocks = blocks(p.Lq, sp);
     const int grid = BH * p.q_blocks;
@@ -86,7 +98,7 @@ int row_one(BwdParamsF32 p, int BH, hipStream_t stream) {
 template <int HD, bool HAS_DO, bool HAS_G, F32Columns COLS>
 int col_one(BwdParamsF32 p, int BH, hipStream_t stream) {
     const int sp = split(BH, p.Lk, p.Lq);
-    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D, HAS_G))
+    if (x3_takes(BH, p.Lq, p.Lr, p.Lk, p.D))
         return bwd_f32x3(p, BH, HAS_DO, HAS_G, SJVP_BWD_COL, x3_width(BH, p.Lk, p.D, false, HAS_G), stream);
     p.k_blocks = blocks(p.Lk, sp);
     const int grid = BH * p.k_blocks;
