@@ -2,8 +2,8 @@
 // with every fp32 operand as a sum of three bf16 values.
 //
 // x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1): 24 significant bits, all of an fp32
-// number's.  Of the nine products of two such operands the three smallest (below 2^-25 of the whole) are left out; the
-// other six are exact in the matrix unit and summed there in fp32, small ones first.  v_mfma_f32_16x16x32_bf16 adds 32 of them
+// number's from 2^-110 on (bf16 ends at 2^-133; no instruction on the way flushes subnormals).
+// Of the nine products of two such operands the three smallest (below 2^-25 of the whole) are left out; the other six are exact in the matrix unit and summed there in fp32, small ones first.  v_mfma_f32_16x16x32_bf16 adds 32 of them
 // per rounding step of the accumulator where v_mfma_f32_16x16x4_f32 adds four, so the error against fp64 is smaller: sums of
 // 32 / 64 / 512 / 4096 products of normal numbers 3.8e-8 / 9.1e-8 / 3.4e-7 / 1.0e-6 relative, on the fp32 unit 1.0e-7 /
 // 1.4e-7 / 4.1e-7 / 1.2e-6.  What was computed in fp32 outside the contractions (exponentials, row sums, statistics,
@@ -23,9 +23,12 @@
 // Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 5.4e-7.
 //
 // Numbers that the split does not hold (infinities, NaN) or whose products could overflow one by one where their sum does
-// not (2^59 and above) are left to the fp32 unit: a wave that met one, in its own rows, in a stage or in a tile, computes its
+// not (2^59 and above) are left to the fp32 unit: a wave that met one, in its own rows, in a stage or in its tiles, computes its
 // 16 rows again as the kernels of sjvp_f32.hpp do, behind its loop (inside it the second form costs the first one 60
 // registers).  So infinite and overflowing scores come out as they do there.
+// So are small numbers: where eight neighbours in a row, or an owned row's tiles of the whole streamed axis, are not all zero and all below
+// 2^-100.  (Beside larger ones what a number loses, at most 2^-134, is nothing.)  Gradients of cotangents at 2^-118 had errors up to 8.5e-5, and have
+// the unit's 4.9e-7 there.
 #pragma once
 #include "sjvp_f32.hpp"
 #include "sjvp_staged16.hpp"
@@ -62,11 +65,39 @@ __device__ __forceinline__ void mfma6_onto(const Op3& a0, const Op3& b0, f32x4& 
     c1 += t1;
 }
 
-// Element i (two neighbours x, y) of the three parts; `sq` collects their squares for the test of kMost.  What a part leaves
-// over is exact in fp32, and the dot product with (-1, 0) or (0, -1) takes it from the packed pair as it is: seven instructions
-// where unpacking and subtracting are eleven.  (The zero beside -1 is a negative one: the pair (-1, +0) is among the constants that
+// The largest of `most` and the magnitudes of x and y; NaN if one is.
+__device__ __forceinline__ float most_of(float most, float x, float y) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(most, fabsf(x)), fabsf(y));
+}
+// Numbers whose largest magnitude is `most` are for the fp32 unit if that is 2^59 or more, or NaN, or below 2^-100 but not zero.  (By the bits:
+// those of magnitudes are in their order, and one less puts zero on the other end.)
+constexpr uint32_t kLeast = 0x0d800000u, kMost = 0x5d000000u;
+__device__ __forceinline__ uint32_t bits_less_one(float most) { return __builtin_bit_cast(uint32_t, most) - 1u; }
+// Groups of numbers, each by its largest magnitude.  (Both ends are compared once for all of a thread's groups: three vector instructions less for
+// every group but one; forward + backward at B=8 H=12 L=500 D=96 904 / 886 us, B=4 H=16 300 on 700 D=80 714 / 698, D <= 64 the same.)
+struct Met {
+    uint32_t least = ~0u;
+    float most = 0.f;
+    __device__ __forceinline__ void add(float group) {
+        least = min(least, bits_less_one(group));
+        most = __builtin_elementwise_maximum(most, group);
+    }
+    __device__ __forceinline__ bool special() const { return (least < kLeast - 1u) | (__builtin_bit_cast(uint32_t, most) >= kMost); }
+};
+// A row of tiles as one group, `most` by the lanes of one n; wave-uniform.
+__device__ __forceinline__ bool tiles_out_of_range(float most) {
+    most = most_of(most, __shfl_xor(most, 16, 64), 0.f);
+    most = most_of(most, __shfl_xor(most, 32, 64), 0.f);
+    Met m;
+    m.add(most);
+    return __builtin_amdgcn_ballot_w64(m.special()) != 0;
+}
+
+// Element i (two neighbours x, y) of the three parts.  What a part leaves over is exact in fp32, and the dot product with
+// (-1, 0) or (0, -1) takes it from the packed pair as it is: seven instructions where unpacking and subtracting are eleven.
+// (A neighbour that is infinite or NaN makes it NaN: such rows go to the fp32 unit.  The zero beside -1 is a negative one: the pair (-1, +0) is among the constants that
 // the compiler writes as the inline operand -1.0, which the instruction reads as the pair (0, -1).)
-__device__ __forceinline__ void split3(Op3& o, int i, float x, float y, float& sq) {
+__device__ __forceinline__ void split3(Op3& o, int i, float x, float y) {
     constexpr uint32_t kLow = 0x8000bf80u, kHigh = 0xbf800000u;
     const uint32_t p0 = Bf16::pack2(x, y);
     x = Bf16::dot2(p0, kLow, x);
@@ -77,18 +108,21 @@ __device__ __forceinline__ void split3(Op3& o, int i, float x, float y, float& s
     o.p[0][i] = p0;
     o.p[1][i] = p1;
     o.p[2][i] = Bf16::pack2(x, y);
-    sq = Bf16::dot2(p0, p0, sq);
 }
 // Two score-like tiles of a stage (32 streamed rows) as the B operand of an output contraction.
-__device__ __forceinline__ Op3 split_tiles(const f32x4& t0, const f32x4& t1, float& sq) {
+__device__ __forceinline__ Op3 split_tiles(const f32x4& t0, const f32x4& t1) {
     Op3 o;
-    split3(o, 0, t0[0], t0[1], sq);
-    split3(o, 1, t0[2], t0[3], sq);
-    split3(o, 2, t1[0], t1[1], sq);
-    split3(o, 3, t1[2], t1[3], sq);
+    split3(o, 0, t0[0], t0[1]);
+    split3(o, 1, t0[2], t0[3]);
+    split3(o, 2, t1[0], t1[1]);
+    split3(o, 3, t1[2], t1[3]);
     return o;
 }
-constexpr float kMost = 0x1p118f;  // of a sum of squares: every element below 2^59 (NaN fails the test too)
+// `most` collects the largest magnitude of the tiles of all stages.
+__device__ __forceinline__ Op3 split_tiles(const f32x4& t0, const f32x4& t1, float& most) {
+    most = most_of(most_of(most_of(most_of(most, t0[0], t0[1]), t0[2], t0[3]), t1[0], t1[1]), t1[2], t1[3]);
+    return split_tiles(t0, t1);
+}
 
 // Eight consecutive fp32 elements from column `col` of a row of D (>= 16); those beyond D become zero.  Read as the row's last
 // eight where they do not all exist, and shifted (piece_col, piece_shift).
@@ -103,10 +137,15 @@ struct F32x8 {
         if (s & 1) a[0] = f32x4{a[0][1], a[0][2], a[0][3], a[1][0]}, a[1] = f32x4{a[1][1], a[1][2], a[1][3], 0.f};
         if (s & 8) zero();
     }
-    __device__ __forceinline__ Op3 split(float& sq) const {
+    __device__ __forceinline__ Op3 split(Met& m) const {
         Op3 o;
+        float most = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) split3(o, i, (*this)[2 * i], (*this)[2 * i + 1], sq);
+        for (int i = 0; i < 4; ++i) {
+            most = most_of(most, (*this)[2 * i], (*this)[2 * i + 1]);
+            split3(o, i, (*this)[2 * i], (*this)[2 * i + 1]);
+        }
+        m.add(most);
         return o;
     }
 };
@@ -127,9 +166,9 @@ __device__ __forceinline__ void own_cut(F32x8* x, int g, int D) {
         for (int c = 0; c < KC; ++c) x[c].shift(piece_shift(32 * c + 8 * g, D));
 }
 template <int KC>
-__device__ __forceinline__ void own_split(Op3* o, const F32x8* x, float& sq) {
+__device__ __forceinline__ void own_split(Op3* o, const F32x8* x, Met& m) {
 #pragma unroll
-    for (int c = 0; c < KC; ++c) o[c] = x[c].split(sq);
+    for (int c = 0; c < KC; ++c) o[c] = x[c].split(m);
 }
 template <int KC>
 __device__ __forceinline__ float own_dot(const F32x8* x, const F32x8* y, float sum) {
@@ -198,15 +237,15 @@ struct TriPlan {
 #pragma unroll
         for (int i = 0; i < N; ++i) src[i] += adv[i];
     }
-    // Whether an element of this thread's was one for the fp32 unit.
+    // Whether elements of this thread's were some for the fp32 unit.
     __device__ __forceinline__ bool commit(elem_t* buffer) {
         constexpr int SE = Slab<HD>::elems;
-        float sq = 0.f;
+        Met m;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             if (total % NT != 0 && row[i] >= kStageRows) continue;
             if (shifted) raw[i].shift(sh);
-            const Op3 o = raw[i].split(sq);
+            const Op3 o = raw[i].split(m);
             constexpr int PPS = NT >= chunks ? 1 : chunks / NT;
             constexpr int SPI = NT >= chunks ? NT / chunks : 1;
             const int slab = NT >= chunks ? j0 + i * SPI : i / PPS;
@@ -214,7 +253,7 @@ struct TriPlan {
 #pragma unroll
             for (int u = 0; u < 3; ++u) *reinterpret_cast<u32x4*>(at + u * SE) = o.p[u];
         }
-        return !(sq < kMost);
+        return m.special();
     }
 };
 
@@ -371,19 +410,20 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void fwd_f32x3_kern
         F32x8 x[KC], tx[KC];
         own_load<KC>(x, q_own, w.g, p.D, qvalid);
         if constexpr (JVP) own_load<KC>(tx, tq_own, w.g, p.D, qvalid);
-        float sq = 0.f;
+        Met m;
         own_cut<KC>(x, w.g, p.D);
-        own_split<KC>(q, x, sq);
+        own_split<KC>(q, x, m);
         if constexpr (JVP) {
             own_cut<KC>(tx, w.g, p.D);
-            own_split<KC>(tq, tx, sq);
+            own_split<KC>(tq, tx, m);
         }
-        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        met = __builtin_amdgcn_ballot_w64(m.special()) != 0;
     }
     f32x4 acc[DT], tacc[DT];
     zero_tiles<DT>(acc);
     zero_tiles<DT>(tacc);
     const float sl2 = p.scale * kLog2e;
+    float pt_most = 0.f;  // (the probabilities are at most 1, and one of a row is)
     float m_i = -INFINITY, l_i = 0.f, mu_i = 0.f;  // maximum (log2 units), exp-sum, sum p * S_dot of the lane's keys
 
     tri_walk<HD, NS, NT>(smem_raw, plan, p.Lk, [&](const elem_t* buf, int k0, bool stage_special) {
@@ -443,11 +483,9 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void fwd_f32x3_kern
                     mu_i += pt[t][j];
                 }
             }
-        float sq = 0.f;
-        const Op3 pb = split_tiles(s[0], s[1], sq);
+        const Op3 pb = split_tiles(s[0], s[1]);
         Op3 ptb;
-        if constexpr (JVP) ptb = split_tiles(pt[0], pt[1], sq);
-        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        if constexpr (JVP) ptb = split_tiles(pt[0], pt[1], pt_most);
         if constexpr (JVP) {
             tri_out<HD, DT>(buf + 3 * SE, w.lane, pb, acc, ptb, tacc);
             tri_out<HD, DT>(buf + 9 * SE, w.lane, pb, tacc);
@@ -456,6 +494,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void fwd_f32x3_kern
         }
     });
     if (!active) return no_query();
+    if constexpr (JVP) met = met || tiles_out_of_range(pt_most);
     if (__builtin_expect(met, 0)) return fwd_f32_wave<HD, JVP, 1, kColumnsCut>(p, w, nullptr, nullptr);
     const float l = group_sum(l_i), mu_un = group_sum(mu_i);
     const float inv_l = 1.0f / l, mu = mu_un * inv_l;
@@ -496,7 +535,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
     bool met;  // an element for the fp32 unit (wave-uniform)
     {
         F32x8 x[KC], o[KC];
-        float sq = 0.f;
+        Met m;
         auto fetch = [&](F32x8* to, const float* row) {
             own_load<KC>(to, row, w.g, p.D, qvalid);
             own_cut<KC>(to, w.g, p.D);
@@ -505,20 +544,20 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
         if constexpr (HAS_DO) {
             fetch(x, do_own);
             s7d = own_dot<KC>(x, o, s7d);
-            own_split<KC>(dO, x, sq);
+            own_split<KC>(dO, x, m);
         }
         if constexpr (HAS_G) {
             fetch(x, g_own);
             s4 = own_dot<KC>(x, o, s4);
             fetch(o, own_row(p.to));
             s7d = own_dot<KC>(x, o, s7d);
-            own_split<KC>(g, x, sq);
+            own_split<KC>(g, x, m);
             fetch(x, tq_own);
-            own_split<KC>(tq, x, sq);
+            own_split<KC>(tq, x, m);
         }
         fetch(x, q_own);
-        own_split<KC>(q, x, sq);
-        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        own_split<KC>(q, x, m);
+        met = __builtin_amdgcn_ballot_w64(m.special()) != 0;
     }
     s4 = group_sum(s4);
     s7d = group_sum(s7d);
@@ -537,6 +576,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
         }
     }
     const float sl2 = p.scale * kLog2e;
+    float ds_most = 0.f, dts_most = 0.f;
 
     tri_walk<HD, NS, NT>(smem_raw, plan, p.Lk, [&](const elem_t* buf, int k0, bool stage_special) {
         met = met || stage_special;
@@ -589,11 +629,9 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
                     dts[t][j] = kvalid ? dts[t][j] : 0.f;
                 }
         }
-        float sq = 0.f;
-        const Op3 dsb = split_tiles(ds[0], ds[1], sq);
+        const Op3 dsb = split_tiles(ds[0], ds[1], ds_most);
         Op3 dtsb;
-        if constexpr (HAS_G) dtsb = split_tiles(dts[0], dts[1], sq);
-        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        if constexpr (HAS_G) dtsb = split_tiles(dts[0], dts[1], dts_most);
         if constexpr (HAS_G) {
             tri_out<HD, DT>(buf, w.lane, dsb, dq, dtsb, dtq);
             tri_out<HD, DT>(buf + 6 * SE, w.lane, dtsb, dq);
@@ -602,6 +640,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_row_f32x3_
         }
     });
     if (!active) return;
+    met = met || tiles_out_of_range(ds_most) || tiles_out_of_range(dts_most);
     if (__builtin_expect(met, 0)) return bwd_row_f32_wave<HD, HAS_DO, HAS_G, 1, kColumnsCut>(p, w, nullptr);
     tri_store<DT>(p.dq.head(w.b, w.h) + (int64_t)qrow * p.dq.sl, dq, p.scale, p.D, w.g, qvalid);
     if constexpr (HAS_G) tri_store<DT>(p.dtq.head(w.b, w.h) + (int64_t)qrow * p.dtq.sl, dtq, p.scale, p.D, w.g, qvalid);
@@ -717,16 +756,16 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_row_f32x3_pair_kernel(con
     bool met;                  // an element for the fp32 unit (wave-uniform)
     {
         F32x8 x[KC], o[KC];
-        float sq = 0.f;
+        Met m;
         auto fetch = [&](F32x8* to, const F32In& t) {
             own_load<KC>(to, t.head(w.b, w.h) + (int64_t)qrow * t.sl, w.g, p.D, qvalid);
             own_cut<KC>(to, w.g, p.D);
         };
         if (role == 0) {
             fetch(x, p.q);
-            own_split<KC>(own, x, sq);
+            own_split<KC>(own, x, m);
             fetch(x, p.tq);
-            own_split<KC>(town, x, sq);
+            own_split<KC>(town, x, m);
             if (active) {
                 c1 = p.lse[so] * kLog2e;
                 c2 = p.mu[so];
@@ -737,13 +776,13 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_row_f32x3_pair_kernel(con
             if constexpr (HAS_DO) {
                 fetch(x, p.dO);
                 c2 = own_dot<KC>(x, o, c2);
-                own_split<KC>(town, x, sq);
+                own_split<KC>(town, x, m);
             }
             fetch(x, p.dTO);
             c1 = own_dot<KC>(x, o, c1);
             fetch(o, p.to);
             c2 = own_dot<KC>(x, o, c2);
-            own_split<KC>(own, x, sq);
+            own_split<KC>(own, x, m);
             c1 = group_sum(c1);
             c2 = group_sum(c2);
             if (active && w.g == 0) {
@@ -751,13 +790,14 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_row_f32x3_pair_kernel(con
                 p.s7d[so] = c2;
             }
         }
-        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        met = __builtin_amdgcn_ballot_w64(m.special()) != 0;
     }
     f32x4 dq[HT], dtq[HT];
     zero_tiles<HT>(dq);
     zero_tiles<HT>(dtq);
     const int col = 16 * HT * role;
     const float sl2 = p.scale * kLog2e;
+    float ds_most = 0.f, dts_most = 0.f;
 
     tri_walk<HD, NS, NT>(smem_raw, plan, p.Lk, [&](const elem_t* buf, int k0, bool stage_special) {
         met = met || stage_special;
@@ -814,12 +854,11 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_row_f32x3_pair_kernel(con
                     dts[t][j] = kvalid ? dts[t][j] : 0.f;
                 }
         }
-        float sq = 0.f;
-        const Op3 dsb = split_tiles(ds[0], ds[1], sq), dtsb = split_tiles(dts[0], dts[1], sq);
-        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        const Op3 dsb = split_tiles(ds[0], ds[1], ds_most), dtsb = split_tiles(dts[0], dts[1], dts_most);
         tri_out<HD, HT>(buf, w.lane, dsb, dq, dtsb, dtq, col);
         tri_out<HD, HT>(buf + 6 * SE, w.lane, dtsb, dq, col);
     });
+    met = met || tiles_out_of_range(ds_most) || tiles_out_of_range(dts_most);
     if (pair_met<HD, NS>(smem_raw, met, wave, w.lane)) {
         if (active && role == 1) bwd_row_f32_unit<HD, HAS_DO>(p, w, c1, c2);
         return;
@@ -857,11 +896,11 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
     bool met;  // an element for the fp32 unit (wave-uniform)
     {
         F32x8 x[KC];
-        float sq = 0.f;
+        Met m;
         auto fetch = [&](Op3* to, const float* row) {
             own_load<KC>(x, row, w.g, p.D, kvalid);
             own_cut<KC>(x, w.g, p.D);
-            own_split<KC>(to, x, sq);
+            own_split<KC>(to, x, m);
         };
         fetch(k, k_own);
         fetch(v, v_own);
@@ -869,7 +908,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             fetch(tk, tk_own);
             fetch(tv, tv_own);
         }
-        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        met = __builtin_amdgcn_ballot_w64(m.special()) != 0;
     }
     f32x4 dk[DT], dv[DT], dtk[DT], dtv[DT];
     zero_tiles<DT>(dk);
@@ -878,6 +917,7 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
     zero_tiles<DT>(dtv);
     const int64_t so = (int64_t)w.bh * p.Lr + 4 * w.g;  // rows below Lr exist in every statistic
     const float sl2 = p.scale * kLog2e;
+    float ds_most = 0.f, dts_most = 0.f, pr_most = 0.f, pn_most = 0.f;
 
     tri_walk<HD, NS, NT>(smem_raw, plan, p.Lq, [&](const elem_t* buf, int q0, bool stage_special) {
         met = met || stage_special;
@@ -941,11 +981,10 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
                 }
             }
         }
-        float sq = 0.f;
         {
-            const Op3 dsb = split_tiles(ds[0], ds[1], sq);
+            const Op3 dsb = split_tiles(ds[0], ds[1], ds_most);
             Op3 dtsb;
-            if constexpr (HAS_G) dtsb = split_tiles(dts[0], dts[1], sq);
+            if constexpr (HAS_G) dtsb = split_tiles(dts[0], dts[1], dts_most);
             if constexpr (HAS_G) {
                 tri_out<HD, DT, ONTO>(buf, w.lane, dsb, dk, dtsb, dtk);
                 tri_out<HD, DT>(buf + kTq * SE, w.lane, dtsb, dk);
@@ -954,15 +993,15 @@ __global__ __launch_bounds__(64 * NW, HD == 32 ? 2 : NW / 4) void bwd_col_f32x3_
             }
         }
         {
-            const Op3 prb = split_tiles(pr[0], pr[1], sq);
+            const Op3 prb = split_tiles(pr[0], pr[1], pr_most);
             Op3 pnb;
-            if constexpr (HAS_G) pnb = split_tiles(pn[0], pn[1], sq);
+            if constexpr (HAS_G) pnb = split_tiles(pn[0], pn[1], pn_most);
             if constexpr (HAS_G) tri_out<HD, DT, ONTO>(buf + kG * SE, w.lane, pnb, dv, prb, dtv);
             if constexpr (HAS_DO) tri_out<HD, DT>(buf + kDo * SE, w.lane, prb, dv);
         }
-        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
     });
     if (!active) return;
+    met = met || tiles_out_of_range(ds_most) || tiles_out_of_range(pr_most) || tiles_out_of_range(dts_most) || tiles_out_of_range(pn_most);
     if (__builtin_expect(met, 0)) return bwd_col_f32_wave<HD, HAS_DO, HAS_G, 1, kColumnsCut>(p, w, nullptr);
     tri_store<DT>(p.dk.head(w.b, w.h) + (int64_t)krow * p.dk.sl, dk, p.scale, p.D, w.g, kvalid);
     tri_store<DT>(p.dv.head(w.b, w.h) + (int64_t)krow * p.dv.sl, dv, 1.0f, p.D, w.g, kvalid);
@@ -1056,21 +1095,22 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_col_f32x3_pair_kernel(con
     bool met;  // an element for the fp32 unit (wave-uniform)
     {
         F32x8 x[KC];
-        float sq = 0.f;
+        Met m;
         auto fetch = [&](Op3* to, const F32In& t) {
             own_load<KC>(x, t.head(w.b, w.h) + (int64_t)krow * t.sl, w.g, p.D, kvalid);
             own_cut<KC>(x, w.g, p.D);
-            own_split<KC>(to, x, sq);
+            own_split<KC>(to, x, m);
         };
         fetch(own, role ? p.v : p.k);
         fetch(town, role ? p.tv : p.tk);
-        met = __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        met = __builtin_amdgcn_ballot_w64(m.special()) != 0;
     }
     f32x4 acc[DT], tacc[DT];
     zero_tiles<DT>(acc);
     zero_tiles<DT>(tacc);
     const int64_t so = (int64_t)w.bh * p.Lr + 4 * w.g;  // rows below Lr exist in every statistic
     const float sl2 = p.scale * kLog2e;
+    float t1_most = 0.f, t2_most = 0.f;
 
     tri_walk<HD, NS, NT>(smem_raw, plan, p.Lq, [&](const elem_t* buf, int q0, bool stage_special) {
         met = met || stage_special;
@@ -1132,12 +1172,11 @@ __global__ __launch_bounds__(128 * kPairs, 2) void bwd_col_f32x3_pair_kernel(con
                     t2[t][j] = valid ? ds : 0.f;
                 }
         }
-        float sq = 0.f;
-        const Op3 b1 = split_tiles(t1[0], t1[1], sq), b2 = split_tiles(t2[0], t2[1], sq);
-        met = met || __builtin_amdgcn_ballot_w64(!(sq < kMost)) != 0;
+        const Op3 b1 = split_tiles(t1[0], t1[1], t1_most), b2 = split_tiles(t2[0], t2[1], t2_most);
         tri_out<HD, DT>(y1, w.lane, b2, acc, b1, tacc);
         if (has_y2) tri_out<HD, DT>(y2, w.lane, b1, acc);
     });
+    met = met || tiles_out_of_range(t1_most) || tiles_out_of_range(t2_most);
     const bool unit = pair_met<HD, NS>(smem_raw, met, wave, w.lane);
     if (!active) return;
     if (unit) return bwd_col_f32_half<HD, HAS_DO>(p, w, role);
