@@ -83,6 +83,37 @@ def test_one_set_for_a_forward_with_tangents_and_a_cotangent_on_o(B, H, Lq, Lk, 
         assert err <= 1.02 * unit_err, (n, err, unit_err)
 
 
+@pytest.mark.parametrize("mode", ["both", "dTO", "plain"])
+@pytest.mark.parametrize("B,H,Lq,Lk,D", [(30, 12, 100, 120, 64), (24, 8, 160, 600, 64), (24, 12, 520, 70, 64), (40, 12, 75, 90, 48),
+                                        (30, 12, 100, 120, 16), (12, 16, 200, 500, 80), (32, 4, 300, 520, 128)])
+def test_error_is_not_above_the_units(mode, B, H, Lq, Lk, D):
+    """Every output against fp64, beside the same heads in calls that the fp32 unit serves (split groups: its smallest error)."""
+    from semicat_amd import kernels as K
+    x = orc.make_inputs(B, H, Lq, Lk, D, seed=11, tangent_scale=0.5, dtype=torch.float32)
+    cot = {n: x[n] for n in ("dO", "dTO") if n in {"both": ("dO", "dTO"), "dTO": ("dTO",), "plain": ("dO",)}[mode]}
+    ref = orc.attention_jvp_autograd(*[x[n] for n in orc.TENSOR_ORDER[:6]], **cot)
+    d = {n: t.cuda() for n, t in x.items()}
+
+    def step(y):
+        if mode != "plain":
+            return _step(y, mode)
+        o, lse = K.attention_forward(y["q"], y["k"], y["v"])
+        g = K.attention_jvp_backward(y["q"], y["k"], y["v"], None, None, None, o, None, lse, None, dO=y["dO"])
+        return {"o": o, **dict(zip(("dq", "dk", "dv"), g))}
+
+    print(f"[f32 error] {(B, H, Lq, Lk, D)} {mode}", flush=True)
+    res, names = _kernels(lambda: step(d))
+    assert len(names) == 3 and all("f32x3" in n for n in names), names
+    unit, names = _kernels(lambda: [step({n: t[b:b + 1] for n, t in d.items()}) for b in range(B)])
+    assert not any("f32x3" in n for n in names), names
+    for n in ("o", "to", "dq", "dk", "dv", "dtq", "dtk", "dtv"):
+        if res.get(n) is not None:
+            r = ref[n.upper() if n in ("o", "to") else n]
+            err, unit_err = (orc.rel_frobenius(t.cpu(), r) for t in (res[n], torch.cat([u[n] for u in unit])))
+            print(f"  {n} {err:.3e} {unit_err:.3e}")
+            assert err <= 1.02 * unit_err, (n, err, unit_err)
+
+
 def _at(name, row, value, column=0):
     def put(x, b):
         x[name][b, 0, row, column] = value
