@@ -110,3 +110,38 @@ def test_rotation_through_the_host_extension(monkeypatch, n, D, half, dtype, out
     monkeypatch.setattr(kernels, "_on_gpu", lambda q: False)
     for a, b in zip(res, kernels.rotary_embedding(xs, *tables, out_dtype=out_dtype, inverse=inverse), strict=True):
         assert torch.equal(a, b) and a.stride() == b.stride() and a.dtype == b.dtype
+
+
+@pytest.mark.parametrize("how", ["a dispatch mode", "deterministic fill"])
+def test_results_that_have_to_be_seen_or_filled_are_made_by_the_dispatcher(how):
+    """Their values and strides are those of results that come straight from the allocator."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x = _inputs(2, 3, 33, 77, 64, torch.bfloat16, True)
+    x[1] = x[1].transpose(1, 2).contiguous().transpose(1, 2)[:, :1].expand(-1, 3, -1, -1)  # no dense strides to keep
+    cos, sin = torch.randn(2, 40, 32, device="cuda")
+
+    def run():
+        return (*_step(x, True, True), *kernels.rotary_embedding((x[0].transpose(1, 2),), cos, sin))
+
+    made = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            made.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    ref = run()
+    if how == "a dispatch mode":
+        with Watch():
+            res = run()
+        # o, to, lse, mu, six gradients, workspace, plain o and lse, one rotated tensor
+        assert sum("empty" in n for n in made) == 14, made
+    else:
+        torch.use_deterministic_algorithms(True)
+        try:
+            assert torch.utils.deterministic.fill_uninitialized_memory
+            res = run()
+        finally:
+            torch.use_deterministic_algorithms(False)
+    for a, b in zip(res, ref, strict=True):
+        assert (a is None and b is None) or (a.stride() == b.stride() and torch.equal(a, b))

@@ -218,3 +218,37 @@ def test_network_block_issues_no_rotary_launch_at_sequence_128():
     names = [e.key for e in prof.key_averages() if e.device_type == torch.autograd.DeviceType.CUDA]
     assert any("fwd16_kernel" in n for n in names) and any("bwd_fused" in n for n in names), names
     assert not any("rope_kernel" in n for n in names), [n for n in names if "rope" in n]
+
+
+@pytest.mark.parametrize("cot", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,H,D", [(2, 256, 4, 64), (2, 150, 3, 128), (1, 40, 2, 48)])
+def test_rotation_in_front_of_the_op_under_jvp(B, S, H, D, dtype, cot):
+    """Shapes that the folded rotation does not serve, q, k and v as slices of a fused projection: one node below the transform, against the
+    rotary function followed by the op."""
+    from semicat_amd import functional
+    from semicat_amd.rotary import apply_rotary
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    qkv, tqkv = ((torch.randn((B, S, 3, H, D), device="cuda", generator=gen) * s).to(dtype).requires_grad_() for s in (1.0, 0.1))
+    cos, sin = tables(S, D)
+    g = [torch.randn((B, S, H, D), device="cuda", generator=gen).to(dtype) for _ in range(2)]
+
+    def whole(x):
+        return functional.safe_sdpa_jvp_rotary(x[:, :, 0], x[:, :, 1], x[:, :, 2], cos, sin)
+
+    def apart(x):
+        return functional.safe_sdpa_jvp(*apply_rotary((x[:, :, 0], x[:, :, 1]), cos, sin), x[:, :, 2])
+
+    applied = []
+
+    def run(f):
+        ys = torch.func.jvp(f, (qkv,), (tqkv,))
+        applied.append(type(torch.func.jvp(f, (qkv,), (tqkv,))[1].grad_fn).__name__)
+        outs = [y for y, c in zip(ys, cot) if c]
+        return (*ys, *torch.autograd.grad(outs, (qkv, tqkv), [t for t, c in zip(g, cot) if c], allow_unused=True))
+
+    for a, b in zip(run(whole), run(apart), strict=True):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.dtype == b.dtype and torch.equal(a, b)
+    assert applied[0].startswith("SDPASeqMajorFunction"), applied
