@@ -18,8 +18,10 @@
  *     flash_jvp_backward.py:2321-2322).  q, tq, o, to, dO, dTO, dq, dtq have L = Lq; the k/v side has
  *     L = Lk.  Any [B,S,H,D] caller layout is expressed through the strides.
  *   - dtype: SJVP_BF16 or SJVP_FP16 for every tensor (MFMA kernels; accumulation and softmax are
- *     fp32), or SJVP_FP32: the correctness mode, fp32 tensors and fp32 arithmetic throughout
- *     (the reference's fp32 math path, ryu_triton.py:426-454; fp32 matrix instructions), or
+ *     fp32), or SJVP_FP32: the correctness mode, fp32 tensors and products, sums and exponentials of fp32
+ *     accuracy (the reference's fp32 math path, ryu_triton.py:426-454; small problems on the fp32 matrix
+ *     instructions, larger ones on the bf16 ones with every operand in three parts, numbers that these
+ *     do not hold on the fp32 ones: 2^59 and above, below 2^-100, infinities, NaN), or
  *     SJVP_FP32_BF16: fp32 tensors whose elements are rounded to bf16 as they are loaded, bf16 MFMA
  *     arithmetic, results stored as fp32, i.e. the casts that functional.py:318-322,330-331 put
  *     around the op for fp32 callers, folded into it (sjvp_fwd, sjvp_bwd*; not sjvp_rope).  Strides

@@ -39,8 +39,8 @@ HIPCC_FLAGS = [
 # to 20 % on staged ones, so they keep the default.
 _ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 UNIT_FLAGS = {name: _ILP for name in ("sjvp_tu_pair16.hip", "sjvp_tu_pair_staged16.hip", "sjvp_f32io_pair.hip")}
-# The waves of these kernels that have 512 registers keep their accumulators among the vector registers: 156 -> 51 spilled in the
-# column-owned kernel at D = 128, 39 -> 0 in the row-owned one.
+# Accumulators among the vector registers.  Forward + backward without tangents, without / with it: B=4 H=16 L=2048 D=64 1756 / 1650 us, B=8
+# H=12 L=500 D=96 448 / 435, twelve shapes 1.035; with tangents 1.004.  The same registers are spilled either way.
 UNIT_FLAGS["sjvp_f32x3.hip"] = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 

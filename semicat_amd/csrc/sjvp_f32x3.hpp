@@ -15,20 +15,23 @@
 // for the score-like tiles, transposing reads for the output ones); the owned side is split once, and each tile
 // once, before the output contractions that it enters.
 //
-// Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4497 / 2198 us (the matrix pipe busy
-// 52, 60 and 55 % of the forward's, row and column kernel's cycles), without tangents at B=8 H=8 L=512 336 / 167, B=64 H=12 L=128
-// D=64 520 / 319, B=8 H=12 L=500 D=32 570 / 259, B=8 H=16 L=512 D=128 2154 / 1475, B=8 H=12 L=500
-// D=96 1936 / 913, B=4 H=16 300 queries on 700 keys D=80 1059 / 724.  What is left between the contractions is the split of the
+// Measured, forward + backward, the fp32 unit's kernels / these: B=8 H=16 L=1024 D=64 4492 / 2177 us (the matrix pipe busy
+// 48, 54 and 52 % of the forward's, row and column kernel's cycles), without tangents 1895 / 853, B=64 H=12 L=128
+// D=64 512 / 308, B=8 H=12 L=500 D=32 567 / 257, B=8 H=16 L=512 D=128 2137 / 1466, B=8 H=12 L=500
+// D=96 1904 / 886, B=4 H=16 300 queries on 700 keys D=80 1039 / 702.  What is left between the contractions is the split of the
 // stage and of the tiles, softmax and barriers.
-// Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 5.4e-7.
+// Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 4.7e-7; over 45 shapes every output's is 0.45 to 1.00 of the unit's.
+// (A float as a sum of bfloat16 values, and which of the products matter: G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", ARITH 2019.)
 //
 // Numbers that the split does not hold (infinities, NaN) or whose products could overflow one by one where their sum does
 // not (2^59 and above) are left to the fp32 unit: a wave that met one, in its own rows, in a stage or in its tiles, computes its
 // 16 rows again as the kernels of sjvp_f32.hpp do, behind its loop (inside it the second form costs the first one 60
 // registers).  So infinite and overflowing scores come out as they do there.
-// So are small numbers: where eight neighbours in a row, or an owned row's tiles of the whole streamed axis, are not all zero and all below
-// 2^-100.  (Beside larger ones what a number loses, at most 2^-134, is nothing.)  Gradients of cotangents at 2^-118 had errors up to 8.5e-5, and have
-// the unit's 4.9e-7 there.
+// So are small numbers, where eight neighbours in a row, or an owned row's tiles of the whole streamed axis, are not all zero and all below
+// 2^-100.  (Beside larger ones what a number loses, at most 2^-134, is nothing.)  Gradients of cotangents at 2^-118 have errors up to 5.3e-7 there, in
+// three parts 8.5e-5 (the unit alone 4.4e-7: the scores meet the log-sum-exp of the other form's).
+// Such waves pay for both forms: where all of a call's are, it takes 1.4 to 1.6 times as long as on the unit alone at D = 64, 2.6 to 3 times at D = 128.
 #pragma once
 #include "sjvp_f32.hpp"
 #include "sjvp_staged16.hpp"
@@ -50,8 +53,8 @@ __device__ __forceinline__ void mfma6(const Op3& a0, const Op3& b0, f32x4& c0, c
 }
 
 // The same into accumulators that live through the loop: the five small products are summed beside them, which leaves two
-// roundings at the accumulator's size per 32 products in the place of six.  (Six, in the column kernel of eight waves: 64 heads, 2000 queries on
-// 70 keys, D = 64 dtK, dtV 7.6e-7 against fp64, so 5.4e-7, the fp32 unit's split groups 5.5e-7; forward + backward 1.3 % shorter.)
+// roundings at the accumulator's size per 32 products in the place of six.  (Six, in the column kernel of eight waves: 288 heads, 2000 queries on
+// 70 keys, D = 64, dtK, dtV 7.6e-7 against fp64, so 4.5e-7, the fp32 unit's split groups 5.5e-7; forward + backward 1.3 % shorter.)
 __device__ __forceinline__ void mfma6_onto(const Op3& a0, const Op3& b0, f32x4& c0, const Op3& a1, const Op3& b1, f32x4& c1) {
     constexpr int pa[5] = {2, 1, 0, 1, 0}, pb[5] = {0, 1, 2, 0, 1};
     f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = t0;

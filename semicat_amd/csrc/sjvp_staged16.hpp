@@ -9,7 +9,7 @@
 // shifted, so no load leaves a row, and columns >= D arrive as zeros.
 //
 // Measured, forward + backward (one element at a time through one stage of LDS under 32-wide tiles before):
-//   bf16 B=8 H=8 L=300 D=36 158 -> 62 us (the aligned D = 40: 54), B=64 H=12 L=128 D=20 174 -> 58,
+//   bf16 B=8 H=8 L=300 D=36 158 -> 54 us (as the aligned D = 40), B=64 H=12 L=128 D=20 174 -> 57,
 //   B=8 H=16 L=512 D=100 1579 -> 325; fp32 rows B=64 H=12 L=128 D=64 248 -> 139 us, B=128 H=12 L=256 1637 -> 745.
 // The shorter life of a stage in registers (one ahead instead of a ring of two or three) costs 15 % against the
 // LDS-DMA form; what is left is bound as that one is.

@@ -21,7 +21,7 @@ import torch
 from . import _lib
 
 # bf16 / fp16: the MFMA kernels (fp32 accumulation).  float32: the fp32 correctness mode of the library
-# (fp32 tensors and arithmetic throughout; about 1e-6 against fp64).
+# (fp32 tensors, contractions of fp32 accuracy; about 1e-6 against fp64).
 _DTYPES = {torch.bfloat16: _lib.SJVP_BF16, torch.float16: _lib.SJVP_FP16, torch.float32: _lib.SJVP_FP32}
 
 

@@ -7,7 +7,7 @@ cotangents ~ N(0,1)), for the shapes the headline benchmark does not cover: long
 head dimensions, keys and queries of different lengths.  Work model 42*B*H*Lq*Lk*D flop per step.
 Prints one JSON line.  A companion measurement, not the headline figure.
 
-``--dtype fp32`` times the library's fp32 correctness mode (fp32 arithmetic throughout);
+``--dtype fp32`` times the library's fp32 correctness mode (contractions of fp32 accuracy);
 ``--dtype fp32io`` and ``fp32cast`` time the two ways of serving a float32 caller with bf16 arithmetic
 (the dtype policy of semicat/jvp_utils/functional.py:318-332): the casts folded into the kernels
 (float32 tensors handed over as they are, SJVP_FP32_BF16), or torch casts around the 16-bit kernels
@@ -140,7 +140,7 @@ def main(argv=None) -> int:
     unit = float(B) * H * Lq * Lk * D
     print(json.dumps({
         "workload": f"attention JVP fwd+bwd, B={B} H={H} Lq={Lq} Lk={Lk} D={D}, "
-                    + {"fp32": "fp32 tensors and fp32 arithmetic throughout (the correctness mode)",
+                    + {"fp32": "fp32 tensors, contractions of fp32 accuracy (the correctness mode)",
                        "fp32io": "fp32 tensors, casts folded into the kernels, bf16 arithmetic",
                        "fp32lib": "fp32 tensors, the library's cast launches around the bf16 kernels",
                        "fp32cast": "fp32 tensors, torch casts around the bf16 kernels"}.get(
