@@ -36,13 +36,13 @@ inline int split(int BH, int rows, int streamed) {
 // Both sides in us, fp32 unit / here, L = 256: D = 64 512 groups 26 / 27 forward, 37 / 34 row, 40 / 44 column; 640 31 / 26, 54 / 33, 59 / 41; 4096 142 / 78, 201 / 105, 250 / 139; D = 80 384 42 / 50, 61 / 53, 74 / 56,
 // 640 62 / 50, 90 / 53, 113 / 57; D = 128 384 43 / 51, 70 / 61, 73 / 70 (L = 1024: 125 / 187, 202 / 206, 218 / 239), 576 64 / 53, 104 / 62,
 // 108 / 72; D = 32 without tangents, forward, 640 9.0 / 11.2, 2048 17 / 13.
-inline int x3_width(int BH, int rows, int D, bool forward, bool tangents) {
+inline int x3_width(int BH, int rows, int D, bool forward, bool tangents, int units = compute_units()) {
     const int64_t four = (int64_t)BH * ((rows + 63) / 64);
-    return D > 64 || four <= compute_units() || (!forward && (D <= 32 || !tangents)) ? 4 : 8;
+    return D > 64 || four <= units || (!forward && (D <= 32 || !tangents)) ? 4 : 8;
 }
 // What a launch saves there, in tenths of fortieths.
-inline int64_t x3_saves(int BH, int groups_of, int rows, int streamed, int D, bool forward, bool tangents) {
-    const int units = compute_units(), waves = x3_width(BH, rows, D, forward, tangents);
+inline int64_t x3_saves(int BH, int groups_of, int rows, int streamed, int D, bool forward, bool tangents, int units) {
+    const int waves = x3_width(BH, rows, D, forward, tangents, units);
     // tenths; workgroups of four that share a compute unit (48 KB of LDS, or less) add 0.7 of a round each
     int64_t rounds = ((int64_t)BH * ((rows + 16 * waves - 1) / (16 * waves)) + units - 1) / units;
     rounds = waves == 4 && (D <= 32 || (D <= 64 && !tangents)) ? 7 * rounds + 3 : 10 * rounds;
@@ -53,21 +53,23 @@ inline int64_t x3_saves(int BH, int groups_of, int rows, int streamed, int D, bo
     const int64_t tiles = (streamed + kF32Rows - 1) / kF32Rows, stages = (streamed + kStageRows - 1) / kStageRows;
     return 10 * tiles * unit - 2 * stages * rounds * per_tile;
 }
-// By the launches of a call with tangents.  Plain calls (the forward without, or a cotangent on O alone) go with them, and what their
-// costs, which are on the high side, say against it counts only where a launch leaves more than half of the compute units without a
-// workgroup.  Forward + backward with and without tangents, fp32 unit / here, us, at shapes where the two kinds' costs disagree:
-//   stays on the unit: 78 heads, 52 queries on 3516 keys, D = 20 505 / 564 and 204 / 313; 24 heads, 250 on 2586, D = 16 349 / 350 and 142 / 193;
-//   goes here: 60 heads, 259 x 259, D = 48 321 / 153 and 125 / 82; 120 heads, 803 x 803, D = 128 5470 / 3742 and 2428 / 1596; the worst
-//   of 80 such shapes 186 heads, 44 on 1663, D = 100 1539 / 1694 and 618 / 739; with half of the units idle at D > 64, 104 heads, 59 on 424,
-//   D = 100 295 / 293 and 122 / 136, 35 heads, 280 on 154, D = 80 220 / 140 and 89 / 74.
-// (Where the plain launches alone would gain: 144 heads, 144 x 144, D = 64 plain 80 / 60; with tangents 221 on the unit.)
+// Where the launches of plain calls (the forward without tangents, or a cotangent on O alone) gain, or those of a call with tangents, whose costs
+// are nearer to what is measured: at D <= 64 only if no launch of theirs leaves more than half of the compute units without a workgroup.
+// Forward + backward with and without tangents, fp32 unit / here, us, at shapes where the two kinds' costs disagree:
+//   plain launches gain, 46 shapes: with tangents 0.81 on average (0.56 to 1.19), plain 0.78: 332 heads, 144 x 144, D = 48 397 / 281 and
+//   145 / 100; the worst, 300 heads, 3170 queries on 24 keys, D = 64 1592 / 1903 and 691 / 605;
+//   launches with tangents gain, 80 shapes: 60 heads, 259 x 259, D = 48 321 / 153 and 125 / 82; 120 heads, 803 x 803, D = 128 5470 / 3742 and
+//   2428 / 1596; the worst, 186 heads, 44 on 1663, D = 100 1539 / 1694 and 618 / 739; with half of the units idle at D > 64, 104 heads, 59 on
+//   424, D = 100 295 / 293 and 122 / 136, 35 heads, 280 on 154, D = 80 220 / 140 and 89 / 74; stays on the unit: 78 heads, 52 on 3516,
+//   D = 20 505 / 564 and 204 / 313; 24 heads, 250 on 2586, D = 16 349 / 350 and 142 / 193.
 inline bool x3_takes(int BH, int Lq, int Lr, int Lk, int D) {
+    const int units = compute_units();  // asks the runtime for the device: once
     auto gains = [&](bool tangents) {  // by the contractions of forward, row and column launch: 6, 9 and 12, without tangents 2, 3 and 4
-        return 2 * x3_saves(BH, Lq, Lr, Lk, D, true, tangents) + 3 * x3_saves(BH, Lq, Lq, Lk, D, false, tangents) +
-                   4 * x3_saves(BH, Lk, Lk, Lq, D, false, tangents) > 0;
+        return 2 * x3_saves(BH, Lq, Lr, Lk, D, true, tangents, units) + 3 * x3_saves(BH, Lq, Lq, Lk, D, false, tangents, units) +
+                   4 * x3_saves(BH, Lk, Lk, Lq, D, false, tangents, units) > 0;
     };
     const int64_t fewest = (int64_t)BH * (((Lq < Lk ? Lq : Lk) + 63) / 64);
-    return gains(true) && (D > 64 || 2 * fewest >= compute_units() || gains(false));
+    return gains(false) || (gains(true) && (D > 64 || 2 * fewest >= units));
 }
 inline int blocks(int rows, int split) {
     const int per = split > 1 ? kF32Rows : kF32Rows * kF32Waves;

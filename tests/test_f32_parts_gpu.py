@@ -63,7 +63,8 @@ def test_parts_at_the_edges(mode, B, H, Lq, Lk, D, offset):
 
 
 @pytest.mark.parametrize("B,H,Lq,Lk,D,parts", [(16, 16, 200, 32, 100, True), (83, 3, 172, 172, 128, True), (15, 8, 76, 76, 80, True),
-                                              (30, 12, 100, 120, 64, True), (12, 16, 200, 500, 80, True), (13, 6, 52, 700, 20, False)])
+                                              (30, 12, 100, 120, 64, True), (12, 16, 200, 500, 80, True), (13, 6, 52, 700, 20, False),
+                                              (36, 4, 144, 144, 64, True)])
 def test_one_set_for_a_forward_with_tangents_and_a_cotangent_on_o(B, H, Lq, Lk, D, parts):
     """The backward knows no tangents there.  Mixed with the other set's forward its error is 1.1 to 1.2 times the fp32 unit's."""
     x = orc.make_inputs(B, H, Lq, Lk, D, seed=7, tangent_scale=0.1, dtype=torch.float32)
