@@ -20,7 +20,7 @@
 // D=64 512 / 308, B=8 H=12 L=500 D=32 567 / 257, B=8 H=16 L=512 D=128 2137 / 1466, B=8 H=12 L=500
 // D=96 1904 / 886, B=4 H=16 300 queries on 700 keys D=80 1039 / 702.  What is left between the contractions is the split of the
 // stage and of the tiles, softmax and barriers.
-// Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 4.7e-7; over 45 shapes every output's is 0.45 to 1.00 of the unit's.
+// Error against fp64 at B=16 H=8 L=512 D=64, worst output: 7.4e-7 / 4.7e-7; over 120 shapes every output's is 0.42 to 1.00 of the unit's.
 // (A float as a sum of bfloat16 values, and which of the products matter: G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 artificial
 // intelligence datatype for higher-precision computations", ARITH 2019.)
 //
